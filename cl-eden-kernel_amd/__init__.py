@@ -92,6 +92,8 @@ EXPORTS = {
     "eh_device_name": (C.c_int, [C.c_char_p, C.c_size_t]),
     "eh_malloc": (C.c_int, [C.POINTER(C.c_void_p), C.c_size_t]),
     "eh_free": (C.c_int, [C.c_void_p]),
+    "eh_host_alloc": (C.c_int, [C.POINTER(C.c_void_p), C.c_size_t]),
+    "eh_host_free": (C.c_int, [C.c_void_p]),
     "eh_memset": (C.c_int, [C.c_void_p, C.c_int, C.c_size_t, C.c_void_p]),
     "eh_h2d": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]),
     "eh_d2h": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]),

@@ -894,6 +894,18 @@ int eh_free(void *ptr) {
     return EH_OK;
 }
 
+int eh_host_alloc(void **ptr, size_t bytes) {
+    EH_REQUIRE(ptr != nullptr, "null result pointer");
+    *ptr = nullptr;
+    EH_HIP(hipHostMalloc(ptr, bytes ? bytes : 1, hipHostMallocDefault));
+    return EH_OK;
+}
+
+int eh_host_free(void *ptr) {
+    if (ptr) EH_HIP(hipHostFree(ptr));
+    return EH_OK;
+}
+
 int eh_memset(void *ptr, int value, size_t bytes, void *stream) {
     if (bytes) EH_HIP(hipMemsetAsync(ptr, value, bytes, as_stream(stream)));
     return EH_OK;

@@ -181,6 +181,8 @@ int eh_init(int device);
 int eh_device_name(char *dst, size_t cap);
 int eh_malloc(void **ptr, size_t bytes);             /* zero-initialised, 256-byte aligned */
 int eh_free(void *ptr);
+int eh_host_alloc(void **ptr, size_t bytes);         /* pinned host memory, for transfers that need not wait */
+int eh_host_free(void *ptr);
 int eh_memset(void *ptr, int value, size_t bytes, void *stream);
 int eh_h2d(void *dst, const void *src, size_t bytes, void *stream);
 int eh_d2h(void *dst, const void *src, size_t bytes, void *stream);

@@ -364,3 +364,23 @@ def test_segmentation_head_with_21_classes_through_the_userdriver():
         finally:
             d.set_store_channels_last(True)
             d.set_image_lanes(2, 12)
+
+
+@pytest.mark.parametrize("count", [1, 257, (1 << 20) - 1, 1 << 20, (1 << 20) + 1], ids=lambda c: "%d_bytes" % c)
+def test_host_transfers_around_the_staging_size(count):
+    """Inputs and outputs through the pinned staging area (up to 1 MiB) and past it, several executions in a row so that
+    the area fills and is reused: c = a + b with equal scales."""
+    d, list_id = driver(), 0x7800
+    ol = ud.OperatorList(list_id, ud.MODEL_ANDROID_NN)
+    ta, tb, tc = (ol.feature_map(i, (1, 1, 1, count), 0.5, 0) for i in range(3))
+    ol.operator("ADD", ud.OP_ADD, [ta, tb], [tc])
+    d.open_subgraph(ol)
+    try:
+        rng = np.random.default_rng(count)
+        for rep in range(4):
+            a, b = (rng.integers(0, 140, count, dtype=np.uint8) for _ in range(2))
+            got = np.zeros(count, np.uint8)
+            d.execute_subgraph(list_id, {0: a, 1: b, 2: got})
+            assert np.array_equal(got, np.minimum(a.astype(int) + b, 255).astype(np.uint8)), rep
+    finally:
+        d.close_subgraph(list_id)
