@@ -420,9 +420,12 @@ class _Plan:
     def __init__(self):
         self.handle = C.c_void_p()
         self._keep = []
+        self._run = getattr(load(), "eh_%s_u8_run" % self._kind)   # looked up once: a call's own cost counts on small layers
 
     def run(self, d_in, d_out, q, stream=None):
-        check(getattr(load(), "eh_%s_u8_run" % self._kind)(self.handle, d_in.ptr, d_out.ptr, C.byref(q), stream))
+        rc = self._run(self.handle, d_in.ptr, d_out.ptr, q, stream)
+        if rc:
+            check(rc)
 
     def repack(self, d_w, d_b, q, stream=None):
         check(getattr(load(), "eh_%s_u8_repack" % self._kind)(self.handle, d_w.ptr, d_b.ptr if d_b else None,

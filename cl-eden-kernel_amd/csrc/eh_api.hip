@@ -237,6 +237,8 @@ int finish_part(GemmPart &g, std::vector<KUnit> &units, const std::vector<int32_
         // 3x3 taps at dilation 1 and stride 1 over all input channels: the patch-in-LDS kernel
         g.cfg.id = GEMM_CONV3X3;
         g.cfg.slab = 32;
+        g.proto.n = g.n;
+        conv3x3_patch_shape(&g.proto);
     } else if (g.vec == 16 && (ktab_fits || (plain_matrix && g.k % 256 == 0)))
         // (a reduction too long for its k-table to fit LDS still runs as a plain matrix of whole slabs: a fully
         // connected layer on 25088 inputs)
@@ -685,6 +687,9 @@ struct eh_dwconv_plan {
     int32_t cout_caller = 0;        // `cout` counts the padded channels; this is what the caller's tensors hold
     bool planar = false;            // the caller's tensors are NCHW
     uint8_t *stage_in = nullptr, *stage_out = nullptr;
+    // geometry of the latest fused launch behind a pointwise layer, and what it was chosen for
+    BlockGeom block{};
+    int32_t block_ks = 0, block_rows = 0, block_cols = 0;
 };
 
 extern "C" {
@@ -1971,7 +1976,16 @@ int eh_conv_dw_block_run(eh_conv_plan *pointwise, eh_dwconv_plan *depthwise, con
     if ((rc = dw_refold(depthwise, *q_depthwise, s))) return rc;
     const GemmProblem pw = pointwise->op.problem(pointwise->op.parts[0], static_cast<const uint8_t *>(input), nullptr, nullptr, nullptr);
     const DwProblem dw = dw_problem(depthwise, nullptr, output);
-    return launch_pwdw_block(pw, dw, rows_per_tile, cols_per_tile, s);
+    const int32_t ks = pw.k_pad / 32;
+    if (depthwise->block_ks != ks || depthwise->block_rows != rows_per_tile || depthwise->block_cols != cols_per_tile) {
+        depthwise->block_ks = 0;
+        EH_REQUIRE(pwdw_block_geometry(pw, dw, rows_per_tile, cols_per_tile, &depthwise->block), "block: no tile of the requested shape (%d x %d outputs) fits",
+                   rows_per_tile, cols_per_tile);
+        depthwise->block_ks = ks;
+        depthwise->block_rows = rows_per_tile;
+        depthwise->block_cols = cols_per_tile;
+    }
+    return launch_pwdw_block(pw, dw, depthwise->block, s);
 }
 
 }  // extern "C"

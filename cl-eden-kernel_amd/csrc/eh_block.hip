@@ -35,25 +35,6 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 namespace {
 
-struct BlockGeom {
-    int32_t th, tw;      // output rows and columns per workgroup
-    int32_t tiles_y, tiles_w;  // workgroups per image, down and across
-    int32_t ih, iwp;     // rows and columns of the expanded image a workgroup holds
-    int32_t pixels;      // ih * iwp
-    int32_t c;           // expanded channels of the layer
-    int32_t nb;          // channel blocks of 32 per workgroup (grid y walks the ranges); bytes per pixel of the LDS image = 32 nb
-    int32_t ks;          // reduction steps of 32 bytes of the pointwise stage
-    int32_t cpitch;      // bytes per pixel of the LDS image
-    int32_t tiles_x;     // depthwise tiles of four output columns per row of the workgroup's tile
-    int32_t units_per_cq;  // th * tiles_x: depthwise thread-units per channel quad
-    int32_t total_tiles; // n * tiles_y * tiles_w
-    int32_t a_pitch;     // LDS bytes per input pixel: 32 ks + 16 (the slack spreads the fragment reads over the banks)
-    FastDiv div_iwp, div_tx, div_tiles_y, div_tiles_w, div_ppp;
-    FastDiv div_cq, div_cq_last;  // by the channel quads of a full range, and of the last one
-    uint32_t a_off;      // byte offset of the staged input pixels
-    uint32_t image_off;  // byte offset of the LDS image behind the staged weights, bias and input pixels
-};
-
 __device__ __forceinline__ int udot4(uint32_t a, uint32_t b, int acc) { return (int)__builtin_amdgcn_udot4(a, b, (uint32_t)acc, false); }
 
 // the four channels of a column's three rows as four words of three bytes each (byte 3 zero)
@@ -391,13 +372,7 @@ bool pwdw_block_preferred(const GemmProblem &pw, const DwProblem &dw) {
     return pwdw_block_applies(pw, dw) && pwdw_block_listed(dw.n, dw.h, dw.w_, pw.k, dw.c, dw.stride_h);
 }
 
-// rows_per_tile / cols_per_tile: the tile a workgroup owns, 0 = chosen here
-int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, int rows_per_tile, int cols_per_tile, hipStream_t stream) {
-    EH_REQUIRE(pwdw_block_applies(pw, caller_dw), "block: the two operators do not fit the fused kernel");
-    EH_REQUIRE((reinterpret_cast<uintptr_t>(pw.a) & 7) == 0 && (reinterpret_cast<uintptr_t>(caller_dw.out) & 3) == 0, "block: unaligned tensors");
-    DwProblem dw = caller_dw;
-    if (dw.w_trip) dw.w_fold = nullptr;                 // the signed form where it applies, as the stand-alone launcher decides
-    if (dw.w_fold) dw.zp_w += dw.w_signed ? 128 : 0;    // zero point of the uint8 values the unsigned form multiplies
+bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, int cols_per_tile, BlockGeom *geom) {
     const int S = dw.stride_h;
     BlockGeom g;
     g.c = dw.c;
@@ -441,13 +416,13 @@ int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, int row
                         }
                     }
             }
-        EH_REQUIRE(best >= 0, "block: no tile of the requested shape fits LDS");
+        if (best < 0) return false;
         th = best_th;
         tw = best_tw;
         nb = best_nb;
     }
     g.nb = nb;
-    EH_REQUIRE(th >= 1 && th <= dw.ho && tw >= 1 && tw <= dw.wo, "block: tile of %d x %d outputs", th, tw);
+    if (!(th >= 1 && th <= dw.ho && tw >= 1 && tw <= dw.wo)) return false;
     g.th = th;
     g.tw = tw;
     g.ih = (th - 1) * S + 3;
@@ -468,9 +443,23 @@ int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, int row
     g.div_cq_last = make_fastdiv((uint32_t)((g.c - (ranges - 1) * g.nb * 32) / 4));
     g.cpitch = block_image_pitch(g.nb, g.c);
     const size_t lds = block_lds_bytes(g.nb, g.ks, g.ih, g.iwp, g.c, &g.a_off, &g.image_off);
-    EH_REQUIRE(lds <= kBlockLdsMax, "block: %zu bytes of LDS", lds);
+    if (lds > kBlockLdsMax) return false;
+    *geom = g;
+    return true;
+}
+
+// `g`: what pwdw_block_geometry gave for the pair (the search over tiles costs the host as much as the launch: callers keep it)
+int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, const BlockGeom &g, hipStream_t stream) {
+    EH_REQUIRE(pwdw_block_applies(pw, caller_dw), "block: the two operators do not fit the fused kernel");
+    EH_REQUIRE((reinterpret_cast<uintptr_t>(pw.a) & 7) == 0 && (reinterpret_cast<uintptr_t>(caller_dw.out) & 3) == 0, "block: unaligned tensors");
+    EH_REQUIRE(g.c == caller_dw.c && g.ks == pw.k_pad / 32, "block: geometry of another pair");
+    DwProblem dw = caller_dw;
+    if (dw.w_trip) dw.w_fold = nullptr;                 // the signed form where it applies, as the stand-alone launcher decides
+    if (dw.w_fold) dw.zp_w += dw.w_signed ? 128 : 0;    // zero point of the uint8 values the unsigned form multiplies
+    const int S = dw.stride_h;
+    const size_t lds = (size_t)g.image_off + (size_t)g.ih * g.iwp * g.cpitch;
     if (g.total_tiles <= 0) return EH_OK;
-    const dim3 grid((unsigned)((g.total_tiles + 7) / 8 * 8), (unsigned)ranges);
+    const dim3 grid((unsigned)((g.total_tiles + 7) / 8 * 8), (unsigned)(((g.c + 31) / 32 + g.nb - 1) / g.nb));
     auto launch_pc = [&](auto s_c, auto fold_c, auto rowsum_c, auto qm_c, auto ks_c, auto pc_c) {
         auto kernel = pwdw_block_kernel<decltype(s_c)::value, decltype(fold_c)::value, decltype(rowsum_c)::value, decltype(qm_c)::value, decltype(ks_c)::value,
                                         decltype(pc_c)::value>;

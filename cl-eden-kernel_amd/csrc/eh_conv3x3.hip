@@ -433,6 +433,13 @@ int conv3x3_patch_prepare() {
     return rc;
 }
 
+void conv3x3_patch_shape(GemmProblem *p) {
+    int th = 1, nb = 1;
+    conv3_shape(p->m / (p->ho * p->wo), p->ho, p->wo, p->cin, p->n, &th, &nb);
+    p->rows_kh = th;
+    p->rows_kw = nb;
+}
+
 int launch_conv3x3_patch(const GemmProblem &p, hipStream_t stream) {
     EH_REQUIRE(p.k == 9 * p.cin && (p.cin & 15) == 0 && p.k_pad == (p.k + 31) / 32 * 32 && p.stride_h == 1 && p.stride_w == 1,
                "conv3x3: unsupported problem (k %d, cin %d)", p.k, p.cin);
@@ -442,8 +449,8 @@ int launch_conv3x3_patch(const GemmProblem &p, hipStream_t stream) {
                p.out_y0, p.out_x0, p.out_sy, p.out_sx, p.ho, p.wo);
     EH_REQUIRE((reinterpret_cast<uintptr_t>(p.a) & 15) == 0, "conv3x3: input pointer is not aligned to 16 bytes");
     const int n_img = p.m / (p.ho * p.wo);
-    int th = 1, nb = 1;
-    conv3_shape(n_img, p.ho, p.wo, p.cin, p.n, &th, &nb);
+    const int th = p.rows_kh, nb = p.rows_kw;
+    EH_REQUIRE(th >= 1 && (nb == 1 || nb == 2), "conv3x3: no tile shape");
     Conv3Launch L;
     L.th = th;
     L.tiles_per_image = (p.ho + th - 1) / th;

@@ -416,7 +416,7 @@ struct GemmProblem {
     // int8 tensors (PrecisionType::INT8) run as their uint8 equivalents (value + 128, zero points + 128):
     uint32_t a_xor;    // turns four stored activation bytes into int8 MFMA operands: 0x80808080 for uint8 data, 0 for int8
     uint32_t out_xor;  // turns four uint8 results into the stored bytes: 0 for uint8 data, 0x80808080 for int8
-    int32_t rows_kh, rows_kw;  // GEMM_ROWS: the kernel's extent (other kernels find their taps in ktab)
+    int32_t rows_kh, rows_kw;  // GEMM_ROWS: the kernel's extent (other kernels find their taps in ktab); GEMM_CONV3X3: output rows per tile, channel blocks per workgroup
     // fused residual add (one-tap and split-reduction kernels only): out = add(residual, result) with `radd`;
     // `residual` is addressed like `out`.  Null: plain convolution.
     const uint8_t *residual;
@@ -447,6 +447,7 @@ int launch_igemm_thin(const GemmProblem *ps, int count, hipStream_t stream);  //
 int launch_splitk_finish(const GemmProblem &p, const int32_t *partial, int32_t partial_ld, int32_t slices, hipStream_t stream);
 int launch_conv_c3k3(const GemmProblem &p, hipStream_t stream);
 int launch_conv3x3_patch(const GemmProblem &p, hipStream_t stream);
+void conv3x3_patch_shape(GemmProblem *p);  // fills rows_kh / rows_kw, once per plan
 // one tap, few output pixels, long reductions: cut along the weights (eh_gemm_skinny.hip)
 bool gemm_skinny_applies(int32_t taps, int32_t cin_group, int32_t pixel_stride, int32_t channel_offset, int64_t m, int64_t n);
 int launch_gemm_skinny(const GemmProblem &p, hipStream_t stream);
@@ -550,7 +551,28 @@ int launch_dwconv_nchw(const DwProblem &p, hipStream_t stream);
 bool pwdw_block_applies(const GemmProblem &pw, const DwProblem &dw);
 bool pwdw_block_listed(int32_t images, int32_t image_h, int32_t image_w, int32_t in_channels, int32_t expanded_channels, int32_t stride);
 bool pwdw_block_preferred(const GemmProblem &pw, const DwProblem &dw);  // the fused launch is the faster one for this shape (measured table)
-int launch_pwdw_block(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, int cols_per_tile, hipStream_t stream);
+// Tile and LDS geometry of a fused launch.
+struct BlockGeom {
+    int32_t th, tw;      // output rows and columns per workgroup
+    int32_t tiles_y, tiles_w;  // workgroups per image, down and across
+    int32_t ih, iwp;     // rows and columns of the expanded image a workgroup holds
+    int32_t pixels;      // ih * iwp
+    int32_t c;           // expanded channels of the layer
+    int32_t nb;          // channel blocks of 32 per workgroup (grid y walks the ranges); bytes per pixel of the LDS image = 32 nb
+    int32_t ks;          // reduction steps of 32 bytes of the pointwise stage
+    int32_t cpitch;      // bytes per pixel of the LDS image
+    int32_t tiles_x;     // depthwise tiles of four output columns per row of the workgroup's tile
+    int32_t units_per_cq;  // th * tiles_x: depthwise thread-units per channel quad
+    int32_t total_tiles; // n * tiles_y * tiles_w
+    int32_t a_pitch;     // LDS bytes per input pixel: 32 ks + 16 (the slack spreads the fragment reads over the banks)
+    FastDiv div_iwp, div_tx, div_tiles_y, div_tiles_w, div_ppp;
+    FastDiv div_cq, div_cq_last;  // by the channel quads of a full range, and of the last one
+    uint32_t a_off;      // byte offset of the staged input pixels
+    uint32_t image_off;  // byte offset of the LDS image behind the staged weights, bias and input pixels
+};
+// the geometry for a pair; rows_per_tile / cols_per_tile: the tile a workgroup owns, 0 = chosen here; false when nothing fits
+bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, int cols_per_tile, BlockGeom *g);
+int launch_pwdw_block(const GemmProblem &pw, const DwProblem &dw, const BlockGeom &g, hipStream_t stream);
 
 // ---------------------------------------------------------------- layout
 int launch_nchw2nhwc(const uint8_t *src, uint8_t *dst, int32_t n, int32_t c, int32_t hw, hipStream_t stream);
