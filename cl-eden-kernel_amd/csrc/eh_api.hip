@@ -183,6 +183,21 @@ static bool units_are_rows(const std::vector<KUnit> &units, int per_tap, int tap
     return true;
 }
 
+// (a geometry that does not fit its fields is never read: such reductions stay with the table-driven kernels)
+TapGeom tap_geom(int cin, int nx, int dy0, int dys, int dx0, int dxs, int c0) {
+    TapGeom t;
+    t.chunks = (uint16_t)(cin / 16 > 0 ? cin / 16 : 1);
+    t.nx = (uint16_t)(nx > 0 ? nx : 1);
+    t.dy0 = (int16_t)dy0;
+    t.dys = (int16_t)dys;
+    t.dx0 = (int16_t)dx0;
+    t.dxs = (int16_t)dxs;
+    t.c0 = c0;
+    t.div_chunks = make_fastdiv(t.chunks);
+    t.div_nx = make_fastdiv(t.nx);
+    return t;
+}
+
 // Allocates a part's device arrays and uploads its tables.  `units` holds one
 // KUnit per `vec` bytes of the real reduction length; padding units are added here.
 // k_floor > 0: the part is one of several whose reductions differ in length and that should share a launch: its
@@ -239,6 +254,9 @@ int finish_part(GemmPart &g, std::vector<KUnit> &units, const std::vector<int32_
         g.cfg.slab = 32;
         g.proto.n = g.n;
         conv3x3_patch_shape(&g.proto);
+    } else if (g.vec == 16 && g.k > 0 && gemm_few_tiles_applies(g.proto.m > m_floor ? g.proto.m : m_floor, g.n, k_len, siblings)) {
+        g.cfg.id = GEMM_FEW_TILES;
+        g.cfg.slab = 32;
     } else if (g.vec == 16 && (ktab_fits || (plain_matrix && g.k % 256 == 0)))
         // (a reduction too long for its k-table to fit LDS still runs as a plain matrix of whole slabs: a fully
         // connected layer on 25088 inputs)
@@ -510,7 +528,7 @@ struct GemmOp {
     // the one-tap kernel, the split-reduction epilogue of the tiled kernel and the kernel for few rows can add a residual tensor
     bool fuses_add() const {
         bool fuse = layout == EH_NHWC && !io_signed && !parts.empty();
-        for (auto &g : parts) fuse = fuse && (g.cfg.id == GEMM_THIN || g.cfg.id == GEMM_DMA_64x64_SPLITK || g.cfg.id == GEMM_SKINNY);
+        for (auto &g : parts) fuse = fuse && (g.cfg.id == GEMM_THIN || g.cfg.id == GEMM_DMA_64x64_SPLITK || g.cfg.id == GEMM_SKINNY || g.cfg.id == GEMM_FEW_TILES);
         return fuse;
     }
 
@@ -1132,6 +1150,7 @@ static int conv_plan_build(eh_conv_plan *pl, const eh_conv_desc *d, hipStream_t 
         p.out_y0 = 0;
         p.out_x0 = 0;
         p.ldc = d->cout;
+        p.tap = tap_geom(cig, d->kw, 0, d->dil_h, 0, d->dil_w, g * cig);
         if ((rc = finish_part(part, units, tap_off, stream, std::min(parts_n, (int)GemmBatch::MAX)))) return rc;
     }
     if (wants_channel_padding(op, G, cig_real)) return conv_plan_build(pl, d, stream);
@@ -1361,6 +1380,7 @@ int eh_fc_q8_plan(eh_fc_plan **plan, int32_t m, int32_t k, int32_t n, int32_t fl
         p.out_y0 = 0;
         p.out_x0 = 0;
         p.ldc = n;
+        p.tap = tap_geom(k, 1, 0, 0, 0, 0, 0);
         rc = finish_part(part, units, tap_off, s);
     }
     if (!rc) rc = op.alloc_staging();
@@ -1540,6 +1560,7 @@ static int deconv_plan_build(eh_deconv_plan *pl, const eh_conv_desc *d, hipStrea
                 p.out_y0 = oy0;
                 p.out_x0 = ox0;
                 p.ldc = d->cout;
+                p.tap = tap_geom(cig, ntx, by, -1, bx, -1, g * cig);
                 // phases (and groups) of equal shape share launches: choose the tile shape for the joint tile count
                 const int siblings = (k_floor > 0 || (d->kh % sh == 0 && d->kw % sw == 0)) ? std::min(G * sh * sw / count, (int)GemmBatch::MAX) : 1;
                 if ((rc = finish_part(part, units, tap_off, stream, siblings, k_floor, k_floor ? m_floor : 0))) return rc;

@@ -290,11 +290,13 @@ int igemm_n_tile(int32_t, int32_t, int32_t) { return 256; }
 
 int launch_igemm(const GemmProblem &p, hipStream_t stream) {
     if (p.m <= 0 || p.n <= 0) return EH_OK;
+    if (gemm_few_tiles_instead(p)) return launch_gemm_few_tiles(&p, 1, stream);
     if (p.cfg.id == GEMM_THIN) return launch_igemm_thin(&p, 1, stream);
     if (p.cfg.id == GEMM_C3K3) return launch_conv_c3k3(p, stream);
     if (p.cfg.id == GEMM_CONV3X3) return launch_conv3x3_patch(p, stream);
     if (p.cfg.id == GEMM_ROWS) return launch_conv_rows(p, stream);
     if (p.cfg.id == GEMM_SKINNY) return launch_gemm_skinny(p, stream);
+    if (p.cfg.id == GEMM_FEW_TILES) return launch_gemm_few_tiles(&p, 1, stream);
     EH_REQUIRE(p.k_pad % BK == 0 && p.k_pad > 0, "igemm: padded reduction length %d is not a multiple of %d", p.k_pad, BK);
     EH_REQUIRE(p.vec == 16 || p.vec == 4 || p.vec == 1, "igemm: bad load unit %d", p.vec);
     if (p.cfg.id != GEMM_STAGED) return launch_igemm_dma(&p, 1, stream);
@@ -313,7 +315,7 @@ int launch_igemm_batch(const GemmProblem *ps, int count, hipStream_t stream) {
     while (i < count) {
         const GemmProblem &p = ps[i];
         int run = 1;
-        const bool dma = p.cfg.id != GEMM_STAGED && p.cfg.id != GEMM_THIN && p.cfg.id != GEMM_C3K3 && p.cfg.id != GEMM_CONV3X3 && p.cfg.id != GEMM_ROWS && p.cfg.id != GEMM_SKINNY && p.m > 0 && p.n > 0;
+        const bool dma = p.cfg.id != GEMM_STAGED && p.cfg.id != GEMM_THIN && p.cfg.id != GEMM_C3K3 && p.cfg.id != GEMM_CONV3X3 && p.cfg.id != GEMM_ROWS && p.cfg.id != GEMM_SKINNY && p.cfg.id != GEMM_FEW_TILES && p.m > 0 && p.n > 0;
         if (dma)
             // (row counts may differ where nothing depends on them: table-driven problems; the launch covers the largest)
             while (i + run < count && run < GemmBatch::MAX && ps[i + run].cfg.id == p.cfg.id && (ps[i + run].m == p.m || (!p.dense && !p.partial)) &&
@@ -331,8 +333,16 @@ int launch_igemm_batch(const GemmProblem *ps, int count, hipStream_t stream) {
                    ps[i + run].y_base == p.y_base && ps[i + run].x_base == p.x_base &&
                    ps[i + run].rq.fast == p.rq.fast && (ps[i + run].rq.pc_multiplier != nullptr) == (p.rq.pc_multiplier != nullptr))
                 ++run;
+        // ... and so do the problems with few tiles, whose row counts may differ
+        const bool few = p.cfg.id == GEMM_FEW_TILES && p.m > 0 && p.n > 0 && p.residual == nullptr;
+        if (few)
+            while (i + run < count && run < GemmBatch::MAX && ps[i + run].cfg.id == GEMM_FEW_TILES && ps[i + run].residual == nullptr && ps[i + run].n == p.n &&
+                   ps[i + run].k_pad == p.k_pad && ps[i + run].zw == p.zw && ps[i + run].rq.fast == p.rq.fast)
+                ++run;
         int rc;
-        if (thin && run > 1) {
+        if (few && run > 1) {
+            rc = launch_gemm_few_tiles(ps + i, run, stream);
+        } else if (thin && run > 1) {
             rc = launch_igemm_thin(ps + i, run, stream);
         } else if (dma && run > 1) {
             EH_REQUIRE(p.k_pad % 64 == 0 && p.k_pad > 0, "igemm: padded reduction length %d", p.k_pad);

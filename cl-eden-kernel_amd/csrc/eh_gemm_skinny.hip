@@ -1,9 +1,9 @@
-// One-tap problems (fully connected layers, 1x1 convolutions) on at most 64 rows of activations and a reduction longer
-// than the one-tap kernel's: batch-1 ... batch-64 classifier heads.  Such a launch is the weights' one trip from memory
+// One-tap problems (fully connected layers, 1x1 convolutions) on at most 16 rows of activations and a reduction longer
+// than the one-tap kernel's: batch-1 ... batch-16 classifier heads (17 to 64 rows take the kernel for few tiles).  Such a launch is the weights' one trip from memory
 // and nothing else, so the work is cut along the WEIGHTS: a workgroup of eight waves owns 32 output channels, its waves
 // take the 32-byte reduction steps round-robin, and a step's weight fragment is one contiguous KiB of the packed weights
 // (MFMA fragment order, as for the one-tap kernel), fetched by one 16-byte-per-lane load straight into the registers the
-// matrix instruction reads, eight such loads in flight per wave.  The activations (at most 64 rows, shared by every
+// matrix instruction reads, eight such loads in flight per wave.  The activations (a few rows, shared by every
 // workgroup through the caches) are read in fragment form as well; rows past the last one multiply as zero.  The eight
 // partial tiles and the rows' partial byte sums add up in LDS, and the first wave(s) requantize and store.
 //
@@ -23,87 +23,69 @@ typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kWaves = 8;    // waves of a workgroup, each on every eighth reduction step
 constexpr int kFlight = 8;   // weight fragments a wave has on their way
 
-// G: groups of 32 activation rows (1 or 2).  FAST: every requantization pair in use is inside the single-shift form's range.
-template <int G, bool ROWSUM, bool FAST>
+// FAST: every requantization pair in use is inside the single-shift form's range.
+template <bool ROWSUM, bool FAST>
 __global__ __launch_bounds__(kWaves * 64) void skinny_gemm_kernel(const GemmProblem p, const int ksteps) {
-    __shared__ int32_t part_s[G][17][64];  // [group][accumulator, then the byte sum][lane]: where the waves' partial tiles add up
+    __shared__ int32_t part_s[17][64];  // [accumulator, then the byte sum][lane]: where the waves' partial tiles add up
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nb = blockIdx.x;
-    for (int i = tid; i < G * 17 * 64; i += kWaves * 64) (&part_s[0][0][0])[i] = 0;
+    for (int i = tid; i < 17 * 64; i += kWaves * 64) (&part_s[0][0])[i] = 0;
     __syncthreads();
     const v4i *wsrc = reinterpret_cast<const v4i *>(p.b) + (size_t)nb * ksteps * 64 + lane;
     // this lane's rows of the activation matrix, from its first reduction byte on
-    const uint8_t *arow[G];
-    bool row_ok[G];
+    const bool row_ok = r < p.m;
+    const uint8_t *arow = p.a + (size_t)(row_ok ? r : 0) * (size_t)p.cin + (size_t)p.a_offset + half * 16;
+    v16i acc;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int row = g * 32 + r;
-        row_ok[g] = row < p.m;
-        arow[g] = p.a + (size_t)(row_ok[g] ? row : 0) * (size_t)p.cin + (size_t)p.a_offset + half * 16;
-    }
-    v16i acc[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[g][i] = 0;
-    int rowsum[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) rowsum[g] = 0;
+    for (int i = 0; i < 16; ++i) acc[i] = 0;
+    int rowsum = 0;
 
     for (int ks0 = wave; ks0 < ksteps; ks0 += kWaves * kFlight) {
-        v4i bf[kFlight], af[kFlight][G];
+        v4i bf[kFlight], af[kFlight];
 #pragma unroll
         for (int u = 0; u < kFlight; ++u) {
             const int ks = ks0 + u * kWaves;
             const int ksc = ks < ksteps ? ks : ksteps - 1;  // (a step past the end: loaded again, not multiplied)
             bf[u] = wsrc[(size_t)ksc * 64];
             const int kb = ksc * 32 + half * 16;
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
+            {
                 // bytes past K (a reduction that ends inside its last step) and rows past M read as the byte that the flip turns into 0
                 u32x4_a4 v = u32x4_a4{p.a_xor, p.a_xor, p.a_xor, p.a_xor};
-                if (row_ok[g] && kb < p.k) v = *reinterpret_cast<const u32x4_a4 *>(arow[g] + ksc * 32);
-                af[u][g] = v4i{(int)(v.x ^ p.a_xor), (int)(v.y ^ p.a_xor), (int)(v.z ^ p.a_xor), (int)(v.w ^ p.a_xor)};
+                if (row_ok && kb < p.k) v = *reinterpret_cast<const u32x4_a4 *>(arow + ksc * 32);
+                af[u] = v4i{(int)(v.x ^ p.a_xor), (int)(v.y ^ p.a_xor), (int)(v.z ^ p.a_xor), (int)(v.w ^ p.a_xor)};
             }
         }
 #pragma unroll
         for (int u = 0; u < kFlight; ++u) {
             if (ks0 + u * kWaves < ksteps) {  // (uniform across the wave)
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    if constexpr (ROWSUM) {
-                        rowsum[g] = __builtin_amdgcn_sdot4(af[u][g].x, 0x01010101, rowsum[g], false);
-                        rowsum[g] = __builtin_amdgcn_sdot4(af[u][g].y, 0x01010101, rowsum[g], false);
-                        rowsum[g] = __builtin_amdgcn_sdot4(af[u][g].z, 0x01010101, rowsum[g], false);
-                        rowsum[g] = __builtin_amdgcn_sdot4(af[u][g].w, 0x01010101, rowsum[g], false);
-                    }
-                    acc[g] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[u], af[u][g], acc[g], 0, 0, 0);
+                if constexpr (ROWSUM) {
+                    rowsum = __builtin_amdgcn_sdot4(af[u].x, 0x01010101, rowsum, false);
+                    rowsum = __builtin_amdgcn_sdot4(af[u].y, 0x01010101, rowsum, false);
+                    rowsum = __builtin_amdgcn_sdot4(af[u].z, 0x01010101, rowsum, false);
+                    rowsum = __builtin_amdgcn_sdot4(af[u].w, 0x01010101, rowsum, false);
                 }
+                acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[u], af[u], acc, 0, 0, 0);
             }
         }
     }
     // the partial tiles meet in LDS (integer adds: the order does not matter)
     if (wave < ksteps) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) atomicAdd(&part_s[g][i][lane], acc[g][i]);
-            if constexpr (ROWSUM) atomicAdd(&part_s[g][16][lane], rowsum[g]);
-        }
+        for (int i = 0; i < 16; ++i) atomicAdd(&part_s[i][lane], acc[i]);
+        if constexpr (ROWSUM) atomicAdd(&part_s[16][lane], rowsum);
     }
     __syncthreads();
-    if (wave >= G) return;
-    const int g = wave;  // wave 0 finishes rows 0 .. 31, wave 1 rows 32 .. 63
+    if (wave != 0) return;
     const int n = nb * 32 + half * 16;  // this lane's sixteen consecutive channels
     // the sixteen residual bytes these outputs are added to, requested before the requantization that hides their way
     u32x4_a4 res4 = u32x4_a4{0, 0, 0, 0};
-    const bool res_vec = p.residual != nullptr && g * 32 + r < p.m && n + 16 <= p.n && (p.ldc & 3) == 0 &&
+    const bool res_vec = p.residual != nullptr && row_ok && n + 16 <= p.n && (p.ldc & 3) == 0 &&
                          (reinterpret_cast<uintptr_t>(p.residual) & 3) == 0;
-    if (res_vec) res4 = *reinterpret_cast<const u32x4_a4 *>(p.residual + (size_t)(g * 32 + r) * (size_t)p.ldc + n);
+    if (res_vec) res4 = *reinterpret_cast<const u32x4_a4 *>(p.residual + (size_t)r * (size_t)p.ldc + n);
     int ncorr = 0;
     if constexpr (ROWSUM) {
-        int rs = part_s[g][16][lane];
+        int rs = part_s[16][lane];
         rs += __shfl_xor(rs, 32);  // the other half of every step's bytes
         ncorr = -p.zw * rs;
     }
@@ -117,7 +99,7 @@ __global__ __launch_bounds__(kWaves * 64) void skinny_gemm_kernel(const GemmProb
         x[q4 * 4 + 3] = bb.w;
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] += ncorr + part_s[g][i][lane];
+    for (int i = 0; i < 16; ++i) x[i] += ncorr + part_s[i][lane];
     const RequantDev rq = p.rq;
     uint32_t packed[4];
     auto produce = [&](auto mode_c) {
@@ -152,16 +134,15 @@ __global__ __launch_bounds__(kWaves * 64) void skinny_gemm_kernel(const GemmProb
         produce(std::integral_constant<int, 2>{});
     else
         produce(std::integral_constant<int, 1>{});
-    const int row = g * 32 + r;
-    if (row < p.m && n < p.n) {
-        uint8_t *dst = p.out + (size_t)row * (size_t)p.ldc + n;
+    if (row_ok && n < p.n) {
+        uint8_t *dst = p.out + (size_t)r * (size_t)p.ldc + n;
         const int cnt = p.n - n;
         if (p.residual) {  // out = add(residual, result)
             if (res_vec) {
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) packed[q4] = add_word(res4[q4], packed[q4], p.radd);
             } else {
-                const uint8_t *res = p.residual + (size_t)row * (size_t)p.ldc + n;
+                const uint8_t *res = p.residual + (size_t)r * (size_t)p.ldc + n;
                 for (int t = 0; t < (cnt < 16 ? cnt : 16); ++t) {
                     const uint32_t v = add_one(res[t], (packed[t >> 2] >> (8 * (t & 3))) & 255u, p.radd);
                     packed[t >> 2] = (packed[t >> 2] & ~(255u << (8 * (t & 3)))) | (v << (8 * (t & 3)));
@@ -189,7 +170,7 @@ bool gemm_skinny_applies(int32_t taps, int32_t cin_group, int32_t pixel_stride, 
 }
 
 int launch_gemm_skinny(const GemmProblem &p, hipStream_t stream) {
-    EH_REQUIRE(p.m >= 1 && p.m <= 64 && p.k_pad % 32 == 0 && p.k_pad >= p.k && (p.k & 15) == 0 && (p.cin & 15) == 0 && (p.a_offset & 15) == 0,
+    EH_REQUIRE(p.m >= 1 && p.m <= 32 && p.k_pad % 32 == 0 && p.k_pad >= p.k && (p.k & 15) == 0 && (p.cin & 15) == 0 && (p.a_offset & 15) == 0,
                "gemm_skinny: %d rows, reduction %d (padded %d), row stride %d", p.m, p.k, p.k_pad, p.cin);
     EH_REQUIRE((reinterpret_cast<uintptr_t>(p.a) & 15) == 0, "gemm_skinny: the activations must start on a 16-byte boundary");
     // pixel m of the problem is row m of a matrix: stride 1, no offsets, dense output
@@ -198,22 +179,15 @@ int launch_gemm_skinny(const GemmProblem &p, hipStream_t stream) {
                "gemm_skinny: the problem is not a plain matrix product");
     const int n_blocks = (p.n + 31) / 32, ksteps = p.k_pad / 32;
     const bool rowsum = p.zw != 0, fast = p.rq.fast != 0;
-    auto launch = [&](auto g_c) {
-        constexpr int G = decltype(g_c)::value;
-        const dim3 grid((unsigned)n_blocks), block(kWaves * 64);
-        if (rowsum && fast)
-            hipLaunchKernelGGL((skinny_gemm_kernel<G, true, true>), grid, block, 0, stream, p, ksteps);
-        else if (rowsum)
-            hipLaunchKernelGGL((skinny_gemm_kernel<G, true, false>), grid, block, 0, stream, p, ksteps);
-        else if (fast)
-            hipLaunchKernelGGL((skinny_gemm_kernel<G, false, true>), grid, block, 0, stream, p, ksteps);
-        else
-            hipLaunchKernelGGL((skinny_gemm_kernel<G, false, false>), grid, block, 0, stream, p, ksteps);
-    };
-    if (p.m <= 32)
-        launch(std::integral_constant<int, 1>{});
+    const dim3 grid((unsigned)n_blocks), block(kWaves * 64);
+    if (rowsum && fast)
+        hipLaunchKernelGGL((skinny_gemm_kernel<true, true>), grid, block, 0, stream, p, ksteps);
+    else if (rowsum)
+        hipLaunchKernelGGL((skinny_gemm_kernel<true, false>), grid, block, 0, stream, p, ksteps);
+    else if (fast)
+        hipLaunchKernelGGL((skinny_gemm_kernel<false, true>), grid, block, 0, stream, p, ksteps);
     else
-        launch(std::integral_constant<int, 2>{});
+        hipLaunchKernelGGL((skinny_gemm_kernel<false, false>), grid, block, 0, stream, p, ksteps);
     EH_HIP(hipGetLastError());
     return EH_OK;
 }

@@ -383,11 +383,21 @@ enum GemmConfigId {
     GEMM_C3K3 = 7,              // 3 input channels, 3x3 taps (first layers); weights row-major [n_pad][32]
     GEMM_CONV3X3 = 8,           // 3x3 taps, stride 1, input patch staged in LDS once; weights in MFMA fragment order
     GEMM_SKINNY = 10,           // one tap, at most 64 output pixels, long reductions; weights in MFMA fragment order
+    GEMM_FEW_TILES = 11,        // few 32 x 32 output tiles; weights in MFMA fragment order
     GEMM_ROWS = 9,              // 1 - 4 input channels, kernel rows of at most 32 bytes; weights row-major [n_pad][32 per kernel row]
 };
 struct GemmConfig {
     int32_t id = GEMM_STAGED;
     int32_t slab = 64;  // reduction bytes per stage; k_pad is a multiple of it
+};
+
+// Where the taps of a reduction over whole 16-byte channel chunks sit: tap t at row dy0 + (t / nx) * dys and column
+// dx0 + (t % nx) * dxs of the output pixel's window, `chunks` chunks per tap from channel c0 on.
+struct TapGeom {
+    uint16_t chunks = 1, nx = 1;
+    int16_t dy0 = 0, dys = 0, dx0 = 0, dxs = 0;
+    int32_t c0 = 0;
+    FastDiv div_chunks, div_nx;
 };
 
 struct GemmProblem {
@@ -416,6 +426,7 @@ struct GemmProblem {
     // int8 tensors (PrecisionType::INT8) run as their uint8 equivalents (value + 128, zero points + 128):
     uint32_t a_xor;    // turns four stored activation bytes into int8 MFMA operands: 0x80808080 for uint8 data, 0 for int8
     uint32_t out_xor;  // turns four uint8 results into the stored bytes: 0 for uint8 data, 0x80808080 for int8
+    TapGeom tap;       // the kernel for few tiles finds its taps by this
     int32_t rows_kh, rows_kw;  // GEMM_ROWS: the kernel's extent (other kernels find their taps in ktab); GEMM_CONV3X3: output rows per tile, channel blocks per workgroup
     // fused residual add (one-tap and split-reduction kernels only): out = add(residual, result) with `radd`;
     // `residual` is addressed like `out`.  Null: plain convolution.
@@ -451,6 +462,10 @@ void conv3x3_patch_shape(GemmProblem *p);  // fills rows_kh / rows_kw, once per 
 // one tap, few output pixels, long reductions: cut along the weights (eh_gemm_skinny.hip)
 bool gemm_skinny_applies(int32_t taps, int32_t cin_group, int32_t pixel_stride, int32_t channel_offset, int64_t m, int64_t n);
 int launch_gemm_skinny(const GemmProblem &p, hipStream_t stream);
+// few output tiles (eh_gemm_few.hip): whether a problem whose weights are packed in fragment order should run there, and the launch
+bool gemm_few_tiles_applies(int64_t m, int64_t n, int64_t k, int32_t siblings);
+bool gemm_few_tiles_instead(const GemmProblem &p);  // ... although it was planned for another kernel of the same weight order
+int launch_gemm_few_tiles(const GemmProblem *ps, int count, hipStream_t stream);  // `count` equally shaped problems as one launch
 // few input channels, a kernel row per reduction step (eh_conv_rows.hip)
 bool conv_rows_applies(int32_t cin_group, int32_t pixel_stride, int32_t kh, int32_t kw);
 int launch_conv_rows(const GemmProblem &p, hipStream_t stream);
@@ -469,7 +484,7 @@ __host__ __device__ inline size_t packed_b_offset(const GemmConfig &cfg, int n, 
     const int ch = n & 31;
     n = (n & ~31) | (((ch & 15) >> 2) << 3) | ((ch >> 4) << 2) | (ch & 3);
     // fragment order: [32-channel block][32-byte step][lane = 32 * (chunk & 1) + row][16 bytes]
-    if (cfg.id == GEMM_THIN || cfg.id == GEMM_CONV3X3 || cfg.id == GEMM_SKINNY) return ((((size_t)(n >> 5) * (k_pad / 32) + (kc16 >> 1)) * 2 + (kc16 & 1)) * 32 + (n & 31)) * 16;
+    if (cfg.id == GEMM_THIN || cfg.id == GEMM_CONV3X3 || cfg.id == GEMM_SKINNY || cfg.id == GEMM_FEW_TILES) return ((((size_t)(n >> 5) * (k_pad / 32) + (kc16 >> 1)) * 2 + (kc16 & 1)) * 32 + (n & 31)) * 16;
     const int cpr = cfg.slab / 16, rpb = 1024 / cfg.slab;
     const int c = kc16 % cpr;
     return ((size_t)(n / rpb) * (k_pad / cfg.slab) + kc16 / cpr) * 1024 + (size_t)(n % rpb) * cfg.slab +
