@@ -11,6 +11,7 @@ import numpy as np
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libedenhip.so")
+CALL_PATH = os.path.join(HERE, "_call.so")
 
 EH_OK = 0
 ACT_NONE, ACT_RELU, ACT_RELU1, ACT_RELU6 = 0, 1, 2, 3
@@ -150,15 +151,20 @@ _lib = None
 
 
 def load():
-    """Loads libedenhip.so and types every export; raises if the library or a symbol is missing."""
-    global _lib
+    """Loads libedenhip.so and types every export, puts the native form of the operator calls (_call.so) on the plan
+    classes; raises if a library or a symbol is missing."""
+    global _lib, conv_dw_block_run
     if _lib is None:
-        if not os.path.exists(LIB_PATH):
-            raise EdenHipError("%s is not built: run `python cl-eden-kernel_amd/build.py`" % LIB_PATH)
+        for path in (LIB_PATH, CALL_PATH):
+            if not os.path.exists(path):
+                raise EdenHipError("%s is not built: run `python cl-eden-kernel_amd/build.py`" % path)
         lib = C.CDLL(LIB_PATH)
         for name, (res, args) in EXPORTS.items():
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = res, args
+        from . import _call
+        _call.install(C.c_void_p, Requant, AddRequant, check, _Plan, ConvPlan, _conv_dw_block_run_general)
+        conv_dw_block_run = _call.conv_dw_block_run
         _lib = lib
     return _lib
 
@@ -369,10 +375,13 @@ def conv_dw_block_preferred(pw, dw):
     return bool(load().eh_conv_dw_block_preferred(pw.handle, dw.handle))
 
 
-def conv_dw_block_run(pointwise, depthwise, d_in, d_out, q_pointwise, q_depthwise, rows_per_tile=0, cols_per_tile=0, stream=None):
+def _conv_dw_block_run_general(pointwise, depthwise, d_in, d_out, q_pointwise, q_depthwise, rows_per_tile=0, cols_per_tile=0, stream=None):
     """pointwise convolution + 3x3 depthwise convolution as one launch (the expanded tensor stays in LDS)"""
     check(load().eh_conv_dw_block_run(pointwise.handle, depthwise.handle, d_in.ptr, d_out.ptr, C.byref(q_pointwise), C.byref(q_depthwise),
                                       rows_per_tile, cols_per_tile, stream))
+
+
+conv_dw_block_run = _conv_dw_block_run_general   # until load() puts the native form in its place
 
 
 class BufferPool:
@@ -421,11 +430,11 @@ class _Plan:
         self.handle = C.c_void_p()
         self._keep = []
         self._run = getattr(load(), "eh_%s_u8_run" % self._kind)   # looked up once: a call's own cost counts on small layers
+        self._entry = C.cast(self._run, C.c_void_p).value
 
-    def run(self, d_in, d_out, q, stream=None):
-        rc = self._run(self.handle, d_in.ptr, d_out.ptr, q, stream)
-        if rc:
-            check(rc)
+    # `run` itself is native (host/py_call.cpp); this is the form for arguments it does not take
+    def _run_general(self, d_in, d_out, q, stream=None):
+        check(self._run(self.handle, d_in.ptr, d_out.ptr, q, stream))
 
     def repack(self, d_w, d_b, q, stream=None):
         check(getattr(load(), "eh_%s_u8_repack" % self._kind)(self.handle, d_w.ptr, d_b.ptr if d_b else None,
@@ -474,7 +483,7 @@ def make_requant_perchannel(s_in, zp_in, filter_scales, s_out, zp_out, act=ACT_N
     return q, mult, shift
 
 
-def _conv_run_add(self, d_in, d_residual, d_out, q, aq, stream=None):
+def _conv_run_add_general(self, d_in, d_residual, d_out, q, aq, stream=None):
     """d_out = add(d_residual, convolution(d_in)) with the add parameters `aq` (the residual is the first operand)"""
     check(load().eh_conv2d_u8_run_add(self.handle, d_in.ptr, d_residual.ptr, d_out.ptr, C.byref(q), C.byref(aq), stream))
 
@@ -486,7 +495,7 @@ def _conv_run_static(self, d_in, d_out, q, stream=None):
 
 STATIC_SCRATCH_BYTES = 32 << 20
 ConvPlan.run_static = _conv_run_static
-ConvPlan.run_add = _conv_run_add
+ConvPlan._run_add_general = _conv_run_add_general
 ConvPlan.fuses_add = lambda self: bool(load().eh_conv2d_u8_fuses_add(self.handle))
 
 

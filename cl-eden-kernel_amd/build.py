@@ -1,10 +1,12 @@
 """Builds libedenhip.so (HIP kernels + the operator-level C ABI, include/eden_hip.h) for gfx950 with hipcc, and
-libedenud.so (the C++ host classes behind the userdriver-level C ABI, include/eden_ud.h) with g++ against it.
+libedenud.so (the C++ host classes behind the userdriver-level C ABI, include/eden_ud.h) and _call.so (the Python
+binding's operator calls) with g++ against it.
 Everything is built in-tree; nothing is installed."""
 import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -14,6 +16,7 @@ HOST = os.path.join(HERE, "host")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libedenhip.so")
 UD_LIB = os.path.join(HERE, "libedenud.so")
+CALL_LIB = os.path.join(HERE, "_call.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
@@ -93,9 +96,17 @@ def build_ud_lib():
     return UD_LIB
 
 
+def build_call_lib():
+    """The Python binding's operator calls (host/py_call.cpp), an extension module linked against libedenhip.so."""
+    _run(["g++", "-O2", "-std=c++17", "-Wall", "-fPIC", "-shared", "-I" + os.path.join(ROOT, "include"), "-I" + sysconfig.get_paths()["include"],
+          os.path.join(HOST, "py_call.cpp"), "-o", CALL_LIB, "-L" + HERE, "-ledenhip", "-Wl,-rpath,$ORIGIN"])
+    return CALL_LIB
+
+
 def build_all():
     lib = build_lib()
     build_ud_lib()
+    build_call_lib()
     return lib
 
 
