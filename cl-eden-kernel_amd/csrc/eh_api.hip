@@ -533,6 +533,21 @@ struct GemmOp {
     }
 
     // residual != null: output = add(residual, result) with `radd`; `fused` tells whether the kernels did it
+    // Whether the plan's kernels write a planar output themselves, instead of a channels-last image that a transposition
+    // then reads (a launch and two trips of the output: 64 channels at 56x56, four images 10.8 -> 8.0 us; 16 -> 96 at
+    // 112x112, 32 images 31 -> 23).  Every epilogue that holds sixteen channels of a pixel per lane has the form, but for
+    // the largest tiles (no registers to spare) and the second launches of sliced reductions; the tiled kernels, whose
+    // workgroups all finish at once, write bytes slower than the transposition moves them from some 6 MB on (128 channels
+    // at 56x56, 32 images, 12.8 MB: 44 -> 48 us; 256 at 28x28, 8 images, 1.6 MB: 18.8 -> 15.6).
+    bool stores_planar() const {
+        bool all = layout == EH_NCHW && (int64_t)in_n * out_hw < (1ll << 31);
+        const bool small = (int64_t)in_n * out_hw * cout <= (6ll << 20);
+        for (auto &g : parts) {
+            const bool per_wave = g.cfg.id == GEMM_THIN || g.cfg.id == GEMM_FEW_TILES || g.cfg.id == GEMM_CONV3X3 || g.cfg.id == GEMM_C3K3 || g.cfg.id == GEMM_ROWS;
+            all = all && g.slices == 0 && g.n_period == 0 && (per_wave || (small && g.cfg.id != GEMM_SKINNY && g.cfg.id != GEMM_DMA_256x256));
+        }
+        return all;
+    }
     // bytes of the two channels-last staging images of a planar plan (each with the slack the kernels' wide loads need)
     size_t stage_in_bytes() const { return ((size_t)in_n * in_c * in_hw + 256 + 255) / 256 * 256; }
     size_t stage_out_bytes() const { return ((size_t)in_n * cout * out_hw + 256 + 255) / 256 * 256; }
@@ -551,13 +566,22 @@ struct GemmOp {
     static constexpr int kInlineParts = 8;  // a run over at most this many parts allocates no host memory
 
     // One part's kernel argument for channels-last tensors `in` / `out`, with the quantization parameters refold() left in `q`
-    GemmProblem problem(const GemmPart &g, const uint8_t *in, uint8_t *out, const uint8_t *residual, const AddDev *radd) const {
+    // (planar_out: `out` is a planar tensor that the kernels write themselves)
+    GemmProblem problem(const GemmPart &g, const uint8_t *in, uint8_t *out, const uint8_t *residual, const AddDev *radd, bool planar_out = false) const {
         GemmProblem p = g.proto;
         p.a = in;
         p.b = g.b;
         p.bias = g.folded;
         p.fillbuf = fillbuf;
-        p.out = out + g.bias_base;
+        p.out = out + (planar_out ? (size_t)g.bias_base * (size_t)out_hw : (size_t)g.bias_base);
+        if (planar_out) {
+            p.ldc = 1;
+            p.out_plane = out_hw;
+            p.out_c = cout;
+            const FastDiv div = make_fastdiv((uint32_t)out_hw);
+            p.out_plane_mul = div.mul;
+            p.out_plane_shift = div.shift;
+        }
         p.zw = zp_w_u8(q) - 128;
         p.out_xor = io_signed ? 0x80808080u : 0u;
         p.a_xor = 0x80808080u ^ p.out_xor;
@@ -588,13 +612,20 @@ struct GemmOp {
         const uint8_t *in = static_cast<const uint8_t *>(input);
         uint8_t *out = static_cast<uint8_t *>(output);
         uint8_t *const st_in = staging ? staging : stage_in, *const st_out = staging ? staging + stage_in_bytes() : stage_out;
+        uint8_t *const st_pad = staging ? staging + (layout == EH_NCHW ? stage_in_bytes() + stage_out_bytes() : 0) : stage_pad;
+        const bool planar_out = stores_planar();
+        bool padded = false;
         if (layout == EH_NCHW) {
-            if ((rc = launch_nchw2nhwc(in, st_in, in_n, in_c, in_hw, stream))) return rc;
-            in = st_in;
-            out = st_out;
+            // (the channel padding as part of the same pass)
+            padded = pad_cg_to != 0 && pad_groups == 1;
+            uint8_t *const to = padded ? st_pad : st_in;
+            rc = padded ? launch_nchw2nhwc_padded(in, to, in_n, in_c, in_hw, pad_cg_to, (uint32_t)(q.zp_in & 0xFF) ^ (io_signed ? 0x80u : 0u), stream)
+                        : launch_nchw2nhwc(in, to, in_n, in_c, in_hw, stream);
+            if (rc) return rc;
+            in = to;
+            if (!planar_out) out = st_out;
         }
-        if (pad_cg_to) {
-            uint8_t *const st_pad = staging ? staging + (layout == EH_NCHW ? stage_in_bytes() + stage_out_bytes() : 0) : stage_pad;
+        if (pad_cg_to && !padded) {
             // (q holds the uint8-equivalent input zero point after refold(); int8 tensors store it minus 128)
             if ((rc = launch_pad_channels(in, st_pad, (int64_t)in_n * in_hw, pad_groups, pad_cg, pad_cg_to,
                                           (uint32_t)(q.zp_in & 0xFF) ^ (io_signed ? 0x80u : 0u), stream)))
@@ -611,7 +642,7 @@ struct GemmOp {
         for (auto &g : parts) {
             EH_REQUIRE((reinterpret_cast<uintptr_t>(in) & (uintptr_t)(g.vec - 1)) == 0,
                        "input pointer is not aligned to %d bytes", g.vec);
-            const GemmProblem whole = problem(g, in, out, fuse ? residual : nullptr, radd);
+            const GemmProblem whole = problem(g, in, out, fuse ? residual : nullptr, radd, planar_out);
             if (g.slices == 0) {
                 problems[filled++] = whole;
                 continue;
@@ -634,7 +665,7 @@ struct GemmOp {
         if ((rc = launch_igemm_batch(problems, filled, stream))) return rc;
         for (auto &g : parts)
             if (g.slices && (rc = launch_splitk_finish(problem(g, in, out, fuse ? residual : nullptr, radd), g.partial, g.n_pad, g.slices, stream))) return rc;
-        if (layout == EH_NCHW) {
+        if (layout == EH_NCHW && !planar_out) {
             if ((rc = launch_nhwc2nchw(st_out, static_cast<uint8_t *>(output), in_n, cout, out_hw, stream))) return rc;
         }
         return EH_OK;

@@ -60,7 +60,7 @@ struct Conv3Launch {
 // that no matrix instruction is spent on repeated pixels).
 // SPLIT (NB == 2 only): a wave works on ONE of the two channel blocks, the waves forming 2 x 2 over (pixel group,
 // channel block): tiles of two pixel groups then keep all four waves busy instead of two.
-template <int NB, bool ROWSUM, int QM, bool PC, int G = 4, bool SPLIT = false>
+template <int NB, bool ROWSUM, int QM, bool PC, int G = 4, bool SPLIT = false, bool PLANAR = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv3x3_patch_kernel(const GemmProblem p, const Conv3Launch L) {
     extern __shared__ __align__(1024) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, half = lane >> 5;
@@ -282,6 +282,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
                 }
                 if (ok && nb < nb_count && n < p.n) {
                     uint8_t *dst = row + n;
+                    if constexpr (PLANAR) {
+                        store_bytes_planar(p, (size_t)(row - p.out), n, packed, p.n - n);
+                        continue;
+                    }
                     if (wide && n + 16 <= p.n) {
                         *reinterpret_cast<uint4 *>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
                     } else {
@@ -357,11 +361,14 @@ int launch_nb(const GemmProblem &p, const Conv3Launch &L, size_t lds, hipStream_
     const dim3 grid((unsigned)((L.tiles + 7) / 8 * 8), (unsigned)((n_blocks + NB - 1) / NB));
     const int rows = L.th < p.ho ? L.th : p.ho;
     const Conv3Variant variant = conv3_variant((rows * p.wo + 31) / 32, NB);
-    auto launch_g = [&](auto rowsum_c, auto qm_c, auto pc_c, auto g_c, auto split_c) {
+    auto launch_planar = [&](auto rowsum_c, auto qm_c, auto pc_c, auto g_c, auto split_c, auto planar_c) {
         auto kernel = conv3x3_patch_kernel<NB, decltype(rowsum_c)::value, decltype(qm_c)::value, decltype(pc_c)::value, decltype(g_c)::value,
-                                           decltype(split_c)::value>;
+                                           decltype(split_c)::value, decltype(planar_c)::value>;
         hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, p, L);
         return (int)EH_OK;
+    };
+    auto launch_g = [&](auto rowsum_c, auto qm_c, auto pc_c, auto g_c, auto split_c) {
+        return p.out_plane ? launch_planar(rowsum_c, qm_c, pc_c, g_c, split_c, std::true_type{}) : launch_planar(rowsum_c, qm_c, pc_c, g_c, split_c, std::false_type{});
     };
     auto launch_pc = [&](auto rowsum_c, auto qm_c, auto pc_c) {
         if constexpr (NB == 2) {
@@ -405,23 +412,27 @@ int conv3x3_patch_prepare() {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
         if (e != hipSuccess && rc == EH_OK) rc = hip_fail(e, "hipFuncSetAttribute(conv3x3_patch_kernel)");
     };
-    auto each_pc = [&](auto nb_c, auto rowsum_c, auto qm_c) {
+    auto each_pc = [&](auto nb_c, auto rowsum_c, auto qm_c, auto planar_c) {
         constexpr int NB = decltype(nb_c)::value;
+        constexpr bool PL = decltype(planar_c)::value;
         constexpr bool RS = decltype(rowsum_c)::value;
         constexpr int QM = decltype(qm_c)::value;
-        raise(conv3x3_patch_kernel<NB, RS, QM, false, 4, false>);
-        raise(conv3x3_patch_kernel<NB, RS, QM, true, 4, false>);
-        raise(conv3x3_patch_kernel<NB, RS, QM, false, 1, false>);
-        raise(conv3x3_patch_kernel<NB, RS, QM, true, 1, false>);
+        raise(conv3x3_patch_kernel<NB, RS, QM, false, 4, false, PL>);
+        raise(conv3x3_patch_kernel<NB, RS, QM, true, 4, false, PL>);
+        raise(conv3x3_patch_kernel<NB, RS, QM, false, 1, false, PL>);
+        raise(conv3x3_patch_kernel<NB, RS, QM, true, 1, false, PL>);
         if constexpr (NB == 2) {
-            raise(conv3x3_patch_kernel<NB, RS, QM, false, 1, true>);
-            raise(conv3x3_patch_kernel<NB, RS, QM, true, 1, true>);
+            raise(conv3x3_patch_kernel<NB, RS, QM, false, 1, true, PL>);
+            raise(conv3x3_patch_kernel<NB, RS, QM, true, 1, true, PL>);
         }
     };
     auto each_qm = [&](auto nb_c, auto rowsum_c) {
-        each_pc(nb_c, rowsum_c, std::integral_constant<int, 0>{});
-        each_pc(nb_c, rowsum_c, std::integral_constant<int, 1>{});
-        each_pc(nb_c, rowsum_c, std::integral_constant<int, 2>{});
+        each_pc(nb_c, rowsum_c, std::integral_constant<int, 0>{}, std::false_type{});
+        each_pc(nb_c, rowsum_c, std::integral_constant<int, 0>{}, std::true_type{});
+        each_pc(nb_c, rowsum_c, std::integral_constant<int, 1>{}, std::false_type{});
+        each_pc(nb_c, rowsum_c, std::integral_constant<int, 1>{}, std::true_type{});
+        each_pc(nb_c, rowsum_c, std::integral_constant<int, 2>{}, std::false_type{});
+        each_pc(nb_c, rowsum_c, std::integral_constant<int, 2>{}, std::true_type{});
     };
     auto each_rowsum = [&](auto nb_c) {
         each_qm(nb_c, std::false_type{});

@@ -87,7 +87,7 @@ __device__ __forceinline__ void gather_c3k3(const GemmProblem &p, const uint32_t
 
 // Matrix-core form.  Grid: x = 256 pixels per workgroup (64 per wave).  With one multiplier and shift per channel,
 // FAST means that every channel's pair is inside the single-shift form's range.
-template <bool ROWSUM, bool FAST>
+template <bool ROWSUM, bool FAST, bool PLANAR>
 __global__ __launch_bounds__(256) void conv_c3k3_mfma_kernel(const GemmProblem p, const uint32_t in_bytes) {
     const int lane = threadIdx.x & 63, r = lane & 31, half = lane >> 5;
     // every XCD (workgroups are dispatched round-robin over the 8 of them) takes one contiguous eighth of the
@@ -181,7 +181,9 @@ __global__ __launch_bounds__(256) void conv_c3k3_mfma_kernel(const GemmProblem p
             if (m < p.m && n < p.n) {
                 uint8_t *dst = p.out + out_off + n;
                 const int cnt = p.n - n;
-                if (cnt >= 16 && (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 3) == 0) {
+                if constexpr (PLANAR) {
+                    store_bytes_planar(p, out_off, n, packed, cnt);
+                } else if (cnt >= 16 && (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 3) == 0) {
                     *reinterpret_cast<u32x4_a4 *>(dst) = u32x4_a4{packed[0], packed[1], packed[2], packed[3]};
                 } else {
                     store_bytes_any_alignment(dst, packed, cnt < 16 ? cnt : 16);
@@ -191,7 +193,7 @@ __global__ __launch_bounds__(256) void conv_c3k3_mfma_kernel(const GemmProblem p
     }
 }
 
-template <bool ROWSUM, bool FAST>
+template <bool ROWSUM, bool FAST, bool PLANAR>
 __global__ __launch_bounds__(256) void conv_c3k3_kernel(const GemmProblem p, const uint32_t in_bytes) {
     const int m = blockIdx.x * 256 + threadIdx.x;
     if (m >= p.m) return;
@@ -280,7 +282,9 @@ __global__ __launch_bounds__(256) void conv_c3k3_kernel(const GemmProblem p, con
         produce(std::integral_constant<int, 1>{});
     uint8_t *dst = p.out + (((size_t)img * p.out_h + (oy * p.out_sy + p.out_y0)) * p.out_w + (ox * p.out_sx + p.out_x0)) * (size_t)p.ldc + n0;
     const bool aligned16 = (p.ldc & 15) == 0 && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
-    if (aligned16 && n0 + 16 <= p.n) {
+    if constexpr (PLANAR) {
+        store_bytes_planar(p, (size_t)(dst - p.out) - (size_t)n0, n0, packed, p.n - n0);
+    } else if (aligned16 && n0 + 16 <= p.n) {
         *reinterpret_cast<uint4 *>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
     } else {
         store_bytes_any_alignment(dst, packed, p.n - n0 < 16 ? p.n - n0 : 16);
@@ -297,29 +301,24 @@ int launch_conv_c3k3(const GemmProblem &p, hipStream_t stream) {
     const uint32_t total_bytes = (uint32_t)(in_bytes * images);
     const bool rowsum = p.zw != 0;
     bool fast = p.rq.fast != 0;
+    auto launch_variant = [&](auto launch) {
+        auto with_planar = [&](auto rs, auto f) { p.out_plane ? launch(rs, f, std::true_type{}) : launch(rs, f, std::false_type{}); };
+        auto with_fast = [&](auto rs) { fast ? with_planar(rs, std::true_type{}) : with_planar(rs, std::false_type{}); };
+        rowsum ? with_fast(std::true_type{}) : with_fast(std::false_type{});
+    };
     if (p.n >= 32) {  // the packed rows and the folded bias are padded to whole tiles of channels
         const dim3 grid_m(((p.m + 255) / 256 + 7) / 8 * 8);  // whole multiples of 8: see the kernel's block numbering
-        if (rowsum && fast)
-            hipLaunchKernelGGL((conv_c3k3_mfma_kernel<true, true>), grid_m, dim3(256), 0, stream, p, total_bytes);
-        else if (rowsum)
-            hipLaunchKernelGGL((conv_c3k3_mfma_kernel<true, false>), grid_m, dim3(256), 0, stream, p, total_bytes);
-        else if (fast)
-            hipLaunchKernelGGL((conv_c3k3_mfma_kernel<false, true>), grid_m, dim3(256), 0, stream, p, total_bytes);
-        else
-            hipLaunchKernelGGL((conv_c3k3_mfma_kernel<false, false>), grid_m, dim3(256), 0, stream, p, total_bytes);
+        launch_variant([&](auto rs, auto f, auto pl) {
+            hipLaunchKernelGGL((conv_c3k3_mfma_kernel<decltype(rs)::value, decltype(f)::value, decltype(pl)::value>), grid_m, dim3(256), 0, stream, p, total_bytes);
+        });
         EH_HIP(hipGetLastError());
         return EH_OK;
     }
     const dim3 grid((p.m + 255) / 256, (p.n + 15) / 16);
     if (p.rq.pc_multiplier) fast = false;  // this kernel's per-channel code is the two-step order
-    if (rowsum && fast)
-        hipLaunchKernelGGL((conv_c3k3_kernel<true, true>), grid, dim3(256), 0, stream, p, total_bytes);
-    else if (rowsum)
-        hipLaunchKernelGGL((conv_c3k3_kernel<true, false>), grid, dim3(256), 0, stream, p, total_bytes);
-    else if (fast)
-        hipLaunchKernelGGL((conv_c3k3_kernel<false, true>), grid, dim3(256), 0, stream, p, total_bytes);
-    else
-        hipLaunchKernelGGL((conv_c3k3_kernel<false, false>), grid, dim3(256), 0, stream, p, total_bytes);
+    launch_variant([&](auto rs, auto f, auto pl) {
+        hipLaunchKernelGGL((conv_c3k3_kernel<decltype(rs)::value, decltype(f)::value, decltype(pl)::value>), grid, dim3(256), 0, stream, p, total_bytes);
+    });
     EH_HIP(hipGetLastError());
     return EH_OK;
 }

@@ -43,7 +43,7 @@ __device__ __forceinline__ uint32_t byte_range_mask(int lo, int hi) {
 // The grid is persistent: as many workgroups as the device keeps resident (a multiple of 8); XCD x (workgroups x, x + 8,
 // ...) walks the x-th contiguous eighth of the 32-pixel blocks, so the input rows that neighbouring output rows share are
 // fetched into one L2 only, and a wave requests its next block's bytes before it multiplies the current one.
-template <int KH, bool ROWSUM, bool FAST>
+template <int KH, bool ROWSUM, bool FAST, bool PLANAR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KH <= 7 ? 4 : 3))) void conv_rows_kernel(const GemmProblem p, const uint32_t in_bytes, const int nbw, const int m_blocks) {
     extern __shared__ __align__(16) uint8_t lds_raw[];
     v4i *w_s = reinterpret_cast<v4i *>(lds_raw);  // [nbw][KH][64 lanes]
@@ -255,7 +255,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KH <= 7 ? 4
             if (m_ok && n < p.n) {
                 uint8_t *dst = p.out + out_off + n;
                 const int cnt = p.n - n;
-                if (cnt >= 16 && (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 3) == 0) {
+                if constexpr (PLANAR) {
+                    store_bytes_planar(p, out_off, n, packed, cnt);
+                } else if (cnt >= 16 && (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 3) == 0) {
                     *reinterpret_cast<u32x4_a4 *>(dst) = u32x4_a4{packed[0], packed[1], packed[2], packed[3]};
                 } else {
                     store_bytes_any_alignment(dst, packed, cnt < 16 ? cnt : 16);
@@ -312,19 +314,14 @@ int launch_conv_rows(const GemmProblem &p, hipStream_t stream) {
     };
     auto launch = [&](auto kh_c) {
         constexpr int KH = decltype(kh_c)::value;
-        static std::atomic<int> resident[4][50];
-        if (rowsum && fast)
-            hipLaunchKernelGGL((conv_rows_kernel<KH, true, true>), grid_for(conv_rows_kernel<KH, true, true>, resident[0]), dim3(256), lds, stream, p, total_bytes, nbw,
-                               m_blocks);
-        else if (rowsum)
-            hipLaunchKernelGGL((conv_rows_kernel<KH, true, false>), grid_for(conv_rows_kernel<KH, true, false>, resident[1]), dim3(256), lds, stream, p, total_bytes, nbw,
-                               m_blocks);
-        else if (fast)
-            hipLaunchKernelGGL((conv_rows_kernel<KH, false, true>), grid_for(conv_rows_kernel<KH, false, true>, resident[2]), dim3(256), lds, stream, p, total_bytes, nbw,
-                               m_blocks);
-        else
-            hipLaunchKernelGGL((conv_rows_kernel<KH, false, false>), grid_for(conv_rows_kernel<KH, false, false>, resident[3]), dim3(256), lds, stream, p, total_bytes, nbw,
-                               m_blocks);
+        auto variant = [&](auto rs, auto f, auto pl) {
+            static std::atomic<int> resident[50];
+            auto kernel = conv_rows_kernel<KH, decltype(rs)::value, decltype(f)::value, decltype(pl)::value>;
+            hipLaunchKernelGGL(kernel, grid_for(kernel, resident), dim3(256), lds, stream, p, total_bytes, nbw, m_blocks);
+        };
+        auto with_planar = [&](auto rs, auto f) { p.out_plane ? variant(rs, f, std::true_type{}) : variant(rs, f, std::false_type{}); };
+        auto with_fast = [&](auto rs) { fast ? with_planar(rs, std::true_type{}) : with_planar(rs, std::false_type{}); };
+        rowsum ? with_fast(std::true_type{}) : with_fast(std::false_type{});
     };
     switch (p.rows_kh) {
         case 3: launch(std::integral_constant<int, 3>{}); break;

@@ -265,6 +265,10 @@ __global__ __launch_bounds__(WGM *WGN * 64) void igemm_u8_kernel(const GemmProbl
         } else {
             const uint4 v = *reinterpret_cast<const uint4 *>(src);
             const uint32_t packed[4] = {v.x, v.y, v.z, v.w};
+            if (p.out_plane) {
+                store_bytes_planar(p, pix, n, packed, p.n - n < 16 ? p.n - n : 16);
+                continue;
+            }
             store_bytes_any_alignment(dst, packed, p.n - n < 16 ? p.n - n : 16);
         }
     }

@@ -519,6 +519,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
                             if constexpr (BM == 256 && BN == 256) {  // (no registers to spare for the dword form's copies)
                                 const int cnt = p.n - n < 16 ? p.n - n : 16;
                                 for (int t = 0; t < cnt; ++t) dst[t] = (uint8_t)(packed[t >> 2] >> (8 * (t & 3)));
+                            } else if (p.out_plane) {
+                                store_bytes_planar(p, row_off[i], n, packed, p.n - n < 16 ? p.n - n : 16);
                             } else {
                                 store_bytes_any_alignment(dst, packed, p.n - n < 16 ? p.n - n : 16);
                             }
@@ -678,6 +680,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
         }
         if (aligned16 && n + 16 <= p.n) {
             *reinterpret_cast<uint4 *>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+        } else if (!p.residual && p.out_plane) {
+            store_bytes_planar(p, out_off - n, n, packed, p.n - n < 16 ? p.n - n : 16);
         } else {
             store_bytes_any_alignment(dst, packed, p.n - n < 16 ? p.n - n : 16);
         }

@@ -252,6 +252,9 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
     uint8_t *dst = p.out + f_off;
     if (f_n + 1 < p.n && ((f_n | 3) < p.n) && (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 3) == 0) {
         if ((f_pair & 1) == 0) *reinterpret_cast<uint32_t *>(dst) = two | (other << 16);
+    } else if (!p.residual && p.out_plane) {
+        const uint32_t packed[4] = {two, 0, 0, 0};
+        store_bytes_planar(p, f_off - (size_t)f_n, f_n, packed, p.n - f_n < 2 ? 1 : 2);
     } else {
         dst[0] = (uint8_t)o0;
         if (f_n + 1 < p.n) dst[1] = (uint8_t)o1;

@@ -56,7 +56,7 @@ struct ThinStage {
 __device__ __forceinline__ const GemmProblem &problem_of(const GemmProblem &one) { return one; }
 __device__ __forceinline__ const GemmProblem &problem_of(const GemmBatch &batch) { return batch.p[blockIdx.z]; }
 
-template <int NBU, int KU, bool ROWSUM, int QM, bool RES, bool BATCHED = false>
+template <int NBU, int KU, bool ROWSUM, int QM, bool RES, bool BATCHED = false, bool PLANAR = false>
 __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional_t<BATCHED, GemmBatch, GemmProblem> arg, const int n_blocks,
                                                           const int ksteps, const int nbw, const int row_blocks, const ThinStage stage) {
     // BATCHED: equally shaped problems of one operator (the output phases of a transposed convolution whose kernel is its
@@ -232,6 +232,10 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
         if (!ok || n >= p.n) return;
         uint8_t *dst = p.out + out_off + n;
         const int cnt = p.n - n;
+        if constexpr (PLANAR) {
+            store_bytes_planar(p, out_off, n, packed, cnt);
+            return;
+        }
         if constexpr (RES) {  // out = add(residual, result); the residual tensor is addressed like the output
             const uint8_t *res = p.residual + out_off + n;
             if (wide && (cnt >= 16 || cnt == 8)) {
@@ -421,13 +425,13 @@ int launch_nbu(const GemmProblem *ps, int count, hipStream_t stream) {
                        p.a_offset >= 0 && p.m < (1 << 24) && p.cin < (1 << 24) && p.ldc < (1 << 24) && reach_in < (1l << 32) &&
                        reach_out < (1l << 32);
     }
-    // row sums, the single-shift requantization and the fused residual add are compile-time variants: a launch pays for
+    // row sums, the single-shift requantization, the fused residual add and planar outputs are compile-time variants: a launch pays for
     // none of the code it does not use
-    auto launch = [&](auto rowsum_c, auto qm_c, auto res_c) {
-        constexpr bool RS = decltype(rowsum_c)::value, RES = decltype(res_c)::value;
+    auto launch = [&](auto rowsum_c, auto qm_c, auto res_c, auto planar_c) {
+        constexpr bool RS = decltype(rowsum_c)::value, RES = decltype(res_c)::value, PL = decltype(planar_c)::value;
         constexpr int QM = decltype(qm_c)::value;
-        const void *kernel = count > 1 ? reinterpret_cast<const void *>(direct_gemm_kernel<NBU, KU, RS, QM, false, true>)
-                                       : reinterpret_cast<const void *>(direct_gemm_kernel<NBU, KU, RS, QM, RES, false>);
+        const void *kernel = count > 1 ? reinterpret_cast<const void *>(direct_gemm_kernel<NBU, KU, RS, QM, false, true, PL>)
+                                       : reinterpret_cast<const void *>(direct_gemm_kernel<NBU, KU, RS, QM, RES, false, PL>);
         // The grid is persistent: as many workgroups as the device holds at once with this variant's registers and
         // this launch's LDS (a wave has one pixel block in flight, so the bytes in flight grow with the waves), and
         // at least four per CU.  The answer is kept per KiB of LDS.
@@ -444,17 +448,19 @@ int launch_nbu(const GemmProblem *ps, int count, hipStream_t stream) {
         const int wg_target = 256 * per_cu / (ranges * count) > 8 ? 256 * per_cu / (ranges * count) / 8 * 8 : 8;
         if (row_wgs > wg_target) row_wgs = wg_target;
         if (count > 1)
-            hipLaunchKernelGGL((direct_gemm_kernel<NBU, KU, RS, QM, false, true>), dim3(row_wgs, ranges, count), dim3(256), lds_all, stream, batch, n_blocks,
+            hipLaunchKernelGGL((direct_gemm_kernel<NBU, KU, RS, QM, false, true, PL>), dim3(row_wgs, ranges, count), dim3(256), lds_all, stream, batch, n_blocks,
                                ksteps, nbw, row_blocks, stage);
         else
-            hipLaunchKernelGGL((direct_gemm_kernel<NBU, KU, RS, QM, RES, false>), dim3(row_wgs, ranges), dim3(256), lds_all, stream, p, n_blocks, ksteps, nbw,
+            hipLaunchKernelGGL((direct_gemm_kernel<NBU, KU, RS, QM, RES, false, PL>), dim3(row_wgs, ranges), dim3(256), lds_all, stream, p, n_blocks, ksteps, nbw,
                                row_blocks, stage);
     };
     auto with_res = [&](auto rowsum_c, auto qm_c) {
         if (p.residual)
-            launch(rowsum_c, qm_c, std::true_type{});
+            launch(rowsum_c, qm_c, std::true_type{}, std::false_type{});
+        else if (p.out_plane)
+            launch(rowsum_c, qm_c, std::false_type{}, std::true_type{});
         else
-            launch(rowsum_c, qm_c, std::false_type{});
+            launch(rowsum_c, qm_c, std::false_type{}, std::false_type{});
     };
     auto with_qm = [&](auto rowsum_c) {
         if (pc_fast)

@@ -431,7 +431,16 @@ struct GemmProblem {
     // fused residual add (one-tap and split-reduction kernels only): out = add(residual, result) with `radd`;
     // `residual` is addressed like `out`.  Null: plain convolution.
     const uint8_t *residual;
-    AddDev radd;
+    union {
+        AddDev radd;
+        // Without a residual: planar output.  Pixels per channel plane (0: channels-last), with ldc = 1, so that what a kernel
+        // computes as an output address is the pixel's number over all images (see store_bytes_planar), the tensor's
+        // channels, and the division by out_plane.
+        struct {
+            int32_t out_plane, out_c;
+            uint32_t out_plane_mul, out_plane_shift;
+        };
+    };
     RequantDev rq;
     // A slice of a reduction that several workgroups share (64 x 64 split-reduction tiles, table-driven): `ktab`, `b`
     // and `k_pad` describe the slice, `b_slabs` is the whole reduction's slab count (the distance between the packed
@@ -441,6 +450,27 @@ struct GemmProblem {
     int32_t partial_ld;
     int32_t b_slabs;
 };
+
+// The first `cnt` (1 .. 16) of a pixel's sixteen result bytes, channels n .. n + 15, to a planar tensor.  Lanes hold
+// neighbouring pixels, so every byte store of a wave writes runs of up to 32 bytes of a plane.
+__device__ __forceinline__ void store_bytes_planar(const GemmProblem &p, size_t pixel, int n, const uint32_t (&packed)[4], int cnt) {
+    FastDiv div;
+    div.mul = p.out_plane_mul;
+    div.shift = p.out_plane_shift;
+    const uint32_t img = fastdiv((uint32_t)pixel, div);
+    uint8_t *dst = p.out + (pixel + ((size_t)img * (size_t)(p.out_c - 1) + (size_t)n) * (size_t)p.out_plane);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        uint32_t w = packed[g];
+        // (a loop: sixteen addresses at once would cost the kernels' main path its registers)
+#pragma unroll 1
+        for (int t = 4 * g; t < 4 * g + 4 && t < cnt; ++t) {
+            *dst = (uint8_t)w;
+            w >>= 8;
+            dst += p.out_plane;
+        }
+    }
+}
 
 // Equally shaped problems of one operator that go out as one launch (kernel argument).
 struct GemmBatch {
@@ -602,6 +632,7 @@ int launch_keep_channels(const uint8_t *src, uint8_t *dst, int64_t pixels, int32
 // dst[pixel][g][0 .. cg_to) = src[pixel][g][0 .. cg) followed by cg_to - cg bytes `fill`, for `groups` channel groups per pixel
 int launch_pad_channels(const uint8_t *src, uint8_t *dst, int64_t pixels, int32_t groups, int32_t cg, int32_t cg_to, uint32_t fill,
                         hipStream_t stream);
+int launch_nchw2nhwc_padded(const uint8_t *src, uint8_t *dst, int32_t n, int32_t c, int32_t hw, int32_t c_to, uint32_t fill, hipStream_t stream);
 int launch_nhwc2nchw(const uint8_t *src, uint8_t *dst, int32_t n, int32_t c, int32_t hw, hipStream_t stream);
 
 }  // namespace eh

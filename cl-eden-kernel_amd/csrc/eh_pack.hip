@@ -117,49 +117,62 @@ __global__ __launch_bounds__(256) void keep_channels_kernel(const uint8_t *__res
     }
 }
 
-// Byte-matrix transpose per batch: src [batch][R][S] -> dst [batch][S][R].
-// 64x64 tiles through LDS; 4-byte global accesses when the extents allow.
-constexpr int TT = 64;
-__global__ __launch_bounds__(256) void transpose_u8_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst,
-                                                           int32_t R, int32_t S) {
-    __shared__ __align__(4) uint8_t tile[TT][TT + 4];
-    const size_t batch_off = (size_t)blockIdx.z * R * S;
-    src += batch_off;
-    dst += batch_off;
-    const int r0 = blockIdx.y * TT, s0 = blockIdx.x * TT;
-    const int t = threadIdx.x;
-    const bool src_wide = (S & 3) == 0 && (reinterpret_cast<uintptr_t>(src) & 3) == 0;
-    const bool dst_wide = (R & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 3) == 0;
+// Byte-matrix transpose per batch, any extents: src [batch][R][S] -> dst [batch][S][pitch], columns R .. pitch - 1 of the
+// result holding `fill` (a planar image to pixels whose channels are rounded up; pitch = R: a plain transpose).  Tiles of TR
+// rows x TS columns through LDS.  Latency-bound at the sizes it serves, so every thread requests its four dwords, at byte
+// addresses, before it waits for one (21 channels at 65 x 47, three images, padded to 32: 2.6 us; single bytes where an
+// extent is odd, and the padding as a pass of its own, took 3.7 and 2.5).
+template <int TR, int TS>
+__global__ __launch_bounds__(256) void transpose_u8_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int32_t R, int32_t S, int32_t pitch,
+                                                           uint32_t fill) {
+    static_assert(TR * TS == 4096, "four dwords per thread");
+    __shared__ __align__(4) uint8_t tile[TR][TS + 4];
+    src += (size_t)blockIdx.z * R * S;
+    dst += (size_t)blockIdx.z * pitch * S;
+    const int r0 = blockIdx.y * TR, s0 = blockIdx.x * TS, t = threadIdx.x;
+    constexpr int LOAD_ROWS = 256 / (TS / 4), STORE_COLS = 256 / (TR / 4);
+    const int lr = t / (TS / 4), ls = t % (TS / 4) * 4;
+    uint32_t v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int r = (t >> 4) + 16 * i, s4 = (t & 15) * 4;
-        const int gr = r0 + r, gs = s0 + s4;
-        uint32_t v = 0;
-        if (gr < R) {
-            if (src_wide && gs + 4 <= S) {
-                v = *reinterpret_cast<const uint32_t *>(src + (size_t)gr * S + gs);
-            } else {
-                for (int b = 0; b < 4; ++b)
-                    if (gs + b < S) v |= (uint32_t)src[(size_t)gr * S + gs + b] << (8 * b);
-            }
+        const int gr = r0 + lr + LOAD_ROWS * i, gs = s0 + ls;
+        v[i] = fill * 0x01010101u;
+        if (gr < R && gs + 4 <= S) {
+            v[i] = *reinterpret_cast<const u32_a1 *>(src + (size_t)gr * S + gs);
+        } else if (gr < R) {
+            v[i] = 0;
+            for (int b = 0; gs + b < S; ++b) v[i] |= (uint32_t)src[(size_t)gr * S + gs + b] << (8 * b);
         }
-        *reinterpret_cast<uint32_t *>(&tile[r][s4]) = v;
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint32_t *>(&tile[lr + LOAD_ROWS * i][ls]) = v[i];
     __syncthreads();
+    const int sr = t % (TR / 4) * 4, gr = r0 + sr;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int s = (t >> 4) + 16 * i, r4 = (t & 15) * 4;
-        const int gs = s0 + s, gr = r0 + r4;
-        if (gs >= S || gr >= R) continue;
-        const uint32_t v = (uint32_t)tile[r4][s] | ((uint32_t)tile[r4 + 1][s] << 8) | ((uint32_t)tile[r4 + 2][s] << 16) |
-                           ((uint32_t)tile[r4 + 3][s] << 24);
-        if (dst_wide && gr + 4 <= R) {
-            *reinterpret_cast<uint32_t *>(dst + (size_t)gs * R + gr) = v;
+        const int s = t / (TR / 4) + STORE_COLS * i, gs = s0 + s;
+        if (gs >= S || gr >= pitch) continue;
+        const uint32_t w = (uint32_t)tile[sr][s] | ((uint32_t)tile[sr + 1][s] << 8) | ((uint32_t)tile[sr + 2][s] << 16) | ((uint32_t)tile[sr + 3][s] << 24);
+        uint8_t *d = dst + (size_t)gs * pitch + gr;
+        if (gr + 4 <= pitch) {
+            *reinterpret_cast<u32_a1 *>(d) = w;
         } else {
-            for (int b = 0; b < 4; ++b)
-                if (gr + b < R) dst[(size_t)gs * R + gr + b] = (uint8_t)(v >> (8 * b));
+            for (int b = 0; gr + b < pitch; ++b) d[b] = (uint8_t)(w >> (8 * b));
         }
     }
+}
+
+int launch_transpose_any(const uint8_t *src, uint8_t *dst, int32_t batch, int32_t R, int32_t S, int32_t pitch, uint32_t fill, hipStream_t stream) {
+    if (pitch <= 32) {
+        hipLaunchKernelGGL((transpose_u8_kernel<32, 128>), dim3((S + 127) / 128, 1, batch), dim3(256), 0, stream, src, dst, R, S, pitch, fill);
+    } else if (S <= 32 && (pitch + 127) / 128 <= 65535) {
+        hipLaunchKernelGGL((transpose_u8_kernel<128, 32>), dim3(1, (pitch + 127) / 128, batch), dim3(256), 0, stream, src, dst, R, S, pitch, fill);
+    } else {
+        EH_REQUIRE((pitch + 63) / 64 <= 65535, "transpose: %d rows exceed the grid limit", pitch);
+        hipLaunchKernelGGL((transpose_u8_kernel<64, 64>), dim3((S + 63) / 64, (pitch + 63) / 64, batch), dim3(256), 0, stream, src, dst, R, S, pitch, fill);
+    }
+    EH_HIP(hipGetLastError());
+    return EH_OK;
 }
 
 // The same transpose for extents that are multiples of 4 on both axes (most feature maps): 16 KiB tiles of
@@ -334,10 +347,7 @@ int launch_transpose(const uint8_t *src, uint8_t *dst, int32_t batch, int32_t R,
             return EH_OK;
         }
     }
-    const dim3 grid((S + TT - 1) / TT, (R + TT - 1) / TT, batch);
-    hipLaunchKernelGGL(transpose_u8_kernel, grid, dim3(256), 0, stream, src, dst, R, S);
-    EH_HIP(hipGetLastError());
-    return EH_OK;
+    return launch_transpose_any(src, dst, batch, R, S, R, 0, stream);
 }
 
 }  // namespace
@@ -395,6 +405,13 @@ int launch_fold_bias(const int32_t *bias, const int32_t *colsum, int32_t *folded
 // out[n][hw][c] = in[n][c][hw]
 int launch_nchw2nhwc(const uint8_t *src, uint8_t *dst, int32_t n, int32_t c, int32_t hw, hipStream_t stream) {
     return launch_transpose(src, dst, n, c, hw, stream);
+}
+
+// out[n][hw][c_to] = in[n][c][hw], bytes c .. c_to - 1 of a pixel `fill`
+int launch_nchw2nhwc_padded(const uint8_t *src, uint8_t *dst, int32_t n, int32_t c, int32_t hw, int32_t c_to, uint32_t fill, hipStream_t stream) {
+    if (n <= 0 || c <= 0 || hw <= 0) return EH_OK;
+    EH_REQUIRE(n <= 65535 && c_to >= c, "transpose: batch %d, %d of %d channels", n, c, c_to);
+    return launch_transpose_any(src, dst, n, c, hw, c_to, fill & 0xFFu, stream);
 }
 
 // out[n][c][hw] = in[n][hw][c]
