@@ -98,6 +98,7 @@ EXPORTS = {
     "eh_memset": (C.c_int, [C.c_void_p, C.c_int, C.c_size_t, C.c_void_p]),
     "eh_h2d": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]),
     "eh_d2h": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]),
+    "eh_copy_pinned": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]),
     "eh_d2d": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]),
     "eh_pool_create": (C.c_int, [C.POINTER(C.c_void_p)]),
     "eh_pool_request": (C.c_int, [C.c_void_p, C.c_int, C.c_size_t, C.POINTER(C.c_int32)]),
@@ -110,6 +111,7 @@ EXPORTS = {
     "eh_pool_destroy": (C.c_int, [C.c_void_p]),
     "eh_stream_create": (C.c_int, [C.POINTER(C.c_void_p)]),
     "eh_stream_destroy": (C.c_int, [C.c_void_p]),
+    "eh_stream_idle": (C.c_int, [C.c_void_p, C.POINTER(C.c_int32)]),
     "eh_stream_sync": (C.c_int, [C.c_void_p]),
     "eh_graph_begin": (C.c_int, [C.c_void_p]),
     "eh_graph_end": (C.c_int, [C.c_void_p, C.POINTER(C.c_void_p)]),
@@ -141,6 +143,7 @@ EXPORTS = {
     "eh_deconv2d_u8_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(Requant), C.c_void_p]),
     "eh_deconv2d_u8_destroy": (C.c_int, [C.c_void_p]),
     "eh_event_create": (C.c_int, [C.POINTER(C.c_void_p)]),
+    "eh_event_create_untimed": (C.c_int, [C.POINTER(C.c_void_p)]),
     "eh_event_record": (C.c_int, [C.c_void_p, C.c_void_p]),
     "eh_stream_wait_event": (C.c_int, [C.c_void_p, C.c_void_p]),
     "eh_event_elapsed_ms": (C.c_int, [C.c_void_p, C.c_void_p, C.POINTER(C.c_float)]),

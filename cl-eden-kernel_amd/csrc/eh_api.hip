@@ -979,6 +979,19 @@ int eh_d2d(void *dst, const void *src, size_t bytes, void *stream) {
     return EH_OK;
 }
 
+int eh_copy_pinned(void *dst, const void *src, size_t bytes, void *stream) {
+    if (bytes == 0) return EH_OK;
+    return launch_copy(dst, src, bytes, as_stream(stream));
+}
+
+int eh_stream_idle(void *stream, int32_t *idle) {
+    EH_REQUIRE(idle != nullptr, "null result pointer");
+    const hipError_t e = hipStreamQuery(as_stream(stream));
+    *idle = e == hipSuccess;
+    if (e != hipSuccess && e != hipErrorNotReady) return hip_fail(e, "hipStreamQuery");
+    return EH_OK;
+}
+
 int eh_stream_sync(void *stream) {
     EH_HIP(hipStreamSynchronize(as_stream(stream)));
     return EH_OK;
@@ -1031,6 +1044,14 @@ int eh_event_create(void **event) {
     EH_REQUIRE(event != nullptr, "null result pointer");
     hipEvent_t e;
     EH_HIP(hipEventCreate(&e));
+    *event = e;
+    return EH_OK;
+}
+
+int eh_event_create_untimed(void **event) {
+    EH_REQUIRE(event != nullptr, "null result pointer");
+    hipEvent_t e;
+    EH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     *event = e;
     return EH_OK;
 }

@@ -623,6 +623,7 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
 int launch_pwdw_block(const GemmProblem &pw, const DwProblem &dw, const BlockGeom &g, hipStream_t stream);
 
 // ---------------------------------------------------------------- layout
+int launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream);  // device and pinned host memory
 int launch_nchw2nhwc(const uint8_t *src, uint8_t *dst, int32_t n, int32_t c, int32_t hw, hipStream_t stream);
 // dst[pixel][c * times + d] = src[pixel][c] for d < times; rows of c_to >= c * times bytes (a multiple of 4), the tail
 // filled with repeats of the pixel's last channel

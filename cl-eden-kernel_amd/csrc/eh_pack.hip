@@ -419,4 +419,28 @@ int launch_nhwc2nchw(const uint8_t *src, uint8_t *dst, int32_t n, int32_t c, int
     return launch_transpose(src, dst, n, hw, c, stream);
 }
 
+// ---- copy by the compute units, for transfers between device memory and pinned host memory that are shorter than what a
+// copy engine's start and its hand-over to and from the compute queue take.  One 16-byte request per thread: a transfer
+// over the bus is bound by how much of it is on its way at once.
+namespace {
+__global__ __launch_bounds__(256) void copy_kernel(uint8_t *__restrict__ dst, const uint8_t *__restrict__ src, const uint32_t pieces, const uint32_t bytes) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < pieces)
+        reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    else if (const uint32_t j = pieces * 16u + (i - pieces); j < bytes)
+        dst[j] = src[j];
+}
+}  // namespace
+
+int launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream) {
+    EH_REQUIRE(dst != nullptr && src != nullptr && bytes > 0 && bytes < (1u << 31), "copy: bad argument");
+    const bool wide = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0;
+    const uint32_t pieces = wide ? (uint32_t)(bytes >> 4) : 0u;
+    const uint32_t threads = pieces + ((uint32_t)bytes - pieces * 16u);
+    hipLaunchKernelGGL(copy_kernel, dim3((threads + 255u) / 256u), dim3(256), 0, stream, static_cast<uint8_t *>(dst), static_cast<const uint8_t *>(src), pieces,
+                       (uint32_t)bytes);
+    EH_HIP(hipGetLastError());
+    return EH_OK;
+}
+
 }  // namespace eh

@@ -814,13 +814,55 @@ public:
         return ENN_RET_SUCCESS;
     }
 
+    // One execution whose inputs arrive share by share: write_share(lane, stream) queues lane's part of the list's inputs
+    // in that stream's order, and the lane's operators follow it there, so that the first lane computes while the inputs
+    // of the next are still crossing the bus.  Only for a list cut into lanes that is recorded already and stands as it
+    // was recorded: *ran stays false otherwise, and nothing has been written.
+    template <typename WriteShare>
+    EnnReturn execute_by_lane(UDOperators &operators, WriteShare write_share, bool *ran) {
+        *ran = false;
+        if (!operators || !replay) return ENN_RET_SUCCESS;
+        auto it = recorded_.find(operators.get());
+        if (it == recorded_.end() || it->second.state != State::RECORDED || lane_count(operators) < 2) return ENN_RET_SUCCESS;
+        Recorded &r = it->second;
+        if (!signature(operators, &scratch_signature_) || scratch_signature_ != r.signature) return ENN_RET_SUCCESS;
+        const auto runtime = compute_library_->runtime();
+        const int lanes = lane_count(operators);
+        auto stream_of = [&](int lane) { return lane == 0 ? runtime->mainStream() : runtime->laneStream((size_t)lane - 1); };
+        if (r.lanes.empty()) {
+            for (int lane = 0; lane < lanes; ++lane) {
+                void *graph = record_on(stream_of(lane), [&] { return run_lane(operators, lane); });
+                if (graph == nullptr) {
+                    drop_lane_graphs(r);
+                    return ENN_RET_SUCCESS;
+                }
+                r.lanes.push_back(graph);
+            }
+        }
+        *ran = true;
+        // (after a blocking read, the usual case, there is nothing to wait for, and the record and its wait cost 14 us)
+        int32_t idle = 0;
+        if ((eh_stream_idle(runtime->mainStream(), &idle) != EH_OK || !idle) && fork_lanes(lanes) != ENN_RET_SUCCESS) return ENN_RET_FAILED;
+        EnnReturn result = ENN_RET_SUCCESS;
+        for (int lane = 0; lane < lanes && result == ENN_RET_SUCCESS; ++lane) {
+            result = write_share(lane, lanes, stream_of(lane));
+            if (result == ENN_RET_SUCCESS && eh_graph_launch(r.lanes[(size_t)lane], stream_of(lane)) != EH_OK) {
+                ERROR_PRINT("OperationExecutor: replay failed: %s\n", eh_last_error());
+                result = ENN_RET_FAILED;
+            }
+        }
+        if (join_lanes(lanes) != ENN_RET_SUCCESS) result = ENN_RET_FAILED;
+        if (result == ENN_RET_SUCCESS) ++counters_.replays;
+        return result;
+    }
+
     static constexpr int kBurst = 4;
 
     // Forgets what was recorded for a list (the userdriver calls this when the list is closed, before its operators go).
     void forget(const UDOperators &operators) {
         auto it = recorded_.find(operators.get());
         if (it == recorded_.end()) return;
-        if (it->second.graph || it->second.burst) {
+        if (it->second.any()) {
             compute_library_->synchronize();
             drop_graphs(it->second);
         }
@@ -835,22 +877,28 @@ private:
     struct Recorded {
         std::vector<uint64_t> signature;
         void *graph = nullptr;
-        void *burst = nullptr;  // kBurst executions in one graph
+        void *burst = nullptr;      // kBurst executions in one graph
+        std::vector<void *> lanes;  // one execution, a graph per lane
         State state = State::WARM;
+        bool any() const { return graph || burst || !lanes.empty(); }
     };
 
+    static void drop_lane_graphs(Recorded &r) {
+        for (void *g : r.lanes) eh_graph_destroy(g);
+        r.lanes.clear();
+    }
     static void drop_graphs(Recorded &r) {
+        drop_lane_graphs(r);
         if (r.graph) eh_graph_destroy(r.graph);
         if (r.burst) eh_graph_destroy(r.burst);
         r.graph = r.burst = nullptr;
     }
 
-    // captures `executions` runs of the list into a graph; null when that fails (the capture is always ended)
-    void *record(UDOperators &operators, int executions) {
-        void *stream = compute_library_->runtime()->mainStream();
+    // captures what `enqueue` puts on `stream` into a graph; null when that fails (the capture is always ended)
+    template <typename Enqueue>
+    void *record_on(void *stream, Enqueue enqueue) {
         if (stream == nullptr || eh_graph_begin(stream) != EH_OK) return nullptr;
-        EnnReturn ran = ENN_RET_SUCCESS;
-        for (int i = 0; i < executions && ran == ENN_RET_SUCCESS; ++i) ran = run_in_order(operators, false);
+        const EnnReturn ran = enqueue();
         void *graph = nullptr;
         const int ended = eh_graph_end(stream, &graph);
         if (ran != ENN_RET_SUCCESS || ended != EH_OK || graph == nullptr) {
@@ -858,6 +906,14 @@ private:
             return nullptr;
         }
         return graph;
+    }
+    // `executions` runs of the list
+    void *record(UDOperators &operators, int executions) {
+        return record_on(compute_library_->runtime()->mainStream(), [&] {
+            EnnReturn ran = ENN_RET_SUCCESS;
+            for (int i = 0; i < executions && ran == ENN_RET_SUCCESS; ++i) ran = run_in_order(operators, false);
+            return ran;
+        });
     }
 
     // one execution, or one burst when `wanted` allows; returns the executions done, 0 on failure
@@ -868,7 +924,7 @@ private:
         const bool can_record = signature(operators, &now);
         if (!can_record || now != r.signature || r.state == State::DIRECT_ONLY) {
             const bool changed = now != r.signature;
-            if ((r.graph || r.burst) && changed) {
+            if (r.any() && changed) {
                 // what was recorded is stale; the operators are about to rewrite the arrays it reads
                 compute_library_->synchronize();
                 drop_graphs(r);
@@ -909,34 +965,54 @@ private:
     // capture the lanes become parallel branches of the graph).  A lane's operators are enqueued in one go.
     EnnReturn run_in_order(UDOperators &operators, bool count = true) {
         if (count) ++counters_.direct;
+        const int lanes = lane_count(operators);
+        if (fork_lanes(lanes) != ENN_RET_SUCCESS) return ENN_RET_FAILED;
+        EnnReturn result = ENN_RET_SUCCESS;
+        for (int lane = 0; lane < lanes && result == ENN_RET_SUCCESS; ++lane) result = run_lane(operators, lane);
+        // the lanes are joined also after a failure: a capture must not end with a lane's stream still forked
+        if (join_lanes(lanes) != ENN_RET_SUCCESS) result = ENN_RET_FAILED;
+        return result;
+    }
+
+    static int lane_count(const UDOperators &operators) {
         int lanes = 1;
         for (auto &op : *operators) lanes = std::max(lanes, op->lane() + 1);
+        return lanes;
+    }
+    // the streams of the lanes beyond the first wait for what the main stream holds
+    EnnReturn fork_lanes(int lanes) {
+        if (lanes < 2) return ENN_RET_SUCCESS;
         const auto runtime = compute_library_->runtime();
-        void *main_stream = runtime->mainStream();
-        if (lanes > 1) {
-            void *fork = runtime->event(0);
-            if (fork == nullptr || eh_event_record(fork, main_stream) != EH_OK) return ENN_RET_FAILED;
-            for (int lane = 1; lane < lanes; ++lane)
-                if (runtime->laneStream((size_t)lane - 1) == nullptr || eh_stream_wait_event(runtime->laneStream((size_t)lane - 1), fork) != EH_OK)
-                    return ENN_RET_FAILED;
-        }
+        void *fork = runtime->event(0);
+        if (fork == nullptr || eh_event_record(fork, runtime->mainStream()) != EH_OK) return ENN_RET_FAILED;
+        for (int lane = 1; lane < lanes; ++lane)
+            if (runtime->laneStream((size_t)lane - 1) == nullptr || eh_stream_wait_event(runtime->laneStream((size_t)lane - 1), fork) != EH_OK)
+                return ENN_RET_FAILED;
+        return ENN_RET_SUCCESS;
+    }
+    // ... and the main stream for what they hold
+    EnnReturn join_lanes(int lanes) {
+        const auto runtime = compute_library_->runtime();
         EnnReturn result = ENN_RET_SUCCESS;
-        for (int lane = 0; lane < lanes && result == ENN_RET_SUCCESS; ++lane) {
-            runtime->launchOn(lane == 0 ? nullptr : runtime->laneStream((size_t)lane - 1));
-            for (auto &op : *operators)
-                if (op->lane() == lane && op->execute(nullptr) != ENN_RET_SUCCESS) {
-                    ERROR_PRINT("OperationExecutor: %s failed\n", op->getName().c_str());
-                    result = ENN_RET_FAILED;
-                    break;
-                }
-        }
-        runtime->launchOn(nullptr);
-        // the lanes are joined also after a failure: a capture must not end with a lane's stream still forked
         for (int lane = 1; lane < lanes; ++lane) {
             void *join = runtime->event((size_t)lane);
-            if (join == nullptr || eh_event_record(join, runtime->laneStream((size_t)lane - 1)) != EH_OK || eh_stream_wait_event(main_stream, join) != EH_OK)
+            if (join == nullptr || eh_event_record(join, runtime->laneStream((size_t)lane - 1)) != EH_OK ||
+                eh_stream_wait_event(runtime->mainStream(), join) != EH_OK)
                 result = ENN_RET_FAILED;
         }
+        return result;
+    }
+    EnnReturn run_lane(UDOperators &operators, int lane) {
+        const auto runtime = compute_library_->runtime();
+        EnnReturn result = ENN_RET_SUCCESS;
+        runtime->launchOn(lane == 0 ? nullptr : runtime->laneStream((size_t)lane - 1));
+        for (auto &op : *operators)
+            if (op->lane() == lane && op->execute(nullptr) != ENN_RET_SUCCESS) {
+                ERROR_PRINT("OperationExecutor: %s failed\n", op->getName().c_str());
+                result = ENN_RET_FAILED;
+                break;
+            }
+        runtime->launchOn(nullptr);
         return result;
     }
 

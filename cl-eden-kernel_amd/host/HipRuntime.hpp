@@ -94,7 +94,7 @@ public:
     void *event(size_t index) {
         while (events_.size() <= index) {
             void *e = nullptr;
-            if (eh_event_create(&e) != EH_OK) return nullptr;
+            if (eh_event_create_untimed(&e) != EH_OK) return nullptr;
             events_.push_back(e);
         }
         return events_[index];
@@ -228,29 +228,32 @@ public:
 
     // The source is ordinary pageable memory that the caller may reuse as soon as this returns (the contract of
     // clEnqueueWriteBuffer(blocking = CL_FALSE) is that the caller waits for the event; callers of the reference's
-    // writeData(false) do not, gpu_userdriver.cc:188-220).  Up to kStagedTransfer bytes go through the runtime's pinned
-    // staging area: the host copies them there (1 us for a 150 KB image), the device takes them in stream order, and a
-    // non-blocking write waits for nothing (the pageable copy of that image and its wait: 66 us).  Larger writes let the
-    // driver pin the caller's pages (measured even at 1.2 MB, 150 against 171 us at 4.8 MB) and wait: that
-    // hipMemcpyAsync has read a pageable source by the time it returns is not what the API promises.
+    // writeData(false) do not, gpu_userdriver.cc:188-220).  It goes through the runtime's pinned staging area: the host
+    // copies it there (75 GB/s) and the device takes it in stream order, so that a non-blocking write waits for nothing.
+    // Larger writes go in pieces of kStagedPiece, the host's copy of one beside the device's of the one before, and the
+    // device's copies are kernels: a copy engine moves 52 GB/s against their 45, but its hand-over costs 9 us per piece
+    // (4.8 MB in front of a network: 562 us per execution by the driver's pageable path or the engine, 540 so, and the
+    // host is free 40 us earlier).
     Status writeBuffer(void *dst, const void *src, size_t type_bytes, uint32_t num, bool blocking) {
         std::lock_guard<std::mutex> lock(mutex_);
-        const size_t bytes = type_bytes * (size_t)num;
-        void *staged = bytes <= kStagedTransfer ? stagingLocked(bytes) : nullptr;
-        if (staged) std::memcpy(staged, src, bytes);
-        CHECK_EXPR_RETURN_FAILURE(eh_h2d(dst, staged ? staged : src, bytes, stream_) == EH_OK, "writeBuffer: %s", eh_last_error());
-        return blocking || !staged ? synchronizeLocked() : Status::SUCCESS;
+        const Status st = writeLocked(dst, src, type_bytes * (size_t)num, stream_);
+        if (st != Status::SUCCESS) return st;
+        return blocking ? synchronizeLocked() : Status::SUCCESS;
+    }
+    // a non-blocking write in the order of a lane's stream (or the main one), which its caller joins to the main stream
+    Status writeBufferOn(void *dst, const void *src, size_t bytes, void *stream) {
+        std::lock_guard<std::mutex> lock(mutex_);
+        return writeLocked(dst, src, bytes, stream);
     }
 
-    // A blocking read of up to kStagedTransfer bytes lands in the staging area first (32 KB: 9 us with its wait and the
-    // host's copy, 21 us straight into pageable memory).  A non-blocking one leaves the caller's pages to the driver: the
+    // A blocking read of up to kStagedRead bytes lands in the staging area first.  A non-blocking one leaves the caller's pages to the driver: the
     // copy is complete only after the stream has drained, and the caller must synchronize() before it looks (as with
     // clEnqueueReadBuffer).
     Status readBuffer(void *dst, const void *src, size_t type_bytes, uint32_t num, bool blocking) {
         std::lock_guard<std::mutex> lock(mutex_);
         const size_t bytes = type_bytes * (size_t)num;
-        void *staged = blocking && bytes <= kStagedTransfer ? stagingLocked(bytes) : nullptr;
-        CHECK_EXPR_RETURN_FAILURE(eh_d2h(staged ? staged : dst, src, bytes, stream_) == EH_OK, "readBuffer: %s", eh_last_error());
+        void *staged = blocking && bytes <= kStagedRead ? stagingLocked(bytes) : nullptr;
+        CHECK_EXPR_RETURN_FAILURE((staged ? eh_copy_pinned(staged, src, bytes, stream_) : eh_d2h(dst, src, bytes, stream_)) == EH_OK, "readBuffer: %s", eh_last_error());
         if (!blocking) return Status::SUCCESS;
         const Status st = synchronizeLocked();
         if (st == Status::SUCCESS && staged) std::memcpy(dst, staged, bytes);
@@ -285,12 +288,32 @@ private:
         staging_used_ = 0;
         return Status::SUCCESS;
     }
+    Status writeLocked(void *dst, const void *src, size_t bytes, void *stream) {
+        for (size_t done = 0; done < bytes;) {
+            const size_t piece = bytes - done <= kStagedPiece + kStagedPiece / 2 ? bytes - done : kStagedPiece;
+            char *to = static_cast<char *>(dst) + done;
+            const char *from = static_cast<const char *>(src) + done;
+            void *staged = stagingLocked(piece);
+            if (!staged) {  // (no pinned memory: the driver pins the caller's pages, and has read them once the stream has drained)
+                CHECK_EXPR_RETURN_FAILURE(eh_h2d(to, from, bytes - done, stream) == EH_OK && eh_stream_sync(stream) == EH_OK, "writeBuffer: %s", eh_last_error());
+                return Status::SUCCESS;
+            }
+            std::memcpy(staged, from, piece);
+            CHECK_EXPR_RETURN_FAILURE(eh_copy_pinned(to, staged, piece, stream) == EH_OK, "writeBuffer: %s", eh_last_error());
+            done += piece;
+        }
+        return Status::SUCCESS;
+    }
     // `bytes` of the pinned staging area that no queued copy reads; null without one.  The area fills from the front and
     // is free again whenever the stream has drained, which every blocking transfer brings about.
     void *stagingLocked(size_t bytes) {
         if (!staging_ || bytes == 0) return nullptr;
         const size_t need = alignTo(bytes, 256);
-        if (staging_used_ + need > kStagingBytes && synchronizeLocked() != Status::SUCCESS) return nullptr;
+        if (staging_used_ + need > kStagingBytes) {
+            for (void *s : lane_streams_)  // (writes in a lane's order may not be joined to the main stream yet)
+                if (eh_stream_sync(s) != EH_OK) return nullptr;
+            if (synchronizeLocked() != Status::SUCCESS) return nullptr;
+        }
         void *p = static_cast<char *>(staging_) + staging_used_;
         staging_used_ += need;
         return p;
@@ -339,7 +362,7 @@ private:
     std::map<void *, void *> allocations_;  // user pointer -> hipMalloc base
     std::mutex mutex_;
     void *stream_ = nullptr;
-    static constexpr size_t kStagedTransfer = (size_t)1 << 20, kStagingBytes = (size_t)2 << 20;
+    static constexpr size_t kStagedPiece = (size_t)1 << 19, kStagedRead = (size_t)1 << 20, kStagingBytes = (size_t)8 << 20;
     void *staging_ = nullptr;  // pinned host memory, kStagingBytes
     size_t staging_used_ = 0;
 };

@@ -187,8 +187,11 @@ int eh_memset(void *ptr, int value, size_t bytes, void *stream);
 int eh_h2d(void *dst, const void *src, size_t bytes, void *stream);
 int eh_d2h(void *dst, const void *src, size_t bytes, void *stream);
 int eh_d2d(void *dst, const void *src, size_t bytes, void *stream);
+/* One kernel instead of a copy engine, in stream order; each side is device memory or memory of eh_host_alloc. */
+int eh_copy_pinned(void *dst, const void *src, size_t bytes, void *stream);
 int eh_stream_create(void **stream);                 /* default priority, non-blocking w.r.t. the null stream */
 int eh_stream_destroy(void *stream);
+int eh_stream_idle(void *stream, int32_t *idle);     /* whether everything queued so far is done */
 int eh_stream_sync(void *stream);
 const char *eh_last_error(void);
 
@@ -427,6 +430,7 @@ int eh_deconv2d_u8_destroy(eh_deconv_plan *plan);
  * eh_event_* wrap hipEventCreate / Record / ElapsedTime so that a harness can
  * time the stream the kernels are launched on without linking HIP itself. */
 int eh_event_create(void **event);
+int eh_event_create_untimed(void **event);           /* orders streams only: cheaper to record, eh_event_elapsed_ms refuses it */
 int eh_event_record(void *event, void *stream);
 int eh_event_elapsed_ms(void *start, void *stop, float *ms); /* synchronises on `stop` */
 /* Work enqueued on `stream` after this call waits for what `event` recorded (hipStreamWaitEvent): the way a caller

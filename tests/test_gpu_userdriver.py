@@ -384,3 +384,25 @@ def test_host_transfers_around_the_staging_size(count):
             assert np.array_equal(got, np.minimum(a.astype(int) + b, 255).astype(np.uint8)), rep
     finally:
         d.close_subgraph(list_id)
+
+
+@pytest.mark.parametrize("count", [7, 4099, (5 << 19) + 1], ids=lambda c: "%d_bytes_per_image" % c)
+def test_inputs_written_lane_by_lane(count):
+    """A list in two lanes is handed its inputs share by share from the third execution on: other inputs in every
+    execution, shares that start on odd addresses, and more bytes in one execution than the staging area holds."""
+    d, list_id, images = driver(), 0x7900, 4
+    d.set_image_lanes(2, 1)
+    try:
+        ol = ud.OperatorList(list_id, ud.MODEL_ANDROID_NN)
+        ta, tb, tc = (ol.feature_map(i, (images, 1, 1, count), 0.5, 0) for i in range(3))
+        ol.operator("ADD", ud.OP_ADD, [ta, tb], [tc])
+        d.open_subgraph(ol)
+        rng = np.random.default_rng(count)
+        for rep in range(5):
+            a, b = (rng.integers(0, 140, images * count, dtype=np.uint8) for _ in range(2))
+            got = np.zeros(images * count, np.uint8)
+            d.execute_subgraph(list_id, {0: a, 1: b, 2: got})
+            assert np.array_equal(got, np.minimum(a.astype(int) + b, 255).astype(np.uint8)), rep
+        d.close_subgraph(list_id)
+    finally:
+        d.set_image_lanes(2, 12)
