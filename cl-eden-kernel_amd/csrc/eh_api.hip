@@ -183,18 +183,18 @@ static bool units_are_rows(const std::vector<KUnit> &units, int per_tap, int tap
     return true;
 }
 
-// (a geometry that does not fit its fields is never read: such reductions stay with the table-driven kernels)
+// (problems without whole chunks or without taps get a geometry too, which nothing reads)
 TapGeom tap_geom(int cin, int nx, int dy0, int dys, int dx0, int dxs, int c0) {
     TapGeom t;
-    t.chunks = (uint16_t)(cin / 16 > 0 ? cin / 16 : 1);
-    t.nx = (uint16_t)(nx > 0 ? nx : 1);
-    t.dy0 = (int16_t)dy0;
-    t.dys = (int16_t)dys;
-    t.dx0 = (int16_t)dx0;
-    t.dxs = (int16_t)dxs;
+    t.chunks = cin / 16 > 0 ? cin / 16 : 1;
+    t.nx = nx > 0 ? nx : 1;
+    t.dy0 = dy0;
+    t.dys = dys;
+    t.dx0 = dx0;
+    t.dxs = dxs;
     t.c0 = c0;
-    t.div_chunks = make_fastdiv(t.chunks);
-    t.div_nx = make_fastdiv(t.nx);
+    t.div_chunks = make_fastdiv((uint32_t)t.chunks);
+    t.div_nx = make_fastdiv((uint32_t)t.nx);
     return t;
 }
 

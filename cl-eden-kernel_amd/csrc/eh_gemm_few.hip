@@ -134,8 +134,8 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
             exists[u] = chunk * 16 < p.k;
             int dy = 0, dx = 0, off = chunk * 16;
             if constexpr (TAPS) {
-                const int tap = (int)fastdiv((uint32_t)chunk, p.tap.div_chunks), c = chunk - tap * (int)p.tap.chunks;
-                const int ty = (int)fastdiv((uint32_t)tap, p.tap.div_nx), tx = tap - ty * (int)p.tap.nx;
+                const int tap = (int)fastdiv((uint32_t)chunk, p.tap.div_chunks), c = chunk - tap * p.tap.chunks;
+                const int ty = (int)fastdiv((uint32_t)tap, p.tap.div_nx), tx = tap - ty * p.tap.nx;
                 dy = p.tap.dy0 + ty * p.tap.dys;
                 dx = p.tap.dx0 + tx * p.tap.dxs;
                 off = (dy * p.w + dx) * p.cin + c * 16;

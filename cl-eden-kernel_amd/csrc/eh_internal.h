@@ -393,9 +393,11 @@ struct GemmConfig {
 
 // Where the taps of a reduction over whole 16-byte channel chunks sit: tap t at row dy0 + (t / nx) * dys and column
 // dx0 + (t % nx) * dxs of the output pixel's window, `chunks` chunks per tap from channel c0 on.
+// (32-bit fields hold whatever a plan accepts: 2^24 terms are 2^20 chunks, and a transposed convolution's taps have no limit of
+// their own.)
 struct TapGeom {
-    uint16_t chunks = 1, nx = 1;
-    int16_t dy0 = 0, dys = 0, dx0 = 0, dxs = 0;
+    int32_t chunks = 1, nx = 1;
+    int32_t dy0 = 0, dys = 0, dx0 = 0, dxs = 0;
     int32_t c0 = 0;
     FastDiv div_chunks, div_nx;
 };

@@ -267,6 +267,20 @@ def test_classifier_heads_take_the_kernel_cut_along_the_weights():
     assert "skinny" not in eden.conv_kernels(eden.conv_desc(1, 512, 9, 9, 48, 1, 1, stride=(2, 2), layout=nhwc))
 
 
+def test_descriptor_queries_up_to_the_longest_reduction():
+    """2^20 terms and more per tap, and a kernel row of 2^16 taps and more: the counts a plan derives from them (16-byte
+    chunks per tap, taps per row) are beyond 16 bits, and multiples of 2^16 must not become 0."""
+    nhwc = eden.NHWC
+    for k in (1 << 20, (1 << 20) + 16, 1 << 21, (1 << 24) - 16, 1 << 24):
+        assert eden.conv_kernels(eden.conv_desc(1, k, 1, 1, 32, 1, 1, layout=nhwc)) == ["skinny"]
+        assert len(eden.conv_kernels(eden.conv_desc(200, k >> 4, 1, 1, 32, 1, 1, layout=nhwc))) == 1
+    for kw in (1 << 16, (1 << 16) + 1, 1 << 17):
+        try:
+            eden.conv_kernels(eden.conv_desc(1, 16, 1, 1, 16, 1, kw, layout=nhwc, weight_layout=eden.W_IOHW), deconv=True)
+        except eden.EdenHipError:
+            pass   # (refused is an answer too)
+
+
 def test_descriptor_queries_answer_or_refuse_whatever_the_descriptor():
     """Descriptors drawn from edge values (zero, negative, 2^31 - 1, unknown layouts): the kernel query, which runs the
     plan builder's host side, either answers or refuses with a status, and does so quickly; the stated limits (a

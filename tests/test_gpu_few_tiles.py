@@ -55,6 +55,17 @@ def test_few_tiles_fully_connected(m, k, n, flags):
     assert want.std() > 4
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 1 << 20, 33), (1, (1 << 20) + 16, 33), (17, (1 << 20) + 32, 5)])
+def test_fully_connected_reductions_beyond_2_to_the_20(m, k, n):
+    # (inputs near their zero points: the sums of the oracle and of the kernels stay far inside 32 bits)
+    a, w = synth.fill_u8_normal((m, k), SEED + 31, 120, 6), synth.fill_u8_normal((n, k), SEED + 32, 128, 6)
+    b = synth.fill_i32((n,), SEED + 33, -1000, 1000)
+    q = O.make_quant(0.01, 120, 0.002, 128, 0.01 * 0.002 * 36 * k ** 0.5 / 40, 128)
+    want, got = O.fc(a, w, b, q), gpu_fc(a, w, b, to_eh_requant(q))
+    assert np.array_equal(got, want), diff_report(got, want)
+    assert want.std() > 4
+
+
 @pytest.mark.parametrize("case", [dict(n=1, c=32, h=5, w=6, cout=8, kh=4, kw=4, stride=(2, 2), pad=(1, 1, 1, 1)),     # phases side by side
                                   dict(n=2, c=48, h=7, w=7, cout=10, kh=3, kw=3, stride=(2, 2), pad=(1, 1, 1, 1)),    # phases of unequal taps and pixel counts
                                   dict(n=1, c=64, h=4, w=5, cout=21, kh=8, kw=8, stride=(4, 4), pad=(2, 2, 2, 2))],
