@@ -143,7 +143,7 @@ struct GemmPart {
     int64_t so = 0, sc = 0;   // source weight strides (out channel, in channel)
     int64_t w_base = 0;       // element offset of this part in the source weights
     int32_t bias_base = 0;    // first output channel
-    GemmProblem proto{};      // geometry; pointers and quantization filled per run
+    TapProblem proto{};      // geometry; pointers and quantization filled per run
 
     void release() {
         dev_free(b);
@@ -567,8 +567,8 @@ struct GemmOp {
 
     // One part's kernel argument for channels-last tensors `in` / `out`, with the quantization parameters refold() left in `q`
     // (planar_out: `out` is a planar tensor that the kernels write themselves)
-    GemmProblem problem(const GemmPart &g, const uint8_t *in, uint8_t *out, const uint8_t *residual, const AddDev *radd, bool planar_out = false) const {
-        GemmProblem p = g.proto;
+    TapProblem problem(const GemmPart &g, const uint8_t *in, uint8_t *out, const uint8_t *residual, const AddDev *radd, bool planar_out = false) const {
+        TapProblem p = g.proto;
         p.a = in;
         p.b = g.b;
         p.bias = g.folded;
@@ -576,11 +576,11 @@ struct GemmOp {
         p.out = out + (planar_out ? (size_t)g.bias_base * (size_t)out_hw : (size_t)g.bias_base);
         if (planar_out) {
             p.ldc = 1;
-            p.out_plane = out_hw;
-            p.out_c = cout;
+            p.planar.out_plane = out_hw;
+            p.planar.out_c = cout;
             const FastDiv div = make_fastdiv((uint32_t)out_hw);
-            p.out_plane_mul = div.mul;
-            p.out_plane_shift = div.shift;
+            p.planar.out_plane_mul = div.mul;
+            p.planar.out_plane_shift = div.shift;
         }
         p.zw = zp_w_u8(q) - 128;
         p.out_xor = io_signed ? 0x80808080u : 0u;
@@ -632,17 +632,17 @@ struct GemmOp {
                 return rc;
             in = st_pad;
         }
-        GemmProblem inline_problems[kInlineParts];
-        std::vector<GemmProblem> many;
+        TapProblem inline_problems[kInlineParts];
+        std::vector<TapProblem> many;
         size_t launches = 0;
         for (auto &g : parts) launches += g.slices ? (size_t)g.slices : 1;
         if (launches > (size_t)kInlineParts) many.resize(launches);
-        GemmProblem *const problems = many.empty() ? inline_problems : many.data();
+        TapProblem *const problems = many.empty() ? inline_problems : many.data();
         int filled = 0;
         for (auto &g : parts) {
             EH_REQUIRE((reinterpret_cast<uintptr_t>(in) & (uintptr_t)(g.vec - 1)) == 0,
                        "input pointer is not aligned to %d bytes", g.vec);
-            const GemmProblem whole = problem(g, in, out, fuse ? residual : nullptr, radd, planar_out);
+            const TapProblem whole = problem(g, in, out, fuse ? residual : nullptr, radd, planar_out);
             if (g.slices == 0) {
                 problems[filled++] = whole;
                 continue;
@@ -650,7 +650,7 @@ struct GemmOp {
             // equal runs of slabs, one problem each: its part of the k-table and of every packed row block
             const int slabs = g.k_pad / g.cfg.slab, run = slabs / g.slices;
             for (int s = 0; s < g.slices; ++s) {
-                GemmProblem slice = whole;
+                TapProblem slice = whole;
                 slice.ktab = whole.ktab + (size_t)s * run * (g.cfg.slab / 16);
                 slice.b = whole.b + (size_t)s * run * 1024;
                 slice.b_slabs = slabs;
@@ -1183,7 +1183,7 @@ static int conv_plan_build(eh_conv_plan *pl, const eh_conv_desc *d, hipStream_t 
             u.offset = (u.dy * d->w + u.dx) * pixel_c + g * cig + c;
             units.push_back(u);
         }
-        GemmProblem &p = part.proto;
+        TapProblem &p = part.proto;
         p.m = d->n * ho * wo;
         p.h = d->h;
         p.w = d->w;
@@ -1413,7 +1413,7 @@ int eh_fc_q8_plan(eh_fc_plan **plan, int32_t m, int32_t k, int32_t n, int32_t fl
             u.offset = kk;
             units.push_back(u);
         }
-        GemmProblem &p = part.proto;
+        TapProblem &p = part.proto;
         p.m = m;
         p.h = 1;
         p.w = 1;
@@ -1593,7 +1593,7 @@ static int deconv_plan_build(eh_deconv_plan *pl, const eh_conv_desc *d, hipStrea
                     u.offset = (u.dy * d->w + u.dx) * pixel_c + g * cig + c;
                     units.push_back(u);
                 }
-                GemmProblem &p = part.proto;
+                TapProblem &p = part.proto;
                 p.m = d->n * ho_p * wo_p;
                 p.h = d->h;
                 p.w = d->w;

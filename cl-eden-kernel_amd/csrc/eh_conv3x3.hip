@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
                 if (ok && nb < nb_count && n < p.n) {
                     uint8_t *dst = row + n;
                     if constexpr (PLANAR) {
-                        store_bytes_planar(p, (size_t)(row - p.out), n, packed, p.n - n);
+                        store_bytes_planar(p.out, p.planar, (size_t)(row - p.out), n, packed, p.n - n);
                         continue;
                     }
                     if (wide && n + 16 <= p.n) {
@@ -368,7 +368,7 @@ int launch_nb(const GemmProblem &p, const Conv3Launch &L, size_t lds, hipStream_
         return (int)EH_OK;
     };
     auto launch_g = [&](auto rowsum_c, auto qm_c, auto pc_c, auto g_c, auto split_c) {
-        return p.out_plane ? launch_planar(rowsum_c, qm_c, pc_c, g_c, split_c, std::true_type{}) : launch_planar(rowsum_c, qm_c, pc_c, g_c, split_c, std::false_type{});
+        return p.planar.out_plane ? launch_planar(rowsum_c, qm_c, pc_c, g_c, split_c, std::true_type{}) : launch_planar(rowsum_c, qm_c, pc_c, g_c, split_c, std::false_type{});
     };
     auto launch_pc = [&](auto rowsum_c, auto qm_c, auto pc_c) {
         if constexpr (NB == 2) {

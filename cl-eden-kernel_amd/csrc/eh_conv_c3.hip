@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void conv_c3k3_mfma_kernel(const GemmProblem p
                 uint8_t *dst = p.out + out_off + n;
                 const int cnt = p.n - n;
                 if constexpr (PLANAR) {
-                    store_bytes_planar(p, out_off, n, packed, cnt);
+                    store_bytes_planar(p.out, p.planar, out_off, n, packed, cnt);
                 } else if (cnt >= 16 && (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 3) == 0) {
                     *reinterpret_cast<u32x4_a4 *>(dst) = u32x4_a4{packed[0], packed[1], packed[2], packed[3]};
                 } else {
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256) void conv_c3k3_kernel(const GemmProblem p, con
     uint8_t *dst = p.out + (((size_t)img * p.out_h + (oy * p.out_sy + p.out_y0)) * p.out_w + (ox * p.out_sx + p.out_x0)) * (size_t)p.ldc + n0;
     const bool aligned16 = (p.ldc & 15) == 0 && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
     if constexpr (PLANAR) {
-        store_bytes_planar(p, (size_t)(dst - p.out) - (size_t)n0, n0, packed, p.n - n0);
+        store_bytes_planar(p.out, p.planar, (size_t)(dst - p.out) - (size_t)n0, n0, packed, p.n - n0);
     } else if (aligned16 && n0 + 16 <= p.n) {
         *reinterpret_cast<uint4 *>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
     } else {
@@ -302,7 +302,7 @@ int launch_conv_c3k3(const GemmProblem &p, hipStream_t stream) {
     const bool rowsum = p.zw != 0;
     bool fast = p.rq.fast != 0;
     auto launch_variant = [&](auto launch) {
-        auto with_planar = [&](auto rs, auto f) { p.out_plane ? launch(rs, f, std::true_type{}) : launch(rs, f, std::false_type{}); };
+        auto with_planar = [&](auto rs, auto f) { p.planar.out_plane ? launch(rs, f, std::true_type{}) : launch(rs, f, std::false_type{}); };
         auto with_fast = [&](auto rs) { fast ? with_planar(rs, std::true_type{}) : with_planar(rs, std::false_type{}); };
         rowsum ? with_fast(std::true_type{}) : with_fast(std::false_type{});
     };

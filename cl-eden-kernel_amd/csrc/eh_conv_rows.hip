@@ -256,7 +256,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KH <= 7 ? 4
                 uint8_t *dst = p.out + out_off + n;
                 const int cnt = p.n - n;
                 if constexpr (PLANAR) {
-                    store_bytes_planar(p, out_off, n, packed, cnt);
+                    store_bytes_planar(p.out, p.planar, out_off, n, packed, cnt);
                 } else if (cnt >= 16 && (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 3) == 0) {
                     *reinterpret_cast<u32x4_a4 *>(dst) = u32x4_a4{packed[0], packed[1], packed[2], packed[3]};
                 } else {
@@ -319,7 +319,7 @@ int launch_conv_rows(const GemmProblem &p, hipStream_t stream) {
             auto kernel = conv_rows_kernel<KH, decltype(rs)::value, decltype(f)::value, decltype(pl)::value>;
             hipLaunchKernelGGL(kernel, grid_for(kernel, resident), dim3(256), lds, stream, p, total_bytes, nbw, m_blocks);
         };
-        auto with_planar = [&](auto rs, auto f) { p.out_plane ? variant(rs, f, std::true_type{}) : variant(rs, f, std::false_type{}); };
+        auto with_planar = [&](auto rs, auto f) { p.planar.out_plane ? variant(rs, f, std::true_type{}) : variant(rs, f, std::false_type{}); };
         auto with_fast = [&](auto rs) { fast ? with_planar(rs, std::true_type{}) : with_planar(rs, std::false_type{}); };
         rowsum ? with_fast(std::true_type{}) : with_fast(std::false_type{});
     };

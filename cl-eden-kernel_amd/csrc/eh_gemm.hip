@@ -265,8 +265,8 @@ __global__ __launch_bounds__(WGM *WGN * 64) void igemm_u8_kernel(const GemmProbl
         } else {
             const uint4 v = *reinterpret_cast<const uint4 *>(src);
             const uint32_t packed[4] = {v.x, v.y, v.z, v.w};
-            if (p.out_plane) {
-                store_bytes_planar(p, pix, n, packed, p.n - n < 16 ? p.n - n : 16);
+            if (p.planar.out_plane) {
+                store_bytes_planar(p.out, p.planar, pix, n, packed, p.n - n < 16 ? p.n - n : 16);
                 continue;
             }
             store_bytes_any_alignment(dst, packed, p.n - n < 16 ? p.n - n : 16);
@@ -292,7 +292,7 @@ int launch_tile(const GemmProblem &p, hipStream_t stream) {
 
 int igemm_n_tile(int32_t, int32_t, int32_t) { return 256; }
 
-int launch_igemm(const GemmProblem &p, hipStream_t stream) {
+int launch_igemm(const TapProblem &p, hipStream_t stream) {
     if (p.m <= 0 || p.n <= 0) return EH_OK;
     if (gemm_few_tiles_instead(p)) return launch_gemm_few_tiles(&p, 1, stream);
     if (p.cfg.id == GEMM_THIN) return launch_igemm_thin(&p, 1, stream);
@@ -314,10 +314,10 @@ int launch_igemm(const GemmProblem &p, hipStream_t stream) {
     return launch_tile<64, 64, 2, 2>(p, stream);
 }
 
-int launch_igemm_batch(const GemmProblem *ps, int count, hipStream_t stream) {
+int launch_igemm_batch(const TapProblem *ps, int count, hipStream_t stream) {
     int i = 0;
     while (i < count) {
-        const GemmProblem &p = ps[i];
+        const TapProblem &p = ps[i];
         int run = 1;
         const bool dma = p.cfg.id != GEMM_STAGED && p.cfg.id != GEMM_THIN && p.cfg.id != GEMM_C3K3 && p.cfg.id != GEMM_CONV3X3 && p.cfg.id != GEMM_ROWS && p.cfg.id != GEMM_SKINNY && p.cfg.id != GEMM_FEW_TILES && p.m > 0 && p.n > 0;
         if (dma)

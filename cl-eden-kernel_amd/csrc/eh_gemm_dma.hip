@@ -519,8 +519,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
                             if constexpr (BM == 256 && BN == 256) {  // (no registers to spare for the dword form's copies)
                                 const int cnt = p.n - n < 16 ? p.n - n : 16;
                                 for (int t = 0; t < cnt; ++t) dst[t] = (uint8_t)(packed[t >> 2] >> (8 * (t & 3)));
-                            } else if (p.out_plane) {
-                                store_bytes_planar(p, row_off[i], n, packed, p.n - n < 16 ? p.n - n : 16);
+                            } else if (p.planar.out_plane) {
+                                store_bytes_planar(p.out, p.planar, row_off[i], n, packed, p.n - n < 16 ? p.n - n : 16);
                             } else {
                                 store_bytes_any_alignment(dst, packed, p.n - n < 16 ? p.n - n : 16);
                             }
@@ -680,8 +680,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
         }
         if (aligned16 && n + 16 <= p.n) {
             *reinterpret_cast<uint4 *>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-        } else if (!p.residual && p.out_plane) {
-            store_bytes_planar(p, out_off - n, n, packed, p.n - n < 16 ? p.n - n : 16);
+        } else if (!p.residual && p.planar.out_plane) {
+            store_bytes_planar(p.out, p.planar, out_off - n, n, packed, p.n - n < 16 ? p.n - n : 16);
         } else {
             store_bytes_any_alignment(dst, packed, p.n - n < 16 ? p.n - n : 16);
         }
@@ -689,10 +689,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
 }
 
 template <int BM, int BN, int WGM, int WGN, int WGK, int SLAB, int STAGES>
-int launch_cfg(const GemmProblem *ps, int count, hipStream_t stream) {
+int launch_cfg(const TapProblem *ps, int count, hipStream_t stream) {
     const GemmProblem &p = ps[0];
     GemmBatch batch;
-    for (int i = 0; i < count; ++i) batch.p[i] = ps[i];
+    for (int i = 0; i < count; ++i) static_cast<GemmProblem &>(batch.p[i]) = ps[i];
     static_assert(STAGES * (BM + BN) * SLAB + WGK * 2 * BM * 4 + BN * 4 <= 160 * 1024 - 12288, "LDS budget with the largest k-table");
     int m_max = p.m;  // (table-driven problems of one launch may differ in their row counts: every kernel tests rows against its own problem's)
     for (int i = 1; i < count; ++i) m_max = ps[i].m > m_max ? ps[i].m : m_max;
@@ -853,7 +853,7 @@ GemmConfig igemm_dma_select(int32_t m, int32_t n, int32_t k, int32_t siblings) {
     return c;
 }
 
-int launch_igemm_dma(const GemmProblem *ps, int count, hipStream_t stream) {
+int launch_igemm_dma(const TapProblem *ps, int count, hipStream_t stream) {
     const GemmProblem &p = ps[0];
     EH_REQUIRE(count >= 1 && count <= GemmBatch::MAX, "igemm_dma: batch of %d", count);
     for (int i = 0; i < count; ++i) {

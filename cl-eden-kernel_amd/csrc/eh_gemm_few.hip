@@ -22,8 +22,40 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr int kWaves = 8;
 constexpr int kLanePitch = 20;  // int32 per lane of a partial tile: 16 and a gap that spreads 16-byte accesses over the banks
 
-__device__ __forceinline__ const GemmProblem &problem_of(const GemmProblem &one) { return one; }
-__device__ __forceinline__ const GemmProblem &problem_of(const GemmBatch &batch) { return batch.p[blockIdx.z]; }
+// What this kernel reads of a problem: fields of GemmProblem by the same names, and the taps' geometry.  (3x3 on 256 channels at
+// 14 x 14, one image: 5.35 us with a GemmProblem that held the geometry, 376 bytes; 6.07 at 512 bytes; 5.30 with this one.)
+struct FewProblem {
+    const uint8_t *a;
+    const int8_t *b;
+    const int32_t *bias;
+    uint8_t *out;
+    const uint8_t *residual;
+    int32_t m, n, k, k_pad;
+    int32_t h, w, cin, ho, wo;
+    int32_t stride_h, stride_w, y_base, x_base;
+    FastDiv div_plane, div_wo;
+    TapGeom tap;
+    uint32_t fill, a_xor, out_xor;
+    int32_t zw;
+    int32_t out_h, out_w, out_sy, out_sx, out_y0, out_x0, ldc;
+    union {
+        AddDev radd;
+        PlanarOut planar;
+    };
+    RequantDev rq;
+
+    FewProblem() {}
+    FewProblem(const TapProblem &p)
+        : a(p.a), b(p.b), bias(p.bias), out(p.out), residual(p.residual), m(p.m), n(p.n), k(p.k), k_pad(p.k_pad), h(p.h), w(p.w), cin(p.cin), ho(p.ho), wo(p.wo),
+          stride_h(p.stride_h), stride_w(p.stride_w), y_base(p.y_base), x_base(p.x_base), div_plane(p.div_plane), div_wo(p.div_wo), tap(p.tap), fill(p.fill),
+          a_xor(p.a_xor), out_xor(p.out_xor), zw(p.zw), out_h(p.out_h), out_w(p.out_w), out_sy(p.out_sy), out_sx(p.out_sx), out_y0(p.out_y0), out_x0(p.out_x0),
+          ldc(p.ldc), radd(p.radd), rq(p.rq) {}  // (radd's bytes are `planar` where that is in use)
+};
+struct FewBatch {
+    FewProblem p[GemmBatch::MAX];
+};
+__device__ __forceinline__ const FewProblem &problem_of(const FewProblem &one) { return one; }
+__device__ __forceinline__ const FewProblem &problem_of(const FewBatch &batch) { return batch.p[blockIdx.z]; }
 
 // the value of lane (lane ^ 1) or (lane ^ 2): a permutation inside every four lanes
 template <int X>
@@ -58,9 +90,9 @@ __device__ __forceinline__ void quad_transpose(int &c0, int &c1, int &c2, int &c
 // may lie outside the image (else: one tap inside it).  ROWSUM: the weights' zero point is not 128.  FAST: every
 // requantization pair in use is inside the single-shift form's range.  BATCHED: equally shaped problems along grid z.
 template <int GROUPS, bool TAPS, bool ROWSUM, bool FAST, bool BATCHED>
-__global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::conditional_t<BATCHED, GemmBatch, GemmProblem> arg, const int m_blocks, const int n_blocks,
+__global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::conditional_t<BATCHED, FewBatch, FewProblem> arg, const int m_blocks, const int n_blocks,
                                                                 const int tiles_per_xcd, const int m_fastest) {
-    const GemmProblem &p = problem_of(arg);
+    const FewProblem &p = problem_of(arg);
     __shared__ __align__(16) int32_t part_s[kWaves][64 * kLanePitch];
     __shared__ int32_t sum_s[ROWSUM ? kWaves * 2 : 1][32];
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, half = lane >> 5;
@@ -252,9 +284,9 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
     uint8_t *dst = p.out + f_off;
     if (f_n + 1 < p.n && ((f_n | 3) < p.n) && (p.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 3) == 0) {
         if ((f_pair & 1) == 0) *reinterpret_cast<uint32_t *>(dst) = two | (other << 16);
-    } else if (!p.residual && p.out_plane) {
+    } else if (!p.residual && p.planar.out_plane) {
         const uint32_t packed[4] = {two, 0, 0, 0};
-        store_bytes_planar(p, f_off - (size_t)f_n, f_n, packed, p.n - f_n < 2 ? 1 : 2);
+        store_bytes_planar(p.out, p.planar, f_off - (size_t)f_n, f_n, packed, p.n - f_n < 2 ? 1 : 2);
     } else {
         dst[0] = (uint8_t)o0;
         if (f_n + 1 < p.n) dst[1] = (uint8_t)o1;
@@ -285,8 +317,8 @@ bool gemm_few_tiles_instead(const GemmProblem &p) {
     return p.cfg.id == GEMM_THIN || p.cfg.id == GEMM_CONV3X3;
 }
 
-int launch_gemm_few_tiles(const GemmProblem *ps, int count, hipStream_t stream) {
-    const GemmProblem &p = ps[0];
+int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream) {
+    const TapProblem &p = ps[0];
     EH_REQUIRE(count >= 1 && count <= GemmBatch::MAX, "few_tiles: batch of %d", count);
     int m_max = p.m;
     for (int i = 0; i < count; ++i) {
@@ -308,7 +340,7 @@ int launch_gemm_few_tiles(const GemmProblem *ps, int count, hipStream_t stream) 
     for (int i = 0; i < count; ++i)
         inside = inside && ps[i].tap.chunks * 16 == ps[i].k && ps[i].tap.dy0 == 0 && ps[i].tap.dx0 == 0 && ps[i].y_base == 0 && ps[i].x_base == 0 &&
                  (ps[i].ho - 1) * ps[i].stride_h < ps[i].h && (ps[i].wo - 1) * ps[i].stride_w < ps[i].w;
-    GemmBatch batch;
+    FewBatch batch;
     if (count > 1)
         for (int i = 0; i < count; ++i) batch.p[i] = ps[i];
     auto launch = [&](auto groups_c, auto taps_c, auto rowsum_c, auto fast_c) {
@@ -317,7 +349,7 @@ int launch_gemm_few_tiles(const GemmProblem *ps, int count, hipStream_t stream) 
         if (count > 1)
             hipLaunchKernelGGL((few_tiles_kernel<S, T, R, F, true>), grid, block, 0, stream, batch, m_blocks, n_blocks, per_xcd, m_fastest);
         else
-            hipLaunchKernelGGL((few_tiles_kernel<S, T, R, F, false>), grid, block, 0, stream, p, m_blocks, n_blocks, per_xcd, m_fastest);
+            hipLaunchKernelGGL((few_tiles_kernel<S, T, R, F, false>), grid, block, 0, stream, FewProblem(p), m_blocks, n_blocks, per_xcd, m_fastest);
     };
     auto with_fast = [&](auto groups_c, auto taps_c, auto rowsum_c) {
         if (p.rq.fast != 0)

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
         uint8_t *dst = p.out + out_off + n;
         const int cnt = p.n - n;
         if constexpr (PLANAR) {
-            store_bytes_planar(p, out_off, n, packed, cnt);
+            store_bytes_planar(p.out, p.planar, out_off, n, packed, cnt);
             return;
         }
         if constexpr (RES) {  // out = add(residual, result); the residual tensor is addressed like the output
@@ -385,10 +385,10 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
 }
 
 template <int NBU, int KU>
-int launch_nbu(const GemmProblem *ps, int count, hipStream_t stream) {
+int launch_nbu(const TapProblem *ps, int count, hipStream_t stream) {
     const GemmProblem &p = ps[0];
     GemmBatch batch;
-    for (int i = 0; i < count; ++i) batch.p[i] = ps[i];
+    for (int i = 0; i < count; ++i) static_cast<GemmProblem &>(batch.p[i]) = ps[i];
     const int n_blocks = (p.n + 31) / 32, ksteps = p.k_pad / 32;
     const int row_blocks = (p.m + 31) / 32;
     // Channel ranges: as few as the LDS budget for the weights allows (32 KiB, so that several workgroups share a CU),
@@ -457,7 +457,7 @@ int launch_nbu(const GemmProblem *ps, int count, hipStream_t stream) {
     auto with_res = [&](auto rowsum_c, auto qm_c) {
         if (p.residual)
             launch(rowsum_c, qm_c, std::true_type{}, std::false_type{});
-        else if (p.out_plane)
+        else if (p.planar.out_plane)
             launch(rowsum_c, qm_c, std::false_type{}, std::true_type{});
         else
             launch(rowsum_c, qm_c, std::false_type{}, std::false_type{});
@@ -492,7 +492,7 @@ bool igemm_thin_applies(int32_t taps, int32_t cin_group, int32_t pixel_stride, i
     return cin_group <= 64 || (cin_group <= 256 && m * n * cin_group <= 1500000000ll);
 }
 
-int launch_igemm_thin(const GemmProblem *ps, int count, hipStream_t stream) {
+int launch_igemm_thin(const TapProblem *ps, int count, hipStream_t stream) {
     const GemmProblem &p = ps[0];
     EH_REQUIRE(count >= 1 && count <= GemmBatch::MAX, "igemm_thin: batch of %d", count);
     for (int i = 1; i < count; ++i)

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "eden_hip.h"
@@ -402,6 +403,13 @@ struct TapGeom {
     FastDiv div_chunks, div_nx;
 };
 
+// A planar output: pixels per channel plane (0: channels-last), the tensor's channels, and the division by out_plane.  The
+// problem's ldc is then 1, so that what a kernel computes as an output address is the pixel's number over all images.
+struct PlanarOut {
+    int32_t out_plane, out_c;
+    uint32_t out_plane_mul, out_plane_shift;
+};
+
 struct GemmProblem {
     const uint8_t *a;     // activations: NHWC image or [M][K] matrix
     const int8_t *b;      // packed weights, value = w - 128, laid out for cfg (see packed_b_offset)
@@ -428,39 +436,36 @@ struct GemmProblem {
     // int8 tensors (PrecisionType::INT8) run as their uint8 equivalents (value + 128, zero points + 128):
     uint32_t a_xor;    // turns four stored activation bytes into int8 MFMA operands: 0x80808080 for uint8 data, 0 for int8
     uint32_t out_xor;  // turns four uint8 results into the stored bytes: 0 for uint8 data, 0x80808080 for int8
-    TapGeom tap;       // the kernel for few tiles finds its taps by this
     int32_t rows_kh, rows_kw;  // GEMM_ROWS: the kernel's extent (other kernels find their taps in ktab); GEMM_CONV3X3: output rows per tile, channel blocks per workgroup
+    int32_t *partial;  // see b_slabs
     // fused residual add (one-tap and split-reduction kernels only): out = add(residual, result) with `radd`;
     // `residual` is addressed like `out`.  Null: plain convolution.
     const uint8_t *residual;
     union {
         AddDev radd;
-        // Without a residual: planar output.  Pixels per channel plane (0: channels-last), with ldc = 1, so that what a kernel
-        // computes as an output address is the pixel's number over all images (see store_bytes_planar), the tensor's
-        // channels, and the division by out_plane.
-        struct {
-            int32_t out_plane, out_c;
-            uint32_t out_plane_mul, out_plane_shift;
-        };
+        PlanarOut planar;  // without a residual
     };
     RequantDev rq;
     // A slice of a reduction that several workgroups share (64 x 64 split-reduction tiles, table-driven): `ktab`, `b`
     // and `k_pad` describe the slice, `b_slabs` is the whole reduction's slab count (the distance between the packed
     // weights' row blocks; 0: k_pad / slab), and the tile's int32 sums minus its activation-sum term go to
     // partial[m * partial_ld + n] instead of being requantized (launch_splitk_finish adds the slices up and does that).
-    int32_t *partial;
     int32_t partial_ld;
     int32_t b_slabs;
 };
+// The order above is one of measured layouts: a kernel's first wait is for these fields, and every further 64-byte line that
+// it has to fetch shows on launches of a few microseconds.  Requantization parameters across three lines instead of two cost
+// the few-row kernel 5.66 -> 5.72 us (1 x 4096 x 4096), an argument of 388 bytes instead of 352 cost it 5.65 -> 5.83.
+static_assert(offsetof(GemmProblem, rq) % 64 == 0 && sizeof(GemmProblem) <= 368, "GemmProblem: requantization parameters from a line's start, and room for the launch's own arguments within six lines");
 
 // The first `cnt` (1 .. 16) of a pixel's sixteen result bytes, channels n .. n + 15, to a planar tensor.  Lanes hold
 // neighbouring pixels, so every byte store of a wave writes runs of up to 32 bytes of a plane.
-__device__ __forceinline__ void store_bytes_planar(const GemmProblem &p, size_t pixel, int n, const uint32_t (&packed)[4], int cnt) {
+__device__ __forceinline__ void store_bytes_planar(uint8_t *out, const PlanarOut &p, size_t pixel, int n, const uint32_t (&packed)[4], int cnt) {
     FastDiv div;
     div.mul = p.out_plane_mul;
     div.shift = p.out_plane_shift;
     const uint32_t img = fastdiv((uint32_t)pixel, div);
-    uint8_t *dst = p.out + (pixel + ((size_t)img * (size_t)(p.out_c - 1) + (size_t)n) * (size_t)p.out_plane);
+    uint8_t *dst = out + (pixel + ((size_t)img * (size_t)(p.out_c - 1) + (size_t)n) * (size_t)p.out_plane);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         uint32_t w = packed[g];
@@ -474,18 +479,26 @@ __device__ __forceinline__ void store_bytes_planar(const GemmProblem &p, size_t 
     }
 }
 
+// A problem as the host hands it to the launchers.  Only the kernel for few tiles is given the taps' geometry.
+struct TapProblem : GemmProblem {
+    TapGeom tap;
+};
+
 // Equally shaped problems of one operator that go out as one launch (kernel argument).
 struct GemmBatch {
     static constexpr int MAX = 8;
-    GemmProblem p[MAX];
+    // (whole lines per problem, for the same reason: transposed convolution 4x4 stride 2, 256 -> 128 at 8 x 32 x 32, two
+    // problems: 11.64 us with slots of 376 bytes, 11.52 with 344, 11.45 with 384)
+    struct alignas(128) Slot : GemmProblem {};
+    Slot p[MAX];
 };
-int launch_igemm(const GemmProblem &p, hipStream_t stream);
+int launch_igemm(const TapProblem &p, hipStream_t stream);
 // `count` problems in order; consecutive equally shaped ones that the direct-to-LDS kernels serve share launches
-int launch_igemm_batch(const GemmProblem *ps, int count, hipStream_t stream);
-int launch_igemm_dma(const GemmProblem *ps, int count, hipStream_t stream);  // vec == 16 and a k-table that fits LDS
+int launch_igemm_batch(const TapProblem *ps, int count, hipStream_t stream);
+int launch_igemm_dma(const TapProblem *ps, int count, hipStream_t stream);  // vec == 16 and a k-table that fits LDS
 GemmConfig igemm_dma_select(int32_t m, int32_t n, int32_t k, int32_t siblings);
 inline size_t igemm_dma_ktab_limit() { return 12288; }
-int launch_igemm_thin(const GemmProblem *ps, int count, hipStream_t stream);  // `count` equally shaped problems as one launch
+int launch_igemm_thin(const TapProblem *ps, int count, hipStream_t stream);  // `count` equally shaped problems as one launch
 // p: the whole problem (bias, requantization, output addressing, residual); partial: [slices][p.m][partial_ld] int32
 int launch_splitk_finish(const GemmProblem &p, const int32_t *partial, int32_t partial_ld, int32_t slices, hipStream_t stream);
 int launch_conv_c3k3(const GemmProblem &p, hipStream_t stream);
@@ -497,7 +510,7 @@ int launch_gemm_skinny(const GemmProblem &p, hipStream_t stream);
 // few output tiles (eh_gemm_few.hip): whether a problem whose weights are packed in fragment order should run there, and the launch
 bool gemm_few_tiles_applies(int64_t m, int64_t n, int64_t k, int32_t siblings);
 bool gemm_few_tiles_instead(const GemmProblem &p);  // ... although it was planned for another kernel of the same weight order
-int launch_gemm_few_tiles(const GemmProblem *ps, int count, hipStream_t stream);  // `count` equally shaped problems as one launch
+int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream);  // `count` equally shaped problems as one launch
 // few input channels, a kernel row per reduction step (eh_conv_rows.hip)
 bool conv_rows_applies(int32_t cin_group, int32_t pixel_stride, int32_t kh, int32_t kw);
 int launch_conv_rows(const GemmProblem &p, hipStream_t stream);
