@@ -851,7 +851,10 @@ public:
                 result = ENN_RET_FAILED;
             }
         }
-        if (join_lanes(lanes) != ENN_RET_SUCCESS) result = ENN_RET_FAILED;
+        if (join_lanes(lanes) == ENN_RET_SUCCESS)
+            runtime->lanesJoined();
+        else
+            result = ENN_RET_FAILED;
         if (result == ENN_RET_SUCCESS) ++counters_.replays;
         return result;
     }

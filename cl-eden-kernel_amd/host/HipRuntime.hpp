@@ -52,7 +52,8 @@ public:
     HipRuntime() = default;
     ~HipRuntime() {
         if (staging_) {
-            if (stream_) eh_stream_sync(stream_);  // copies out of the staging area may still be on their way
+            for (void *s : lane_streams_) eh_stream_sync(s);  // copies out of the staging area may still be on their way
+            if (stream_) eh_stream_sync(stream_);
             eh_host_free(staging_);
         }
         for (auto &kv : allocations_) eh_free(kv.second);
@@ -84,6 +85,7 @@ public:
     // Streams for the lanes of an operator list beyond the first (default priority, made on first use), and events to
     // fork them from the main stream and join them to it.
     void *laneStream(size_t lane) {
+        std::lock_guard<std::mutex> lock(mutex_);  // (another thread's transfer may be draining the lanes' streams)
         while (lane_streams_.size() <= lane) {
             void *s = nullptr;
             if (eh_stream_create(&s) != EH_OK) return nullptr;
@@ -240,10 +242,16 @@ public:
         if (st != Status::SUCCESS) return st;
         return blocking ? synchronizeLocked() : Status::SUCCESS;
     }
-    // a non-blocking write in the order of a lane's stream (or the main one), which its caller joins to the main stream
+    // A non-blocking write in the order of a lane's stream (or the main one).  The caller joins the lanes' streams to the main
+    // one and says so with lanesJoined().
     Status writeBufferOn(void *dst, const void *src, size_t bytes, void *stream) {
         std::lock_guard<std::mutex> lock(mutex_);
         return writeLocked(dst, src, bytes, stream);
+    }
+    // Everything queued on the lanes' streams so far runs ahead of what the main stream is given from now on.
+    void lanesJoined() {
+        std::lock_guard<std::mutex> lock(mutex_);
+        lanes_staged_ = false;
     }
 
     // A blocking read of up to kStagedRead bytes lands in the staging area first.  A non-blocking one leaves the caller's pages to the driver: the
@@ -283,7 +291,12 @@ public:
     }
 
 private:
+    // Waits for the main stream, and for the lanes' streams too while copies out of the staging area are queued there that
+    // the main stream does not wait for yet (another thread is between writeBufferOn() and lanesJoined()).
     Status synchronizeLocked() {
+        if (lanes_staged_)
+            for (void *s : lane_streams_) CHECK_EXPR_RETURN_FAILURE(eh_stream_sync(s) == EH_OK, "synchronize: %s", eh_last_error());
+        lanes_staged_ = false;
         CHECK_EXPR_RETURN_FAILURE(eh_stream_sync(stream_) == EH_OK, "synchronize: %s", eh_last_error());
         staging_used_ = 0;
         return Status::SUCCESS;
@@ -299,21 +312,18 @@ private:
                 return Status::SUCCESS;
             }
             std::memcpy(staged, from, piece);
+            lanes_staged_ = lanes_staged_ || stream != stream_;
             CHECK_EXPR_RETURN_FAILURE(eh_copy_pinned(to, staged, piece, stream) == EH_OK, "writeBuffer: %s", eh_last_error());
             done += piece;
         }
         return Status::SUCCESS;
     }
     // `bytes` of the pinned staging area that no queued copy reads; null without one.  The area fills from the front and
-    // is free again whenever the stream has drained, which every blocking transfer brings about.
+    // is free again whenever every stream with a copy out of it has drained, which every blocking transfer brings about.
     void *stagingLocked(size_t bytes) {
         if (!staging_ || bytes == 0) return nullptr;
         const size_t need = alignTo(bytes, 256);
-        if (staging_used_ + need > kStagingBytes) {
-            for (void *s : lane_streams_)  // (writes in a lane's order may not be joined to the main stream yet)
-                if (eh_stream_sync(s) != EH_OK) return nullptr;
-            if (synchronizeLocked() != Status::SUCCESS) return nullptr;
-        }
+        if (staging_used_ + need > kStagingBytes && synchronizeLocked() != Status::SUCCESS) return nullptr;
         void *p = static_cast<char *>(staging_) + staging_used_;
         staging_used_ += need;
         return p;
@@ -365,6 +375,7 @@ private:
     static constexpr size_t kStagedPiece = (size_t)1 << 19, kStagedRead = (size_t)1 << 20, kStagingBytes = (size_t)8 << 20;
     void *staging_ = nullptr;  // pinned host memory, kStagingBytes
     size_t staging_used_ = 0;
+    bool lanes_staged_ = false;  // a lane's stream holds copies out of the staging area that the main stream does not wait for
 };
 
 }  // namespace hip
