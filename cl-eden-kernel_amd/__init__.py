@@ -11,7 +11,6 @@ import numpy as np
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libedenhip.so")
-CALL_PATH = os.path.join(HERE, "_call.so")
 
 EH_OK = 0
 ACT_NONE, ACT_RELU, ACT_RELU1, ACT_RELU6 = 0, 1, 2, 3
@@ -154,20 +153,24 @@ _lib = None
 
 
 def load():
-    """Loads libedenhip.so and types every export, puts the native form of the operator calls (_call.so) on the plan
-    classes; raises if a library or a symbol is missing."""
+    """Loads libedenhip.so and types every export; raises if the library or a symbol is missing.  The native form of the
+    operator calls (the extension module _call, built for one interpreter) takes the ctypes form's place where it is there
+    and loads; without it the calls go through ctypes, with the same results."""
     global _lib, conv_dw_block_run
     if _lib is None:
-        for path in (LIB_PATH, CALL_PATH):
-            if not os.path.exists(path):
-                raise EdenHipError("%s is not built: run `python cl-eden-kernel_amd/build.py`" % path)
+        if not os.path.exists(LIB_PATH):
+            raise EdenHipError("%s is not built: run `python cl-eden-kernel_amd/build.py`" % LIB_PATH)
         lib = C.CDLL(LIB_PATH)
         for name, (res, args) in EXPORTS.items():
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = res, args
-        from . import _call
-        _call.install(C.c_void_p, Requant, AddRequant, check, _Plan, ConvPlan, _conv_dw_block_run_general)
-        conv_dw_block_run = _call.conv_dw_block_run
+        try:
+            from . import _call
+        except ImportError:
+            _call = None
+        if _call is not None:
+            _call.install(C.c_void_p, Requant, AddRequant, check, _Plan, ConvPlan, _conv_dw_block_run_general)
+            conv_dw_block_run = _call.conv_dw_block_run
         _lib = lib
     return _lib
 
@@ -384,7 +387,7 @@ def _conv_dw_block_run_general(pointwise, depthwise, d_in, d_out, q_pointwise, q
                                       rows_per_tile, cols_per_tile, stream))
 
 
-conv_dw_block_run = _conv_dw_block_run_general   # until load() puts the native form in its place
+conv_dw_block_run = _conv_dw_block_run_general   # load() puts the native form in its place
 
 
 class BufferPool:
@@ -435,9 +438,12 @@ class _Plan:
         self._run = getattr(load(), "eh_%s_u8_run" % self._kind)   # looked up once: a call's own cost counts on small layers
         self._entry = C.cast(self._run, C.c_void_p).value
 
-    # `run` itself is native (host/py_call.cpp); this is the form for arguments it does not take
     def _run_general(self, d_in, d_out, q, stream=None):
+        """d_out = operator(d_in)"""
         check(self._run(self.handle, d_in.ptr, d_out.ptr, q, stream))
+
+    # load() puts the native form (host/py_call.cpp) in its place, which hands arguments it does not take to the general one
+    run = _run_general
 
     def repack(self, d_w, d_b, q, stream=None):
         check(getattr(load(), "eh_%s_u8_repack" % self._kind)(self.handle, d_w.ptr, d_b.ptr if d_b else None,
@@ -498,7 +504,7 @@ def _conv_run_static(self, d_in, d_out, q, stream=None):
 
 STATIC_SCRATCH_BYTES = 32 << 20
 ConvPlan.run_static = _conv_run_static
-ConvPlan._run_add_general = _conv_run_add_general
+ConvPlan.run_add = ConvPlan._run_add_general = _conv_run_add_general
 ConvPlan.fuses_add = lambda self: bool(load().eh_conv2d_u8_fuses_add(self.handle))
 
 

@@ -1,6 +1,6 @@
 """Builds libedenhip.so (HIP kernels + the operator-level C ABI, include/eden_hip.h) for gfx950 with hipcc, and
-libedenud.so (the C++ host classes behind the userdriver-level C ABI, include/eden_ud.h) and _call.so (the Python
-binding's operator calls) with g++ against it.
+libedenud.so (the C++ host classes behind the userdriver-level C ABI, include/eden_ud.h) and the extension module _call
+(the Python binding's operator calls, for the running interpreter) with g++ against it.
 Everything is built in-tree; nothing is installed."""
 import os
 import re
@@ -16,7 +16,7 @@ HOST = os.path.join(HERE, "host")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libedenhip.so")
 UD_LIB = os.path.join(HERE, "libedenud.so")
-CALL_LIB = os.path.join(HERE, "_call.so")
+CALL_LIB = os.path.join(HERE, "_call" + sysconfig.get_config_var("EXT_SUFFIX"))  # (the interpreter it is built for is part of its name)
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
@@ -97,8 +97,16 @@ def build_ud_lib():
 
 
 def build_call_lib():
-    """The Python binding's operator calls (host/py_call.cpp), an extension module linked against libedenhip.so."""
-    _run(["g++", "-O2", "-std=c++17", "-Wall", "-fPIC", "-shared", "-I" + os.path.join(ROOT, "include"), "-I" + sysconfig.get_paths()["include"],
+    """The Python binding's operator calls (host/py_call.cpp), an extension module linked against libedenhip.so.  Where the
+    interpreter's headers are not installed there is none, and the binding makes its calls through ctypes."""
+    include = sysconfig.get_paths()["include"]
+    for f in os.listdir(HERE):   # (one without the interpreter in its name would be taken by any of them)
+        if f.startswith("_call.") and f.endswith(".so"):
+            os.remove(os.path.join(HERE, f))
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print("no Python.h in %s: operator calls go through ctypes" % include)
+        return None
+    _run(["g++", "-O2", "-std=c++17", "-Wall", "-fPIC", "-shared", "-I" + os.path.join(ROOT, "include"), "-I" + include,
           os.path.join(HOST, "py_call.cpp"), "-o", CALL_LIB, "-L" + HERE, "-ledenhip", "-Wl,-rpath,$ORIGIN"])
     return CALL_LIB
 

@@ -115,6 +115,44 @@ def test_make_requant_perchannel_matches_per_channel_oracle_multipliers():
         assert (q.multiplier, q.shift) == (0, 0)  # the per-tensor pair is unused in this mode
 
 
+@pytest.mark.parametrize("module", ["missing", "foreign"])
+def test_operator_calls_without_the_native_call_module(module, tmp_path):
+    """libedenhip.so alone serves any interpreter: without the extension module, or with one that does not load, the calls
+    are made through ctypes (here up to the library's own refusal of a null plan)."""
+    import os
+    import subprocess
+    import sys
+    pkg = os.path.dirname(os.path.abspath(eden.__file__))
+    copy = tmp_path / os.path.basename(pkg)
+    copy.mkdir()
+    for f in os.listdir(pkg):
+        if f.endswith(".py") or f == "libedenhip.so":
+            os.symlink(os.path.join(pkg, f), copy / f)
+    os.unlink(copy / "__init__.py")   # (its own place is where it looks for the libraries)
+    (copy / "__init__.py").write_text(open(os.path.join(pkg, "__init__.py")).read())
+    if module == "foreign":
+        (copy / "_call.so").write_bytes(b"not for this interpreter")
+    program = """
+import importlib, sys
+sys.path.insert(0, %r)
+eden = importlib.import_module(%r)
+eden.load()
+plan = eden.ConvPlan.__new__(eden.ConvPlan)
+eden._Plan.__init__(plan)
+class Mem: ptr = None
+q, aq = eden.Requant(), eden.AddRequant()
+for call in (lambda: plan.run(Mem, Mem, q), lambda: plan.run_add(Mem, Mem, Mem, q, aq), lambda: eden.conv_dw_block_run(plan, plan, Mem, Mem, q, q)):
+    try:
+        call()
+    except eden.EdenHipError as e:
+        assert "null" in str(e), e
+    else:
+        raise SystemExit("not refused")
+""" % (str(tmp_path), os.path.basename(pkg))
+    r = subprocess.run([sys.executable, "-c", program], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert r.returncode == 0, r.stdout
+
+
 def test_output_dim_formulas_match_oracle():
     lib = eden.load()
     rng = np.random.default_rng(22)
