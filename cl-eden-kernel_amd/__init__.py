@@ -83,6 +83,8 @@ EXPORTS = {
     "eh_conv2d_u8_run_static": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(Requant), C.c_void_p]),
     "eh_conv2d_u8_kernels": (C.c_int, [C.POINTER(ConvDesc), C.c_void_p, C.c_int32]),
     "eh_deconv2d_u8_kernels": (C.c_int, [C.POINTER(ConvDesc), C.c_void_p, C.c_int32]),
+    "eh_conv2d_u8_launch_kernels": (C.c_int, [C.POINTER(ConvDesc), C.c_void_p, C.c_int32]),
+    "eh_deconv2d_u8_launch_kernels": (C.c_int, [C.POINTER(ConvDesc), C.c_void_p, C.c_int32]),
     "eh_conv2d_u8_set_perchannel": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p]),
     "eh_dwconv2d_u8_set_perchannel": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p]),
     "eh_deconv2d_u8_set_perchannel": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p]),
@@ -278,10 +280,11 @@ def conv_desc(n, c, h, w, cout, kh, kw, stride=(1, 1), pad=(0, 0, 0, 0), dil=(1,
 KERNEL_NAMES = ("staged", "dma_256x128", "dma_128x128", "dma_128x64", "dma_64x64_splitk", "dma_256x256", "one_tap", "c3k3", "conv3x3_patch", "few_channel_rows", "skinny", "few_tiles")
 
 
-def conv_kernels(desc, deconv=False):
-    """Kernel family (a KERNEL_NAMES entry) per part of a convolution / deconvolution plan made from `desc`; no GPU."""
+def conv_kernels(desc, deconv=False, launched=False):
+    """Kernel family (a KERNEL_NAMES entry) per part of a convolution / deconvolution plan made from `desc`: the one it is
+    planned for, or the one a run launches; no GPU."""
     ids = (C.c_int32 * 64)()
-    fn = load().eh_deconv2d_u8_kernels if deconv else load().eh_conv2d_u8_kernels
+    fn = getattr(load(), "eh_%s2d_u8_%skernels" % ("deconv" if deconv else "conv", "launch_" if launched else ""))
     count = fn(C.byref(desc), ids, 64)
     if count < 0:
         check(count)

@@ -1228,12 +1228,27 @@ static int conv_desc_checked(const eh_conv_desc *desc, eh_conv_desc *plain) {
     return EH_OK;
 }
 
-static int report_kernels(const GemmOp &op, int32_t *kernel_ids, int32_t cap) {
-    for (size_t i = 0; i < op.parts.size() && (int32_t)i < cap; ++i) kernel_ids[i] = op.parts[i].cfg.id;
-    return (int)op.parts.size();
+// launched: the kernels that a run's launches take (see igemm_next_launch), instead of those the parts are planned for
+static int report_kernels(const GemmOp &op, int32_t *kernel_ids, int32_t cap, bool launched) {
+    std::vector<int32_t> ids;
+    for (auto &g : op.parts) ids.push_back(g.cfg.id);
+    for (size_t i = 0; launched && i < op.parts.size();) {
+        std::vector<TapProblem> problems;  // (a sliced part is launched by itself, by the kernel it is planned for)
+        while (i + problems.size() < op.parts.size() && op.parts[i + problems.size()].slices == 0)
+            problems.push_back(op.problem(op.parts[i + problems.size()], nullptr, nullptr, nullptr, nullptr));
+        for (size_t j = 0; j < problems.size();) {
+            int32_t id;
+            const int run = igemm_next_launch(problems.data() + j, (int)(problems.size() - j), &id);
+            std::fill(ids.begin() + (long)(i + j), ids.begin() + (long)(i + j) + run, id);
+            j += (size_t)run;
+        }
+        i += problems.size() + 1;
+    }
+    for (size_t i = 0; i < ids.size() && (int32_t)i < cap; ++i) kernel_ids[i] = ids[i];
+    return (int)ids.size();
 }
 
-int eh_conv2d_u8_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap) {
+static int conv_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap, bool launched) {
     EH_REQUIRE(kernel_ids != nullptr || cap == 0, "null result array");
     eh_conv_desc plain;
     int rc = conv_desc_checked(desc, &plain);
@@ -1244,8 +1259,11 @@ int eh_conv2d_u8_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t 
     g_dry_run = true;
     rc = conv_plan_build(&pl, &plain, nullptr);
     g_dry_run = false;
-    return rc ? rc : report_kernels(pl.op, kernel_ids, cap);
+    return rc ? rc : report_kernels(pl.op, kernel_ids, cap, launched);
 }
+
+int eh_conv2d_u8_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap) { return conv_kernels(desc, kernel_ids, cap, false); }
+int eh_conv2d_u8_launch_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap) { return conv_kernels(desc, kernel_ids, cap, true); }
 
 int eh_conv2d_u8_plan(eh_conv_plan **plan, const eh_conv_desc *desc, const void *weight, const void *bias,
                       const eh_requant *q, void *stream) {
@@ -1641,7 +1659,7 @@ static int deconv_desc_checked(const eh_conv_desc *desc, eh_conv_desc *plain) {
     return EH_OK;
 }
 
-int eh_deconv2d_u8_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap) {
+static int deconv_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap, bool launched) {
     EH_REQUIRE(kernel_ids != nullptr || cap == 0, "null result array");
     eh_conv_desc plain;
     int rc = deconv_desc_checked(desc, &plain);
@@ -1652,8 +1670,11 @@ int eh_deconv2d_u8_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_
     g_dry_run = true;
     rc = deconv_plan_build(&pl, &plain, nullptr);
     g_dry_run = false;
-    return rc ? rc : report_kernels(pl.op, kernel_ids, cap);
+    return rc ? rc : report_kernels(pl.op, kernel_ids, cap, launched);
 }
+
+int eh_deconv2d_u8_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap) { return deconv_kernels(desc, kernel_ids, cap, false); }
+int eh_deconv2d_u8_launch_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap) { return deconv_kernels(desc, kernel_ids, cap, true); }
 
 int eh_deconv2d_u8_plan(eh_deconv_plan **plan, const eh_conv_desc *desc, const void *weight, const void *bias,
                         const eh_requant *q, void *stream) {

@@ -292,18 +292,9 @@ int launch_tile(const GemmProblem &p, hipStream_t stream) {
 
 int igemm_n_tile(int32_t, int32_t, int32_t) { return 256; }
 
-int launch_igemm(const TapProblem &p, hipStream_t stream) {
-    if (p.m <= 0 || p.n <= 0) return EH_OK;
-    if (gemm_few_tiles_instead(p)) return launch_gemm_few_tiles(&p, 1, stream);
-    if (p.cfg.id == GEMM_THIN) return launch_igemm_thin(&p, 1, stream);
-    if (p.cfg.id == GEMM_C3K3) return launch_conv_c3k3(p, stream);
-    if (p.cfg.id == GEMM_CONV3X3) return launch_conv3x3_patch(p, stream);
-    if (p.cfg.id == GEMM_ROWS) return launch_conv_rows(p, stream);
-    if (p.cfg.id == GEMM_SKINNY) return launch_gemm_skinny(p, stream);
-    if (p.cfg.id == GEMM_FEW_TILES) return launch_gemm_few_tiles(&p, 1, stream);
+static int launch_staged(const GemmProblem &p, hipStream_t stream) {
     EH_REQUIRE(p.k_pad % BK == 0 && p.k_pad > 0, "igemm: padded reduction length %d is not a multiple of %d", p.k_pad, BK);
     EH_REQUIRE(p.vec == 16 || p.vec == 4 || p.vec == 1, "igemm: bad load unit %d", p.vec);
-    if (p.cfg.id != GEMM_STAGED) return launch_igemm_dma(&p, 1, stream);
     // Pick the largest tile that still spreads the problem over the 256 CUs.
     const long tiles128 = (long)((p.m + 127) / 128) * ((p.n + 127) / 128);
     const long tiles64 = (long)((p.m + 63) / 64) * ((p.n + 63) / 64);
@@ -314,46 +305,55 @@ int launch_igemm(const TapProblem &p, hipStream_t stream) {
     return launch_tile<64, 64, 2, 2>(p, stream);
 }
 
+static bool is_dma(int32_t id) {
+    return id == GEMM_DMA_256x256 || id == GEMM_DMA_256x128 || id == GEMM_DMA_128x128 || id == GEMM_DMA_128x64 || id == GEMM_DMA_64x64_SPLITK;
+}
+
+int igemm_next_launch(const TapProblem *ps, int count, int32_t *kernel_id) {
+    const TapProblem &p = ps[0];
+    *kernel_id = p.cfg.id;
+    int run = 1;
+    if (p.m <= 0 || p.n <= 0) return run;
+    if (is_dma(p.cfg.id))
+        // (row counts may differ where nothing depends on them: table-driven problems; the launch covers the largest)
+        while (run < count && run < GemmBatch::MAX && ps[run].cfg.id == p.cfg.id && (ps[run].m == p.m || (!p.dense && !p.partial)) && ps[run].n == p.n &&
+               ps[run].k_pad == p.k_pad && ps[run].dense == p.dense && ps[run].zw == p.zw)
+            ++run;
+    // ... and so do equally shaped one-tap problems (the phases of a transposed convolution whose kernel is its stride,
+    // the groups of a grouped 1x1 convolution)
+    if (p.cfg.id == GEMM_THIN && p.residual == nullptr)
+        while (run < count && run < GemmBatch::MAX && ps[run].cfg.id == GEMM_THIN && ps[run].residual == nullptr && ps[run].m == p.m && ps[run].n == p.n &&
+               ps[run].k == p.k && ps[run].k_pad == p.k_pad && ps[run].cin == p.cin && ps[run].ldc == p.ldc && ps[run].zw == p.zw && ps[run].ho == p.ho &&
+               ps[run].wo == p.wo && ps[run].h == p.h && ps[run].w == p.w && ps[run].stride_h == p.stride_h && ps[run].stride_w == p.stride_w &&
+               ps[run].out_sy == p.out_sy && ps[run].out_sx == p.out_sx && ps[run].out_h == p.out_h && ps[run].out_w == p.out_w &&
+               ps[run].y_base == p.y_base && ps[run].x_base == p.x_base && ps[run].rq.fast == p.rq.fast &&
+               (ps[run].rq.pc_multiplier != nullptr) == (p.rq.pc_multiplier != nullptr))
+            ++run;
+    // ... and so do the problems with few tiles, whose row counts may differ
+    if (p.cfg.id == GEMM_FEW_TILES && p.residual == nullptr)
+        while (run < count && run < GemmBatch::MAX && ps[run].cfg.id == GEMM_FEW_TILES && ps[run].residual == nullptr && ps[run].n == p.n &&
+               ps[run].k_pad == p.k_pad && ps[run].zw == p.zw && ps[run].rq.fast == p.rq.fast)
+            ++run;
+    if (run == 1 && gemm_few_tiles_instead(p)) *kernel_id = GEMM_FEW_TILES;
+    return run;
+}
+
 int launch_igemm_batch(const TapProblem *ps, int count, hipStream_t stream) {
-    int i = 0;
-    while (i < count) {
+    for (int i = 0; i < count;) {
         const TapProblem &p = ps[i];
-        int run = 1;
-        const bool dma = p.cfg.id != GEMM_STAGED && p.cfg.id != GEMM_THIN && p.cfg.id != GEMM_C3K3 && p.cfg.id != GEMM_CONV3X3 && p.cfg.id != GEMM_ROWS && p.cfg.id != GEMM_SKINNY && p.cfg.id != GEMM_FEW_TILES && p.m > 0 && p.n > 0;
-        if (dma)
-            // (row counts may differ where nothing depends on them: table-driven problems; the launch covers the largest)
-            while (i + run < count && run < GemmBatch::MAX && ps[i + run].cfg.id == p.cfg.id && (ps[i + run].m == p.m || (!p.dense && !p.partial)) &&
-                   ps[i + run].n == p.n && ps[i + run].k_pad == p.k_pad && ps[i + run].dense == p.dense && ps[i + run].zw == p.zw)
-                ++run;
-        // ... and so do equally shaped one-tap problems (the phases of a transposed convolution whose kernel is its stride,
-        // the groups of a grouped 1x1 convolution)
-        const bool thin = p.cfg.id == GEMM_THIN && p.m > 0 && p.n > 0 && p.residual == nullptr;
-        if (thin)
-            while (i + run < count && run < GemmBatch::MAX && ps[i + run].cfg.id == GEMM_THIN && ps[i + run].residual == nullptr &&
-                   ps[i + run].m == p.m && ps[i + run].n == p.n && ps[i + run].k == p.k && ps[i + run].k_pad == p.k_pad && ps[i + run].cin == p.cin &&
-                   ps[i + run].ldc == p.ldc && ps[i + run].zw == p.zw && ps[i + run].ho == p.ho && ps[i + run].wo == p.wo && ps[i + run].h == p.h &&
-                   ps[i + run].w == p.w && ps[i + run].stride_h == p.stride_h && ps[i + run].stride_w == p.stride_w && ps[i + run].out_sy == p.out_sy &&
-                   ps[i + run].out_sx == p.out_sx && ps[i + run].out_h == p.out_h && ps[i + run].out_w == p.out_w &&
-                   ps[i + run].y_base == p.y_base && ps[i + run].x_base == p.x_base &&
-                   ps[i + run].rq.fast == p.rq.fast && (ps[i + run].rq.pc_multiplier != nullptr) == (p.rq.pc_multiplier != nullptr))
-                ++run;
-        // ... and so do the problems with few tiles, whose row counts may differ
-        const bool few = p.cfg.id == GEMM_FEW_TILES && p.m > 0 && p.n > 0 && p.residual == nullptr;
-        if (few)
-            while (i + run < count && run < GemmBatch::MAX && ps[i + run].cfg.id == GEMM_FEW_TILES && ps[i + run].residual == nullptr && ps[i + run].n == p.n &&
-                   ps[i + run].k_pad == p.k_pad && ps[i + run].zw == p.zw && ps[i + run].rq.fast == p.rq.fast)
-                ++run;
-        int rc;
-        if (few && run > 1) {
-            rc = launch_gemm_few_tiles(ps + i, run, stream);
-        } else if (thin && run > 1) {
-            rc = launch_igemm_thin(ps + i, run, stream);
-        } else if (dma && run > 1) {
-            EH_REQUIRE(p.k_pad % 64 == 0 && p.k_pad > 0, "igemm: padded reduction length %d", p.k_pad);
-            rc = launch_igemm_dma(ps + i, run, stream);
-        } else {
-            rc = launch_igemm(p, stream);
-        }
+        int32_t id;
+        const int run = igemm_next_launch(ps + i, count - i, &id);
+        int rc = EH_OK;
+        if (p.m > 0 && p.n > 0) switch (id) {
+                case GEMM_FEW_TILES: rc = launch_gemm_few_tiles(ps + i, run, stream); break;
+                case GEMM_THIN: rc = launch_igemm_thin(ps + i, run, stream); break;
+                case GEMM_C3K3: rc = launch_conv_c3k3(p, stream); break;
+                case GEMM_CONV3X3: rc = launch_conv3x3_patch(p, stream); break;
+                case GEMM_ROWS: rc = launch_conv_rows(p, stream); break;
+                case GEMM_SKINNY: rc = launch_gemm_skinny(p, stream); break;
+                case GEMM_STAGED: rc = launch_staged(p, stream); break;
+                default: rc = launch_igemm_dma(ps + i, run, stream);
+            }
         if (rc) return rc;
         i += run;
     }

@@ -857,7 +857,7 @@ int launch_igemm_dma(const TapProblem *ps, int count, hipStream_t stream) {
     const GemmProblem &p = ps[0];
     EH_REQUIRE(count >= 1 && count <= GemmBatch::MAX, "igemm_dma: batch of %d", count);
     for (int i = 0; i < count; ++i) {
-        EH_REQUIRE(ps[i].vec == 16 && ps[i].k_pad % ps[i].cfg.slab == 0, "igemm_dma: unsupported problem");
+        EH_REQUIRE(ps[i].vec == 16 && ps[i].k_pad > 0 && ps[i].k_pad % ps[i].cfg.slab == 0, "igemm_dma: unsupported problem");
         EH_REQUIRE(ps[i].cfg.id == p.cfg.id && (ps[i].m == p.m || (!p.dense && !p.partial)) && ps[i].n == p.n && ps[i].k_pad == p.k_pad &&
                        ps[i].dense == p.dense && ps[i].zw == p.zw,
                    "igemm_dma: a batch must hold equally shaped problems");

@@ -492,8 +492,9 @@ struct GemmBatch {
     struct alignas(128) Slot : GemmProblem {};
     Slot p[MAX];
 };
-int launch_igemm(const TapProblem &p, hipStream_t stream);
-// `count` problems in order; consecutive equally shaped ones that the direct-to-LDS kernels serve share launches
+// How many of the `count` >= 1 problems from ps[0] on go out as one launch, and the kernel that it takes.
+int igemm_next_launch(const TapProblem *ps, int count, int32_t *kernel_id);
+// `count` problems in order; consecutive equally shaped ones share launches
 int launch_igemm_batch(const TapProblem *ps, int count, hipStream_t stream);
 int launch_igemm_dma(const TapProblem *ps, int count, hipStream_t stream);  // vec == 16 and a k-table that fits LDS
 GemmConfig igemm_dma_select(int32_t m, int32_t n, int32_t k, int32_t siblings);

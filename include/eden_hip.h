@@ -303,7 +303,9 @@ int eh_conv2d_u8_plan(eh_conv_plan **plan, const eh_conv_desc *desc, const void 
 /* Which kernel family a plan made from `desc` would run, one eh_kernel_id per part (convolution group;
  * deconvolution output phase and group), without a GPU: the choice CLConvolution::initialize makes among its
  * implementations (gpu/operators/CLConvolution.cpp:139-218).  Writes at most `cap` ids, returns the number of
- * parts or a negative eh_status. */
+ * parts or a negative eh_status.  *_kernels name the kernel a part is planned, and its weights are laid out, for;
+ * *_launch_kernels the one that a run launches: parts of few output tiles go to EH_KERNEL_FEW_TILES, which reads the
+ * same weight order as the one-tap, the 3x3 patch and the few-row kernel, where that is the faster one. */
 typedef enum eh_kernel_id {
     EH_KERNEL_STAGED = 0,         /* register-staged implicit GEMM, any channel count               */
     EH_KERNEL_DMA_256x128 = 1,    /* direct-to-LDS implicit GEMM tiles                              */
@@ -320,6 +322,8 @@ typedef enum eh_kernel_id {
 } eh_kernel_id;
 int eh_conv2d_u8_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap);
 int eh_deconv2d_u8_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap);
+int eh_conv2d_u8_launch_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap);
+int eh_deconv2d_u8_launch_kernels(const eh_conv_desc *desc, int32_t *kernel_ids, int32_t cap);
 /* Per-channel mode (conv_per_channel_quantized, gpu/operators/cl_kernels/ConvolutionKernels.cpp:1317-1375):
  * `count` == cout host arrays of multipliers and shifts replace the requant's single pair on every
  * following run; two null pointers return to per-tensor mode.  Copies synchronously. */

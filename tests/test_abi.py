@@ -319,6 +319,32 @@ def test_descriptor_queries_up_to_the_longest_reduction():
             pass   # (refused is an answer too)
 
 
+def test_launch_query_names_the_kernel_that_runs():
+    """Plans for the one-tap, the 3x3 patch and the few-row kernel that have few output tiles are launched on the kernel for
+    few tiles; the launch query says so, on both sides of each rule."""
+    nhwc = eden.NHWC
+    launched = lambda *a, deconv=False, **kw: eden.conv_kernels(eden.conv_desc(*a, layout=nhwc, **kw), deconv=deconv, launched=True)
+    # 3x3 patch plans: 4 x 62 = 248 tiles of 32 pixels x 32 channels, 4 x 66 = 264
+    same = dict(pad=(1, 1, 1, 1))
+    assert launched(1, 64, 48, 41, 128, 3, 3, **same) == ["few_tiles"]
+    assert launched(1, 64, 48, 44, 128, 3, 3, **same) == ["conv3x3_patch"]
+    # one tap: 256 tiles, 272; 24 channels a pixel are not read in 16-byte chunks
+    assert launched(1, 64, 16, 32, 512, 1, 1) == ["few_tiles"]
+    assert launched(1, 64, 16, 33, 512, 1, 1) == ["one_tap"]
+    assert launched(2, 24, 14, 14, 144, 1, 1) == ["one_tap"]
+    # few rows: up to 16 stay with the kernel that is cut along the weights
+    assert launched(16, 4096, 1, 1, 4096, 1, 1) == ["skinny"]
+    assert launched(17, 4096, 1, 1, 4096, 1, 1) == ["few_tiles"]
+    # parts that share a launch stay together: phases of a transposed convolution, groups; a single one goes by itself
+    assert launched(1, 16, 6, 6, 32, 2, 2, stride=(2, 2), weight_layout=eden.W_IOHW, deconv=True) == ["one_tap"] * 4
+    assert launched(1, 64, 14, 14, 64, 1, 1, groups=2) == ["one_tap"] * 2
+    assert launched(1, 64, 14, 14, 64, 1, 1) == ["few_tiles"]
+    assert launched(1, 144, 14, 14, 144, 1, 1, groups=9) == ["one_tap"] * 8 + ["few_tiles"]
+    # the others run what they are planned for
+    for a, kw in (((1, 3, 64, 64, 32, 3, 3), {}), ((64, 256, 14, 14, 256, 3, 3), same), ((8, 512, 7, 7, 4096, 7, 7), {}), ((1, 256, 14, 14, 256, 3, 3), same)):
+        assert launched(*a, **kw) == eden.conv_kernels(eden.conv_desc(*a, layout=nhwc, **kw))
+
+
 def test_descriptor_queries_answer_or_refuse_whatever_the_descriptor():
     """Descriptors drawn from edge values (zero, negative, 2^31 - 1, unknown layouts): the kernel query, which runs the
     plan builder's host side, either answers or refuses with a status, and does so quickly; the stated limits (a
