@@ -301,7 +301,10 @@ static long few_tiles_count(int64_t m, int64_t n) { return (long)(((m + 31) / 32
 // tiles, in us: 3x3 on 256 channels at 14 x 14, images 1 / 4 / 8 (56 / 200 / 392 tiles) 9.3 / 9.1 / 9.1 -> 5.3 / 5.4 / 8.9; on
 // 512 channels at 7 x 7, 1 / 16 images (32 / 400 tiles) 13.1 / 13.4 -> 7.1 / 12.5; fully connected 100 x 4096 x 1000 (128
 // tiles) 9.8 -> 6.6, 1364 x 640 x 192 (258) 5.8 -> 4.8, 64 x 4096 x 4096 (256) 10.4 -> 7.4; deconvolution 4x4 stride 2
-// 256 -> 128 at 16 x 16, one image (128 in four phases) 7.3 -> 5.0.  (Reductions beyond 8 KiB were not measured.)
+// 256 -> 128 at 16 x 16, one image (128 in four phases) 7.3 -> 5.0.  Beyond 8 KiB, where a wave's loads no longer travel together,
+// the tiles win or lose by their number: 3x3 on 1024 channels at 7 x 7, one image (64 tiles, 9 KiB) 14.3 -> 11.1, fully connected
+// 100 x 9216 x 1000 (128) 15.0 -> 10.0, but 128 x 16384 x 4096 (512) 24.7 -> 31.7, 200 x 65536 x 256 (56) 37.3 -> 49.9 and 3x3 on
+// 1024 at 14 x 14, eight images (392, 9 KiB) 21.1 -> 21.0; such plans keep the tiles.
 bool gemm_few_tiles_applies(int64_t m, int64_t n, int64_t k, int32_t siblings) {
     return m > 0 && few_tiles_count(m, n) * siblings <= 512 && k <= 8192;
 }
@@ -309,11 +312,14 @@ bool gemm_few_tiles_applies(int64_t m, int64_t n, int64_t k, int32_t siblings) {
 // The one-tap, few-row and 3x3 patch kernels keep their weights in the same order, so that the choice can be made at the
 // launch.  Up to one round of tiles this kernel is the faster one: 3x3 on 128 channels at 28 x 28, one image (100 tiles)
 // 6.1 -> 4.6, on 64 at 28 x 28, four images (196) 4.7 -> 4.1, but eight (392) 4.7 -> 4.9; one tap 256 -> 64 at 14 x 14, eight
-// images (98) 5.6 -> 4.0, 96 -> 576 (882) 4.3 -> 6.3; fully connected 64 x 1280 x 1000 7.3 -> 4.6, 64 x 3456 x 184 11.2 -> 6.0,
-// 32 x 4096 x 4096 8.1 -> 7.1, while 16 x 4096 x 4096 takes 6.6 on the few-row kernel and 6.9 here.
+// images (98) 5.6 -> 4.0, 96 -> 576 (882) 4.3 -> 6.3; fully connected 64 x 1280 x 1000 7.3 -> 4.6, 64 x 3456 x 184 11.2 -> 6.0.
+// The few-row kernel fetches a row's activations once per lane and step, which costs by the row, this one 32 rows' whether they
+// exist or not.  Few rows -> here, us at 1000 channels: 32 x 4096 7.3 -> 6.4, 17 x 4096 6.1 -> 6.4, 16 x 4096 6.0 -> 6.3, 16 x 8192
+// 9.1 -> 9.1, 16 x 9216 10.5 -> 9.6, 12 x 9216 9.7 -> 9.7, 10 x 9216 9.2 -> 9.6, 1 x 9216 8.5 -> 9.6; 12 x 25088 20.9 -> 20.7,
+// 10 x 25088 19.9 -> 20.7, 1 x 25088 17.6 -> 20.7; 12 x 65536 50.3 -> 48.3, 10 x 65536 46.7 -> 48.0.
 bool gemm_few_tiles_instead(const GemmProblem &p) {
     if (p.vec != 16 || (reinterpret_cast<uintptr_t>(p.a) & 15) != 0 || few_tiles_count(p.m, p.n) > 256) return false;
-    if (p.cfg.id == GEMM_SKINNY) return p.m > 16 || p.k > 8192;
+    if (p.cfg.id == GEMM_SKINNY) return p.m > 16 || (p.m > 10 && p.k > 8192);
     return p.cfg.id == GEMM_THIN || p.cfg.id == GEMM_CONV3X3;
 }
 

@@ -1,6 +1,8 @@
-// One-tap problems (fully connected layers, 1x1 convolutions) on at most 16 rows of activations and a reduction longer
-// than the one-tap kernel's: batch-1 ... batch-16 classifier heads (17 to 64 rows take the kernel for few tiles).  Such a launch is the weights' one trip from memory
-// and nothing else, so the work is cut along the WEIGHTS: a workgroup of eight waves owns 32 output channels, its waves
+// One-tap problems (fully connected layers, 1x1 convolutions) on few rows of activations and a reduction longer than the
+// one-tap kernel's: classifier heads at batch 1 to 16 (to 10 beyond 8192 terms).  Plans of up to 64 rows are made for this
+// kernel, whose weight order the kernel for few tiles shares; that one is launched for the others wherever it has at most 256
+// tiles (gemm_few_tiles_instead), which leaves this one up to 32 rows of more than 8192 channels.  Such a launch is the
+// weights' one trip from memory and nothing else, so the work is cut along the WEIGHTS: a workgroup of eight waves owns 32 output channels, its waves
 // take the 32-byte reduction steps round-robin, and a step's weight fragment is one contiguous KiB of the packed weights
 // (MFMA fragment order, as for the one-tap kernel), fetched by one 16-byte-per-lane load straight into the registers the
 // matrix instruction reads, eight such loads in flight per wave.  The activations (a few rows, shared by every
@@ -161,9 +163,9 @@ __global__ __launch_bounds__(kWaves * 64) void skinny_gemm_kernel(const GemmProb
 
 // One tap at the pixel itself over rows of whole 16-byte chunks, at most 64 output pixels, which the problem addresses as a
 // plain matrix (pixel m reads at m * pixel_stride + channel_offset and writes at m * ldc), and a reduction beyond the
-// one-tap kernel's.  Every workgroup reads all of the activations: beyond 32 rows that pays only while the channels are
-// too few for the tiled kernels to spread (measured at 64 rows: 1280 -> 1000 channels 6.5 against 7.5 us, 4096 -> 4096
-// 11.4 against 7.7 us).
+// one-tap kernel's.  From 17 rows on the launch goes to the kernel for few tiles (above), which such a plan's weights serve
+// as well, at any length of the reduction: beyond 32 rows this holds up to 2048 channels, where it always has its 256 tiles or
+// fewer, and wider layers are planned by the rules of the tiled kernels.
 bool gemm_skinny_applies(int32_t taps, int32_t cin_group, int32_t pixel_stride, int32_t channel_offset, int64_t m, int64_t n) {
     if (!(taps == 1 && m >= 1 && m <= 64 && cin_group > 256 && (cin_group & 15) == 0 && (pixel_stride & 15) == 0 && (channel_offset & 15) == 0)) return false;
     return m <= 32 || n <= 2048;

@@ -335,6 +335,17 @@ def test_launch_query_names_the_kernel_that_runs():
     # few rows: up to 16 stay with the kernel that is cut along the weights
     assert launched(16, 4096, 1, 1, 4096, 1, 1) == ["skinny"]
     assert launched(17, 4096, 1, 1, 4096, 1, 1) == ["few_tiles"]
+    # ... and up to 10 whatever the reduction; from 11 on only 8192 terms
+    assert launched(1, 25088, 1, 1, 4096, 1, 1) == ["skinny"]
+    assert launched(10, 9216, 1, 1, 4096, 1, 1) == ["skinny"]
+    assert launched(11, 9216, 1, 1, 4096, 1, 1) == ["few_tiles"]
+    assert launched(11, 8192, 1, 1, 4096, 1, 1) == ["skinny"]
+    assert launched(1, 8208, 1, 1, 10, 1, 1) == ["skinny"]
+    # more than 256 tiles: back to the planned kernel, which takes 32 rows; beyond those a plan has at most 128 tiles
+    assert launched(32, 512, 1, 1, 8192, 1, 1) == ["few_tiles"]
+    assert launched(32, 512, 1, 1, 8224, 1, 1) == ["skinny"]
+    assert launched(64, 512, 1, 1, 2048, 1, 1) == ["few_tiles"]
+    assert launched(33, 512, 1, 1, 8224, 1, 1) != ["skinny"]
     # parts that share a launch stay together: phases of a transposed convolution, groups; a single one goes by itself
     assert launched(1, 16, 6, 6, 32, 2, 2, stride=(2, 2), weight_layout=eden.W_IOHW, deconv=True) == ["one_tap"] * 4
     assert launched(1, 64, 14, 14, 64, 1, 1, groups=2) == ["one_tap"] * 2

@@ -55,7 +55,7 @@ def test_few_tiles_fully_connected(m, k, n, flags):
     assert want.std() > 4
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 1 << 20, 33), (1, (1 << 20) + 16, 33), (17, (1 << 20) + 32, 5)])
+@pytest.mark.parametrize("m,k,n", [(1, 1 << 20, 33), (1, (1 << 20) + 16, 33), (11, (1 << 20) + 16, 33), (17, (1 << 20) + 32, 5)])
 def test_fully_connected_reductions_beyond_2_to_the_20(m, k, n):
     # (inputs near their zero points: the sums of the oracle and of the kernels stay far inside 32 bits)
     a, w = synth.fill_u8_normal((m, k), SEED + 31, 120, 6), synth.fill_u8_normal((n, k), SEED + 32, 128, 6)
