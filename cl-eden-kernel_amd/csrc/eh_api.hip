@@ -532,13 +532,20 @@ struct GemmOp {
         return fuse;
     }
 
-    // residual != null: output = add(residual, result) with `radd`; `fused` tells whether the kernels did it
     // Whether the plan's kernels write a planar output themselves, instead of a channels-last image that a transposition
-    // then reads (a launch and two trips of the output: 64 channels at 56x56, four images 10.8 -> 8.0 us; 16 -> 96 at
-    // 112x112, 32 images 31 -> 23).  Every epilogue that holds sixteen channels of a pixel per lane has the form, but for
-    // the largest tiles (no registers to spare) and the second launches of sliced reductions; the tiled kernels, whose
-    // workgroups all finish at once, write bytes slower than the transposition moves them from some 6 MB on (128 channels
-    // at 56x56, 32 images, 12.8 MB: 44 -> 48 us; 256 at 28x28, 8 images, 1.6 MB: 18.8 -> 15.6).
+    // then reads (a launch and two trips of the output).  Every epilogue that holds sixteen channels of a pixel per lane has
+    // the form, but for the largest tiles (no registers to spare) and the second launches of sliced reductions.  Transposed ->
+    // written, us, whole runs, over 16 .. 512 output channels, planes of 7x7 .. 224x224 and 1 .. 64 images:
+    //   kernels that finish wave by wave gain at every size, some 3 us on small outputs, and at worst break even:
+    //     one tap      64 -> 256 at 56x56, 4 / 64 images (3.2 / 51 MB) 11.8 -> 9.5 / 47.3 -> 40.7; 64 -> 256 at 112x112, 64 images (206 MB) 185 -> 115
+    //     3x3 patch    64 -> 96 at 56x56, 4 images (1.2 MB) 11.7 -> 8.7; 64 -> 16 at 112x112, 64 images (13 MB) 70.1 -> 70.8, 64 -> 256, 16 images (51 MB)
+    //                  80.4 -> 80.8, 64 images (206 MB) 324 -> 284
+    //     first layers 3 -> 64 at 224x224 stride 2, 64 images (51 MB) 3x3 45.9 -> 38.4, 7x7 59.3 -> 54.4
+    //     few tiles    5x5, 64 -> 256 at 28x28, 1 image 10.4 -> 7.7
+    //   the tiled kernels, whose workgroups finish together, gain while the output is small (128x128 tiles: 5x5, 64 -> 256 at 14x14, 64 images,
+    //   3.2 MB 21.0 -> 19.1; 256 -> 512 at 56x56, 4 images, 6.4 MB 17.5 -> 14.2) and lose on 256x128 tiles beyond (256 -> 256 at 56x56, 16 images,
+    //   12.8 MB 30.3 -> 37.6; 5x5, 64 -> 96 at 112x112, 16 images, 19 MB 94 -> 110); at the line those tiles go both ways
+    //   (20 images at 56x56, 6.0 MB: 5x5, 64 -> 96 33.2 -> 31.6, 256 -> 96 23.6 -> 26.0)
     bool stores_planar() const {
         bool all = layout == EH_NCHW && (int64_t)in_n * out_hw < (1ll << 31);
         const bool small = (int64_t)in_n * out_hw * cout <= (6ll << 20);
@@ -600,6 +607,7 @@ struct GemmOp {
         return p;
     }
 
+    // residual != null: output = add(residual, result) with `radd`; `fused` tells whether the kernels did it
     // staging != null: the plan uses [staging, staging + staging_bytes()) instead of its own images
     int run(const void *input, void *output, const eh_requant *nq, hipStream_t stream, const uint8_t *residual = nullptr,
             const AddDev *radd = nullptr, bool *fused = nullptr, uint8_t *staging = nullptr) {
