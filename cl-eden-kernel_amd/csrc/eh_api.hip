@@ -1582,6 +1582,8 @@ static int deconv_plan_build(eh_deconv_plan *pl, const eh_conv_desc *d, hipStrea
                 const int count = (int)(last - first);
                 first = last;
                 const int px = x0.px, ox0 = x0.ox0, wo_p = x0.wo_p, ntx = x0.ntx, bx = x0.bx;
+                // (the taps' positions are 16-bit in the tables)
+                EH_REQUIRE(by < 32000 && nty - by < 32000 && bx < 32000 && ntx - bx < 32000, "kernel extent or padding too large");
                 op.parts.emplace_back();
                 GemmPart &part = op.parts.back();
                 part.n = cog * count;

@@ -312,11 +312,13 @@ def test_descriptor_queries_up_to_the_longest_reduction():
     for k in (1 << 20, (1 << 20) + 16, 1 << 21, (1 << 24) - 16, 1 << 24):
         assert eden.conv_kernels(eden.conv_desc(1, k, 1, 1, 32, 1, 1, layout=nhwc)) == ["skinny"]
         assert len(eden.conv_kernels(eden.conv_desc(200, k >> 4, 1, 1, 32, 1, 1, layout=nhwc))) == 1
-    for kw in (1 << 16, (1 << 16) + 1, 1 << 17):
-        try:
-            eden.conv_kernels(eden.conv_desc(1, 16, 1, 1, 16, 1, kw, layout=nhwc, weight_layout=eden.W_IOHW), deconv=True)
-        except eden.EdenHipError:
-            pass   # (refused is an answer too)
+    # positions beyond the tables' 16 bits are refused: by the kernel's extent or by a padding that moves it
+    deconv = lambda kw, stride=1, left=0, right=0: eden.conv_kernels(
+        eden.conv_desc(1, 16, 1, 1, 16, 1, kw, stride=(1, stride), pad=(0, 0, left, right), layout=nhwc, weight_layout=eden.W_IOHW), deconv=True)
+    for args in ((1 << 15,), ((1 << 15) + 1,), (1 << 16,), ((1 << 16) + 1,), (1 << 17,), (3, 1, 40000, -40000)):
+        with pytest.raises(eden.EdenHipError, match="too large"):
+            deconv(*args)
+    assert len(deconv(31000)) == 1 and len(deconv(1 << 15, 2)) == 1 and len(deconv(3, 1, 31000, -31000)) == 1
 
 
 def test_launch_query_names_the_kernel_that_runs():
