@@ -50,3 +50,54 @@ def test_matrix_depthwise_two_step_requantization(k, scale):
     got = gpu_dwconv(x, wt, b, s, to_eh_requant(q), layout=eden.NHWC)
     assert np.array_equal(got, want), diff_report(got, want)
     assert want.std() > 4
+
+
+@pytest.mark.parametrize("quant", ["u8pc", "s8", "s8pc"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(str(v) for v in c[:6]))
+def test_matrix_depthwise_per_channel_and_int8(case, quant):
+    n, c, h, w, k, stride, pad = case
+    s = O.conv_shape(n, c, h, w, c, k, k, stride=(stride, stride), pad=pad)
+    signed, pc = quant.startswith("s8"), quant.endswith("pc")
+    x = synth.fill_u8((n, c, h, w), SEED + 41)
+    if signed:
+        x = (x.astype(np.int16) - 128).astype(np.int8)
+    wt = (synth.fill_u8((c, 1, k, k), SEED + 42).astype(np.int16) - 128).astype(np.int8)   # the whole range, -128 among it
+    b = synth.fill_i32((c,), SEED + 43, -1000, 1000)
+    desc = eden.conv_desc(n, c, h, w, c, k, k, (stride,) * 2, pad, (1, 1), 1, 1, eden.NHWC | (eden.IO_SIGNED if signed else 0), eden.W_OIHW | eden.W_SIGNED)
+    d_x, d_w, d_b = eden.DeviceBuffer(host=np.ascontiguousarray(x.transpose(0, 2, 3, 1))), eden.DeviceBuffer(host=wt), eden.DeviceBuffer(host=b)
+    d_o = eden.DeviceBuffer(nbytes=int(np.prod(O.conv_out_hw(s))) * n * c)
+
+    def compare(plan, q, want):
+        plan.run(d_x, d_o, q)
+        got = d_o.download((n, want.shape[2], want.shape[3], c)).transpose(0, 3, 1, 2).view(want.dtype)
+        assert np.array_equal(got, want), diff_report(got, want)
+        assert want.std() > 4
+
+    if not pc:
+        # weights about zero points at the ends of int8 too: differences of up to 255
+        for zp_w, spread in ((3, 74), (-128, 147), (127, 147)):
+            oq = O.make_quant_s8(0.02, -14, 0.005, zp_w, 0.02 * 0.005 * 74 * spread * k / 40, -3)
+            q = to_eh_requant(oq)
+            compare(eden.DwConvPlan(desc, d_w, d_b, q), q, O.dwconv2d_s8(x, wt, b, s, oq))
+        return
+    zp_in, zp_out = (-14, 5) if signed else (93, 131)
+    scales = (0.002 * (1.0 + 9.0 * synth.fill_u8((c,), SEED + 44) / 255.0)).astype(np.float32)
+    q, mults, shifts = eden.make_requant_perchannel(0.02, zp_in, scales, float(0.02 * 0.02 * 74 * 74 * k / 60), zp_out)
+    oq = O.raw_quant(zp_in=zp_in, zp_w=0, zp_out=zp_out)
+    if signed:
+        q.act_min, q.act_max = oq.act_min, oq.act_max = -128, 127
+    oracle = lambda sh: O.dwconv2d_s8(x, wt, b, s, oq, mults, sh) if signed else O.dwconv2d_perchannel(x, wt, b, s, oq, mults, sh)
+    plan = eden.DwConvPlan(desc, d_w, d_b, q)
+    plan.set_perchannel(mults, shifts)
+    compare(plan, q, oracle(shifts))
+    # one channel's shift outside the single-shift form's range: the whole launch takes the two-step order
+    odd = shifts.copy()
+    odd[c // 3] = 0
+    plan.set_perchannel(mults, odd)
+    compare(plan, q, oracle(odd))
+    # the clamp's floor at the output zero point: the single-shift form without its sign test
+    q.act_min = oq.act_min = zp_out
+    plan.set_perchannel(mults, shifts)
+    plan.run(d_x, d_o, q)
+    want = oracle(shifts)
+    assert np.array_equal(d_o.download((n, want.shape[2], want.shape[3], c)).transpose(0, 3, 1, 2).view(want.dtype), want)

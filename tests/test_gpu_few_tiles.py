@@ -19,7 +19,7 @@ CASES = [
     dict(n=1, c=272, h=6, w=6, cout=64, kh=1, kw=1, stride=(2, 2), pad=(1, 1, 1, 1)),      # a tap that leaves the image
     dict(n=2, c=64, h=10, w=10, cout=64, kh=3, kw=3, pad=(1, 1, 1, 1), groups=4),          # channel groups
     dict(n=1, c=21, h=9, w=8, cout=21, kh=3, kw=3, pad=(1, 1, 1, 1)),                      # on the channel-padded copy
-    dict(n=1, c=64, h=16, w=31, cout=512, kh=1, kw=1),                                     # one tile short of the largest launch of a one-tap plan
+    dict(n=1, c=64, h=16, w=31, cout=512, kh=1, kw=1),                                     # 256 tiles, the largest launch of a one-tap plan
 ]
 
 
@@ -101,3 +101,22 @@ def test_few_tiles_residual_add_and_per_channel(cout):
     assert np.array_equal(d_o.download(conv.shape), conv)
     plan.run_add(d_x, d_r, d_o, q, to_eh_add(aq))
     assert np.array_equal(d_o.download(conv.shape), O.add(res, conv, aq))
+
+
+def test_the_cases_above_run_on_the_kernel_for_few_tiles():
+    for case in CASES:
+        s = O.conv_shape(**case)
+        for layout in (eden.NHWC, eden.NCHW):
+            desc = eden.conv_desc(s.n, s.c, s.h, s.w, s.cout, s.kh, s.kw, (s.stride_h, s.stride_w), (s.pad_t, s.pad_b, s.pad_l, s.pad_r), (s.dil_h, s.dil_w), s.groups,
+                                  layout=layout)
+            assert set(eden.conv_kernels(desc, launched=True)) == {"few_tiles"}, (case, eden.conv_kernels(desc, launched=True))
+    rows = [(17, 272, 10), (31, 4096, 65), (33, 512, 31), (64, 3456, 184), (257, 640, 30), (100, 8192, 34), (11, (1 << 20) + 16, 33), (17, (1 << 20) + 32, 5)]
+    for m, k, n in rows:
+        assert eden.conv_kernels(eden.conv_desc(m, k, 1, 1, n, 1, 1, layout=eden.NHWC), launched=True) == ["few_tiles"], (m, k, n)
+    for m, k, n in ((1, 1 << 20, 33), (1, (1 << 20) + 16, 33)):
+        assert eden.conv_kernels(eden.conv_desc(m, k, 1, 1, n, 1, 1, layout=eden.NHWC), launched=True) == ["skinny"], (m, k, n)
+    for c, h, w, cout, k, st, pad, n in ((32, 5, 6, 8, 4, 2, 1, 1), (48, 7, 7, 10, 3, 2, 1, 2), (64, 4, 5, 21, 8, 4, 2, 1)):
+        desc = eden.conv_desc(n, c, h, w, cout, k, k, (st, st), (pad,) * 4, layout=eden.NHWC, weight_layout=eden.W_IOHW)
+        assert set(eden.conv_kernels(desc, deconv=True, launched=True)) == {"few_tiles"}, (c, cout, k)
+    for cout in (160, 34, 5):
+        assert eden.conv_kernels(eden.conv_desc(2, 320, 7, 7, cout, 1, 1, layout=eden.NHWC), launched=True) == ["few_tiles"]
