@@ -178,7 +178,8 @@ private:
 
     // Whether the list's inputs can be handed over lane by lane: as they are, and at least one of them at all.  (A list cut
     // into lanes gains at every size: two linear graphs also start sooner than one with branches, MobileNetV2 on 24 images
-    // of 96 x 96 387 -> 300 us, 24 of 160 x 160 425 -> 366, 32 of 224 x 224 562 -> 530.)
+    // of 96 x 96 400 -> 276 us, 24 of 160 x 160 451 -> 342, 32 of 224 x 224 577 -> 493, as a planar list with per-channel
+    // weights 604 -> 518; the same list executed in turn with others, on inputs that are not in the host's caches, 625 -> 618.)
     static bool inputs_go_by_lane(const UDTensors &in_tensors, const BufferTable &buffer_table) {
         bool any = false;
         for (const auto &in : in_tensors) {
