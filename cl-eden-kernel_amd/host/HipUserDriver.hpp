@@ -48,6 +48,16 @@ public:
 
     EnnReturn OpenSubGraph(const OperatorListDesc &operator_list) {
         std::lock_guard<std::mutex> lock_guard(mutex_constructor);
+        return open_locked(operator_list);
+    }
+    EnnReturn OpenSubGraph(const OperatorListDesc &operator_list, bool fuse_residual_adds) {
+        std::lock_guard<std::mutex> lock_guard(mutex_constructor);
+        if (op_constructor) op_constructor->fuse_residual_adds = fuse_residual_adds;
+        return open_locked(operator_list);
+    }
+
+private:
+    EnnReturn open_locked(const OperatorListDesc &operator_list) {
         if (!compute_library || compute_library->initialize_queue() != Status::SUCCESS) return ENN_RET_FAILED;
         {
             std::lock_guard<std::mutex> lock_guard_map(mutex_operators_map);
@@ -67,6 +77,7 @@ public:
                                 op_constructor->get_out_tensors());
     }
 
+public:
     // nothing to prepare: buffers are bound at execution (gpu_userdriver.cc:72-76)
     EnnReturn PrepareSubGraph(uint64_t) { return ENN_RET_SUCCESS; }
 
@@ -142,6 +153,10 @@ public:
         compute_library->flush();
         return ENN_RET_SUCCESS;
     }
+
+    // For entry points beside the six: whoever holds this runs alone.  A transfer or a wait while another thread records a
+    // list's graph would become part of the recording or end it.
+    std::unique_lock<std::mutex> serialise() { return std::unique_lock<std::mutex>(mutex_constructor); }
 
     const std::shared_ptr<HipComputeLibrary> &computeLibrary() const { return compute_library; }
     OperationExecutor *executor() { return op_executor.get(); }

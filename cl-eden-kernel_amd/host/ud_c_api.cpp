@@ -243,8 +243,7 @@ int eud_oplist_destroy(eud_oplist *list) {
 int eud_open_subgraph(eud_driver *driver, const eud_oplist *list, int32_t fuse_residual_adds) {
     return guarded([&] {
         if (driver == nullptr || list == nullptr) return fail("eud_open_subgraph: null argument");
-        driver->ud.constructor()->fuse_residual_adds = fuse_residual_adds != 0;
-        return driver->ud.OpenSubGraph(list->desc) == ENN_RET_SUCCESS ? 0 : fail_below("eud_open_subgraph");
+        return driver->ud.OpenSubGraph(list->desc, fuse_residual_adds != 0) == ENN_RET_SUCCESS ? 0 : fail_below("eud_open_subgraph");
     });
 }
 
@@ -277,6 +276,7 @@ int eud_execute_operators(eud_driver *driver, uint64_t list_id, int32_t times) {
 
 int eud_set_replay(eud_driver *driver, int32_t replay) {
     if (driver == nullptr || driver->ud.executor() == nullptr) return fail("eud_set_replay: no driver");
+    const auto alone = driver->ud.serialise();
     driver->ud.executor()->replay = replay != 0;
     return 0;
 }
@@ -284,6 +284,7 @@ int eud_set_replay(eud_driver *driver, int32_t replay) {
 int eud_set_image_lanes(eud_driver *driver, int32_t lanes, int32_t min_lane_images) {
     if (driver == nullptr || driver->ud.constructor() == nullptr) return fail("eud_set_image_lanes: no driver");
     if (lanes < 1 || min_lane_images < 1) return fail("eud_set_image_lanes: lanes and min_lane_images start at 1");
+    const auto alone = driver->ud.serialise();
     driver->ud.constructor()->image_lanes = lanes;
     driver->ud.constructor()->min_lane_images = min_lane_images;
     return 0;
@@ -292,6 +293,7 @@ int eud_set_image_lanes(eud_driver *driver, int32_t lanes, int32_t min_lane_imag
 int eud_set_fuse_expansions(eud_driver *driver, int32_t mode) {
     if (driver == nullptr || driver->ud.constructor() == nullptr) return fail("eud_set_fuse_expansions: no driver");
     if (mode < 0 || mode > 2) return fail("eud_set_fuse_expansions: mode is 0, 1 or 2");
+    const auto alone = driver->ud.serialise();
     driver->ud.constructor()->fuse_expansions = mode != 0;
     driver->ud.constructor()->fuse_unlisted_expansions = mode == 2;
     return 0;
@@ -299,23 +301,26 @@ int eud_set_fuse_expansions(eud_driver *driver, int32_t mode) {
 
 int eud_set_store_channels_last(eud_driver *driver, int32_t on) {
     if (driver == nullptr || driver->ud.constructor() == nullptr) return fail("eud_set_store_channels_last: no driver");
+    const auto alone = driver->ud.serialise();
     driver->ud.constructor()->store_channels_last = on != 0;
     return 0;
 }
 
 int eud_synchronize(eud_driver *driver) {
     if (driver == nullptr || !driver->ud.computeLibrary()) return fail("eud_synchronize: no driver");
+    const auto alone = driver->ud.serialise();
     return driver->ud.computeLibrary()->runtime()->synchronize() == Status::SUCCESS ? 0 : fail_below("eud_synchronize");
 }
 
 void *eud_stream(eud_driver *driver) {
-    return driver && driver->ud.computeLibrary() ? driver->ud.computeLibrary()->runtime()->stream() : nullptr;
+    return driver && driver->ud.computeLibrary() ? driver->ud.computeLibrary()->runtime()->mainStream() : nullptr;
 }
 
 int eud_stats(eud_driver *driver, uint64_t list_id, int32_t *operator_count, uint64_t *direct, uint64_t *recordings, uint64_t *replays,
               size_t *pool_bytes) {
     return guarded([&] {
         if (driver == nullptr || driver->ud.executor() == nullptr) return fail("eud_stats: no driver");
+        const auto alone = driver->ud.serialise();
         UDOperators ops;
         if (driver->ud.get_graph_for_TC(list_id, ops) != ENN_RET_SUCCESS) return fail("eud_stats: list is not open");
         const auto &c = driver->ud.executor()->counters();
@@ -328,8 +333,10 @@ int eud_stats(eud_driver *driver, uint64_t list_id, int32_t *operator_count, uin
     });
 }
 
-static int list_tensor(eud_driver *driver, uint64_t list_id, bool output, int32_t i, std::shared_ptr<ITensor> *t) {
+// A tensor of an open list, and the driver's lock for as long as the caller uses it.
+static int list_tensor(eud_driver *driver, uint64_t list_id, bool output, int32_t i, std::shared_ptr<ITensor> *t, std::unique_lock<std::mutex> *alone) {
     if (driver == nullptr) return fail("no driver");
+    *alone = driver->ud.serialise();
     UDOperators ops;
     UDTensors in, out;
     if (driver->ud.get_ud_operators(list_id, ops, in, out) != ENN_RET_SUCCESS) return fail("list is not open");
@@ -341,8 +348,9 @@ static int list_tensor(eud_driver *driver, uint64_t list_id, bool output, int32_
 
 int eud_write_input(eud_driver *driver, uint64_t list_id, int32_t i, const void *host, size_t bytes) {
     return guarded([&] {
+        std::unique_lock<std::mutex> alone;
         std::shared_ptr<ITensor> t;
-        if (list_tensor(driver, list_id, false, i, &t)) return 1;
+        if (list_tensor(driver, list_id, false, i, &t, &alone)) return 1;
         if (host == nullptr || bytes != t->getNumOfBytes()) return fail("eud_write_input: %zu bytes given, the tensor holds %zu", bytes, t->getNumOfBytes());
         return t->writeData(const_cast<void *>(host), true) == Status::SUCCESS ? 0 : fail_below("eud_write_input");
     });
@@ -350,8 +358,9 @@ int eud_write_input(eud_driver *driver, uint64_t list_id, int32_t i, const void 
 
 int eud_read_output(eud_driver *driver, uint64_t list_id, int32_t i, void *host, size_t bytes) {
     return guarded([&] {
+        std::unique_lock<std::mutex> alone;
         std::shared_ptr<ITensor> t;
-        if (list_tensor(driver, list_id, true, i, &t)) return 1;
+        if (list_tensor(driver, list_id, true, i, &t, &alone)) return 1;
         if (host == nullptr || bytes != t->getNumOfBytes()) return fail("eud_read_output: %zu bytes given, the tensor holds %zu", bytes, t->getNumOfBytes());
         return t->readData(host, true) == Status::SUCCESS ? 0 : fail_below("eud_read_output");
     });
@@ -359,8 +368,9 @@ int eud_read_output(eud_driver *driver, uint64_t list_id, int32_t i, void *host,
 
 int eud_set_quant(eud_driver *driver, uint64_t list_id, int32_t is_output, int32_t i, float scale, int32_t zero_point) {
     return guarded([&] {
+        std::unique_lock<std::mutex> alone;
         std::shared_ptr<ITensor> t;
-        if (list_tensor(driver, list_id, is_output != 0, i, &t)) return 1;
+        if (list_tensor(driver, list_id, is_output != 0, i, &t, &alone)) return 1;
         t->setScale(scale);
         t->setZeroPoint(zero_point);
         return 0;
