@@ -31,17 +31,8 @@ namespace eh {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) uint8_t lds_byte;
 
 namespace {
-
-
-__device__ __forceinline__ uint32_t lds_offset(const void *p) { return (uint32_t)(uintptr_t)(lds_byte *)p; }
-
-// One wave copies up to 64 x 16 bytes: active lane i's 16 bytes land at lds_base + 16 * i.
-__device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base_uniform) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_base_uniform) : "memory");
-}
 
 struct Conv3Launch {
     int32_t th;               // output rows per tile
@@ -88,7 +79,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     {
         const uint8_t *wsrc = reinterpret_cast<const uint8_t *>(p.b) + (size_t)nb_first * KS * 1024;
         const int w_instr = nb_count * KS;  // 1 KiB each
-        for (int i = wave; i < w_instr; i += 4) dma16(wsrc + (size_t)i * 1024 + lane * 16, lds_offset(lds) + (uint32_t)i * 1024u);
+        dma_linear<4>(wsrc, lds_offset(lds), w_instr, wave, lane);
         const int pch = L.pitch >> 4, cpp = p.cin >> 4;  // chunks per pixel with and without the slack
         const int patch_pixels = (rows + 2) * L.pc;
         const int chunks = patch_pixels * pch;
@@ -114,7 +105,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
             // (the half step past the ninth tap of a 16 (mod 32) channel count multiplies zero weights: any bytes will do)
             step_s[tid] = tap < 9 ? (ky * L.pc + kx) * L.pitch + c0 : 0;
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        wait_vmcnt<0>();
         __syncthreads();
         // One pass over the patch in place: bytes to the signed operands the matrix cores take (a ^ 0x80), and each
         // pixel's sum of them over the channels into the pixel's slack chunk.  The nine taps then need neither a flip

@@ -37,30 +37,10 @@ namespace eh {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) uint8_t lds_byte;
 
 namespace {
 
 constexpr int16_t KPAD_MARK = INT16_MIN;
-
-__device__ __forceinline__ uint32_t lds_offset(const void *p) { return (uint32_t)(uintptr_t)(lds_byte *)p; }
-
-// One wave copies 64 x 16 bytes: lane i's 16 bytes land at lds_base + 16 * i.
-__device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base_uniform) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_base_uniform) : "memory");
-}
-
-// The same with the address split into a wave-uniform base and a 32-bit per-lane offset.
-__device__ __forceinline__ void dma16_off(const void *base_uniform, uint32_t lane_offset, uint32_t lds_base_uniform) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base_uniform),
-                 "s"(lds_base_uniform)
-                 : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 __device__ __forceinline__ v4i xor128(v4i v, int x) {
     v.x ^= x;

@@ -10,6 +10,34 @@
 
 namespace eh {
 
+// ---------------------------------------------------------------- direct-to-LDS copies
+typedef __attribute__((address_space(3))) uint8_t lds_byte;
+__device__ __forceinline__ uint32_t lds_offset(const void *p) { return (uint32_t)(uintptr_t)(lds_byte *)p; }
+
+// One wave copies 64 x 16 bytes: active lane i's 16 bytes land at lds_base + 16 * i.  Nothing waits: s_waitcnt vmcnt before the bytes are read.
+__device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base_uniform) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_base_uniform) : "memory");
+}
+
+// The same with the address split into a wave-uniform base and a 32-bit per-lane offset.
+__device__ __forceinline__ void dma16_off(const void *base_uniform, uint32_t lane_offset, uint32_t lds_base_uniform) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base_uniform),
+                 "s"(lds_base_uniform)
+                 : "memory");
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// A workgroup of WAVES waves copies `kib` KiB of global memory (16-byte aligned) to LDS, every KiB on its way before anything waits.
+template <int WAVES>
+__device__ __forceinline__ void dma_linear(const void *src_uniform, uint32_t lds_base_uniform, int kib, int wave_uniform, int lane) {
+    const uint8_t *src = static_cast<const uint8_t *>(src_uniform);
+    for (int i = wave_uniform; i < kib; i += WAVES) dma16_off(src + (size_t)i * 1024, (uint32_t)lane * 16u, lds_base_uniform + (uint32_t)i * 1024u);
+}
+
 // ---------------------------------------------------------------- errors
 void set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 int hip_fail(hipError_t e, const char *what);  // records the text, returns EH_DEVICE_FAILURE
