@@ -727,7 +727,7 @@ struct eh_dwconv_plan {
     int32_t *w_trip = nullptr, *bias_trip = nullptr;
     int32_t *w_fold = nullptr, *bias_fold = nullptr;  // the unsigned form of the same plans, for weights of any range
     bool fold_valid = false;
-    uint8_t *w_mm = nullptr;      // 5x5 / 7x7 channels-last plans: the matrix form of the weights and its bias
+    uint8_t *w_mm = nullptr;      // 3x3 / 5x5 / 7x7 channels-last plans: the matrix form of the weights and its bias
     int32_t *bias_mm = nullptr;
     bool range_known = false;   // w_lo / w_hi hold the extremes of the weight bytes (in the caller's own domain)
     int32_t w_lo = 0, w_hi = 0;
@@ -1882,7 +1882,7 @@ int eh_dwconv2d_u8_plan(eh_dwconv_plan **plan, const eh_conv_desc *desc, const v
         if (!rc) rc = dev_alloc(&pl->w_fold, (size_t)3 * pl->cout);
         if (!rc) rc = dev_alloc(&pl->bias_fold, (size_t)pl->cout + 4);
     }
-    const bool tile_form_k = pl->d.layout == EH_NHWC && pl->d.kh == pl->d.kw && (pl->d.kh == 5 || pl->d.kh == 7) && pl->d.depth_multiplier == 1 &&
+    const bool tile_form_k = pl->d.layout == EH_NHWC && pl->d.kh == pl->d.kw && (pl->d.kh == 3 || pl->d.kh == 5 || pl->d.kh == 7) && pl->d.depth_multiplier == 1 &&
                              pl->d.dil_h == 1 && pl->d.dil_w == 1;
     if (!rc && tile_form_k) {
         rc = dev_alloc(&pl->w_mm, dw_mfma_weight_bytes(pl->cout, pl->d.kh));

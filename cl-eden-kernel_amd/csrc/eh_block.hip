@@ -16,6 +16,9 @@
 //   2. after one barrier the threads compute the depthwise outputs from that image, four horizontally adjacent output
 //      pixels of four channels per thread, with the arithmetic of the stand-alone depthwise kernel (8-bit dot products,
 //      signed or unsigned form), and store them.
+//      Small tiles (a network on few images) do this stage on the matrix cores: a unit of sixteen outputs is some 300 vector
+//      instructions, and with fewer units than half the threads a workgroup waits for that chain (2 of the 4.1 us that a launch of
+//      such tiles lasts beyond an empty one).
 // The rows and columns two neighbouring workgroups both need (the halo) are computed twice; nothing else is.  Tiles are
 // cut in both directions because the halo of a stride-2 window costs (2 TH + 1)(2 TW + 1) / (4 TH TW): 1.53 for one full
 // row of 28 outputs, 1.21 for 4 x 7.
@@ -47,13 +50,18 @@ __device__ __forceinline__ void column_words(uint32_t r0, uint32_t r1, uint32_t 
     out[3] = __builtin_amdgcn_perm(r2, t23, 0x0c070302u);
 }
 
-// S: depthwise stride.  FOLD: the depthwise stage multiplies raw bytes (unsigned form, weights of any range) instead of
-// a - 128 against w - zp_w.  ROWSUM: the pointwise weights' zero point is not 128, so a pixel's byte sum enters.
+// S: depthwise stride.  FORM: how the depthwise stage multiplies (DwForm).  ROWSUM: the pointwise weights' zero point is not 128, so a pixel's byte sum enters.
 // QM: pointwise requantization, 0 two-step order, 1 / 2 the single-shift forms.  KS: reduction steps of the pointwise
 // stage when they are 1, 2 or 3 (a lane then keeps its pixel's operand bytes in registers across the channel blocks),
 // 0 for any number (read from LDS for every product).
-template <int S, bool FOLD, bool ROWSUM, int QM, int KS, bool PC>
+enum class DwForm {
+    DOT,   // 8-bit dot products of a - 128 and w - zp_w
+    FOLD,  // ... of the raw bytes: the unsigned form, for weights of any range
+    MATRIX // on the matrix cores, weights of any range
+};
+template <int S, DwForm FORM, bool ROWSUM, int QM, int KS, bool PC>
 __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, const DwProblem dw, const BlockGeom g) {
+    constexpr bool FOLD = FORM == DwForm::FOLD, MATRIX = FORM == DwForm::MATRIX;
     const int ksteps = KS ? KS : g.ks;
     extern __shared__ __align__(16) uint8_t lds_raw[];
     v4i *b_s = reinterpret_cast<v4i *>(lds_raw);                              // [nb][ks][64 lanes]: pointwise weights, fragment order
@@ -81,6 +89,34 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
     const int iy_first = oy0 * S - dw.pad_t, ix_first = ox_first * S - dw.pad_l;  // image coordinates of the LDS image's corner
     uint8_t *a_s = lds_raw + g.a_off;  // [pixels][a_pitch]: the input pixels' reduction bytes as signed operands (a ^ 0x80), 0 past the reduction length
 
+    // MATRIX: units of (chunk of 16 channels, 16 output pixels), a contiguous share per wave; lane (i, q) holds the weights of
+    // channel i of the chunk in kernel column q.  A wave's first chunk is requested ahead of everything else.
+    const int lane16 = lane & 15, quarter = lane >> 4, cpad = (g.c + 15) & ~15;
+    const int out_pixels = g.th * g.tw, groups = (out_pixels + 15) >> 4, w_uniform = __builtin_amdgcn_readfirstlane(wave);
+    const int unit_first = ((c_here >> 4) * groups * w_uniform) >> 2, unit_last = ((c_here >> 4) * groups * (w_uniform + 1)) >> 2;
+    struct DwPart {
+        uint32_t w[3], neg;  // by kernel row; minus what the stored weights lack (dw_pack_mfma_kernel)
+        int4 bias, mult, shift;
+    };
+    auto request_dw = [&](int chunk) {
+        const int c0 = c_first + chunk * 16;
+        DwPart d;
+#pragma unroll
+        for (int ky = 0; ky < 3; ++ky) d.w[ky] = dw.w_mm[(ky * 4 + quarter) * cpad + c0 + lane16];  // (column 3 is padding: zero)
+        d.neg = dw.w_mm[12 * cpad + c0 + lane16];
+        d.bias = *reinterpret_cast<const int4 *>(dw.bias_mm + c0 + quarter * 4);
+        if constexpr (PC) {
+            d.mult = *reinterpret_cast<const int4 *>(dw.rq.pc_multiplier + c0 + quarter * 4);
+            d.shift = *reinterpret_cast<const int4 *>(dw.rq.pc_shift + c0 + quarter * 4);
+        }
+        return d;
+    };
+    int chunk = unit_first / groups, group = unit_first - chunk * groups;
+    DwPart part{};
+    if constexpr (MATRIX) {
+        if (unit_first < unit_last) part = request_dw(chunk);
+    }
+
     // ---- stage 0: weights, bias and the tile's input pixels into LDS (8-byte pieces: pixels start on 8-byte boundaries)
     auto inside_image = [&](int q, int &iy, int &ix) {
         const int ry = (int)fastdiv((uint32_t)q, g.div_iwp), rx = q - ry * g.iwp;
@@ -89,22 +125,38 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
         return (unsigned)iy < (unsigned)pw.h && (unsigned)ix < (unsigned)pw.w;
     };
     {
+        // the weights as direct-to-LDS copies, all on their way at once beside the input pixels
+        dma_linear<4>(pw.b + (size_t)nb_first * ksteps * 1024, lds_offset(lds_raw), nb_here * ksteps, w_uniform, lane);
         const int ppp = ksteps * 4;  // 8-byte pieces per pixel
         const int pieces = g.pixels * ppp;
-        for (int i = tid; i < pieces; i += 256) {
-            const int q = KS ? i / (KS * 4) : (int)fastdiv((uint32_t)i, g.div_ppp), piece = i - q * ppp;
-            int iy, ix;
-            uint2 v = make_uint2(0u, 0u);  // bytes past the reduction length, and whole pixels outside the image: operand 0
-            if (inside_image(q, iy, ix) && piece * 8 < pw.k) {
-                v = *reinterpret_cast<const uint2 *>(pw.a + (((img * (uint32_t)pw.h + (uint32_t)iy) * (uint32_t)pw.w + (uint32_t)ix) * (uint32_t)pw.cin +
-                                                               (uint32_t)pw.a_offset + (uint32_t)piece * 8u));
-                v.x ^= pw.a_xor;
-                v.y ^= pw.a_xor;
+        // Longer reductions have several pieces for every thread: four are requested, from addresses clamped into the image so that
+        // no branch separates the loads, before the first is used.  (One step has hardly more than a piece per thread, and the
+        // instructions of idle turns cost a small launch more than the trips they save.)
+        constexpr int FLIGHT = KS == 1 ? 1 : 4;
+        for (int first = 0; first < pieces; first += 256 * FLIGHT) {
+            uint2 v[FLIGHT];
+            uint8_t *to[FLIGHT];
+            bool exists[FLIGHT];
+#pragma unroll
+            for (int f = 0; f < FLIGHT; ++f) {
+                if (first + f * 256 >= pieces) break;  // (uniform)
+                const int i = first + f * 256 + tid < pieces ? first + f * 256 + tid : pieces - 1;
+                const int q = KS ? i / (KS * 4) : (int)fastdiv((uint32_t)i, g.div_ppp), piece = i - q * ppp;
+                int iy, ix;
+                exists[f] = inside_image(q, iy, ix) && piece * 8 < pw.k;  // (else operand 0: bytes past the reduction length, whole pixels outside the image)
+                iy = iy < 0 ? 0 : (iy < pw.h ? iy : pw.h - 1);
+                ix = ix < 0 ? 0 : (ix < pw.w ? ix : pw.w - 1);
+                v[f] = *reinterpret_cast<const uint2 *>(pw.a + (((img * (uint32_t)pw.h + (uint32_t)iy) * (uint32_t)pw.w + (uint32_t)ix) * (uint32_t)pw.cin +
+                                                                (uint32_t)pw.a_offset + (piece * 8 < pw.k ? (uint32_t)piece * 8u : 0u)));
+                to[f] = a_s + q * g.a_pitch + piece * 8;
             }
-            *reinterpret_cast<uint2 *>(a_s + q * g.a_pitch + piece * 8) = v;
+#pragma unroll
+            for (int f = 0; f < FLIGHT; ++f) {
+                if (first + f * 256 >= pieces) break;
+                // (a thread past the last piece holds that piece as well and writes the same bytes)
+                *reinterpret_cast<uint2 *>(to[f]) = make_uint2(exists[f] ? v[f].x ^ pw.a_xor : 0u, exists[f] ? v[f].y ^ pw.a_xor : 0u);
+            }
         }
-        const v4i *src = reinterpret_cast<const v4i *>(pw.b) + (size_t)nb_first * ksteps * 64;
-        for (int i = tid; i < nb_here * ksteps * 64; i += 256) b_s[i] = src[i];
         for (int i = tid; i < nb_here * 32; i += 256) bias_s[i] = pw.bias[c_first + i];
         if constexpr (PC) {  // (the per-channel arrays are padded to whole channel blocks)
             for (int i = tid; i < nb_here * 32; i += 256) {
@@ -114,11 +166,12 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
                 pch_s[i] = QM != 0 ? channel_table_pos_hi(pw.rq.zp_out, -sh) : 0;
             }
         }
+        wait_vmcnt<0>();
         __syncthreads();
     }
 
     // ---- stage 1: the expanded pixels into the LDS image.  Units of (pixel block, channel block), a contiguous share per wave.
-    const uint32_t flip_store = FOLD ? 0u : 0x80808080u;  // the signed depthwise form reads a - 128
+    const uint32_t flip_store = FOLD ? 0u : 0x80808080u;  // the signed depthwise forms read a - 128
     const uint32_t pad_word = ((uint32_t)dw.zp_in * 0x01010101u) ^ flip_store;
     const int blocks = (g.pixels + 31) >> 5;
     const RequantDev rq = pw.rq;
@@ -215,11 +268,71 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
     __syncthreads();
 
     // ---- stage 2: the depthwise outputs from the LDS image
+    // four channels' accumulators to four bytes
+    auto finish = [&](int a0, int a1, int a2, int a3, const int4 &m, const int4 &sh) {
+        const RequantDev &drq = dw.rq;
+        if constexpr (PC) {
+            if (drq.fast == 2)
+                return pack_bytes(requant_u8_channel_fast<2>(a0, m.x, sh.x, drq), requant_u8_channel_fast<2>(a1, m.y, sh.y, drq),
+                                  requant_u8_channel_fast<2>(a2, m.z, sh.z, drq), requant_u8_channel_fast<2>(a3, m.w, sh.w, drq));
+            if (drq.fast)
+                return pack_bytes(requant_u8_channel_fast<1>(a0, m.x, sh.x, drq), requant_u8_channel_fast<1>(a1, m.y, sh.y, drq),
+                                  requant_u8_channel_fast<1>(a2, m.z, sh.z, drq), requant_u8_channel_fast<1>(a3, m.w, sh.w, drq));
+            return pack_bytes(requant_u8_channel(a0, m.x, sh.x, drq), requant_u8_channel(a1, m.y, sh.y, drq), requant_u8_channel(a2, m.z, sh.z, drq),
+                              requant_u8_channel(a3, m.w, sh.w, drq));
+        }
+        if (drq.fast == 2) return requant4_fast<2>(a0, a1, a2, a3, 0, drq);
+        if (drq.fast) return requant4_fast<1>(a0, a1, a2, a3, 0, drq);
+        return pack_bytes(requant_u8(a0, drq), requant_u8(a1, drq), requant_u8(a2, drq), requant_u8(a3, drq));
+    };
+    if constexpr (MATRIX) {
+        // As in eh_dwconv_mfma.hip: lane (i, q) fetches the sixteen channels of output pixel i's window at kernel column q, one
+        // 16-byte piece per kernel row, and three products against diagonal weights leave every lane with four neighbouring
+        // channels of one pixel.
+        const int column = quarter < 3 ? quarter : 2;  // (the fourth column's weights are zero: any pixel will do)
+        auto diagonal = [&](uint32_t byte) {
+            const int v = (int)(byte << (8 * (lane16 & 3))), d = lane16 >> 2;
+            return v4i{d == 0 ? v : 0, d == 1 ? v : 0, d == 2 ? v : 0, d == 3 ? v : 0};
+        };
+        for (int left = unit_last - unit_first; left > 0; group = 0, ++chunk) {
+            v4i wf[3];
+#pragma unroll
+            for (int ky = 0; ky < 3; ++ky) wf[ky] = diagonal(part.w[ky]);
+            const v4i df = diagonal(quarter < 3 ? part.neg : 0u);
+            const bool lacks = __builtin_amdgcn_ballot_w64(part.neg != 0) != 0;
+            const DwPart now = part;
+            const int last_group = left < groups - group ? group + left : groups;
+            left -= last_group - group;
+            if (left > 0) part = request_dw(chunk + 1);  // (on its way under this chunk's products)
+            const int c0 = c_first + chunk * 16;
+            for (int grp = group; grp < last_group; ++grp) {
+                const int p = grp * 16 + lane16, pc = p < out_pixels ? p : out_pixels - 1;
+                const int row = (int)fastdiv((uint32_t)pc, g.div_tw), col = pc - row * g.tw, oy = oy0 + row, ox = ox_first + col;
+                const uint8_t *const src = img_s + (row * S * g.iwp + col * S + column) * cpitch + chunk * 16;
+                v4i x[3];
+#pragma unroll
+                for (int ky = 0; ky < 3; ++ky) x[ky] = *reinterpret_cast<const v4i *>(src + ky * g.iwp * cpitch);
+                v4i acc = v4i{now.bias.x, now.bias.y, now.bias.z, now.bias.w};
+#pragma unroll
+                for (int ky = 0; ky < 3; ++ky) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[ky], x[ky], acc, 0, 0, 0);
+                if (lacks) {
+                    v4i lack = v4i{0, 0, 0, 0};
+#pragma unroll
+                    for (int ky = 0; ky < 3; ++ky) lack = __builtin_amdgcn_mfma_i32_16x16x64_i8(df, x[ky], lack, 0, 0, 0);
+                    acc -= lack;
+                }
+                const uint32_t o = finish(acc.x, acc.y, acc.z, acc.w, now.mult, now.shift);
+                if (p < out_pixels && oy < dw.ho && ox < dw.wo)
+                    *reinterpret_cast<uint32_t *>(dw.out + (((img * (uint32_t)dw.ho + (uint32_t)oy) * (uint32_t)dw.wo + (uint32_t)ox) * (uint32_t)dw.cout +
+                                                            (uint32_t)(c0 + quarter * 4))) = o;
+            }
+        }
+        return;
+    }
     constexpr int TW = 4, IW = (TW - 1) * S + 3;  // a thread's four adjacent output pixels
     const uint32_t cq_count = (uint32_t)c_here >> 2;
     const uint32_t units = (uint32_t)g.units_per_cq * cq_count;
     const uint32_t cq_first = (uint32_t)c_first >> 2;
-    const RequantDev drq = dw.rq;
     const FastDiv div_cq = blockIdx.y + 1 == gridDim.y ? g.div_cq_last : g.div_cq;
     for (uint32_t u = (uint32_t)tid; u < units; u += 256u) {
         const uint32_t t = fastdiv(u, div_cq);
@@ -243,8 +356,8 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
         const int4 b4 = *reinterpret_cast<const int4 *>((FOLD ? dw.bias_fold : dw.bias_trip) + cq * 4u);
         int4 dm = make_int4(0, 0, 0, 0), ds = dm;  // PC: the depthwise stage's four pairs
         if constexpr (PC) {
-            dm = *reinterpret_cast<const int4 *>(drq.pc_multiplier + cq * 4u);
-            ds = *reinterpret_cast<const int4 *>(drq.pc_shift + cq * 4u);
+            dm = *reinterpret_cast<const int4 *>(dw.rq.pc_multiplier + cq * 4u);
+            ds = *reinterpret_cast<const int4 *>(dw.rq.pc_shift + cq * 4u);
         }
         uint32_t colw[IW][4];
         int cs[FOLD ? IW : 1][4];
@@ -280,23 +393,7 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
                 acc2 += __mul24(-dw.zp_w, cs[j * S][2] + cs[j * S + 1][2] + cs[j * S + 2][2]);
                 acc3 += __mul24(-dw.zp_w, cs[j * S][3] + cs[j * S + 1][3] + cs[j * S + 2][3]);
             }
-            uint32_t o;
-            if constexpr (PC) {
-                if (drq.fast == 2)
-                    o = pack_bytes(requant_u8_channel_fast<2>(acc0, dm.x, ds.x, drq), requant_u8_channel_fast<2>(acc1, dm.y, ds.y, drq),
-                                   requant_u8_channel_fast<2>(acc2, dm.z, ds.z, drq), requant_u8_channel_fast<2>(acc3, dm.w, ds.w, drq));
-                else if (drq.fast)
-                    o = pack_bytes(requant_u8_channel_fast<1>(acc0, dm.x, ds.x, drq), requant_u8_channel_fast<1>(acc1, dm.y, ds.y, drq),
-                                   requant_u8_channel_fast<1>(acc2, dm.z, ds.z, drq), requant_u8_channel_fast<1>(acc3, dm.w, ds.w, drq));
-                else
-                    o = pack_bytes(requant_u8_channel(acc0, dm.x, ds.x, drq), requant_u8_channel(acc1, dm.y, ds.y, drq),
-                                   requant_u8_channel(acc2, dm.z, ds.z, drq), requant_u8_channel(acc3, dm.w, ds.w, drq));
-            } else if (drq.fast == 2)
-                o = requant4_fast<2>(acc0, acc1, acc2, acc3, 0, drq);
-            else if (drq.fast)
-                o = requant4_fast<1>(acc0, acc1, acc2, acc3, 0, drq);
-            else
-                o = pack_bytes(requant_u8(acc0, drq), requant_u8(acc1, drq), requant_u8(acc2, drq), requant_u8(acc3, drq));
+            const uint32_t o = finish(acc0, acc1, acc2, acc3, dm, ds);
             if (lx0 + j < g.tw && ox0 + j < dw.wo) *reinterpret_cast<uint32_t *>(dst + (uint32_t)j * (uint32_t)dw.cout) = o;
         }
     }
@@ -386,6 +483,14 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     // the one that computes the fewest pixel slots wins, counting the slots that pixel blocks of 32 and output tiles of
     // four leave empty and, at a lower weight, the input bytes staged again for every channel range.
     int th = rows_per_tile, tw = cols_per_tile, nb = nb_all;
+    // Where the vector form's units (sixteen outputs, some 300 instructions each) would keep at most half of a workgroup's threads
+    // busy, the matrix form spreads the depthwise stage over all four waves.  One image, us: 28x28 32 -> 192 stride 2 (8 units)
+    // 5.9 -> 4.2, 14x14 64 -> 384 (8) 5.2 -> 4.0, 7x7 160 -> 960 (8) 5.8 -> 4.5, 56x56 24 -> 144 (48) 4.4 -> 4.2; 16 images: 14x14 64 -> 384
+    // (96) 6.0 -> 5.8, but 28x28 32 -> 192 (240) 5.9 -> 6.4; 32 images: 28x28 (480) 8.7 -> 9.0, 56x56 24 -> 144 stride 2 (252) 10.9 -> 11.4.
+    auto matrix_form = [&](int rows, int cols, int blocks) {
+        const int quads = blocks * 8 < dw.c / 4 ? blocks * 8 : dw.c / 4;
+        return dw.w_mm != nullptr && rows * ((cols + 3) / 4) * quads <= 128;
+    };
     {
         double best = -1;
         int best_th = 1, best_tw = dw.wo < 4 ? dw.wo : 4, best_nb = 1;
@@ -405,7 +510,9 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
                         const int px = ih * iw;
                         const double tiles = (double)dw.n * ((dw.ho + ch - 1) / ch) * ((dw.wo + cw - 1) / cw);
                         const double stage1 = (double)((px + 31) / 32 * 32) * tiles / ((double)dw.n * dw.h * dw.w_);   // pixel slots computed per real pixel
-                        const double stage2 = (double)ch * ((cw + 3) / 4 * 4) * tiles / ((double)dw.n * dw.ho * dw.wo);  // output slots per real output
+                        // (a slot of the matrix form, which works on sixteen outputs, counts three quarters)
+                        const double slots = matrix_form(ch, cw, cn) ? 0.75 * ((ch * cw + 15) / 16 * 16) : (double)(ch * ((cw + 3) / 4 * 4));
+                        const double stage2 = slots * tiles / ((double)dw.n * dw.ho * dw.wo);  // output slots per real output
                         const double restage = (double)px * tiles * ranges * (g.ks * 32) / ((double)dw.n * dw.h * dw.w_ * dw.c);  // staged input bytes per expanded byte
                         const double cost = stage1 + 0.5 * stage2 + 2.0 * restage;
                         if (best < 0 || cost < best) {
@@ -435,6 +542,7 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     g.units_per_cq = th * g.tiles_x;
     g.div_iwp = make_fastdiv((uint32_t)g.iwp);
     g.div_tx = make_fastdiv((uint32_t)g.tiles_x);
+    g.div_tw = make_fastdiv((uint32_t)tw);
     g.div_tiles_y = make_fastdiv((uint32_t)g.tiles_y);
     g.div_tiles_w = make_fastdiv((uint32_t)g.tiles_w);
     g.div_ppp = make_fastdiv((uint32_t)(g.ks * 4));
@@ -442,6 +550,7 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     g.div_cq = make_fastdiv((uint32_t)(g.nb * 8 < g.c / 4 ? g.nb * 8 : g.c / 4));
     g.div_cq_last = make_fastdiv((uint32_t)((g.c - (ranges - 1) * g.nb * 32) / 4));
     g.cpitch = block_image_pitch(g.nb, g.c);
+    g.matrix = matrix_form(th, tw, nb) ? 1 : 0;
     const size_t lds = block_lds_bytes(g.nb, g.ks, g.ih, g.iwp, g.c, &g.a_off, &g.image_off);
     if (lds > kBlockLdsMax) return false;
     *geom = g;
@@ -460,8 +569,8 @@ int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, const B
     const size_t lds = (size_t)g.image_off + (size_t)g.ih * g.iwp * g.cpitch;
     if (g.total_tiles <= 0) return EH_OK;
     const dim3 grid((unsigned)((g.total_tiles + 7) / 8 * 8), (unsigned)(((g.c + 31) / 32 + g.nb - 1) / g.nb));
-    auto launch_pc = [&](auto s_c, auto fold_c, auto rowsum_c, auto qm_c, auto ks_c, auto pc_c) {
-        auto kernel = pwdw_block_kernel<decltype(s_c)::value, decltype(fold_c)::value, decltype(rowsum_c)::value, decltype(qm_c)::value, decltype(ks_c)::value,
+    auto launch_pc = [&](auto s_c, auto form_c, auto rowsum_c, auto qm_c, auto ks_c, auto pc_c) {
+        auto kernel = pwdw_block_kernel<decltype(s_c)::value, decltype(form_c)::value, decltype(rowsum_c)::value, decltype(qm_c)::value, decltype(ks_c)::value,
                                         decltype(pc_c)::value>;
         if (lds > 64 * 1024) {
             // (a driver call, made per launch of the tall-tile shapes only; the default tile height stays below 64 KiB)
@@ -471,25 +580,28 @@ int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, const B
         hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, pw, dw, g);
         return (int)EH_OK;
     };
-    auto launch = [&](auto s_c, auto fold_c, auto rowsum_c, auto qm_c, auto ks_c) {
-        return pw.rq.pc_multiplier ? launch_pc(s_c, fold_c, rowsum_c, qm_c, ks_c, std::true_type{}) : launch_pc(s_c, fold_c, rowsum_c, qm_c, ks_c, std::false_type{});
+    auto launch = [&](auto s_c, auto form_c, auto rowsum_c, auto qm_c, auto ks_c) {
+        return pw.rq.pc_multiplier ? launch_pc(s_c, form_c, rowsum_c, qm_c, ks_c, std::true_type{}) : launch_pc(s_c, form_c, rowsum_c, qm_c, ks_c, std::false_type{});
     };
-    auto with_ks = [&](auto s_c, auto fold_c, auto rowsum_c, auto qm_c) {
-        if (g.ks == 1) return launch(s_c, fold_c, rowsum_c, qm_c, std::integral_constant<int, 1>{});
-        if (g.ks == 2) return launch(s_c, fold_c, rowsum_c, qm_c, std::integral_constant<int, 2>{});
-        if (g.ks == 3) return launch(s_c, fold_c, rowsum_c, qm_c, std::integral_constant<int, 3>{});
-        return launch(s_c, fold_c, rowsum_c, qm_c, std::integral_constant<int, 0>{});
+    auto with_ks = [&](auto s_c, auto form_c, auto rowsum_c, auto qm_c) {
+        if (g.ks == 1) return launch(s_c, form_c, rowsum_c, qm_c, std::integral_constant<int, 1>{});
+        if (g.ks == 2) return launch(s_c, form_c, rowsum_c, qm_c, std::integral_constant<int, 2>{});
+        if (g.ks == 3) return launch(s_c, form_c, rowsum_c, qm_c, std::integral_constant<int, 3>{});
+        return launch(s_c, form_c, rowsum_c, qm_c, std::integral_constant<int, 0>{});
     };
-    auto with_qm = [&](auto s_c, auto fold_c, auto rowsum_c) {
-        if (pw.rq.fast == 2) return with_ks(s_c, fold_c, rowsum_c, std::integral_constant<int, 2>{});
-        if (pw.rq.fast == 1) return with_ks(s_c, fold_c, rowsum_c, std::integral_constant<int, 1>{});
-        return with_ks(s_c, fold_c, rowsum_c, std::integral_constant<int, 0>{});
+    auto with_qm = [&](auto s_c, auto form_c, auto rowsum_c) {
+        if (pw.rq.fast == 2) return with_ks(s_c, form_c, rowsum_c, std::integral_constant<int, 2>{});
+        if (pw.rq.fast == 1) return with_ks(s_c, form_c, rowsum_c, std::integral_constant<int, 1>{});
+        return with_ks(s_c, form_c, rowsum_c, std::integral_constant<int, 0>{});
     };
-    auto with_rowsum = [&](auto s_c, auto fold_c) {
-        return pw.zw != 0 ? with_qm(s_c, fold_c, std::true_type{}) : with_qm(s_c, fold_c, std::false_type{});
+    auto with_rowsum = [&](auto s_c, auto form_c) {
+        return pw.zw != 0 ? with_qm(s_c, form_c, std::true_type{}) : with_qm(s_c, form_c, std::false_type{});
     };
-    auto with_fold = [&](auto s_c) { return dw.w_trip ? with_rowsum(s_c, std::false_type{}) : with_rowsum(s_c, std::true_type{}); };
-    const int rc = S == 1 ? with_fold(std::integral_constant<int, 1>{}) : with_fold(std::integral_constant<int, 2>{});
+    auto with_form = [&](auto s_c) {
+        if (g.matrix) return with_rowsum(s_c, std::integral_constant<DwForm, DwForm::MATRIX>{});
+        return dw.w_trip ? with_rowsum(s_c, std::integral_constant<DwForm, DwForm::DOT>{}) : with_rowsum(s_c, std::integral_constant<DwForm, DwForm::FOLD>{});
+    };
+    const int rc = S == 1 ? with_form(std::integral_constant<int, 1>{}) : with_form(std::integral_constant<int, 2>{});
     if (rc) return rc;
     EH_HIP(hipGetLastError());
     return EH_OK;

@@ -612,7 +612,7 @@ struct DwProblem {
     // weight bytes (int8 weights: byte + 128), and the bias with -zp_in * sum w + 9 zp_in zp_w folded in
     const int32_t *w_fold;
     const int32_t *bias_fold;
-    // 5x5 and 7x7 weights for the matrix form (else null), laid out by launch_dw_pack_mfma
+    // 3x3, 5x5 and 7x7 weights for the matrix form (else null), laid out by launch_dw_pack_mfma
     const uint8_t *w_mm;
     const int32_t *bias_mm;
     uint8_t *out;
@@ -655,9 +655,10 @@ struct BlockGeom {
     int32_t cpitch;      // bytes per pixel of the LDS image
     int32_t tiles_x;     // depthwise tiles of four output columns per row of the workgroup's tile
     int32_t units_per_cq;  // th * tiles_x: depthwise thread-units per channel quad
+    int32_t matrix;      // the depthwise stage runs on the matrix cores (see pwdw_block_geometry)
     int32_t total_tiles; // n * tiles_y * tiles_w
     int32_t a_pitch;     // LDS bytes per input pixel: 32 ks + 16 (the slack spreads the fragment reads over the banks)
-    FastDiv div_iwp, div_tx, div_tiles_y, div_tiles_w, div_ppp;
+    FastDiv div_iwp, div_tx, div_tw, div_tiles_y, div_tiles_w, div_ppp;
     FastDiv div_cq, div_cq_last;  // by the channel quads of a full range, and of the last one
     uint32_t a_off;      // byte offset of the staged input pixels
     uint32_t image_off;  // byte offset of the LDS image behind the staged weights, bias and input pixels
