@@ -9,11 +9,16 @@
 // w - 128 with the zero-point terms folded into the bias and a per-pixel
 // correction -(zp_w - 128) * sum(a').
 //
-//
 // With 32 output channels or more the multiply-adds go to the matrix cores instead (conv_c3k3_mfma_kernel): a
 // lane still gathers one pixel, the two halves of the wave then exchange half of what they gathered so that each
 // of the wave's two 32-pixel blocks has its 27 (+5 zero) reduction bytes in 32x32x32 fragment form, and one
 // v_mfma_i32_32x32x32_i8 per block and 32 channels leaves every lane with 16 consecutive channels of one pixel.
+//
+// Bound by its instructions (about 350 to a wavefront of 64 pixels x 32 channels, half of them requantization) once the
+// loads are together: 224x224, stride 2, 32 channels, before and after the rows, the weights and the bias (and a channel's
+// pair) were requested ahead of their first use: one image 3.95 -> 3.20 us, 32 images 9.31 -> 7.77, 64 images
+// 13.54 -> 11.50; with a pair per channel 4.62 -> 3.47, 11.43 -> 9.76 and 18.74 -> 15.61; 160x160 to 96 channels,
+// 8 images 8.81 -> 5.96.  With fewer than 32 channels: 224x224 to 16, 32 images 7.17 -> 6.89.
 //
 // Stands in for the reference's direct convolution kernels on this shape
 // (gpu/operators/cl_kernels/DirectConvolutionKernel.cpp, 3x3 uint8 variants).
@@ -29,45 +34,77 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// The 27 reduction bytes of output pixel m as seven dwords of a' = a ^ a_xor (the 28th byte zero), out-of-image taps
-// reading the input zero point; all zero for m past the last pixel.
-__device__ __forceinline__ void gather_c3k3(const GemmProblem &p, const uint32_t in_bytes, int m, uint32_t (&A)[7]) {
+// The 27 reduction bytes of output pixel m < p.m as seven dwords of a' = a ^ a_xor (the 28th byte zero), out-of-image
+// taps reading the input zero point; `pixel` is where the output pixel lies in the output's rows.
+//
+// Every row is read, the ones outside the image from the nearest inside, and all three before the first is used: with
+// each row's loads in a branch of its own the compiler waited for one row before it asked for the next.  Where twelve
+// bytes would leave the tensor at its first or last pixels, the twelve inside are read and the bytes moved into place.
+__device__ __forceinline__ void gather_c3k3(const GemmProblem &p, const uint32_t in_bytes, int m, uint32_t (&A)[7], uint32_t &pixel) {
     const int plane = p.ho * p.wo;
     const int img = (int)fastdiv((uint32_t)m, p.div_plane), rem = m - img * plane;
     const int oy = (int)fastdiv((uint32_t)rem, p.div_wo), ox = rem - oy * p.wo;
+    pixel = (uint32_t)((img * p.out_h + (oy * p.out_sy + p.out_y0)) * p.out_w + (ox * p.out_sx + p.out_x0));
     const int iy0 = oy * p.stride_h + p.y_base, ix0 = ox * p.stride_w + p.x_base;
     const bool c0 = (unsigned)ix0 < (unsigned)p.w, c1 = (unsigned)(ix0 + 1) < (unsigned)p.w, c2 = (unsigned)(ix0 + 2) < (unsigned)p.w;
-    const int row_bytes = p.w * 3, a_row0 = ((img * p.h + iy0) * p.w + ix0) * 3;
+    // (tensors stay below 2 GiB: 32-bit offsets)
+    uint32_t d[3][3];
+    int past[3];  // how far a row's nine bytes lie past the twelve that were read
+    const int last = (int)in_bytes - 12;
+    if (last >= 0) {
+#pragma unroll
+        for (int ky = 0; ky < 3; ++ky) {
+            const int iy = iy0 + ky, iyc = iy < 0 ? 0 : (iy < p.h ? iy : p.h - 1);
+            const int a = ((img * p.h + iyc) * p.w + ix0) * 3, ac = a < 0 ? 0 : (a < last ? a : last);
+            past[ky] = a - ac;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) d[ky][i] = *reinterpret_cast<const u32_unaligned *>(p.a + ac + 4 * i);  // (a three-element vector would read sixteen bytes)
+        }
+        if (__builtin_amdgcn_ballot_w64((past[0] | past[1] | past[2]) != 0) != 0) {
+#pragma unroll
+            for (int ky = 0; ky < 3; ++ky)
+#pragma unroll
+                for (int step = 3; step <= 9; step += 3) {  // (a multiple of three, like every pixel's address and the tensor's length)
+                    uint32_t &x = d[ky][0], &y = d[ky][1], &z = d[ky][2];
+                    if (past[ky] >= step) {
+                        x = __builtin_amdgcn_alignbyte(y, x, 3);
+                        y = __builtin_amdgcn_alignbyte(z, y, 3);
+                        z = z >> 24;
+                    }
+                    if (past[ky] <= -step) {
+                        z = __builtin_amdgcn_alignbyte(z, y, 1);
+                        y = __builtin_amdgcn_alignbyte(y, x, 1);
+                        x = x << 24;
+                    }
+                }
+        }
+    } else {  // a tensor of three pixels at most
+#pragma unroll
+        for (int ky = 0; ky < 3; ++ky) {
+            const int iy = iy0 + ky, iyc = iy < 0 ? 0 : (iy < p.h ? iy : p.h - 1);
+            uint32_t lo = 0, mid = 0, hi = 0;
+#pragma unroll 1
+            for (int j = 0; j < 9; ++j) {  // the first byte is shifted in last
+                const int b = ((img * p.h + iyc) * p.w + ix0) * 3 + 8 - j;
+                const uint32_t v = b >= 0 && (uint32_t)b < in_bytes ? p.a[b] : 0u;
+                hi = __builtin_amdgcn_alignbyte(hi, mid, 3);
+                mid = __builtin_amdgcn_alignbyte(mid, lo, 3);
+                lo = lo << 8 | v;
+            }
+            d[ky][0] = lo, d[ky][1] = mid, d[ky][2] = hi;
+        }
+    }
     uint32_t seg[3][3];  // per kernel row: bytes 0..8 = 3 pixels x 3 channels, the rest zero
 #pragma unroll
     for (int ky = 0; ky < 3; ++ky) {
-        const int iy = iy0 + ky;
-        const bool row_ok = (unsigned)iy < (unsigned)p.h;
-        // (tensors stay below 2 GiB: 32-bit offsets, one multiplication chain per pixel instead of one per row)
-        const int a = a_row0 + ky * row_bytes;
-        uint32_t d0 = 0, d1 = 0, d2 = 0;
-        if (row_ok) {
-            if (a >= 0 && (uint32_t)a + 12u <= in_bytes) {
-                d0 = *reinterpret_cast<const u32_unaligned *>(p.a + a);
-                d1 = *reinterpret_cast<const u32_unaligned *>(p.a + a + 4);
-                d2 = *reinterpret_cast<const u32_unaligned *>(p.a + a + 8);
-            } else {  // the first pixel of the first image and the last of the last: byte by byte, inside the tensor
-                for (int j = 0; j < 9; ++j) {
-                    const int b = a + j;
-                    const uint32_t v = b >= 0 && (uint32_t)b < in_bytes ? p.a[b] : 0u;
-                    if (j < 4) d0 |= v << (8 * j);
-                    else if (j < 8) d1 |= v << (8 * (j - 4));
-                    else d2 |= v;
-                }
-            }
-        }
+        const bool row_ok = (unsigned)(iy0 + ky) < (unsigned)p.h;
         const bool v0 = row_ok && c0, v1 = row_ok && c1, v2 = row_ok && c2;
         const uint32_t m0 = (v0 ? 0x00FFFFFFu : 0u) | (v1 ? 0xFF000000u : 0u);
         const uint32_t m1 = (v1 ? 0x0000FFFFu : 0u) | (v2 ? 0xFFFF0000u : 0u);
         const uint32_t m2 = v2 ? 0x000000FFu : 0u;
-        seg[ky][0] = (d0 & m0) | (p.fill & ~m0);
-        seg[ky][1] = (d1 & m1) | (p.fill & ~m1);
-        seg[ky][2] = ((d2 & m2) | (p.fill & ~m2)) & 0xFFu;
+        seg[ky][0] = (d[ky][0] & m0) | (p.fill & ~m0);
+        seg[ky][1] = (d[ky][1] & m1) | (p.fill & ~m1);
+        seg[ky][2] = ((d[ky][2] & m2) | (p.fill & ~m2)) & 0xFFu;
     }
     A[0] = seg[0][0];
     A[1] = seg[0][1];
@@ -79,27 +116,36 @@ __device__ __forceinline__ void gather_c3k3(const GemmProblem &p, const uint32_t
 #pragma unroll
     for (int i = 0; i < 7; ++i) A[i] ^= p.a_xor;
     A[6] &= 0x00FFFFFFu;
-    if (m >= p.m) {
-#pragma unroll
-        for (int i = 0; i < 7; ++i) A[i] = 0;
-    }
 }
 
 // Matrix-core form.  Grid: x = 256 pixels per workgroup (64 per wave).  With one multiplier and shift per channel,
 // FAST means that every channel's pair is inside the single-shift form's range.
-template <bool ROWSUM, bool FAST, bool PLANAR>
+template <bool ROWSUM, bool FAST, bool PLANAR, bool PC>
 __global__ __launch_bounds__(256) void conv_c3k3_mfma_kernel(const GemmProblem p, const uint32_t in_bytes) {
     const int lane = threadIdx.x & 63, r = lane & 31, half = lane >> 5;
     // every XCD (workgroups are dispatched round-robin over the 8 of them) takes one contiguous eighth of the
     // pixel range, so the input rows that neighbouring output rows share are fetched into one L2 only
     const int block = (int)((blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3));
     const int m_own = block * 256 + threadIdx.x;  // the pixel this lane gathers
-    uint32_t A[7];
-    gather_c3k3(p, in_bytes, m_own < p.m ? m_own : p.m - 1, A);
-    if (m_own >= p.m) {
+    // weight rows are stored plainly, [channel][32 bytes]: row `r` of the fragment is channel 16 h + 4 g + t of the block
+    const int8_t *const w_own = p.b + (size_t)(16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3)) * 32 + half * 16;
+    v4i wf;
+    int4 bias[4], mult[4], shift[4];
+    auto request = [&](int nb) {
+        const int n = nb * 32 + half * 16;
+        wf = *reinterpret_cast<const v4i *>(w_own + (size_t)nb * (32 * 32));
 #pragma unroll
-        for (int i = 0; i < 7; ++i) A[i] = 0;
-    }
+        for (int g = 0; g < 4; ++g) {
+            bias[g] = *reinterpret_cast<const int4 *>(p.bias + n + g * 4);
+            if constexpr (PC) {  // (the arrays are padded past the last channel block)
+                mult[g] = *reinterpret_cast<const int4 *>(p.rq.pc_multiplier + n + g * 4);
+                shift[g] = *reinterpret_cast<const int4 *>(p.rq.pc_shift + n + g * 4);
+            }
+        }
+    };
+    request(0);  // on its way while the pixels are gathered
+    uint32_t A[7], pixel_own;
+    gather_c3k3(p, in_bytes, m_own < p.m ? m_own : p.m - 1, A, pixel_own);
     int rs_own = 0;
     if constexpr (ROWSUM) {
 #pragma unroll
@@ -115,34 +161,26 @@ __global__ __launch_bounds__(256) void conv_c3k3_mfma_kernel(const GemmProblem p
     af[0] = half ? v4i{(int)got[0], (int)got[1], (int)got[2], (int)got[3]} : v4i{(int)A[0], (int)A[1], (int)A[2], (int)A[3]};
     af[1] = half ? v4i{(int)A[4], (int)A[5], (int)A[6], 0} : v4i{(int)got[0], (int)got[1], (int)got[2], (int)got[3]};
     const int rs_got = ROWSUM ? __shfl_xor(rs_own, 32) : 0;
+    const uint32_t pixel_got = (uint32_t)__shfl_xor((int)pixel_own, 32);
     const int wave_base = m_own - lane;
     const RequantDev rq = p.rq;
-    const int plane = p.ho * p.wo;
     const int n_blocks = (p.n + 31) >> 5;
+    for (int nb = 0; nb < n_blocks; ++nb) {
+        const int n = nb * 32 + half * 16;
+        if (nb != 0) request(nb);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const int m = wave_base + 32 * b + r;  // the pixel whose 16 channels this lane finishes in block b
-        const int ncorr = ROWSUM ? -p.zw * (b == half ? rs_own : rs_got) : 0;
-        size_t out_off = 0;
-        if (m < p.m) {
-            const int img = (int)fastdiv((uint32_t)m, p.div_plane), rem = m - img * plane;
-            const int oy = (int)fastdiv((uint32_t)rem, p.div_wo), ox = rem - oy * p.wo;
-            out_off = (((size_t)img * p.out_h + (oy * p.out_sy + p.out_y0)) * p.out_w + (ox * p.out_sx + p.out_x0)) * (size_t)p.ldc;
-        }
-        for (int nb = 0; nb < n_blocks; ++nb) {
-            // weight rows are stored plainly, [channel][32 bytes]: row `r` of the fragment is channel 16 h + 4 g + t of the block
-            const int ch = nb * 32 + 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
-            const v4i wf = *reinterpret_cast<const v4i *>(p.b + (size_t)ch * 32 + half * 16);
-            const int n = nb * 32 + half * 16;
+        for (int b = 0; b < 2; ++b) {
+            const int m = wave_base + 32 * b + r;  // the pixel whose 16 channels this lane finishes in block b
+            const int ncorr = ROWSUM ? -p.zw * (b == half ? rs_own : rs_got) : 0;
+            const size_t out_off = (size_t)(b == half ? pixel_own : pixel_got) * (size_t)p.ldc;
             // the accumulators start from the folded bias and the pixel's row-sum term: nothing left to add afterwards
             v16i acc;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int4 bb = *reinterpret_cast<const int4 *>(p.bias + n + g * 4);
-                acc[g * 4 + 0] = bb.x + ncorr;
-                acc[g * 4 + 1] = bb.y + ncorr;
-                acc[g * 4 + 2] = bb.z + ncorr;
-                acc[g * 4 + 3] = bb.w + ncorr;
+                acc[g * 4 + 0] = bias[g].x + ncorr;
+                acc[g * 4 + 1] = bias[g].y + ncorr;
+                acc[g * 4 + 2] = bias[g].z + ncorr;
+                acc[g * 4 + 3] = bias[g].w + ncorr;
             }
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf, af[b], acc, 0, 0, 0);
             uint32_t packed[4];
@@ -150,21 +188,22 @@ __global__ __launch_bounds__(256) void conv_c3k3_mfma_kernel(const GemmProblem p
                 constexpr int mode = decltype(mode_c)::value;
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    if (rq.pc_multiplier) {  // (the arrays are padded past the last channel block)
-                        const int4 cm = *reinterpret_cast<const int4 *>(rq.pc_multiplier + n + g * 4);
-                        const int4 cs = *reinterpret_cast<const int4 *>(rq.pc_shift + n + g * 4);
-                        auto one = [&](int x, int32_t mult, int32_t shift) {
+                    if constexpr (PC) {
+                        auto one = [&](int x, int32_t mu, int32_t sh) {
+#if defined(__HIP_DEVICE_COMPILE__)
+                            // (the channel's rounding term is worked out for each block: 16 of them kept for both, at two
+                            // registers each, would leave two wavefronts to a SIMD)
+                            asm("" : "+v"(sh));
+#endif
                             if constexpr (mode == 0)
-                                return requant_u8_channel(x, mult, shift, rq);
+                                return requant_u8_channel(x, mu, sh, rq);
                             else
-                                return requant_u8_channel_fast<mode>(x, mult, shift, rq);
+                                return requant_u8_channel_fast<mode>(x, mu, sh, rq);
                         };
-                        packed[g] = pack_bytes(one(acc[g * 4 + 0], cm.x, cs.x), one(acc[g * 4 + 1], cm.y, cs.y),
-                                               one(acc[g * 4 + 2], cm.z, cs.z), one(acc[g * 4 + 3], cm.w, cs.w)) ^
+                        packed[g] = pack_bytes(one(acc[g * 4 + 0], mult[g].x, shift[g].x), one(acc[g * 4 + 1], mult[g].y, shift[g].y),
+                                               one(acc[g * 4 + 2], mult[g].z, shift[g].z), one(acc[g * 4 + 3], mult[g].w, shift[g].w)) ^
                                     p.out_xor;
-                        continue;
-                    }
-                    if constexpr (mode != 0)
+                    } else if constexpr (mode != 0)
                         packed[g] = requant4_fast<mode>(acc[g * 4 + 0], acc[g * 4 + 1], acc[g * 4 + 2], acc[g * 4 + 3], 0, rq) ^ p.out_xor;
                     else
                         packed[g] = pack_bytes(requant_u8_as<mode>(acc[g * 4 + 0], rq), requant_u8_as<mode>(acc[g * 4 + 1], rq),
@@ -198,55 +237,9 @@ __global__ __launch_bounds__(256) void conv_c3k3_kernel(const GemmProblem p, con
     const int m = blockIdx.x * 256 + threadIdx.x;
     if (m >= p.m) return;
     const int n0 = blockIdx.y * 16;
-    const int plane = p.ho * p.wo;
-    const int img = (int)fastdiv((uint32_t)m, p.div_plane), rem = m - img * plane;
-    const int oy = (int)fastdiv((uint32_t)rem, p.div_wo), ox = rem - oy * p.wo;
-    const int iy0 = oy * p.stride_h + p.y_base, ix0 = ox * p.stride_w + p.x_base;
-    const bool c0 = (unsigned)ix0 < (unsigned)p.w, c1 = (unsigned)(ix0 + 1) < (unsigned)p.w, c2 = (unsigned)(ix0 + 2) < (unsigned)p.w;
-
-    uint32_t seg[3][3];  // per kernel row: bytes 0..8 = 3 pixels x 3 channels, the rest zero
-#pragma unroll
-    for (int ky = 0; ky < 3; ++ky) {
-        const int iy = iy0 + ky;
-        const bool row_ok = (unsigned)iy < (unsigned)p.h;
-        const long a = ((long)(img * p.h + iy) * p.w + ix0) * 3;
-        uint32_t d0 = 0, d1 = 0, d2 = 0;
-        if (row_ok) {
-            if (a >= 0 && a + 12 <= (long)in_bytes) {
-                d0 = *reinterpret_cast<const u32_unaligned *>(p.a + a);
-                d1 = *reinterpret_cast<const u32_unaligned *>(p.a + a + 4);
-                d2 = *reinterpret_cast<const u32_unaligned *>(p.a + a + 8);
-            } else {  // the first pixel of the first image and the last of the last: byte by byte, inside the tensor
-                for (int j = 0; j < 9; ++j) {
-                    const long b = a + j;
-                    const uint32_t v = b >= 0 && b < (long)in_bytes ? p.a[b] : 0u;
-                    if (j < 4) d0 |= v << (8 * j);
-                    else if (j < 8) d1 |= v << (8 * (j - 4));
-                    else d2 |= v;
-                }
-            }
-        }
-        // keep the bytes of pixels inside the image, the others read the input zero point
-        const bool v0 = row_ok && c0, v1 = row_ok && c1, v2 = row_ok && c2;
-        const uint32_t m0 = (v0 ? 0x00FFFFFFu : 0u) | (v1 ? 0xFF000000u : 0u);
-        const uint32_t m1 = (v1 ? 0x0000FFFFu : 0u) | (v2 ? 0xFFFF0000u : 0u);
-        const uint32_t m2 = v2 ? 0x000000FFu : 0u;
-        seg[ky][0] = (d0 & m0) | (p.fill & ~m0);
-        seg[ky][1] = (d1 & m1) | (p.fill & ~m1);
-        seg[ky][2] = ((d2 & m2) | (p.fill & ~m2)) & 0xFFu;
-    }
     // reduction order (kernel row, kernel column, channel): 27 bytes in seven dwords, the 28th byte is zero
-    uint32_t A[7];
-    A[0] = seg[0][0];
-    A[1] = seg[0][1];
-    A[2] = seg[0][2] | (seg[1][0] << 8);
-    A[3] = __builtin_amdgcn_alignbyte(seg[1][1], seg[1][0], 3);
-    A[4] = (__builtin_amdgcn_alignbyte(seg[1][2], seg[1][1], 3) & 0xFFFFu) | (seg[2][0] << 16);
-    A[5] = __builtin_amdgcn_alignbyte(seg[2][1], seg[2][0], 2);
-    A[6] = __builtin_amdgcn_alignbyte(seg[2][2], seg[2][1], 2);
-#pragma unroll
-    for (int i = 0; i < 7; ++i) A[i] ^= p.a_xor;
-    A[6] &= 0x00FFFFFFu;
+    uint32_t A[7], pixel;
+    gather_c3k3(p, in_bytes, m, A, pixel);
     int ncorr = 0;
     if constexpr (ROWSUM) {
         int rs = 0;
@@ -280,7 +273,7 @@ __global__ __launch_bounds__(256) void conv_c3k3_kernel(const GemmProblem p, con
         produce(std::integral_constant<int, 2>{});
     else
         produce(std::integral_constant<int, 1>{});
-    uint8_t *dst = p.out + (((size_t)img * p.out_h + (oy * p.out_sy + p.out_y0)) * p.out_w + (ox * p.out_sx + p.out_x0)) * (size_t)p.ldc + n0;
+    uint8_t *dst = p.out + (size_t)pixel * (size_t)p.ldc + n0;
     const bool aligned16 = (p.ldc & 15) == 0 && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
     if constexpr (PLANAR) {
         store_bytes_planar(p.out, p.planar, (size_t)(dst - p.out) - (size_t)n0, n0, packed, p.n - n0);
@@ -309,7 +302,11 @@ int launch_conv_c3k3(const GemmProblem &p, hipStream_t stream) {
     if (p.n >= 32) {  // the packed rows and the folded bias are padded to whole tiles of channels
         const dim3 grid_m(((p.m + 255) / 256 + 7) / 8 * 8);  // whole multiples of 8: see the kernel's block numbering
         launch_variant([&](auto rs, auto f, auto pl) {
-            hipLaunchKernelGGL((conv_c3k3_mfma_kernel<decltype(rs)::value, decltype(f)::value, decltype(pl)::value>), grid_m, dim3(256), 0, stream, p, total_bytes);
+            constexpr bool ROWSUM = decltype(rs)::value, FAST = decltype(f)::value, PLANAR = decltype(pl)::value;
+            if (p.rq.pc_multiplier)
+                hipLaunchKernelGGL((conv_c3k3_mfma_kernel<ROWSUM, FAST, PLANAR, true>), grid_m, dim3(256), 0, stream, p, total_bytes);
+            else
+                hipLaunchKernelGGL((conv_c3k3_mfma_kernel<ROWSUM, FAST, PLANAR, false>), grid_m, dim3(256), 0, stream, p, total_bytes);
         });
         EH_HIP(hipGetLastError());
         return EH_OK;
