@@ -28,6 +28,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 namespace {
 
+typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 
@@ -56,8 +57,9 @@ struct ThinStage {
 __device__ __forceinline__ const GemmProblem &problem_of(const GemmProblem &one) { return one; }
 __device__ __forceinline__ const GemmProblem &problem_of(const GemmBatch &batch) { return batch.p[blockIdx.z]; }
 
+// (six steps in flight: bounded to four wavefronts per SIMD; with three, 96 -> 24 with a pair per channel took 5.69 us instead of 4.28)
 template <int NBU, int KU, bool ROWSUM, int QM, bool RES, bool BATCHED = false, bool PLANAR = false>
-__global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional_t<BATCHED, GemmBatch, GemmProblem> arg, const int n_blocks,
+__global__ __launch_bounds__(256, KU == 6 ? 4 : 1) void direct_gemm_kernel(const std::conditional_t<BATCHED, GemmBatch, GemmProblem> arg, const int n_blocks,
                                                           const int ksteps, const int nbw, const int row_blocks, const ThinStage stage) {
     // BATCHED: equally shaped problems of one operator (the output phases of a transposed convolution whose kernel is its
     // stride) that differ in their weights and in where their outputs go.  (A kernel of its own: indexing the argument
@@ -121,13 +123,14 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
     const int rb_first = (int)(blockIdx.x & 7u) * rb_per_xcd + (int)(blockIdx.x >> 3) * 4 + wave;
     const int rb_end = ((int)(blockIdx.x & 7u) + 1) * rb_per_xcd < row_blocks ? ((int)(blockIdx.x & 7u) + 1) * rb_per_xcd : row_blocks;
     const int rb_stride = (int)(gridDim.x >> 3) * 4;
-    constexpr bool SINGLE = KU < 4;  // the whole reduction is one group of KU steps (the launcher guarantees ksteps <= KU)
+    constexpr bool SINGLE = KU < 4;  // the whole reduction is one group of KU steps (the launcher guarantees ksteps == KU)
+    constexpr int WHOLE = KU == 6 ? 2 : KU == 2 ? 1 : 0;  // steps at the front that every launch of the variant has whole
 
     // where the lane's pixel of row block `rb` reads and writes
     auto locate = [&](int rb, bool &ok, size_t &in_off, size_t &out_off) {
         const int m = rb * 32 + r;
         ok = rb < rb_end && m < p.m;
-        in_off = 0;
+        in_off = (size_t)(p.a_offset + half * 16);  // (a lane without a pixel reads the first one: no branch around its loads)
         out_off = 0;
         if (ok && stage.linear) {
             in_off = (size_t)(__umul24((uint32_t)m, (uint32_t)p.cin) + (uint32_t)p.a_offset + (uint32_t)half * 16u);
@@ -140,13 +143,27 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
             out_off = (((size_t)img * p.out_h + (oy * p.out_sy + p.out_y0)) * p.out_w + (ox * p.out_sx + p.out_x0)) * (size_t)p.ldc;
         }
     };
-    // 16 reduction bytes of step ks; bytes past K read as the byte that the sign flip turns into 0
-    auto load_a = [&](bool ok, size_t in_off, int ks, uint2 &lo, uint2 &hi) {
-        const int kb = ks * 32 + half * 16;
-        lo = make_uint2(p.a_xor, p.a_xor);
-        hi = lo;
-        if (ok && kb < p.k) lo = *reinterpret_cast<const uint2 *>(p.a + in_off + ks * 32);
-        if (ok && kb + 8 < p.k) hi = *reinterpret_cast<const uint2 *>(p.a + in_off + ks * 32 + 8);
+    // 16 reduction bytes of step ks < ksteps, in one load.  In a last step that ends early the bytes past K are read from the
+    // pixel's first ones and replaced by the byte that the sign flip turns into 0.  (Two loads of 8 bytes, each in a branch of its
+    // lane's own, and the steps that a reduction lacks read all the same, took at 32 images 4.48 us instead of 4.08 for 96 -> 24 at
+    // 56x56, 5.36 instead of 4.45 for 144 -> 24, 4.63 instead of 4.20 for 96 -> 576 at 14x14, 5.33 instead of 4.40 for 256 -> 40.)
+    const int full = p.k >> 5, tail = p.k & ~31, behind = p.k - tail - half * 16;  // (whole steps; bytes this lane has in the last one)
+    const int tail_lo = behind > 0 ? tail : -(half * 16), tail_hi = behind > 8 ? tail + 8 : -(half * 16);
+    auto load_a = [&](size_t in_off, int ks, uint2 &lo, uint2 &hi) {
+        const uint8_t *const row = p.a + in_off;
+        if (ks < WHOLE || ks < full) {
+            const u32x4_a8 v = *reinterpret_cast<const u32x4_a8 *>(row + ks * 32);
+            lo = make_uint2(v.x, v.y);
+            hi = make_uint2(v.z, v.w);
+        } else {
+            lo = *reinterpret_cast<const uint2 *>(row + tail_lo);
+            hi = *reinterpret_cast<const uint2 *>(row + tail_hi);
+        }
+    };
+    auto cut_a = [&](int ks, uint2 &lo, uint2 &hi) {
+        if (ks < WHOLE || ks < full) return;
+        if (behind <= 0) lo = make_uint2(p.a_xor, p.a_xor);
+        if (behind <= 8) hi = make_uint2(p.a_xor, p.a_xor);
     };
     auto to_fragment = [&](uint2 lo, uint2 hi, int &rowsum) {
         v4i af;
@@ -189,6 +206,7 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
             for (int g = 0; g < 4; ++g) {
                 uint32_t o0, o1, o2, o3;
                 if constexpr (QM == 2) {
+                    if (KU >= 4 && g != 0) __builtin_amdgcn_sched_barrier(0);  // (all four groups' pairs at once would cost a wavefront)
                     const int tab = nb_local * 32 + half * 16 + g * 4;
                     const int4 cm = *reinterpret_cast<const int4 *>(pcm_s + tab);
                     const int4 cf = *reinterpret_cast<const int4 *>(pcf_s + tab);
@@ -295,16 +313,19 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
         int rb = rb_first;
         locate(rb, ok, in_off, out_off);
 #pragma unroll
-        for (int t = 0; t < KU; ++t) load_a(ok, in_off, t, lo[t], hi[t]);
+        for (int t = 0; t < KU; ++t) load_a(in_off, t, lo[t], hi[t]);
         stage_weights();  // after the first activation loads are on their way: the two latencies overlap
         for (; rb < rb_end; rb += rb_stride) {
             locate(rb + rb_stride, ok_next, in_next, out_next);
 #pragma unroll
-            for (int t = 0; t < KU; ++t) load_a(ok_next, in_next, t, lo_next[t], hi_next[t]);
+            for (int t = 0; t < KU; ++t) load_a(in_next, t, lo_next[t], hi_next[t]);
             v4i af[KU];
             int rowsum = 0;
 #pragma unroll
-            for (int t = 0; t < KU; ++t) af[t] = to_fragment(lo[t], hi[t], rowsum);
+            for (int t = 0; t < KU; ++t) {
+                cut_a(t, lo[t], hi[t]);
+                af[t] = to_fragment(lo[t], hi[t], rowsum);
+            }
             int ncorr = 0;
             if constexpr (ROWSUM) {
                 rowsum += __shfl_xor(rowsum, 32);  // the other half of this pixel's reduction bytes
@@ -316,7 +337,7 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
                 for (int u = 0; u < NBU; ++u) {
                     const int nb = nb0 + u < nb_count ? nb0 + u : nb_count - 1;
 #pragma unroll
-                    for (int t = 0; t < KU; ++t) bf[u][t] = b_s[(nb * ksteps + (t < ksteps ? t : ksteps - 1)) * 64 + lane];
+                    for (int t = 0; t < KU; ++t) bf[u][t] = b_s[(nb * ksteps + t) * 64 + lane];
                 }
 #pragma unroll
                 for (int u = 0; u < NBU; ++u) {
@@ -351,15 +372,18 @@ __global__ __launch_bounds__(256) void direct_gemm_kernel(const std::conditional
 #pragma unroll
                 for (int u = 0; u < NBU; ++u) acc[u] = start_block(nb0 + u < nb_count ? nb0 + u : nb_count - 1, 0);
                 int rowsum = 0;
-                for (int ks0 = 0; ks0 < ksteps; ks0 += KU) {
-                    // steps past the last one read bytes that flip to 0, so they multiply whatever weights they re-read by zero
+                for (int ks0 = 0; ks0 < (KU == 6 ? 1 : ksteps); ks0 += KU) {  // (six: the launcher guarantees 3 <= ksteps <= 6)
                     uint2 lo[KU], hi[KU];
+                    const int steps = ksteps - ks0;
 #pragma unroll
-                    for (int t = 0; t < KU; ++t) load_a(ok, in_off, ks0 + t, lo[t], hi[t]);
+                    for (int t = 0; t < KU; ++t)
+                        if (t < (KU == 6 ? 3 : 1) || t < steps) load_a(in_off, ks0 + t, lo[t], hi[t]);
 #pragma unroll
                     for (int t = 0; t < KU; ++t) {
+                        if (t >= (KU == 6 ? 3 : 1) && t >= steps) break;
+                        const int ks = ks0 + t;
+                        cut_a(ks, lo[t], hi[t]);
                         const v4i af = to_fragment(lo[t], hi[t], rowsum);
-                        const int ks = ks0 + t < ksteps ? ks0 + t : ksteps - 1;
 #pragma unroll
                         for (int u = 0; u < NBU; ++u) {
                             const int nb = nb0 + u < nb_count ? nb0 + u : nb_count - 1;
