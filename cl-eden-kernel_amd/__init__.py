@@ -260,7 +260,8 @@ def probe_mfma_i8(iterations=100000, toggling_operands=True):
 
 def requant_apply(q, acc, two_step=False, channel_form=None):
     """Host evaluation of the kernels' requantization of int32 accumulators; returns (uint8 array, used_single_shift).
-    channel_form: "registers" or "table" evaluates the per-channel single-shift forms with q's pair as the channel's;
+    channel_form: "registers" or "table" evaluates the per-channel single-shift forms with q's pair as the channel's
+    (one value from the pair as it is; four values from multipliers and shift bytes, as kernels keep them in tables);
     "packed" the per-tensor single-shift form four outputs at a time with a row term folded into the rounding term."""
     acc = np.ascontiguousarray(acc, np.int32)
     out = np.empty(acc.shape, np.uint8)

@@ -446,7 +446,7 @@ struct GemmOp {
         // padded so that the kernels may read whole channel blocks
         if (!pc_multiplier && (rc = dev_alloc(&pc_multiplier, (size_t)cout + 512))) return rc;
         if (!pc_shift && (rc = dev_alloc(&pc_shift, (size_t)cout + 512))) return rc;
-        pc_fast = all_pairs_fast(multipliers, shifts, cout, -2);  // the table form's rounding term needs rs >= 2
+        pc_fast = all_pairs_fast(multipliers, shifts, cout, -2);  // (the four-channel form needs shifts of two and more)
         if ((rc = upload_padded_pairs(pc_multiplier, pc_shift, multipliers, shifts, cout, 512, stream))) return rc;
         for (auto &g : parts) {
             if (g.n_period == 0) continue;
@@ -722,7 +722,8 @@ struct eh_dwconv_plan {
     bool packed_valid = false;
     bool w_signed = false, io_signed = false, has_bias = true;
     int32_t *pc_multiplier = nullptr, *pc_shift = nullptr;  // [cout + 4] once per-channel pairs are set
-    bool pc_fast = false;  // every pair is inside the single-shift form's range
+    bool pc_fast = false;   // every pair is inside the single-shift form's range
+    bool pc_fours = false;  // ... and inside that of its four-channel form
     // 3x3 channels-last plans: the 8-bit dot product form of the weights, usable while every w - zp_w fits int8
     int32_t *w_trip = nullptr, *bias_trip = nullptr;
     int32_t *w_fold = nullptr, *bias_fold = nullptr;  // the unsigned form of the same plans, for weights of any range
@@ -760,15 +761,22 @@ int eh_requant_apply(const eh_requant *q, const int32_t *acc, uint8_t *out, int6
     if (form == 2 || form == 3) {  // the per-channel single-shift forms, with the requant's pair as the channel's
         EH_REQUIRE(channel_pair_is_fast(q->multiplier, q->shift, form == 3 ? -2 : -1) && channel_fast_mode(*q) != 0,
                    "requant_apply: multiplier %d, shift %d, zero point %d are outside form %d", q->multiplier, q->shift, q->zp_out, form);
-        const int mode = channel_fast_mode(*q), rs = -q->shift;
+        const int mode = channel_fast_mode(*q);
         if (single_shift) *single_shift = 1;
         for (int64_t i = 0; i < count; ++i) {
             uint32_t v;
-            if (form == 2)
+            if (form == 2) {
                 v = mode == 2 ? requant_u8_channel_fast<2>(acc[i], q->multiplier, q->shift, r) : requant_u8_channel_fast<1>(acc[i], q->multiplier, q->shift, r);
-            else
-                v = mode == 2 ? requant_u8_channel_table<2>(acc[i], q->multiplier, rs - 1, channel_table_pos_hi(q->zp_out, rs), r)
-                              : requant_u8_channel_table<1>(acc[i], q->multiplier, rs - 1, channel_table_pos_hi(q->zp_out, rs), r);
+            } else {  // (four at a time: the value in each place in turn, beside others)
+                const int4 m = make_int4(q->multiplier, q->multiplier, q->multiplier, q->multiplier);
+                const int32_t other = acc[count - 1 - i];
+                const int place = (int)(i & 3);
+                int32_t x[4] = {other, other, other, other};
+                x[place] = acc[i];
+                const uint32_t e4 = channel_shift_bytes(make_int4(q->shift, q->shift, q->shift, q->shift));
+                const uint32_t w = mode == 2 ? requant4_channel<2>(x[0], x[1], x[2], x[3], m, e4, r) : requant4_channel<1>(x[0], x[1], x[2], x[3], m, e4, r);
+                v = (w >> (8 * place)) & 255u;
+            }
             out[i] = (uint8_t)v;
         }
         return EH_OK;
@@ -1937,6 +1945,7 @@ int eh_dwconv2d_u8_set_perchannel(eh_dwconv_plan *plan, const int32_t *multiplie
     if (!plan->pc_multiplier && (rc = dev_alloc(&plan->pc_multiplier, padded))) return rc;
     if (!plan->pc_shift && (rc = dev_alloc(&plan->pc_shift, padded))) return rc;
     plan->pc_fast = all_pairs_fast(multipliers, shifts, count);
+    plan->pc_fours = all_pairs_fast(multipliers, shifts, count, -2);
     return upload_padded_pairs(plan->pc_multiplier, plan->pc_shift, multipliers, shifts, count, 4, s);
 }
 
@@ -2076,7 +2085,8 @@ int eh_conv_dw_block_run(eh_conv_plan *pointwise, eh_dwconv_plan *depthwise, con
     if ((rc = pointwise->op.refold(*q_pointwise, s))) return rc;
     if ((rc = dw_refold(depthwise, *q_depthwise, s))) return rc;
     const GemmProblem pw = pointwise->op.problem(pointwise->op.parts[0], static_cast<const uint8_t *>(input), nullptr, nullptr, nullptr);
-    const DwProblem dw = dw_problem(depthwise, nullptr, output);
+    DwProblem dw = dw_problem(depthwise, nullptr, output);
+    if (depthwise->pc_multiplier && !depthwise->pc_fours) dw.rq.fast = 0;  // (a shift of -1: the kernel's other form is the two-step order)
     const int32_t ks = pw.k_pad / 32;
     if (depthwise->block_ks != ks || depthwise->block_rows != rows_per_tile || depthwise->block_cols != cols_per_tile) {
         depthwise->block_ks = 0;

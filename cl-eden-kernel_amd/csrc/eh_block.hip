@@ -66,9 +66,10 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
     extern __shared__ __align__(16) uint8_t lds_raw[];
     v4i *b_s = reinterpret_cast<v4i *>(lds_raw);                              // [nb][ks][64 lanes]: pointwise weights, fragment order
     int32_t *bias_s = reinterpret_cast<int32_t *>(lds_raw + (size_t)g.nb * ksteps * 1024);  // [nb * 32]
-    // PC (one multiplier and shift per channel in both operators): the pointwise stage's pairs beside the bias, as the
-    // single-shift form's table (multiplier, right shift - 1, high word of the rounding term) or, two-step, as they are
-    int32_t *pcm_s = bias_s + g.nb * 32, *pcf_s = pcm_s + g.nb * 32, *pch_s = pcf_s + g.nb * 32;
+    // PC (one multiplier and shift per channel in both operators): the pointwise stage's pairs beside the bias; the shifts as the
+    // bytes that requant4_channel wants or, two-step, as they are
+    int32_t *pcm_s = bias_s + g.nb * 32, *pcf_s = pcm_s + g.nb * 32;
+    uint8_t *pce_s = reinterpret_cast<uint8_t *>(pcf_s);
     uint8_t *img_s = lds_raw + g.image_off;                                   // [ih][iwp][cpitch] uint8 (xor 0x80 for the signed form)
     const int nb_first = blockIdx.y * g.nb;                                   // this workgroup's channel range
     const int c_first = nb_first * 32;
@@ -162,8 +163,10 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
             for (int i = tid; i < nb_here * 32; i += 256) {
                 const int32_t m = pw.rq.pc_multiplier[c_first + i], sh = pw.rq.pc_shift[c_first + i];
                 pcm_s[i] = m;
-                pcf_s[i] = QM != 0 ? -sh - 1 : sh;
-                pch_s[i] = QM != 0 ? channel_table_pos_hi(pw.rq.zp_out, -sh) : 0;
+                if constexpr (QM != 0)
+                    pce_s[i] = (uint8_t)(-2 - sh);
+                else
+                    pcf_s[i] = sh;
             }
         }
         wait_vmcnt<0>();
@@ -227,26 +230,21 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
                     acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(bw[ks * 64], *reinterpret_cast<const v4i *>(arow + ks * 32), acc, 0, 0, 0);
             }
             uint32_t packed[4];
+            v4i e16 = {0, 0, 0, 0};
+            if constexpr (PC && QM != 0) e16 = *reinterpret_cast<const v4i *>(pce_s + nb * 32 + half * 16);
 #pragma unroll
             for (int gq = 0; gq < 4; ++gq) {
                 if constexpr (PC) {
                     const int tab = nb * 32 + half * 16 + gq * 4;
                     const int4 cm = *reinterpret_cast<const int4 *>(pcm_s + tab);
-                    const int4 cf = *reinterpret_cast<const int4 *>(pcf_s + tab);
-                    uint32_t o0, o1, o2, o3;
                     if constexpr (QM != 0) {
-                        const int4 ch = *reinterpret_cast<const int4 *>(pch_s + tab);
-                        o0 = requant_u8_channel_table<QM>(acc[gq * 4 + 0] + ncorr, cm.x, cf.x, ch.x, rq);
-                        o1 = requant_u8_channel_table<QM>(acc[gq * 4 + 1] + ncorr, cm.y, cf.y, ch.y, rq);
-                        o2 = requant_u8_channel_table<QM>(acc[gq * 4 + 2] + ncorr, cm.z, cf.z, ch.z, rq);
-                        o3 = requant_u8_channel_table<QM>(acc[gq * 4 + 3] + ncorr, cm.w, cf.w, ch.w, rq);
+                        packed[gq] = requant4_channel<QM>(acc[gq * 4 + 0] + ncorr, acc[gq * 4 + 1] + ncorr, acc[gq * 4 + 2] + ncorr, acc[gq * 4 + 3] + ncorr, cm,
+                                                          (uint32_t)e16[gq], rq);
                     } else {
-                        o0 = requant_u8_channel(acc[gq * 4 + 0] + ncorr, cm.x, cf.x, rq);
-                        o1 = requant_u8_channel(acc[gq * 4 + 1] + ncorr, cm.y, cf.y, rq);
-                        o2 = requant_u8_channel(acc[gq * 4 + 2] + ncorr, cm.z, cf.z, rq);
-                        o3 = requant_u8_channel(acc[gq * 4 + 3] + ncorr, cm.w, cf.w, rq);
+                        const int4 cf = *reinterpret_cast<const int4 *>(pcf_s + tab);
+                        packed[gq] = pack_bytes(requant_u8_channel(acc[gq * 4 + 0] + ncorr, cm.x, cf.x, rq), requant_u8_channel(acc[gq * 4 + 1] + ncorr, cm.y, cf.y, rq),
+                                                requant_u8_channel(acc[gq * 4 + 2] + ncorr, cm.z, cf.z, rq), requant_u8_channel(acc[gq * 4 + 3] + ncorr, cm.w, cf.w, rq));
                     }
-                    packed[gq] = pack_bytes(o0, o1, o2, o3);
                 } else if constexpr (QM != 0) {
                     packed[gq] = requant4_fast<QM>(acc[gq * 4 + 0], acc[gq * 4 + 1], acc[gq * 4 + 2], acc[gq * 4 + 3], ncorr, rq);
                 } else {
@@ -272,12 +270,9 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
     auto finish = [&](int a0, int a1, int a2, int a3, const int4 &m, const int4 &sh) {
         const RequantDev &drq = dw.rq;
         if constexpr (PC) {
-            if (drq.fast == 2)
-                return pack_bytes(requant_u8_channel_fast<2>(a0, m.x, sh.x, drq), requant_u8_channel_fast<2>(a1, m.y, sh.y, drq),
-                                  requant_u8_channel_fast<2>(a2, m.z, sh.z, drq), requant_u8_channel_fast<2>(a3, m.w, sh.w, drq));
-            if (drq.fast)
-                return pack_bytes(requant_u8_channel_fast<1>(a0, m.x, sh.x, drq), requant_u8_channel_fast<1>(a1, m.y, sh.y, drq),
-                                  requant_u8_channel_fast<1>(a2, m.z, sh.z, drq), requant_u8_channel_fast<1>(a3, m.w, sh.w, drq));
+            // (the caller clears `fast` unless every pair fits the four-channel form)
+            if (drq.fast == 2) return requant4_channel<2>(a0, a1, a2, a3, m, channel_shift_bytes(sh), drq);
+            if (drq.fast) return requant4_channel<1>(a0, a1, a2, a3, m, channel_shift_bytes(sh), drq);
             return pack_bytes(requant_u8_channel(a0, m.x, sh.x, drq), requant_u8_channel(a1, m.y, sh.y, drq), requant_u8_channel(a2, m.z, sh.z, drq),
                               requant_u8_channel(a3, m.w, sh.w, drq));
         }
@@ -411,7 +406,7 @@ int block_image_pitch(int nb, int c) {
 }
 
 size_t block_lds_bytes(int nb, int ks, int ih, int iwp, int c, uint32_t *a_off, uint32_t *image_off) {
-    const size_t head = ((size_t)nb * ks * 1024 + (size_t)nb * 512 + 15) & ~(size_t)15;  // weights, bias, three per-channel tables
+    const size_t head = ((size_t)nb * ks * 1024 + (size_t)nb * 512 + 15) & ~(size_t)15;  // weights, bias, per-channel pairs
     const size_t a_bytes = ((size_t)ih * iwp * (ks * 32 + 16) + 15) & ~(size_t)15;
     if (a_off) *a_off = (uint32_t)head;
     if (image_off) *image_off = (uint32_t)(head + a_bytes);

@@ -235,6 +235,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         if (ks < KS) multiply(b0{});  // odd step count: the last step sits in the first set
 
         // ---- epilogue: 16 consecutive channels of one pixel per lane and channel block
+        int4 cm[PC && QM != 0 ? NBW : 1][4];
+        uint32_t e4[PC && QM != 0 ? NBW : 1][4];
+        if constexpr (PC && QM != 0) {  // (read ahead of the stores, which may alias them as far as the compiler knows; the arrays cover whole blocks)
+#pragma unroll
+            for (int nbw = 0; nbw < NBW; ++nbw)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    const int n = (nb_first + nb_lo + nbw) * 32 + half * 16 + q4 * 4;
+                    cm[nbw][q4] = *reinterpret_cast<const int4 *>(rq.pc_multiplier + n);
+                    e4[nbw][q4] = channel_shift_bytes(*reinterpret_cast<const int4 *>(rq.pc_shift + n));
+                }
+        }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const int pidx = (g0 + GW * g) * 32 + r;
@@ -252,16 +264,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
                     const int32_t x0 = acc[g][nbw][q4 * 4 + 0], x1 = acc[g][nbw][q4 * 4 + 1];
                     const int32_t x2 = acc[g][nbw][q4 * 4 + 2], x3 = acc[g][nbw][q4 * 4 + 3];
                     uint32_t o0, o1, o2, o3;
-                    if constexpr (PC) {  // the padded per-channel arrays cover whole blocks
-                        const int4 cm = *reinterpret_cast<const int4 *>(rq.pc_multiplier + n + q4 * 4);
-                        const int4 cs = *reinterpret_cast<const int4 *>(rq.pc_shift + n + q4 * 4);
-                        if constexpr (QM != 0) {
-                            o0 = requant_u8_channel_fast<QM>(x0, cm.x, cs.x, rq), o1 = requant_u8_channel_fast<QM>(x1, cm.y, cs.y, rq);
-                            o2 = requant_u8_channel_fast<QM>(x2, cm.z, cs.z, rq), o3 = requant_u8_channel_fast<QM>(x3, cm.w, cs.w, rq);
-                        } else {
-                            o0 = requant_u8_channel(x0, cm.x, cs.x, rq), o1 = requant_u8_channel(x1, cm.y, cs.y, rq);
-                            o2 = requant_u8_channel(x2, cm.z, cs.z, rq), o3 = requant_u8_channel(x3, cm.w, cs.w, rq);
-                        }
+                    if constexpr (PC && QM != 0) {
+                        packed[q4] = requant4_channel<QM>(x0, x1, x2, x3, cm[nbw][q4], e4[nbw][q4], rq) ^ p.out_xor;
+                        continue;
+                    } else if constexpr (PC) {
+                        const int4 m = *reinterpret_cast<const int4 *>(rq.pc_multiplier + n + q4 * 4);
+                        const int4 sh = *reinterpret_cast<const int4 *>(rq.pc_shift + n + q4 * 4);
+                        o0 = requant_u8_channel(x0, m.x, sh.x, rq), o1 = requant_u8_channel(x1, m.y, sh.y, rq);
+                        o2 = requant_u8_channel(x2, m.z, sh.z, rq), o3 = requant_u8_channel(x3, m.w, sh.w, rq);
                     } else if constexpr (QM != 0) {
                         packed[q4] = requant4_fast<QM>(x0, x1, x2, x3, late, rq) ^ p.out_xor;
                         continue;

@@ -17,8 +17,8 @@
 // Bound by its instructions (about 350 to a wavefront of 64 pixels x 32 channels, half of them requantization) once the
 // loads are together: 224x224, stride 2, 32 channels, before and after the rows, the weights and the bias (and a channel's
 // pair) were requested ahead of their first use: one image 3.95 -> 3.20 us, 32 images 9.31 -> 7.77, 64 images
-// 13.54 -> 11.50; with a pair per channel 4.62 -> 3.47, 11.43 -> 9.76 and 18.74 -> 15.61; 160x160 to 96 channels,
-// 8 images 8.81 -> 5.96.  With fewer than 32 channels: 224x224 to 16, 32 images 7.17 -> 6.89.
+// 13.54 -> 11.50; with a pair per channel 4.62 -> 3.47, 11.43 -> 9.76 and 18.74 -> 15.61 (14.41 with the four-channel
+// requantization); 160x160 to 96 channels, 8 images 8.81 -> 5.96.  With fewer than 32 channels: 224x224 to 16, 32 images 7.17 -> 6.89.
 //
 // Stands in for the reference's direct convolution kernels on this shape
 // (gpu/operators/cl_kernels/DirectConvolutionKernel.cpp, 3x3 uint8 variants).
@@ -188,17 +188,14 @@ __global__ __launch_bounds__(256) void conv_c3k3_mfma_kernel(const GemmProblem p
                 constexpr int mode = decltype(mode_c)::value;
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    if constexpr (PC) {
+                    if constexpr (PC && mode != 0)
+                        packed[g] = requant4_channel<mode>(acc[g * 4 + 0], acc[g * 4 + 1], acc[g * 4 + 2], acc[g * 4 + 3], mult[g], channel_shift_bytes(shift[g]), rq) ^ p.out_xor;
+                    else if constexpr (PC) {
                         auto one = [&](int x, int32_t mu, int32_t sh) {
 #if defined(__HIP_DEVICE_COMPILE__)
-                            // (the channel's rounding term is worked out for each block: 16 of them kept for both, at two
-                            // registers each, would leave two wavefronts to a SIMD)
-                            asm("" : "+v"(sh));
+                            asm("" : "+v"(sh));  // (a channel's terms are worked out for each block: kept for both they would cost a wavefront)
 #endif
-                            if constexpr (mode == 0)
-                                return requant_u8_channel(x, mu, sh, rq);
-                            else
-                                return requant_u8_channel_fast<mode>(x, mu, sh, rq);
+                            return requant_u8_channel(x, mu, sh, rq);
                         };
                         packed[g] = pack_bytes(one(acc[g * 4 + 0], mult[g].x, shift[g].x), one(acc[g * 4 + 1], mult[g].y, shift[g].y),
                                                one(acc[g * 4 + 2], mult[g].z, shift[g].z), one(acc[g * 4 + 3], mult[g].w, shift[g].w)) ^

@@ -59,7 +59,7 @@ __device__ __forceinline__ const GemmProblem &problem_of(const GemmBatch &batch)
 
 // (six steps in flight: bounded to four wavefronts per SIMD; with three, 96 -> 24 with a pair per channel took 5.69 us instead of 4.28)
 template <int NBU, int KU, bool ROWSUM, int QM, bool RES, bool BATCHED = false, bool PLANAR = false>
-__global__ __launch_bounds__(256, KU == 6 ? 4 : 1) void direct_gemm_kernel(const std::conditional_t<BATCHED, GemmBatch, GemmProblem> arg, const int n_blocks,
+__global__ __launch_bounds__(256, KU == 6 && !BATCHED ? 4 : 1) void direct_gemm_kernel(const std::conditional_t<BATCHED, GemmBatch, GemmProblem> arg, const int n_blocks,
                                                           const int ksteps, const int nbw, const int row_blocks, const ThinStage stage) {
     // BATCHED: equally shaped problems of one operator (the output phases of a transposed convolution whose kernel is its
     // stride) that differ in their weights and in where their outputs go.  (A kernel of its own: indexing the argument
@@ -77,21 +77,19 @@ __global__ __launch_bounds__(256, KU == 6 ? 4 : 1) void direct_gemm_kernel(const
     int32_t *bias_s = reinterpret_cast<int32_t *>(lds_raw + (size_t)nbw * ksteps * 1024);  // [nbw * 32]
     // fused residual add: the rescaled value of every possible residual byte and of every possible result byte, so that
     // an output costs two lookups and one rescaling instead of three rescalings
-    // per-channel single-shift tables, only with QM == 2: multiplier, right shift - 1, high word of the rounding term
-    int32_t *pcm_s = bias_s + nbw * 32, *pcf_s = pcm_s + nbw * 32, *pch_s = pcf_s + nbw * 32;
-    int32_t *add_a_s = bias_s + (QM == 2 ? 4 : 1) * nbw * 32, *add_b_s = add_a_s + 256;  // [256] each, only with RES
+    // only with QM == 2: the channels' multipliers and, a byte each, what requant4_channel wants of their shifts
+    int32_t *pcm_s = bias_s + nbw * 32;
+    uint8_t *pce_s = reinterpret_cast<uint8_t *>(pcm_s + nbw * 32);
+    int32_t *add_a_s = bias_s + (QM == 2 ? 2 * 32 + 8 : 32) * nbw, *add_b_s = add_a_s + 256;  // [256] each, only with RES
     auto stage_weights = [&]() {
         // direct-to-LDS copies, every KiB on its way at once (a loop of loads and LDS stores waits a trip to L2 for each of its up to
         // eight turns; MobileNetV2 on 64 images, whose launches are mostly this kernel's, 444.3 -> 437.8 us)
         dma_linear<4>(p.b + (size_t)nb_first * ksteps * 1024, lds_offset(lds_raw), nb_count * ksteps, __builtin_amdgcn_readfirstlane(wave), lane);
         for (int i = threadIdx.x; i < nb_count * 32; i += 256) bias_s[i] = p.bias[nb_first * 32 + i];
         if constexpr (QM == 2) {
-            // rounding term 2^30 + (1 + 2 zp_out) 2^(30 + rs) for rs >= 2: low word 2^30, high word (1 + 2 zp_out) 2^(rs - 2)
             for (int i = threadIdx.x; i < nb_count * 32; i += 256) {
-                const int32_t rs = -p.rq.pc_shift[nb_first * 32 + i];
                 pcm_s[i] = p.rq.pc_multiplier[nb_first * 32 + i];
-                pcf_s[i] = rs - 1;
-                pch_s[i] = channel_table_pos_hi(p.rq.zp_out, rs);
+                pce_s[i] = (uint8_t)(-2 - p.rq.pc_shift[nb_first * 32 + i]);
             }
         }
         if constexpr (RES) {
@@ -202,19 +200,17 @@ __global__ __launch_bounds__(256, KU == 6 ? 4 : 1) void direct_gemm_kernel(const
         uint32_t packed[4];
         auto quantize = [&](auto mode_c) {
             constexpr int mode = decltype(mode_c)::value;
+            v4i e16 = {0, 0, 0, 0};
+            if constexpr (QM == 2) e16 = *reinterpret_cast<const v4i *>(pce_s + nb_local * 32 + half * 16);
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 uint32_t o0, o1, o2, o3;
                 if constexpr (QM == 2) {
-                    if (KU >= 4 && g != 0) __builtin_amdgcn_sched_barrier(0);  // (all four groups' pairs at once would cost a wavefront)
-                    const int tab = nb_local * 32 + half * 16 + g * 4;
-                    const int4 cm = *reinterpret_cast<const int4 *>(pcm_s + tab);
-                    const int4 cf = *reinterpret_cast<const int4 *>(pcf_s + tab);
-                    const int4 ch = *reinterpret_cast<const int4 *>(pch_s + tab);
-                    o0 = requant_u8_channel_table<mode>(acc[g * 4 + 0] + ncorr, cm.x, cf.x, ch.x, rq);
-                    o1 = requant_u8_channel_table<mode>(acc[g * 4 + 1] + ncorr, cm.y, cf.y, ch.y, rq);
-                    o2 = requant_u8_channel_table<mode>(acc[g * 4 + 2] + ncorr, cm.z, cf.z, ch.z, rq);
-                    o3 = requant_u8_channel_table<mode>(acc[g * 4 + 3] + ncorr, cm.w, cf.w, ch.w, rq);
+                    const int4 cm = *reinterpret_cast<const int4 *>(pcm_s + nb_local * 32 + half * 16 + g * 4);
+                    packed[g] = requant4_channel<mode>(acc[g * 4 + 0] + ncorr, acc[g * 4 + 1] + ncorr, acc[g * 4 + 2] + ncorr, acc[g * 4 + 3] + ncorr, cm,
+                                                       (uint32_t)e16[g], rq) ^
+                                p.out_xor;
+                    continue;
                 } else if (mode == 0 && rq.pc_multiplier) {  // per-channel parameters (the padded arrays cover whole blocks)
                     const int4 cm = *reinterpret_cast<const int4 *>(rq.pc_multiplier + n + g * 4);
                     const int4 cs = *reinterpret_cast<const int4 *>(rq.pc_shift + n + g * 4);
@@ -429,7 +425,7 @@ int launch_nbu(const TapProblem *ps, int count, hipStream_t stream) {
     const int nbw = (groups_total + ranges - 1) / ranges * NBU;
     ranges = (n_blocks + nbw - 1) / nbw;
     const bool pc_fast = p.rq.fast && p.rq.pc_multiplier;
-    const size_t lds = (size_t)nbw * ksteps * 1024 + (size_t)nbw * 32 * sizeof(int32_t) * (pc_fast ? 4 : 1) +
+    const size_t lds = (size_t)nbw * ksteps * 1024 + (size_t)nbw * 32 * (pc_fast ? 2 * sizeof(int32_t) + 1 : sizeof(int32_t)) +
                        (p.residual ? 2 * 256 * sizeof(int32_t) : 0);
     EH_REQUIRE(lds <= 64 * 1024, "igemm_thin: %zu bytes of LDS for the weights", lds);
     // Staged output where a workgroup owns whole, densely stored pixels of at most 256 bytes (wider pixels already fill

@@ -211,28 +211,61 @@ __host__ __device__ __forceinline__ uint32_t requant_u8_channel_fast(int32_t x, 
     return (uint32_t)v;
 }
 
-// The same with the channel's terms from a table: `fs` = rs - 1 and `pos_hi` = (1 + 2 zp) 2^(rs - 2), the high word
-// of the rounding term, whose low word is 2^30 for every rs >= 2.  For a negative accumulator the term is 2^31
-// less: the low word gains bit 31 and the high word lends one.
+// Four channels at a time, for shifts of two and more.  With z = 1 + 2 zp the numerator's channel term is z 2^(rs - 2) in the high
+// word, so with h the high word of x M + 2^30 (2^31 less where x < 0)
+//     result + zp = (h + z 2^(rs - 2)) >> (rs - 1) = ((h >> (rs - 2)) + z) >> 1,
+// and all that a kernel keeps per channel is the multiplier and a byte, rs - 2: four of them to a word, `e4` (see
+// channel_shift_bytes), from which the first shift takes its amount as an SDWA operand.  The clamp goes before the last shift,
+// which then writes the byte, as in requant4_fast (its bounds on act_min and act_max hold here).
+// Before, kernels kept a table of multiplier, rs - 1 and z 2^(rs - 2) in LDS, twelve reads of 16 bytes for sixteen results instead of
+// five and 48 registers instead of 20, or worked the 64-bit term out for each use.  32 images, us: one tap 16 -> 96 at 112x112
+// 19.8 -> 15.8, 32 -> 16 7.5 -> 7.0, 24 -> 144 at 56x56 9.7 -> 8.9, 64 -> 256 15.3 -> 13.4, 64 -> 384 at 14x14 4.7 -> 4.45; first layer
+// of 64 images 15.6 -> 14.4; 3x3 128 -> 128 at 28x28 11.0 -> 10.7; expansion and depthwise 16 -> 96 at 112x112 stride 2, 16 images
+// 17.5 -> 16.5.
+// (Kernels that finish each value once from global memory, without a register to spare, or two of a channel quad, keep
+// requant_u8_channel_fast: packing the bytes costs what the shorter form saves.  7x7 first layer 10.1 us, with this form 10.4.)
 template <int MODE>
-__host__ __device__ __forceinline__ uint32_t requant_u8_channel_table(int32_t x, int32_t multiplier, int32_t fs, int32_t pos_hi,
-                                                                      const RequantDev &r) {
-    uint32_t lo = 0x40000000u;
-    int32_t hi = pos_hi;
-    if (MODE != 2) {
-        lo |= (uint32_t)x & 0x80000000u;
-        hi += x >> 31;
-    }
-    const int64_t t = (int64_t)x * (int64_t)multiplier + (int64_t)(((uint64_t)(uint32_t)hi << 32) | lo);
-    int32_t v = (int32_t)(t >> 32) >> fs;
-    v = v < r.act_min ? r.act_min : v;
-    v = v > r.act_max ? r.act_max : v;
-    return (uint32_t)v;
+__host__ __device__ __forceinline__ uint32_t requant4_channel(int32_t x0, int32_t x1, int32_t x2, int32_t x3, const int4 &m, uint32_t e4, const RequantDev &r) {
+    static_assert(MODE == 1 || MODE == 2, "single-shift forms only");
+    auto high = [&](int32_t x, int32_t multiplier) {
+        const uint32_t lo = MODE == 1 ? ((uint32_t)x & 0x80000000u) | 0x40000000u : 0x40000000u;
+        const uint32_t hi = MODE == 1 ? (uint32_t)(x >> 31) : 0u;
+        return (int32_t)(((int64_t)x * (int64_t)multiplier + (int64_t)(((uint64_t)hi << 32) | lo)) >> 32);
+    };
+    const int32_t z = 1 + 2 * r.zp_out, lowest = 2 * r.act_min, highest = 2 * r.act_max + 1;
+    int32_t h0 = high(x0, m.x), h1 = high(x1, m.y), h2 = high(x2, m.z), h3 = high(x3, m.w);
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_ashrrev_i32_sdwa %0, %1, %0 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0 src1_sel:DWORD" : "+v"(h0) : "v"(e4));
+    asm("v_ashrrev_i32_sdwa %0, %1, %0 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1 src1_sel:DWORD" : "+v"(h1) : "v"(e4));
+    asm("v_ashrrev_i32_sdwa %0, %1, %0 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2 src1_sel:DWORD" : "+v"(h2) : "v"(e4));
+    asm("v_ashrrev_i32_sdwa %0, %1, %0 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3 src1_sel:DWORD" : "+v"(h3) : "v"(e4));
+    auto clamp = [&](int32_t h) {
+        int32_t o;
+        asm("v_med3_i32 %0, %1, %2, %3" : "=v"(o) : "v"(h + z), "s"(lowest), "v"(highest));
+        return o;
+    };
+    h0 = clamp(h0);
+    h1 = clamp(h1);
+    h2 = clamp(h2);
+    h3 = clamp(h3);
+    uint32_t w;
+    asm("v_lshrrev_b32_sdwa %0, %1, %2 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:DWORD" : "=v"(w) : "v"(1), "v"(h0));
+    asm("v_lshrrev_b32_sdwa %0, %1, %2 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD" : "+v"(w) : "v"(1), "v"(h1));
+    asm("v_lshrrev_b32_sdwa %0, %1, %2 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD" : "+v"(w) : "v"(1), "v"(h2));
+    asm("v_lshrrev_b32_sdwa %0, %1, %2 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD" : "+v"(w) : "v"(1), "v"(h3));
+    return w;
+#else
+    auto rest = [&](int32_t h, int k) {
+        const int32_t v = (h >> ((e4 >> (8 * k)) & 31u)) + z;
+        return (uint32_t)((v < lowest ? lowest : v > highest ? highest : v) >> 1);
+    };
+    return rest(h0, 0) | rest(h1, 1) << 8 | rest(h2, 2) << 16 | rest(h3, 3) << 24;
+#endif
 }
 
-// high word of the table form's rounding term for a right shift rs >= 2
-__host__ __device__ __forceinline__ int32_t channel_table_pos_hi(int32_t zp_out, int32_t rs) {
-    return (int32_t)((uint32_t)(1 + 2 * zp_out) << (rs - 2));
+// four channels' shifts (each -2 or less) as requant4_channel wants them
+__host__ __device__ __forceinline__ uint32_t channel_shift_bytes(const int4 &shift) {
+    return (uint32_t)(-2 - shift.x) | (uint32_t)(-2 - shift.y) << 8 | (uint32_t)(-2 - shift.z) << 16 | (uint32_t)(-2 - shift.w) << 24;
 }
 
 // whether the single-shift form covers a channel's pair
