@@ -479,12 +479,18 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     // four leave empty and, at a lower weight, the input bytes staged again for every channel range.
     int th = rows_per_tile, tw = cols_per_tile, nb = nb_all;
     // Where the vector form's units (sixteen outputs, some 300 instructions each) would keep at most half of a workgroup's threads
-    // busy, the matrix form spreads the depthwise stage over all four waves.  One image, us: 28x28 32 -> 192 stride 2 (8 units)
-    // 5.9 -> 4.2, 14x14 64 -> 384 (8) 5.2 -> 4.0, 7x7 160 -> 960 (8) 5.8 -> 4.5, 56x56 24 -> 144 (48) 4.4 -> 4.2; 16 images: 14x14 64 -> 384
-    // (96) 6.0 -> 5.8, but 28x28 32 -> 192 (240) 5.9 -> 6.4; 32 images: 28x28 (480) 8.7 -> 9.0, 56x56 24 -> 144 stride 2 (252) 10.9 -> 11.4.
+    // busy, the matrix form spreads the depthwise stage over all four waves, in groups of sixteen outputs by sixteen channels: one
+    // group a wave, or groups that are more than half full.  Same tiles, vector -> matrix form, us (with a pair per channel): 28x28
+    // 32 -> 192 stride 2, one image (two groups) 5.7 -> 4.2 (6.3 -> 4.8), 7x7 160 -> 960, one image 5.4 -> 4.5 (6.2 -> 4.9), four (four
+    // groups a quarter full) 5.5 -> 5.2 (6.3 -> 5.9); 14x14 96 -> 576, eight images (eight groups of twelve) 5.9 -> 5.4 (6.8 -> 6.5), but
+    // four (six groups of six) 5.1 -> 5.4 (5.8 -> 6.4), at stride 2 with sixteen images (ten groups of four) 5.9 -> 6.3 (6.8 -> 7.7);
+    // 7x7 160 -> 960, eight images (eight groups of six) 5.4 -> 5.7 (6.1 -> 6.9).  Beyond 128 units: 28x28 32 -> 192, 16 images (240)
+    // 5.9 -> 6.4, 32 images (480) 8.7 -> 9.0, 56x56 24 -> 144 stride 2 (252) 10.9 -> 11.4.
+    auto quads_of = [&](int blocks) { return blocks * 8 < dw.c / 4 ? blocks * 8 : dw.c / 4; };
+    auto small = [&](int rows, int cols, int blocks) { return dw.w_mm != nullptr && rows * ((cols + 3) / 4) * quads_of(blocks) <= 128; };
     auto matrix_form = [&](int rows, int cols, int blocks) {
-        const int quads = blocks * 8 < dw.c / 4 ? blocks * 8 : dw.c / 4;
-        return dw.w_mm != nullptr && rows * ((cols + 3) / 4) * quads <= 128;
+        const int pixel_groups = (rows * cols + 15) / 16;
+        return small(rows, cols, blocks) && (pixel_groups * (quads_of(blocks) / 4) <= 4 || rows * cols > pixel_groups * 8);
     };
     {
         double best = -1;
@@ -505,8 +511,11 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
                         const int px = ih * iw;
                         const double tiles = (double)dw.n * ((dw.ho + ch - 1) / ch) * ((dw.wo + cw - 1) / cw);
                         const double stage1 = (double)((px + 31) / 32 * 32) * tiles / ((double)dw.n * dw.h * dw.w_);   // pixel slots computed per real pixel
-                        // (a slot of the matrix form, which works on sixteen outputs, counts three quarters)
-                        const double slots = matrix_form(ch, cw, cn) ? 0.75 * ((ch * cw + 15) / 16 * 16) : (double)(ch * ((cw + 3) / 4 * 4));
+                        // (A slot of the matrix form, which works on sixteen outputs, counts three quarters.  Small tiles all count like
+                        // that: by the vector form's slots the search prefers still smaller ones, of two outputs or four, which lose to
+                        // the matrix form's: 56x56 24 -> 144 stride 2, one image 4.75 us against 3.90, 14x14 96 -> 576 stride 2, four images
+                        // 5.45 against 4.66.)
+                        const double slots = small(ch, cw, cn) ? 0.75 * ((ch * cw + 15) / 16 * 16) : (double)(ch * ((cw + 3) / 4 * 4));
                         const double stage2 = slots * tiles / ((double)dw.n * dw.ho * dw.wo);  // output slots per real output
                         const double restage = (double)px * tiles * ranges * (g.ks * 32) / ((double)dw.n * dw.h * dw.w_ * dw.c);  // staged input bytes per expanded byte
                         const double cost = stage1 + 0.5 * stage2 + 2.0 * restage;

@@ -1,7 +1,7 @@
 """The fused expansion + depthwise launch with its depthwise stage on the matrix cores, which small tiles take (up to 128 units of
-four output pixels x four channels per workgroup), and tiles just beyond that: bit for bit the oracle's chain, at groups of sixteen
-output pixels that end early, several chunks and groups per wave, waves without work, and weights whose differences from their zero
-point leave int8 on either side."""
+four output pixels x four channels per workgroup, in groups of sixteen outputs x sixteen channels, one a wave or more than half full),
+and tiles just beyond that: bit for bit the oracle's chain, at groups of sixteen output pixels that end early, several chunks and
+groups per wave, waves without work, and weights whose differences from their zero point leave int8 on either side."""
 import numpy as np
 import pytest
 
@@ -20,7 +20,9 @@ CASES = [
     (1, 11, 13, 32, 80, 1, 3, 7, 100),   # two groups, the second of five; a range that ends inside a block
     (1, 16, 16, 40, 32, 1, 8, 8, 150),   # 128 units: four groups
     (1, 16, 17, 40, 32, 1, 8, 9, 150),   # 192 units: the vector form
-    (3, 8, 8, 160, 96, 2, 2, 3, 127),    # five reduction steps
+    (3, 8, 8, 160, 96, 2, 2, 3, 127),    # five reduction steps; groups of six outputs
+    (2, 8, 8, 24, 64, 1, 2, 4, 127),     # eight outputs, half a group: the matrix form with up to four chunks to a workgroup
+    (2, 8, 8, 24, 64, 1, 3, 3, 127),     # nine: with any number
     (1, 5, 6, 16, 16, 1, 5, 6, 90),      # the whole image in one workgroup
 ]
 
