@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
             bool exists[FLIGHT];
 #pragma unroll
             for (int f = 0; f < FLIGHT; ++f) {
-                if (first + f * 256 >= pieces) break;  // (uniform)
+                if (FLIGHT > 1 && first + f * 256 + w_uniform * 64 >= pieces) break;  // (a wave without a piece fetches nothing: 7x7 160 -> 960, four images 5.22 -> 5.05 us)
                 const int i = first + f * 256 + tid < pieces ? first + f * 256 + tid : pieces - 1;
                 const int q = KS ? i / (KS * 4) : (int)fastdiv((uint32_t)i, g.div_ppp), piece = i - q * ppp;
                 int iy, ix;
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
             }
 #pragma unroll
             for (int f = 0; f < FLIGHT; ++f) {
-                if (first + f * 256 >= pieces) break;
+                if (FLIGHT > 1 && first + f * 256 + w_uniform * 64 >= pieces) break;
                 // (a thread past the last piece holds that piece as well and writes the same bytes)
                 *reinterpret_cast<uint2 *>(to[f]) = make_uint2(exists[f] ? v[f].x ^ pw.a_xor : 0u, exists[f] ? v[f].y ^ pw.a_xor : 0u);
             }
