@@ -37,7 +37,7 @@ typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 // y = channel ranges of `nbw` blocks.
 // QM: how results are requantized.  0: the two-step order (one pair, or one per channel read from global memory);
 // 1: the single-shift form with the requant's one pair; 2: the single-shift form with one pair per channel, whose
-// multiplier, shift and rounding term sit in LDS beside the bias.
+// multiplier and shift byte sit in LDS beside the bias (requant4_channel).
 // Output staging (stage_pitch != 0; launches whose workgroups own whole pixels of a densely stored output, no residual):
 // a lane's sixteen bytes go to a per-wave LDS image of the block's 32 pixels first, and the wave then writes that
 // image out as one contiguous span, 16 bytes per lane.  A pixel block's output is contiguous in memory (32 x ldc
