@@ -15,14 +15,18 @@ typedef __attribute__((address_space(3))) uint8_t lds_byte;
 __device__ __forceinline__ uint32_t lds_offset(const void *p) { return (uint32_t)(uintptr_t)(lds_byte *)p; }
 
 // One wave copies 64 x 16 bytes: active lane i's 16 bytes land at lds_base + 16 * i.  Nothing waits: s_waitcnt vmcnt before the bytes are read.
+// (m0 is an output, so that the compiler knows what it held is gone: it takes a second setting of the same value for redundant.)
 __device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base_uniform) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_base_uniform) : "memory");
+    register uint32_t m0 asm("m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : "=s"(m0) : "v"(gptr), "s"(lds_base_uniform) : "memory");
 }
 
 // The same with the address split into a wave-uniform base and a 32-bit per-lane offset.
 __device__ __forceinline__ void dma16_off(const void *base_uniform, uint32_t lane_offset, uint32_t lds_base_uniform) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base_uniform),
-                 "s"(lds_base_uniform)
+    register uint32_t m0 asm("m0");
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 : "=s"(m0)
+                 : "v"(lane_offset), "s"(base_uniform), "s"(lds_base_uniform)
                  : "memory");
 }
 

@@ -58,7 +58,8 @@ __global__ __launch_bounds__(256) void stream_probe_kernel(const uint4 *__restri
 typedef __attribute__((address_space(3))) uint8_t lds_byte;
 
 __device__ __forceinline__ void probe_dma16(const void *base_uniform, uint32_t lane_offset, uint32_t lds_base_uniform) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base_uniform), "s"(lds_base_uniform) : "memory");
+    register uint32_t m0 asm("m0");  // (written here: an output)
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : "=s"(m0) : "v"(lane_offset), "s"(base_uniform), "s"(lds_base_uniform) : "memory");
 }
 __device__ __forceinline__ v4i probe_dsread(uint32_t a) {
     v4i r;
