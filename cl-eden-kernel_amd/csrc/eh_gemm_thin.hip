@@ -455,15 +455,15 @@ int launch_nbu(const TapProblem *ps, int count, hipStream_t stream) {
                                        : reinterpret_cast<const void *>(direct_gemm_kernel<NBU, KU, RS, QM, RES, false, PL>);
         // The grid is persistent: as many workgroups as the device holds at once with this variant's registers and
         // this launch's LDS (a wave has one pixel block in flight, so the bytes in flight grow with the waves), and
-        // at least four per CU.  The answer is kept per KiB of LDS.
-        static std::atomic<int> resident[65];
-        const size_t slot = (lds_all + 1023) / 1024;
-        int per_cu = resident[slot].load(std::memory_order_relaxed);
+        // at least four per CU.  The answer is kept per kernel (a batch's has register bounds of its own) and KiB of LDS.
+        static std::atomic<int> resident[2][65];
+        std::atomic<int> &known = resident[count > 1 ? 1 : 0][(lds_all + 1023) / 1024];
+        int per_cu = known.load(std::memory_order_relaxed);
         if (per_cu == 0) {
             int n = 0;
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, 256, lds_all) != hipSuccess || n < 1) n = 4;
             per_cu = n < 4 ? 4 : (n > 8 ? 8 : n);
-            resident[slot].store(per_cu, std::memory_order_relaxed);
+            known.store(per_cu, std::memory_order_relaxed);
         }
         int row_wgs = ((row_blocks + 7) / 8 + 3) / 4 * 8;   // a multiple of 8: every XCD walks its own eighth of the row blocks
         const int wg_target = 256 * per_cu / (ranges * count) > 8 ? 256 * per_cu / (ranges * count) / 8 * 8 : 8;

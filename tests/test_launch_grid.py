@@ -1,0 +1,55 @@
+"""What is launched, without a GPU: the library runs on a stand-in for the HIP runtime (tests/hip_stub.cpp) that notes each
+launch's kernel and grid."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import importlib, sys
+import numpy as np
+sys.path.insert(0, %r)
+eden = importlib.import_module("cl-eden-kernel_amd")
+eden.init(0)
+q = eden.make_requant(0.02, 117, 0.004, 121, 0.03, 5)
+def buf(*shape, dtype=np.uint8):
+    return eden.DeviceBuffer(host=np.full(shape, 121, dtype))
+def run(plan_type, n, c, h, cout, k, stride):
+    out = h * stride if plan_type is eden.DeconvPlan else h
+    w = (c, cout, k, k) if plan_type is eden.DeconvPlan else (cout, c, k, k)
+    desc = eden.conv_desc(n, c, h, h, cout, k, k, (stride, stride), layout=eden.NHWC,
+                          weight_layout=eden.W_IOHW if plan_type is eden.DeconvPlan else eden.W_OIHW)
+    plan_type(desc, buf(*w), buf(cout, dtype=np.int32), q).run(buf(n, h, h, c), eden.DeviceBuffer(nbytes=n * out * out * cout), q)
+""" % ROOT
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-shared", "-fPIC", os.path.join(HERE, "hip_stub.cpp"), "-o", so], check=True)
+    return so
+
+
+def launches(stub, tmp_path, program, full=""):
+    """[(kernel, grid x, y, z, LDS bytes)] of a program on the stand-in"""
+    log = tmp_path / "launches"
+    log.write_text("")
+    env = dict(os.environ, LD_PRELOAD=stub, HIP_STUB_LOG=str(log), HIP_STUB_FULL=full)
+    subprocess.run([sys.executable, "-c", PRELUDE + program], check=True, env=env, cwd=ROOT)
+    return [(a[0],) + tuple(int(v) for v in a[1:]) for a in (line.split() for line in log.read_text().splitlines())]
+
+
+def test_one_tap_grid_does_not_depend_on_what_ran_before(stub, tmp_path):
+    """96 -> 16 channels as the four phases of a transposed convolution (one launch of the batched kernel) and 96 -> 24 as a
+    convolution (the plain one), of equal LDS: each grid follows its own kernel's occupancy, in either order."""
+    batched, plain = "run(eden.DeconvPlan, 16, 96, 56, 16, 2, 2)\n", "run(eden.ConvPlan, 64, 96, 56, 24, 1, 1)\n"
+    grids = []
+    for program in (batched + plain, plain + batched):
+        own = sorted(l for l in launches(stub, tmp_path, program, full="ELb0ELb1ELb0EEEv") if "direct_gemm_kernel" in l[0])
+        assert len(own) == 2 and {l[3] for l in own} == {1, 4} and own[0][4] == own[1][4], own
+        grids.append(own)
+    assert grids[0] == grids[1]
