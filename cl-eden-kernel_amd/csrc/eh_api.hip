@@ -728,7 +728,7 @@ struct eh_dwconv_plan {
     int32_t *w_trip = nullptr, *bias_trip = nullptr;
     int32_t *w_fold = nullptr, *bias_fold = nullptr;  // the unsigned form of the same plans, for weights of any range
     bool fold_valid = false;
-    uint8_t *w_mm = nullptr;      // 3x3 / 5x5 / 7x7 channels-last plans: the matrix form of the weights and its bias
+    uint8_t *w_mm = nullptr;      // 5x5 / 7x7 channels-last plans, and 3x3 ones that a fused launch takes: the matrix form of the weights and its bias
     int32_t *bias_mm = nullptr;
     bool range_known = false;   // w_lo / w_hi hold the extremes of the weight bytes (in the caller's own domain)
     int32_t w_lo = 0, w_hi = 0;
@@ -1791,6 +1791,8 @@ static int dw_set_weights(eh_dwconv_plan *pl, const void *weight, const void *bi
     return EH_OK;
 }
 
+static DwProblem dw_problem(const eh_dwconv_plan *plan, const void *input, void *output);
+
 static int dw_refold(eh_dwconv_plan *pl, const eh_requant &caller_q, hipStream_t stream) {
     const eh_requant q = pl->io_signed ? io_as_uint8(caller_q) : caller_q;  // pl->q: the uint8-equivalent input/output side
     if (!(pl->packed_valid && q.zp_in == pl->q.zp_in && q.zp_w == pl->q.zp_w)) {
@@ -1890,9 +1892,10 @@ int eh_dwconv2d_u8_plan(eh_dwconv_plan **plan, const eh_conv_desc *desc, const v
         if (!rc) rc = dev_alloc(&pl->w_fold, (size_t)3 * pl->cout);
         if (!rc) rc = dev_alloc(&pl->bias_fold, (size_t)pl->cout + 4);
     }
-    const bool tile_form_k = pl->d.layout == EH_NHWC && pl->d.kh == pl->d.kw && (pl->d.kh == 3 || pl->d.kh == 5 || pl->d.kh == 7) && pl->d.depth_multiplier == 1 &&
+    const bool wide_window = pl->d.layout == EH_NHWC && pl->d.kh == pl->d.kw && (pl->d.kh == 5 || pl->d.kh == 7) && pl->d.depth_multiplier == 1 &&
                              pl->d.dil_h == 1 && pl->d.dil_w == 1;
-    if (!rc && tile_form_k) {
+    const bool fusable = pl->d.layout == EH_NHWC && !pl->rep_dm && !pl->planar && pwdw_block_takes(dw_problem(pl, nullptr, nullptr));
+    if (!rc && (wide_window || fusable)) {
         rc = dev_alloc(&pl->w_mm, dw_mfma_weight_bytes(pl->cout, pl->d.kh));
         if (!rc) rc = dev_alloc(&pl->bias_mm, (size_t)(pl->cout + 15) / 16 * 16);
     }

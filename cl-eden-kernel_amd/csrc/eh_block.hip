@@ -415,6 +415,13 @@ size_t block_lds_bytes(int nb, int ks, int ih, int iwp, int c, uint32_t *a_off, 
 
 }  // namespace
 
+// What a depthwise layer has to be to end a fused launch, of what is fixed when its plan is made: those plans keep the matrix form of
+// their weights.
+bool pwdw_block_takes(const DwProblem &dw) {
+    return dw.kh == 3 && dw.kw == 3 && dw.dil_h == 1 && dw.dil_w == 1 && dw.stride_h == dw.stride_w && (dw.stride_h == 1 || dw.stride_h == 2) && dw.dm == 1 &&
+           dw.c == dw.cout && (dw.c & 15) == 0 && !dw.io_flip && dw.pad_t >= 0 && dw.pad_l >= 0 && dw.pad_t <= 2 && dw.pad_l <= 2;
+}
+
 // The pointwise problem is a one-tap problem of at most eight 32-byte reduction steps on whole dense images whose
 // weights are packed in fragment order, the depthwise one a 3x3 channels-last layer of stride 1 or 2 on the pointwise
 // output with the 8-bit dot product weights at hand; uint8 tensors; one requantization pair per operator, or one pair per
@@ -424,10 +431,7 @@ bool pwdw_block_applies(const GemmProblem &pw, const DwProblem &dw) {
     if (pw.stride_h != 1 || pw.stride_w != 1 || pw.y_base != 0 || pw.x_base != 0 || pw.ho != pw.h || pw.wo != pw.w) return false;
     if (pw.a_xor != 0x80808080u || pw.out_xor != 0u || pw.residual) return false;
     if ((pw.rq.pc_multiplier != nullptr) != (dw.rq.pc_multiplier != nullptr)) return false;
-    if (dw.kh != 3 || dw.kw != 3 || dw.dil_h != 1 || dw.dil_w != 1 || dw.stride_h != dw.stride_w || (dw.stride_h != 1 && dw.stride_h != 2)) return false;
-    if (dw.dm != 1 || dw.c != dw.cout || dw.c != pw.n || (dw.c & 15) != 0 || dw.h != pw.h || dw.w_ != pw.w) return false;
-    if (dw.io_flip || (!dw.w_trip && !dw.w_fold)) return false;
-    if (dw.pad_t < 0 || dw.pad_l < 0 || dw.pad_t > 2 || dw.pad_l > 2) return false;
+    if (!pwdw_block_takes(dw) || dw.c != pw.n || dw.h != pw.h || dw.w_ != pw.w || (!dw.w_trip && !dw.w_fold)) return false;
     if ((size_t)dw.n * dw.h * dw.w_ * pw.cin >= (1ull << 31) || (size_t)dw.n * dw.ho * dw.wo * dw.cout >= (1ull << 31)) return false;
     return block_lds_bytes(1, pw.k_pad / 32, 3, 3 * dw.stride_w + 3, dw.c, nullptr, nullptr) <= kBlockLdsMax;  // one row of four outputs, one channel block
 }

@@ -677,6 +677,7 @@ bool dw_mfma_applies(const DwProblem &p);
 int launch_dw_mfma(const DwProblem &p, hipStream_t stream);
 
 // ---------------------------------------------------------------- pointwise + depthwise in one launch (eh_block.hip)
+bool pwdw_block_takes(const DwProblem &dw);
 bool pwdw_block_applies(const GemmProblem &pw, const DwProblem &dw);
 bool pwdw_block_listed(int32_t images, int32_t image_h, int32_t image_w, int32_t in_channels, int32_t expanded_channels, int32_t stride);
 bool pwdw_block_preferred(const GemmProblem &pw, const DwProblem &dw);  // the fused launch is the faster one for this shape (measured table)

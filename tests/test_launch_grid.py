@@ -53,3 +53,29 @@ def test_one_tap_grid_does_not_depend_on_what_ran_before(stub, tmp_path):
         assert len(own) == 2 and {l[3] for l in own} == {1, 4} and own[0][4] == own[1][4], own
         grids.append(own)
     assert grids[0] == grids[1]
+
+
+@pytest.mark.parametrize("desc,packs", [
+    ("1, 32, 9, 9, 32, 3, 3, (1, 1), (1, 1, 1, 1)", 1),
+    ("1, 32, 9, 9, 32, 3, 3, (2, 2), (0, 1, 0, 1)", 1),
+    ("1, 32, 9, 9, 32, 3, 3, (3, 3), (1, 1, 1, 1)", 0),
+    ("1, 32, 9, 9, 32, 3, 3, (1, 1), (2, 2, 2, 2), (2, 2)", 0),
+    ("1, 24, 9, 9, 24, 3, 3, (1, 1), (1, 1, 1, 1)", 0),
+    ("1, 16, 9, 9, 32, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1, 2", 0),
+    ("1, 32, 9, 9, 32, 3, 3, (1, 1), (1, 1, 1, 1), layout=eden.NCHW", 0),
+    ("1, 32, 9, 9, 32, 3, 3, (1, 1), (1, 1, 1, 1), layout=eden.NHWC | eden.IO_SIGNED", 0),
+    ("1, 20, 9, 9, 20, 5, 5, (1, 1), (2, 2, 2, 2)", 1),
+])
+def test_matrix_form_of_depthwise_weights_is_packed_where_a_kernel_reads_it(stub, tmp_path, desc, packs):
+    """5x5 and 7x7 layers, and of the 3x3 ones those that the fused expansion + depthwise launch can end with."""
+    if "layout" not in desc:
+        desc += ", layout=eden.NHWC"
+    if "dm" not in desc and ", 1, 2" not in desc:
+        desc += ", dm=1"
+    program = """
+d = eden.conv_desc(%s)
+if d.layout & eden.IO_SIGNED:
+    q = eden.make_requant_s8(0.02, 3, 0.004, 121, 0.03, 5)
+plan = eden.DwConvPlan(d, buf(d.cout, 1, d.kh, d.kw), buf(d.cout, dtype=np.int32), q)
+""" % desc
+    assert sum("dw_pack_mfma_kernel" in l[0] for l in launches(stub, tmp_path, program)) == packs
