@@ -78,6 +78,7 @@ EXPORTS = {
     "eh_conv_dw_block_applies": (C.c_int, [C.c_void_p, C.c_void_p]),
     "eh_conv_dw_block_preferred": (C.c_int, [C.c_void_p, C.c_void_p]),
     "eh_conv_dw_block_listed": (C.c_int, [C.c_int32] * 6),
+    "eh_conv_dw_block_tile": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32] + [C.POINTER(C.c_int32)] * 4),
     "eh_conv_dw_block_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(Requant), C.POINTER(Requant), C.c_int32,
                                        C.c_int32, C.c_void_p]),
     "eh_conv2d_u8_run_static": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(Requant), C.c_void_p]),
@@ -383,6 +384,13 @@ def conv_dw_block_applies(pointwise, depthwise):
 def conv_dw_block_preferred(pw, dw):
     """True when the fused launch is also the faster choice for the pair's shape (the library's measured table)."""
     return bool(load().eh_conv_dw_block_preferred(pw.handle, dw.handle))
+
+
+def conv_dw_block_tile(pw, dw, rows_per_tile=0, cols_per_tile=0):
+    """(rows, columns, blocks of 32 channels, depthwise stage on the matrix cores) of the tile that a fused launch of the pair takes"""
+    out = [C.c_int32() for _ in range(4)]
+    check(load().eh_conv_dw_block_tile(pw.handle, dw.handle, rows_per_tile, cols_per_tile, *(C.byref(v) for v in out)))
+    return tuple(v.value for v in out[:3]) + (bool(out[3].value),)
 
 
 def _conv_dw_block_run_general(pointwise, depthwise, d_in, d_out, q_pointwise, q_depthwise, rows_per_tile=0, cols_per_tile=0, stream=None):

@@ -2073,6 +2073,35 @@ int eh_conv_dw_block_preferred(const eh_conv_plan *pointwise, const eh_dwconv_pl
     return pwdw_block_preferred(pw, dw) ? 1 : 0;
 }
 
+// The geometry of a fused launch of two plans that fit.  The search over tiles costs the host as much as the launch, so the depthwise
+// plan keeps its latest result and what it was for.
+static int block_geometry(const GemmProblem &pw, const DwProblem &dw, eh_dwconv_plan *depthwise, int32_t rows_per_tile, int32_t cols_per_tile) {
+    const int32_t ks = pw.k_pad / 32;
+    if (depthwise->block_ks != ks || depthwise->block_rows != rows_per_tile || depthwise->block_cols != cols_per_tile) {
+        depthwise->block_ks = 0;
+        EH_REQUIRE(pwdw_block_geometry(pw, dw, rows_per_tile, cols_per_tile, &depthwise->block), "block: no tile of the requested shape (%d x %d outputs) fits",
+                   rows_per_tile, cols_per_tile);
+        depthwise->block_ks = ks;
+        depthwise->block_rows = rows_per_tile;
+        depthwise->block_cols = cols_per_tile;
+    }
+    return EH_OK;
+}
+
+int eh_conv_dw_block_tile(eh_conv_plan *pointwise, eh_dwconv_plan *depthwise, int32_t rows_per_tile, int32_t cols_per_tile, int32_t *rows, int32_t *cols,
+                          int32_t *channel_blocks, int32_t *matrix) {
+    EH_REQUIRE(rows != nullptr && cols != nullptr && channel_blocks != nullptr && matrix != nullptr, "null result pointer");
+    EH_REQUIRE(eh_conv_dw_block_applies(pointwise, depthwise), "block: these two plans do not fit the fused kernel");
+    const int rc = block_geometry(pointwise->op.problem(pointwise->op.parts[0], nullptr, nullptr, nullptr, nullptr), dw_problem(depthwise, nullptr, nullptr), depthwise,
+                                  rows_per_tile, cols_per_tile);
+    if (rc) return rc;
+    *rows = depthwise->block.th;
+    *cols = depthwise->block.tw;
+    *channel_blocks = depthwise->block.nb;
+    *matrix = depthwise->block.matrix;
+    return EH_OK;
+}
+
 int eh_conv_dw_block_run(eh_conv_plan *pointwise, eh_dwconv_plan *depthwise, const void *input, void *output,
                          const eh_requant *q_pointwise, const eh_requant *q_depthwise, int32_t rows_per_tile, int32_t cols_per_tile, void *stream) {
     EH_REQUIRE(pointwise != nullptr && depthwise != nullptr, "null plan");
@@ -2090,15 +2119,7 @@ int eh_conv_dw_block_run(eh_conv_plan *pointwise, eh_dwconv_plan *depthwise, con
     const GemmProblem pw = pointwise->op.problem(pointwise->op.parts[0], static_cast<const uint8_t *>(input), nullptr, nullptr, nullptr);
     DwProblem dw = dw_problem(depthwise, nullptr, output);
     if (depthwise->pc_multiplier && !depthwise->pc_fours) dw.rq.fast = 0;  // (a shift of -1: the kernel's other form is the two-step order)
-    const int32_t ks = pw.k_pad / 32;
-    if (depthwise->block_ks != ks || depthwise->block_rows != rows_per_tile || depthwise->block_cols != cols_per_tile) {
-        depthwise->block_ks = 0;
-        EH_REQUIRE(pwdw_block_geometry(pw, dw, rows_per_tile, cols_per_tile, &depthwise->block), "block: no tile of the requested shape (%d x %d outputs) fits",
-                   rows_per_tile, cols_per_tile);
-        depthwise->block_ks = ks;
-        depthwise->block_rows = rows_per_tile;
-        depthwise->block_cols = cols_per_tile;
-    }
+    if ((rc = block_geometry(pw, dw, depthwise, rows_per_tile, cols_per_tile))) return rc;
     return launch_pwdw_block(pw, dw, depthwise->block, s);
 }
 

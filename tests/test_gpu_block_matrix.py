@@ -13,24 +13,24 @@ pytestmark = pytest.mark.gpu
 SEED = 0xB10D
 
 CASES = [
-    # n, h, w, cin, c, stride, rows, cols, depthwise zp_w
-    (1, 3, 3, 8, 16, 1, 1, 1, 128),      # one output per workgroup, one chunk: three waves without work
-    (2, 9, 7, 16, 48, 1, 3, 5, 0),       # fifteen pixels; differences up to 255
-    (1, 9, 7, 24, 48, 2, 4, 4, 255),     # sixteen pixels; differences down to -255
-    (1, 11, 13, 32, 80, 1, 3, 7, 100),   # two groups, the second of five; a range that ends inside a block
-    (1, 16, 16, 40, 32, 1, 8, 8, 150),   # 128 units: four groups
-    (1, 16, 17, 40, 32, 1, 8, 9, 150),   # 192 units: the vector form
-    (3, 8, 8, 160, 96, 2, 2, 3, 127),    # five reduction steps; groups of six outputs
-    (2, 8, 8, 24, 64, 1, 2, 4, 127),     # eight outputs, half a group: the matrix form with up to four chunks to a workgroup
-    (2, 8, 8, 24, 64, 1, 3, 3, 127),     # nine: with any number
-    (1, 5, 6, 16, 16, 1, 5, 6, 90),      # the whole image in one workgroup
+    # n, h, w, cin, c, stride, rows, cols, depthwise zp_w, on the matrix cores
+    (1, 3, 3, 8, 16, 1, 1, 1, 128, True),      # one output per workgroup, one chunk: three waves without work
+    (2, 9, 7, 16, 48, 1, 3, 5, 0, True),       # fifteen pixels; differences up to 255
+    (1, 9, 7, 24, 48, 2, 4, 4, 255, True),     # sixteen pixels; differences down to -255
+    (1, 11, 13, 32, 80, 1, 3, 7, 100, True),   # two groups, the second of five; a range that ends inside a block
+    (1, 16, 16, 40, 32, 1, 8, 8, 150, True),   # 128 units: four groups
+    (1, 16, 17, 40, 32, 1, 8, 9, 150, False),   # 192 units: the vector form
+    (3, 8, 8, 160, 96, 2, 2, 3, 127, False),    # five reduction steps; six groups of six outputs: the vector form
+    (2, 8, 8, 24, 64, 1, 2, 4, 127, True),     # eight outputs, half a group: the matrix form with up to four chunks to a workgroup
+    (2, 8, 8, 24, 64, 1, 3, 3, 127, True),     # nine
+    (1, 5, 6, 16, 16, 1, 5, 6, 90, True),      # the whole image in one workgroup
 ]
 
 
 @pytest.mark.parametrize("per_channel", [False, True], ids=["tensor", "channel"])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(str(v) for v in c))
 def test_matrix_form_matches_oracle(case, per_channel):
-    n, h, w, cin, c, stride, rows, cols, zp_w = case
+    n, h, w, cin, c, stride, rows, cols, zp_w, matrix = case
     print("block", case, per_channel, flush=True)
     x, w1 = synth.fill_u8((n, h, w, cin), SEED + h), synth.fill_u8((c, cin, 1, 1), SEED + 1)
     b1, b2 = synth.fill_i32((c,), SEED + 2, -1000, 1000), synth.fill_i32((c,), SEED + 4, -1000, 1000)
@@ -47,7 +47,7 @@ def test_matrix_form_matches_oracle(case, per_channel):
     if per_channel:   # the tensors' own pair for every channel: the same results through the per-channel code
         for plan, e in ((pw, e1), (dw, e2)):
             plan.set_perchannel(np.full(c, e.multiplier), np.full(c, e.shift))
-    assert eden.conv_dw_block_applies(pw, dw)
+    assert eden.conv_dw_block_applies(pw, dw) and eden.conv_dw_block_tile(pw, dw, rows, cols)[3] == matrix
     d_x, d_o = eden.DeviceBuffer(host=x), eden.DeviceBuffer(nbytes=n * ho * wo * c)
     eden.conv_dw_block_run(pw, dw, d_x, d_o, e1, e2, rows, cols)
     got = d_o.download((n, ho, wo, c))

@@ -41,9 +41,9 @@ def test_shift_range_matches_oracle(case, act_min):
     assert want.std() > 4
 
 
-@pytest.mark.parametrize("rows, cols", [(3, 4), (8, 9)], ids=["matrix", "vector"])
+@pytest.mark.parametrize("rows, cols, matrix", [(3, 4, True), (8, 9, False)], ids=["matrix", "vector"])
 @pytest.mark.parametrize("depthwise_shift", [-1, -2])
-def test_fused_launch_at_the_largest_depthwise_scales(depthwise_shift, rows, cols):
+def test_fused_launch_at_the_largest_depthwise_scales(depthwise_shift, rows, cols, matrix):
     n, h, w, cin, c = 2, 9, 11, 24, 64
     x, w1, w2 = synth.fill_u8((n, h, w, cin), SEED + 7), int8((c, cin, 1, 1), SEED + 8), int8((c, 1, 3, 3), SEED + 9)
     b1, b2 = synth.fill_i32((c,), SEED + 10, -500, 500), synth.fill_i32((c,), SEED + 11, -500, 500)
@@ -60,7 +60,7 @@ def test_fused_launch_at_the_largest_depthwise_scales(depthwise_shift, rows, col
                          keep[3], q2)
     pw.set_perchannel(m1, sh1)
     dw.set_perchannel(m2, sh2)
-    assert eden.conv_dw_block_applies(pw, dw)
+    assert eden.conv_dw_block_applies(pw, dw) and eden.conv_dw_block_tile(pw, dw, rows, cols)[3] == matrix
     d_x, d_o = eden.DeviceBuffer(host=x), eden.DeviceBuffer(nbytes=n * h * w * c)
     eden.conv_dw_block_run(pw, dw, d_x, d_o, q1, q2, rows, cols)
     got = d_o.download((n, h, w, c))
