@@ -747,6 +747,7 @@ struct eh_dwconv_plan {
     // geometry of the latest fused launch behind a pointwise layer, and what it was chosen for
     BlockGeom block{};
     int32_t block_ks = 0, block_rows = 0, block_cols = 0;
+    bool block_per_channel = false;
 };
 
 extern "C" {
@@ -2077,13 +2078,15 @@ int eh_conv_dw_block_preferred(const eh_conv_plan *pointwise, const eh_dwconv_pl
 // plan keeps its latest result and what it was for.
 static int block_geometry(const GemmProblem &pw, const DwProblem &dw, eh_dwconv_plan *depthwise, int32_t rows_per_tile, int32_t cols_per_tile) {
     const int32_t ks = pw.k_pad / 32;
-    if (depthwise->block_ks != ks || depthwise->block_rows != rows_per_tile || depthwise->block_cols != cols_per_tile) {
+    const bool per_channel = pw.rq.pc_multiplier != nullptr;
+    if (depthwise->block_ks != ks || depthwise->block_rows != rows_per_tile || depthwise->block_cols != cols_per_tile || depthwise->block_per_channel != per_channel) {
         depthwise->block_ks = 0;
         EH_REQUIRE(pwdw_block_geometry(pw, dw, rows_per_tile, cols_per_tile, &depthwise->block), "block: no tile of the requested shape (%d x %d outputs) fits",
                    rows_per_tile, cols_per_tile);
         depthwise->block_ks = ks;
         depthwise->block_rows = rows_per_tile;
         depthwise->block_cols = cols_per_tile;
+        depthwise->block_per_channel = per_channel;
     }
     return EH_OK;
 }

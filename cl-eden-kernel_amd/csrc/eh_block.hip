@@ -482,19 +482,24 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     // the one that computes the fewest pixel slots wins, counting the slots that pixel blocks of 32 and output tiles of
     // four leave empty and, at a lower weight, the input bytes staged again for every channel range.
     int th = rows_per_tile, tw = cols_per_tile, nb = nb_all;
-    // Where the vector form's units (sixteen outputs, some 300 instructions each) would keep at most half of a workgroup's threads
-    // busy, the matrix form spreads the depthwise stage over all four waves, in groups of sixteen outputs by sixteen channels: one
-    // group a wave, or groups that are more than half full.  Same tiles, vector -> matrix form, us (with a pair per channel): 28x28
-    // 32 -> 192 stride 2, one image (two groups) 5.7 -> 4.2 (6.3 -> 4.8), 7x7 160 -> 960, one image 5.4 -> 4.5 (6.2 -> 4.9), four (four
-    // groups a quarter full) 5.5 -> 5.2 (6.3 -> 5.9); 14x14 96 -> 576, eight images (eight groups of twelve) 5.9 -> 5.4 (6.8 -> 6.5), but
-    // four (six groups of six) 5.1 -> 5.4 (5.8 -> 6.4), at stride 2 with sixteen images (ten groups of four) 5.9 -> 6.3 (6.8 -> 7.7);
-    // 7x7 160 -> 960, eight images (eight groups of six) 5.4 -> 5.7 (6.1 -> 6.9).  Beyond 128 units: 28x28 32 -> 192, 16 images (240)
-    // 5.9 -> 6.4, 32 images (480) 8.7 -> 9.0, 56x56 24 -> 144 stride 2 (252) 10.9 -> 11.4.
+    // Form of the depthwise stage.  The matrix form works in units of sixteen output pixels by sixteen channels, spread over the four
+    // waves, the vector form in units of four by four, some 300 instructions each, one to a thread: with few of them a workgroup waits
+    // for that chain, however few threads walk it.  One matrix unit to a wave wins, or comes within 3 %; with more it is a matter
+    // of their fill and of their epilogue, which a pair per channel doubles.  The same tiles, vector -> matrix form, us (with a pair per
+    // channel):
+    //   up to 4 units  28x28 32 -> 192 stride 2, 2 images 5.4 -> 4.2 (6.1 -> 4.6), stride 1, 4 images 4.7 -> 4.8 (5.25 -> 5.4),
+    //                  7x7 160 -> 960, 1 image 5.3 -> 4.55 (6.1 -> 5.05), 4 images 5.4 -> 5.2 (5.85 -> 5.8)
+    //   6, full        56x56 24 -> 144 stride 2, 6 images 5.8 -> 5.1 (6.6 -> 6.0), 28x28 32 -> 192, 8 images 6.2 -> 6.0 (6.8 -> 7.1), at
+    //                  stride 2, 24 images 6.5 -> 6.0 (7.4 -> 7.15)
+    //   6, half full   28x28 32 -> 192 stride 2, 8 images 5.2 -> 5.35 (5.6 -> 6.4), 14x14 96 -> 576, 4 images 5.2 -> 5.7 (5.9 -> 6.7)
+    //   8, full        14x14 96 -> 576, 8 images 5.9 -> 5.6 (6.6 -> 6.7), 64 -> 384, 16 images 6.0 -> 6.05 (6.85 -> 7.3)
+    //   9 and 10, full 56x56 24 -> 144 stride 2, 12 images 7.1 -> 7.5 (8.4 -> 9.2), 14x14 96 -> 576, 12 images 6.5 -> 6.6 (7.3 -> 8.0),
+    //                  33x33 48 -> 288, 4 images 5.8 -> 6.2 (6.5 -> 7.6)
+    const bool per_channel = pw.rq.pc_multiplier != nullptr;
     auto quads_of = [&](int blocks) { return blocks * 8 < dw.c / 4 ? blocks * 8 : dw.c / 4; };
-    auto small = [&](int rows, int cols, int blocks) { return dw.w_mm != nullptr && rows * ((cols + 3) / 4) * quads_of(blocks) <= 128; };
     auto matrix_form = [&](int rows, int cols, int blocks) {
-        const int pixel_groups = (rows * cols + 15) / 16;
-        return small(rows, cols, blocks) && (pixel_groups * (quads_of(blocks) / 4) <= 4 || rows * cols > pixel_groups * 8);
+        const int groups = (rows * cols + 15) / 16, units = groups * (quads_of(blocks) / 4);
+        return dw.w_mm != nullptr && (units <= 4 || (units <= (!per_channel ? 8 : S == 2 ? 6 : 4) && rows * cols > groups * 8));
     };
     {
         double best = -1;
@@ -515,11 +520,14 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
                         const int px = ih * iw;
                         const double tiles = (double)dw.n * ((dw.ho + ch - 1) / ch) * ((dw.wo + cw - 1) / cw);
                         const double stage1 = (double)((px + 31) / 32 * 32) * tiles / ((double)dw.n * dw.h * dw.w_);   // pixel slots computed per real pixel
-                        // (A slot of the matrix form, which works on sixteen outputs, counts three quarters.  Small tiles all count like
-                        // that: by the vector form's slots the search prefers still smaller ones, of two outputs or four, which lose to
-                        // the matrix form's: 56x56 24 -> 144 stride 2, one image 4.75 us against 3.90, 14x14 96 -> 576 stride 2, four images
-                        // 5.45 against 4.66.)
-                        const double slots = small(ch, cw, cn) ? 0.75 * ((ch * cw + 15) / 16 * 16) : (double)(ch * ((cw + 3) / 4 * 4));
+                        // A tile of up to 128 vector units (half the threads) is priced by whole groups of sixteen outputs, a slot of them at
+                        // three quarters, whichever form will run it: by the vector form's own slots the search prefers tiles of two outputs
+                        // or four, whose chain is as long and whose halo is larger.  Tiles by groups and by slots, us (with a pair per
+                        // channel): both matrix, 56x56 24 -> 144 stride 2, one image 4.15 and 4.5 (4.6 and 5.0); matrix and vector, 28x28
+                        // 32 -> 192 stride 2, 16 images 5.0 and 5.8 (5.8 and 6.6); both vector, 56x56 24 -> 144 stride 2, two images 5.0 and
+                        // 5.15 (5.3 and 5.35), 14x14 96 -> 576 stride 2, 24 images 6.2 and 6.3 (7.15 and 7.1).
+                        const bool small = ch * ((cw + 3) / 4) * quads_of(cn) <= 128;
+                        const double slots = small ? 0.75 * ((ch * cw + 15) / 16 * 16) : (double)(ch * ((cw + 3) / 4 * 4));
                         const double stage2 = slots * tiles / ((double)dw.n * dw.ho * dw.wo);  // output slots per real output
                         const double restage = (double)px * tiles * ranges * (g.ks * 32) / ((double)dw.n * dw.h * dw.w_ * dw.c);  // staged input bytes per expanded byte
                         const double cost = stage1 + 0.5 * stage2 + 2.0 * restage;

@@ -79,3 +79,31 @@ if d.layout & eden.IO_SIGNED:
 plan = eden.DwConvPlan(d, buf(d.cout, 1, d.kh, d.kw), buf(d.cout, dtype=np.int32), q)
 """ % desc
     assert sum("dw_pack_mfma_kernel" in l[0] for l in launches(stub, tmp_path, program)) == packs
+
+
+@pytest.mark.parametrize("shape,tensor,channel", [
+    # n, cin, expanded, extent, stride
+    ((1, 32, 192, 28, 2), 1, 1),      # up to four units of sixteen outputs by sixteen channels
+    ((16, 64, 384, 14, 1), 1, 0),     # eight, three quarters full
+    ((6, 24, 144, 56, 2), 1, 1),      # six at stride 2
+    ((8, 32, 192, 28, 1), 1, 0),      # six at stride 1
+    ((4, 96, 576, 14, 1), 0, 0),      # six, less than half full
+    ((12, 24, 144, 56, 2), 0, 0),     # nine
+    ((4, 48, 288, 33, 1), 0, 0),      # ten
+    ((32, 24, 144, 56, 2), 0, 0),     # large tiles
+])
+def test_form_of_the_fused_launchs_depthwise_stage(stub, tmp_path, shape, tensor, channel):
+    """On the matrix cores where that is the faster form, with one pair per tensor and with one per channel; the plan notices
+    that its pairs have changed."""
+    program = """
+n, cin, c, h, stride = %r
+pw = eden.ConvPlan(eden.conv_desc(n, cin, h, h, c, 1, 1, layout=eden.NHWC), buf(c, cin, 1, 1), buf(c, dtype=np.int32), q)
+dw = eden.DwConvPlan(eden.conv_desc(n, c, h, h, c, 3, 3, (stride,) * 2, (1,) * 4, dm=1, layout=eden.NHWC), buf(c, 1, 3, 3), buf(c, dtype=np.int32), q)
+forms = []
+for pairs in (False, True, False):
+    for plan in (pw, dw):
+        plan.set_perchannel(*((np.full(c, q.multiplier), np.full(c, q.shift)) if pairs else (None, None)))
+    forms.append(eden.conv_dw_block_tile(pw, dw)[3])
+assert forms == [%d, %d, %d], forms
+""" % (shape, tensor, channel, tensor)
+    launches(stub, tmp_path, program)
