@@ -126,38 +126,25 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
         return (unsigned)iy < (unsigned)pw.h && (unsigned)ix < (unsigned)pw.w;
     };
     {
-        // the weights as direct-to-LDS copies, all on their way at once beside the input pixels
-        dma_linear<4>(pw.b + (size_t)nb_first * ksteps * 1024, lds_offset(lds_raw), nb_here * ksteps, w_uniform, lane);
+        // The input pixels first, then the weights as direct-to-LDS copies, all on their way at once beside the bias.  (The pieces four
+        // at a time behind the weights' copies, from clamped addresses without a branch, cost a small launch more instructions than they
+        // save trips: 40 -> 240 at 20x20 stride 2, six images, 5.13 us as here, 5.44 like that; 48 -> 288 at 33x33, four images 5.57
+        // and 5.81; 64 -> 384 at 14x14, eight images 5.46 and 5.69.)
         const int ppp = ksteps * 4;  // 8-byte pieces per pixel
         const int pieces = g.pixels * ppp;
-        // Longer reductions have several pieces for every thread: four are requested, from addresses clamped into the image so that
-        // no branch separates the loads, before the first is used.  (One step has hardly more than a piece per thread, and the
-        // instructions of idle turns cost a small launch more than the trips they save.)
-        constexpr int FLIGHT = KS == 1 ? 1 : 4;
-        for (int first = 0; first < pieces; first += 256 * FLIGHT) {
-            uint2 v[FLIGHT];
-            uint8_t *to[FLIGHT];
-            bool exists[FLIGHT];
-#pragma unroll
-            for (int f = 0; f < FLIGHT; ++f) {
-                if (FLIGHT > 1 && first + f * 256 + w_uniform * 64 >= pieces) break;  // (a wave without a piece fetches nothing: 7x7 160 -> 960, four images 5.22 -> 5.05 us)
-                const int i = first + f * 256 + tid < pieces ? first + f * 256 + tid : pieces - 1;
-                const int q = KS ? i / (KS * 4) : (int)fastdiv((uint32_t)i, g.div_ppp), piece = i - q * ppp;
-                int iy, ix;
-                exists[f] = inside_image(q, iy, ix) && piece * 8 < pw.k;  // (else operand 0: bytes past the reduction length, whole pixels outside the image)
-                iy = iy < 0 ? 0 : (iy < pw.h ? iy : pw.h - 1);
-                ix = ix < 0 ? 0 : (ix < pw.w ? ix : pw.w - 1);
-                v[f] = *reinterpret_cast<const uint2 *>(pw.a + (((img * (uint32_t)pw.h + (uint32_t)iy) * (uint32_t)pw.w + (uint32_t)ix) * (uint32_t)pw.cin +
-                                                                (uint32_t)pw.a_offset + (piece * 8 < pw.k ? (uint32_t)piece * 8u : 0u)));
-                to[f] = a_s + q * g.a_pitch + piece * 8;
+        for (int i = tid; i < pieces; i += 256) {
+            const int q = KS ? i / (KS * 4) : (int)fastdiv((uint32_t)i, g.div_ppp), piece = i - q * ppp;
+            int iy, ix;
+            uint2 v = make_uint2(0u, 0u);  // bytes past the reduction length, and whole pixels outside the image: operand 0
+            if (inside_image(q, iy, ix) && piece * 8 < pw.k) {
+                v = *reinterpret_cast<const uint2 *>(pw.a + (((img * (uint32_t)pw.h + (uint32_t)iy) * (uint32_t)pw.w + (uint32_t)ix) * (uint32_t)pw.cin +
+                                                               (uint32_t)pw.a_offset + (uint32_t)piece * 8u));
+                v.x ^= pw.a_xor;
+                v.y ^= pw.a_xor;
             }
-#pragma unroll
-            for (int f = 0; f < FLIGHT; ++f) {
-                if (FLIGHT > 1 && first + f * 256 + w_uniform * 64 >= pieces) break;
-                // (a thread past the last piece holds that piece as well and writes the same bytes)
-                *reinterpret_cast<uint2 *>(to[f]) = make_uint2(exists[f] ? v[f].x ^ pw.a_xor : 0u, exists[f] ? v[f].y ^ pw.a_xor : 0u);
-            }
+            *reinterpret_cast<uint2 *>(a_s + q * g.a_pitch + piece * 8) = v;
         }
+        dma_linear<4>(pw.b + (size_t)nb_first * ksteps * 1024, lds_offset(lds_raw), nb_here * ksteps, w_uniform, lane);
         for (int i = tid; i < nb_here * 32; i += 256) bias_s[i] = pw.bias[c_first + i];
         if constexpr (PC) {  // (the per-channel arrays are padded to whole channel blocks)
             for (int i = tid; i < nb_here * 32; i += 256) {
