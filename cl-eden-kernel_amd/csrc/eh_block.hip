@@ -471,11 +471,12 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     int th = rows_per_tile, tw = cols_per_tile, nb = nb_all;
     // Form of the depthwise stage.  The matrix form works in units of sixteen output pixels by sixteen channels, spread over the four
     // waves, the vector form in units of four by four, some 300 instructions each, one to a thread: with few of them a workgroup waits
-    // for that chain, however few threads walk it.  One matrix unit to a wave wins, or comes within 3 %; with more it is a matter
-    // of their fill and of their epilogue, which a pair per channel doubles.  The same tiles, vector -> matrix form, us (with a pair per
-    // channel):
-    //   up to 4 units  28x28 32 -> 192 stride 2, 2 images 5.4 -> 4.2 (6.1 -> 4.6), stride 1, 4 images 4.7 -> 4.8 (5.25 -> 5.4),
-    //                  7x7 160 -> 960, 1 image 5.3 -> 4.55 (6.1 -> 5.05), 4 images 5.4 -> 5.2 (5.85 -> 5.8)
+    // for that chain, however few threads walk it.  With more than a matrix unit to a wave it is a matter of their fill and of their
+    // epilogue, which a pair per channel doubles.  The same tiles, vector -> matrix form, us (with a pair per channel):
+    //   up to 3 units  28x28 32 -> 192 stride 2, 2 images 5.4 -> 4.2 (6.1 -> 4.6), stride 1, 2 images 4.6 -> 4.3 (4.9 -> 4.6),
+    //                  7x7 160 -> 960, 1 image 5.3 -> 4.55 (6.1 -> 5.05)
+    //   4              56x56 24 -> 144 stride 2, 4 images 5.4 -> 4.75 (6.1 -> 5.5), 28x28 32 -> 192 stride 1, 4 images 4.7 -> 4.8
+    //                  (5.25 -> 5.4), 14x14 64 -> 384, 4 images 4.9 -> 4.8 (5.35 -> 5.5), 7x7 160 -> 960, 4 images 5.4 -> 5.2 (5.85 -> 5.8)
     //   6, full        56x56 24 -> 144 stride 2, 6 images 5.8 -> 5.1 (6.6 -> 6.0), 28x28 32 -> 192, 8 images 6.2 -> 6.0 (6.8 -> 7.1), at
     //                  stride 2, 24 images 6.5 -> 6.0 (7.4 -> 7.15)
     //   6, half full   28x28 32 -> 192 stride 2, 8 images 5.2 -> 5.35 (5.6 -> 6.4), 14x14 96 -> 576, 4 images 5.2 -> 5.7 (5.9 -> 6.7)
@@ -486,7 +487,7 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     auto quads_of = [&](int blocks) { return blocks * 8 < dw.c / 4 ? blocks * 8 : dw.c / 4; };
     auto matrix_form = [&](int rows, int cols, int blocks) {
         const int groups = (rows * cols + 15) / 16, units = groups * (quads_of(blocks) / 4);
-        return dw.w_mm != nullptr && (units <= 4 || (units <= (!per_channel ? 8 : S == 2 ? 6 : 4) && rows * cols > groups * 8));
+        return dw.w_mm != nullptr && units <= (!per_channel ? 8 : S == 2 ? 6 : 3) && (units <= 4 || rows * cols > groups * 8);
     };
     {
         double best = -1;

@@ -1,5 +1,5 @@
 """The fused expansion + depthwise launch with its depthwise stage on the matrix cores, which small tiles take (up to four
-units of sixteen outputs x sixteen channels per workgroup, or up to eight, six or four of them more than half full), and tiles just
+units of sixteen outputs x sixteen channels per workgroup, up to eight that are more than half full; fewer with one pair per channel), and tiles just
 beyond that: bit for bit the oracle's chain, at groups of sixteen output pixels that end early, several chunks and
 groups per wave, waves without work, and weights whose differences from their zero point leave int8 on either side."""
 import numpy as np
@@ -25,8 +25,9 @@ CASES = [
     (1, 16, 17, 40, 32, 1, 8, 9, 150, False, False),  # ten
     (3, 8, 8, 160, 96, 2, 2, 3, 127, False, False),   # six units of six pixels
     (3, 8, 8, 160, 64, 2, 2, 3, 127, True, True),     # four of them, behind five reduction steps
-    (2, 8, 8, 24, 64, 1, 2, 4, 127, True, True),      # four units of eight pixels, half a group
-    (2, 8, 8, 24, 64, 1, 3, 3, 127, True, True),      # of nine
+    (2, 8, 8, 24, 64, 1, 2, 4, 127, True, False),     # four units of eight pixels, half a group
+    (2, 8, 8, 24, 64, 2, 2, 4, 127, True, True),      # ... at stride 2
+    (2, 8, 8, 24, 64, 1, 3, 3, 127, True, False),     # of nine
     (1, 5, 6, 16, 16, 1, 5, 6, 90, True, True),       # the whole image in one workgroup
 ]
 

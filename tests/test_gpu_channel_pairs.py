@@ -41,10 +41,10 @@ def test_shift_range_matches_oracle(case, act_min):
     assert want.std() > 4
 
 
-@pytest.mark.parametrize("rows, cols, matrix", [(3, 4, True), (8, 9, False)], ids=["matrix", "vector"])
+@pytest.mark.parametrize("rows, cols, c, matrix", [(3, 4, 48, True), (8, 9, 64, False)], ids=["matrix", "vector"])
 @pytest.mark.parametrize("depthwise_shift", [-1, -2])
-def test_fused_launch_at_the_largest_depthwise_scales(depthwise_shift, rows, cols, matrix):
-    n, h, w, cin, c = 2, 9, 11, 24, 64
+def test_fused_launch_at_the_largest_depthwise_scales(depthwise_shift, rows, cols, c, matrix):
+    n, h, w, cin = 2, 9, 11, 24
     x, w1, w2 = synth.fill_u8((n, h, w, cin), SEED + 7), int8((c, cin, 1, 1), SEED + 8), int8((c, 1, 3, 3), SEED + 9)
     b1, b2 = synth.fill_i32((c,), SEED + 10, -500, 500), synth.fill_i32((c,), SEED + 11, -500, 500)
     m1, sh1 = edge_pairs(c, -8)

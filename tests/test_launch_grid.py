@@ -83,7 +83,9 @@ plan = eden.DwConvPlan(d, buf(d.cout, 1, d.kh, d.kw), buf(d.cout, dtype=np.int32
 
 @pytest.mark.parametrize("shape,tensor,channel", [
     # n, cin, expanded, extent, stride
-    ((1, 32, 192, 28, 2), 1, 1),      # up to four units of sixteen outputs by sixteen channels
+    ((1, 32, 192, 28, 2), 1, 1),      # two units of sixteen outputs by sixteen channels
+    ((4, 24, 144, 56, 2), 1, 1),      # four at stride 2
+    ((4, 64, 384, 14, 1), 1, 0),      # four at stride 1
     ((16, 64, 384, 14, 1), 1, 0),     # eight, three quarters full
     ((6, 24, 144, 56, 2), 1, 1),      # six at stride 2
     ((8, 32, 192, 28, 1), 1, 0),      # six at stride 1
