@@ -16,9 +16,9 @@
 //   2. after one barrier the threads compute the depthwise outputs from that image, four horizontally adjacent output
 //      pixels of four channels per thread, with the arithmetic of the stand-alone depthwise kernel (8-bit dot products,
 //      signed or unsigned form), and store them.
-//      Small tiles (a network on few images) do this stage on the matrix cores: a unit of sixteen outputs is some 300 vector
-//      instructions, and with fewer units than half the threads a workgroup waits for that chain (2 of the 4.1 us that a launch of
-//      such tiles lasts beyond an empty one).
+//      Small tiles (a network on few images) do this stage on the matrix cores: a thread's sixteen outputs are a chain of some 300
+//      vector instructions that a workgroup of few such threads waits for.  28x28 32 -> 192 at stride 2, two images, 5.4 -> 4.2 us
+//      (pwdw_block_geometry has the rule and both sides of it).
 // The rows and columns two neighbouring workgroups both need (the halo) are computed twice; nothing else is.  Tiles are
 // cut in both directions because the halo of a stride-2 window costs (2 TH + 1)(2 TW + 1) / (4 TH TW): 1.53 for one full
 // row of 28 outputs, 1.21 for 4 x 7.
@@ -427,19 +427,20 @@ bool pwdw_block_applies(const GemmProblem &pw, const DwProblem &dw) {
 // requantizes every expanded value on the vector ALU just as the stand-alone kernels do, so what it saves is the
 // expanded tensor's trip through memory and one launch; whether that pays depends on the shape, and the answer here
 // is a table of the shapes that were timed inside a network (MobileNetV2 at 224 x 224, 32 images per launch, each
-// pair switched to the fused kernel on its own; microseconds per network pass against 445):
+// pair switched to the fused kernel on its own; microseconds per network pass against 345 with none fused):
 //   image  in -> expanded  stride   change        image  in -> expanded  stride   change
-//   112     16 ->  96        2      +1.9           14    64 -> 384         1      -6.1 / -5.0 / -5.4 / -3.8
-//    56     24 -> 144        1      -0.8           14    96 -> 576         1      +0.1 / -0.4
-//    56     24 -> 144        2      -6.9           14    96 -> 576         2      -1.5
-//    28     32 -> 192        1      -5.2 / -3.8     7   160 -> 960         1      +0.4 / -0.6 / -0.4
-//    28     32 -> 192        2      -6.4
-// (changes within +-1.5 are noise; the listed shapes are the ones beyond it.)
+//   112     16 ->  96        2      +6.4           14    64 -> 384         1      -0.8 / -0.4 / -0.8 / -0.5
+//    56     24 -> 144        1      -3.1           14    96 -> 576         1      -0.3 / +1.5
+//    56     24 -> 144        2      -4.6           14    96 -> 576         2      -0.6
+//    28     32 -> 192        1      -3.3 / +1.3     7   160 -> 960         1      +0.1 / +1.2 / +0.8
+//    28     32 -> 192        2      -1.1
+// (changes within +-1.5 are noise.  With the listed pairs fused the pass takes 324.6; 14 x 14 64 -> 384 alone runs in 6.6 us against 8.0
+// for the two launches, 28 x 28 32 -> 192 in 9.2 against 9.2 and at stride 2 in 6.8 against 7.8, 56 x 56 24 -> 144 in 20.9 against 21.1.)
 // A shape that is not in the table runs as two launches.
 bool pwdw_block_listed(int32_t images, int32_t image_h, int32_t image_w, int32_t in_channels, int32_t expanded_channels, int32_t stride) {
-    // Below 32 images a launch is mostly latency, and one launch instead of two wins for every pair the kernel fits:
-    // MobileNetV2 with all 16 fitting pairs fused against the listed ones, 198 against 220 us at batch 1, 209 against 256
-    // at 4, 247 against 263 at 8, 287 against 294 at 16, 325 against 328 at 24; at 32 the list wins, 350 against 354.
+    // Below 32 images a launch is mostly latency, and one launch instead of two wins for the whole network:
+    // MobileNetV2 with all 16 fitting pairs fused against the listed ones, 144 against 162 us at batch 1, 168 against 176
+    // at 4, 206 against 222 at 8, 246 against 260 at 16, 288 against 294 at 24; at 32 it is a draw, 324.2 against 324.6.
     if (images < 32) return true;
     if (image_h != image_w) return false;
     struct Shape {

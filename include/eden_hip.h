@@ -155,9 +155,11 @@ void eh_make_requant_s8(float input_scale, int32_t input_zp, float filter_scale,
  * the two-step reference order.  Forms 2 and 3 are the single-shift forms the
  * kernels use with one multiplier and shift per channel (conv_per_channel_quantized,
  * gpu/operators/cl_kernels/ConvolutionKernels.cpp:1317-1375), q's pair standing for
- * the channel's: 2 with the rounding term computed from the shift (-20 <= shift <= -1),
- * 3 with it taken from a per-channel table (-20 <= shift <= -2); parameters outside
- * those ranges are an error, as the kernels then take the two-step order.  Form 4 is
+ * the channel's: 2 one value at a time from the pair as it is (-20 <= shift <= -1),
+ * 3 four values at a time from the multipliers and a byte, -2 - shift, per channel, the
+ * zero-point term added after the first shift and the clamp applied before the last
+ * (-20 <= shift <= -2); parameters outside those ranges are an error, as the kernels then
+ * take the two-step order.  Form 4 is
  * the per-tensor single-shift form as the kernels' epilogues evaluate it: four accumulators
  * at a time, the clamp applied before the shift, and a row term (here a value that varies
  * with the group of four) kept out of the accumulators and folded into the rounding term. */

@@ -79,7 +79,7 @@ def test_other_shifts_take_the_two_step_form(shift):
 
 @pytest.mark.parametrize("rs", [1, 2, 3, 7, 8, 11, 16, 20])
 def test_per_channel_single_shift_forms_equal_oracle(rs):
-    """The two per-channel forms (rounding term from the shift in registers; from a table, for rs >= 2), with and
+    """The two per-channel forms (one value from the pair as it is; four values from multipliers and shift bytes, for rs >= 2), with and
     without the sign test (clamp floor below / at the output zero point)."""
     rng = np.random.default_rng(3000 + rs)
     for mult in MULTIPLIERS:
