@@ -82,6 +82,13 @@ __global__ __launch_bounds__(256, KU == 6 && !BATCHED ? 4 : 1) void direct_gemm_
     uint8_t *pce_s = reinterpret_cast<uint8_t *>(pcm_s + nbw * 32);
     int32_t *add_a_s = bias_s + (QM == 2 ? 2 * 32 + 8 : 32) * nbw, *add_b_s = add_a_s + 256;  // [256] each, only with RES
     auto stage_weights = [&]() {
+        if constexpr (RES) {
+            // ahead of the weights: behind their copies and the bias's trip the tables lengthen every small launch (144 -> 24 at 56x56 with
+            // the add, four images 4.79 us, here 4.55, with a pair per channel 5.16 and 4.95; 96 -> 16 at 40x40, 16 images 4.93 and 4.78)
+            const int byte = threadIdx.x;  // 256 threads, 256 byte values
+            add_a_s[byte] = mul_round_shift((int32_t)((uint32_t)(byte - p.radd.zp_a) << p.radd.left_shift), p.radd.mult_a, p.radd.rs_a);
+            add_b_s[byte] = mul_round_shift((int32_t)((uint32_t)(byte - p.radd.zp_b) << p.radd.left_shift), p.radd.mult_b, p.radd.rs_b);
+        }
         // direct-to-LDS copies, every KiB on its way at once (a loop of loads and LDS stores waits a trip to L2 for each of its up to
         // eight turns; MobileNetV2 on 64 images, whose launches are mostly this kernel's, 444.3 -> 437.8 us)
         dma_linear<4>(p.b + (size_t)nb_first * ksteps * 1024, lds_offset(lds_raw), nb_count * ksteps, __builtin_amdgcn_readfirstlane(wave), lane);
@@ -91,11 +98,6 @@ __global__ __launch_bounds__(256, KU == 6 && !BATCHED ? 4 : 1) void direct_gemm_
                 pcm_s[i] = p.rq.pc_multiplier[nb_first * 32 + i];
                 pce_s[i] = (uint8_t)(-2 - p.rq.pc_shift[nb_first * 32 + i]);
             }
-        }
-        if constexpr (RES) {
-            const int byte = threadIdx.x;  // 256 threads, 256 byte values
-            add_a_s[byte] = mul_round_shift((int32_t)((uint32_t)(byte - p.radd.zp_a) << p.radd.left_shift), p.radd.mult_a, p.radd.rs_a);
-            add_b_s[byte] = mul_round_shift((int32_t)((uint32_t)(byte - p.radd.zp_b) << p.radd.left_shift), p.radd.mult_b, p.radd.rs_b);
         }
         wait_vmcnt<0>();
         __syncthreads();
