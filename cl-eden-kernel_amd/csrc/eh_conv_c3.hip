@@ -14,11 +14,12 @@
 // of the wave's two 32-pixel blocks has its 27 (+5 zero) reduction bytes in 32x32x32 fragment form, and one
 // v_mfma_i32_32x32x32_i8 per block and 32 channels leaves every lane with 16 consecutive channels of one pixel.
 //
-// Bound by its instructions (about 350 to a wavefront of 64 pixels x 32 channels, half of them requantization) once the
-// loads are together: 224x224, stride 2, 32 channels, before and after the rows, the weights and the bias (and a channel's
-// pair) were requested ahead of their first use: one image 3.95 -> 3.20 us, 32 images 9.31 -> 7.77, 64 images
-// 13.54 -> 11.50; with a pair per channel 4.62 -> 3.47, 11.43 -> 9.76 and 18.74 -> 15.61 (14.41 with the four-channel
-// requantization); 160x160 to 96 channels, 8 images 8.81 -> 5.96.  With fewer than 32 channels: 224x224 to 16, 32 images 7.17 -> 6.89.
+// A wavefront of 64 pixels x 32 channels is 358 vector instructions, 426 with a pair per channel (SQ_INSTS_VALU / SQ_WAVES; multiply,
+// clamp and shift of a lane's 32 values are 96 of them): at 32 images 3.7 of the 7.9 us, the rest is waiting, 45 % of the waves' cycles.
+// 224x224, stride 2, 32 channels, before and after the rows, the weights and the bias (and a channel's pair) were requested
+// ahead of their first use: one image 3.95 -> 3.20 us, 32 images 9.31 -> 7.77, 64 images 13.54 -> 11.50; with a pair per
+// channel 4.62 -> 3.47, 11.43 -> 9.76 and 18.74 -> 15.61 (14.41 with the four-channel requantization); 160x160 to 96
+// channels, 8 images 8.81 -> 5.96.  With fewer than 32 channels: 224x224 to 16, 32 images 7.17 -> 6.89.
 //
 // Stands in for the reference's direct convolution kernels on this shape
 // (gpu/operators/cl_kernels/DirectConvolutionKernel.cpp, 3x3 uint8 variants).
