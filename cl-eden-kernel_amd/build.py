@@ -21,6 +21,11 @@ CALL_LIB = os.path.join(HERE, "_call" + sysconfig.get_config_var("EXT_SUFFIX")) 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+             # Every joining block of a conditional restores the execution mask itself.  Left to itself the compiler drops the
+             # restore where an enclosing conditional ends right behind it, and then, out of registers, puts a spilled value's
+             # reload between the two, where the lanes that need it are off: the per-channel epilogue of a 256 x 256 tile wrote
+             # to addresses made of stale registers (tests/test_exec_restore.py reads the built code for this).
+             "-mllvm", "-amdgpu-remove-redundant-endcf=0",
              "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
 
 
