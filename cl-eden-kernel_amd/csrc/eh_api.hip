@@ -260,7 +260,7 @@ int finish_part(GemmPart &g, std::vector<KUnit> &units, const std::vector<int32_
     } else if (g.vec == 16 && (ktab_fits || (plain_matrix && g.k % 256 == 0)))
         // (a reduction too long for its k-table to fit LDS still runs as a plain matrix of whole slabs: a fully
         // connected layer on 25088 inputs)
-        g.cfg = igemm_dma_select(g.proto.m > m_floor ? g.proto.m : m_floor, g.n, g.k, siblings);  // (m_floor: the siblings' largest row count)
+        g.cfg = igemm_dma_select(g.proto.m > m_floor ? g.proto.m : m_floor, g.n, k_len, siblings);  // (m_floor: the siblings' largest row count)
     bool must_slice = false;
     if (g.cfg.id == GEMM_STAGED && g.vec == 16 && !ktab_fits && siblings == 1 && g.n_period == 0) {
         // table-driven and too long for one k-table (a 7x7 convolution over 512 channels): the split-reduction tiles

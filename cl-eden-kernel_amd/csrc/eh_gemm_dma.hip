@@ -14,7 +14,13 @@
 // compute their own addresses (implicit im2col), and lanes whose tap falls
 // outside the image fetch a 16-byte constant holding the input zero point.
 //
-// The 4 waves of a workgroup are arranged WGM x WGN x WGK.  WGK > 1 splits the
+// The waves of a workgroup (four, one per SIMD, or eight) are arranged WGM x WGN x WGK.  One wave alone issues an instruction
+// every 8 clocks, two waves together one every 2 to 5 (measured, ns per vector instruction and SIMD: one wave 3.35, two 1.1 for
+// additions and logic, 2.4 for three-operand forms, four 1.1 and 2.1).  The 256 x 256 tile therefore has eight waves of 128 x 64
+// instead of four of 128 x 128: its registers then hold the per-channel forms and the dword stores of output rows off 16-byte
+// boundaries, whose absence (a byte at a time) cost 1x1 96 -> 168 behind its expansion at 44 x 88x88 251 -> 105 us in all and the
+// transposed convolution 16x16 stride 8, 48 -> 40 at 4 x 45x45, 81 -> 30 us.  On whole rows the two are equal: 8192 x 4096 x 4096
+// is held by power (random bytes 121.5 us, all zero 88).  WGK > 1 splits the
 // slab along the reduction axis between waves (each wave still owns the whole
 // BM/WGM x BN/WGN sub-tile): for problems with few output tiles this keeps LDS
 // traffic per MFMA low; the partial tiles meet in LDS at the end (exact: int32).
@@ -108,15 +114,16 @@ __device__ __forceinline__ void static_for(F &&f) {
 // DENSE: 0 table-driven operand gather; 1 a plain matrix of whole slabs; 2 a plain matrix whose reduction ends inside
 // its last slab (the chunks past the end read a constant that the sign flip turns into 0).
 template <int BM, int BN, int WGM, int WGN, int WGK, int SLAB, int STAGES, int DENSE, bool ROWSUM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 && BN == 64 ? 3 : (BM == 128 && BN == 128 ? 2 : 1)))) void igemm_dma_kernel(const GemmBatch batch, const int count, const int tiles_m, const int tiles_n,
+__global__ __launch_bounds__(WGM * WGN * WGK * 64) __attribute__((amdgpu_waves_per_eu(BM == 128 && BN == 64 ? 3 : (BM == 128 && BN == 128 ? WGM * WGN * WGK / 2 : WGM * WGN * WGK / 4)))) void igemm_dma_kernel(const GemmBatch batch, const int count, const int tiles_m, const int tiles_n,
                                                         const int gm, const int gn) {
-    static_assert(WGM * WGN * WGK == 4, "four waves per workgroup");
+    constexpr int WAVES = WGM * WGN * WGK;
+    static_assert(WAVES == 4 || WAVES == 8, "one or two waves per SIMD");
     constexpr int CPR = SLAB / 16;            // 16-byte chunks per LDS row
     constexpr int RPB = 1024 / SLAB;          // rows per 1 KiB DMA block
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
     constexpr int FM = WTM / 32, FN = WTN / 32;
     constexpr int KSTEPS = SLAB / WGK / 32;   // 32-byte MFMA steps per wave per stage
-    constexpr int A_LOADS = BM / RPB / 4, B_LOADS = BN / RPB / 4;  // DMA instructions per wave per stage
+    constexpr int A_LOADS = BM / RPB / WAVES, B_LOADS = BN / RPB / WAVES;  // DMA instructions per wave per stage
     constexpr int LPS = A_LOADS + B_LOADS;
     constexpr int STAGE_BYTES = (BM + BN) * SLAB;
     constexpr int PART_ROW = BN + 4;          // int32 per row of a partial tile: 8 consecutive rows cover all banks
@@ -126,16 +133,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
     constexpr int WINDOW = STAGES == 2 ? KSTEPS / 2 : KSTEPS;        // steps over which the DMA of one stage is issued
     constexpr int DPS = (LPS + WINDOW * NMF - 1) / (WINDOW * NMF);   // DMA instructions placed behind one MFMA
     static_assert(WTM % 32 == 0 && WTN % 32 == 0 && KSTEPS >= 2 && KSTEPS % 2 == 0, "wave tile is made of 32x32x32 MFMA steps; fragment registers alternate between two sets");
-    static_assert(BM % (RPB * 4) == 0 && BN % (RPB * 4) == 0, "whole DMA blocks per wave");
+    static_assert(BM % (RPB * WAVES) == 0 && BN % (RPB * WAVES) == 0, "whole DMA blocks per wave");
     static_assert((STAGES - 1) * LPS <= 63, "vmcnt is a 6-bit counter");
     // the WGK partial tiles of the split reduction reuse the operand stages; with two stages they need a little more
     constexpr int PARTIAL_BYTES = WGK == 1 ? 0 : WGK * BM * PART_ROW * 4;
     constexpr int STAGE_AREA = STAGES * STAGE_BYTES > PARTIAL_BYTES ? STAGES * STAGE_BYTES : PARTIAL_BYTES;
-    static_assert(WGK == 1 || (BM == 64 && BN == 64 && WGM == 1 && WGN == 1), "the split-reduction epilogue is written for one 64x64 tile");
+    static_assert(WGK == 1 || (BM == 64 && BN == 64 && WGM == 1 && WGN == 1 && WAVES == 4), "the split-reduction epilogue is written for one 64x64 tile");
     static_assert(WTM % CPR == 0 && WTN % CPR == 0, "every fragment row of a lane has the same swizzle");
 
     __shared__ __align__(1024) uint8_t stages[STAGE_AREA];
-    __shared__ int32_t rowsum_s[WGK * 2][BM];
+    // Two waves per SIMD: the WGN waves of one row block hold the same activation fragments, and each sums those of every WGN-th
+    // step.  (One wave per SIMD: all sum all of them in the shadow of their products, and the first one's sums count; a branch
+    // per step costs more there, 11.27 -> 11.43 us for the transposed convolution of 256 -> 128 channels at 8 x 32x32.)
+    constexpr bool SHARED_SUMS = WAVES == 8;
+    constexpr int SUM_PARTS = WGK * (SHARED_SUMS ? WGN : 1) * 2;
+    __shared__ int32_t rowsum_s[SUM_PARTS][BM];
     __shared__ __align__(16) int32_t bias_s[BN];  // read in the epilogue from LDS: a global load there would have to
                                                    // wait for the stores issued before it (one counter for both)
     // fused residual add (split-reduction epilogue only): the rescaled value of every possible residual byte and of
@@ -219,13 +231,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
     if constexpr (DENSE) {
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i) {
-            int m = m0 + (i * 4 + wave) * RPB + slot_row;
+            int m = m0 + (i * WAVES + wave) * RPB + slot_row;
             m = m < p.m ? m : p.m - 1;  // rows past M re-read the last row; their results are never stored
             a_voff[i] = (uint32_t)m * (uint32_t)p.cin + my_chunk * 16;
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) rows[i] = make_row(p, m0 + (i * 4 + wave) * RPB + slot_row, plane);
+        for (int i = 0; i < A_LOADS; ++i) rows[i] = make_row(p, m0 + (i * WAVES + wave) * RPB + slot_row, plane);
     }
     // dense operands whose reduction is not whole slabs: which lanes' chunks lie past its end in the last slab
     constexpr bool ragged = DENSE == 2;
@@ -239,14 +251,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
     // (only the split-reduction tile runs slices of a reduction, whose row blocks lie a whole reduction apart)
     const int b_block_slabs = (WGK != 1 && p.b_slabs) ? p.b_slabs : k_slabs;
 #pragma unroll
-    for (int i = 0; i < B_LOADS; ++i) b_base[i] = p.b + ((size_t)(n0 / RPB + i * 4 + wave) * b_block_slabs) * 1024;
+    for (int i = 0; i < B_LOADS; ++i) b_base[i] = p.b + ((size_t)(n0 / RPB + i * WAVES + wave) * b_block_slabs) * 1024;
     uint32_t b_voff = lane * 16;    // advances by one block per issued stage
     const uint32_t wave_lds = lds_offset(stages) + (wave << 10);
 
     auto issue_piece = [&](auto idx_c, const uint32_t stage_off, const KUnit ku) {
         constexpr int idx = decltype(idx_c)::value;
         if constexpr (idx < A_LOADS) {
-            const uint32_t dst = wave_lds + stage_off + idx * 4096;
+            const uint32_t dst = wave_lds + stage_off + idx * (WAVES * 1024);
             if constexpr (DENSE) {
                 // (ku.dy marks the last slab of a reduction that ends inside it: the chunks past its end read the
                 // constant that the sign flip turns into 0 instead of the next pixel's bytes)
@@ -258,7 +270,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
                 dma16(a_chunk_address(p, rows[idx], ku), dst);
         } else {
             constexpr int bi = idx - A_LOADS;
-            dma16_off(b_base[bi], b_voff, wave_lds + stage_off + BM * SLAB + bi * 4096);
+            dma16_off(b_base[bi], b_voff, wave_lds + stage_off + BM * SLAB + bi * (WAVES * 1024));
         }
     };
     auto advance_slab = [&]() {
@@ -281,7 +293,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
     // blocks of the first stage ahead, so the copy of the k-table to LDS runs under their latency.
     if constexpr (!DENSE) {
         static_for<B_LOADS>([&](auto bi) { issue_piece(std::integral_constant<int, A_LOADS + decltype(bi)::value>{}, 0u, KUnit()); });
-        for (int i = tid; i < k_slabs * CPR; i += 256) ktab_s[i] = p.ktab[i];
+        for (int i = tid; i < k_slabs * CPR; i += WAVES * 64) ktab_s[i] = p.ktab[i];
         __syncthreads();
         const KUnit ku = ktab_s[my_chunk];
         static_for<A_LOADS>([&](auto ai) { issue_piece(ai, 0u, ku); });
@@ -328,7 +340,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
     auto flip = [&](auto buf_c, auto i_c) {
         constexpr int buf = decltype(buf_c)::value, i = decltype(i_c)::value;
         af[buf][i] = xor128(af[buf][i], a_xor);
-        if constexpr (ROWSUM) rowsum[i] = sum_bytes_signed(af[buf][i], rowsum[i]);
+        if constexpr (ROWSUM && !SHARED_SUMS) rowsum[i] = sum_bytes_signed(af[buf][i], rowsum[i]);
     };
     typedef std::integral_constant<int, 0> c0;
     typedef std::integral_constant<int, -1> no_wait;
@@ -370,6 +382,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
                     // the buffer being refilled is the one whose last fragments were read a step ago
                     if constexpr (idx < LPS) issue_piece(std::integral_constant<int, idx>{}, cross ? rd_off : next_off, ku);
                 });
+            }
+            if constexpr (ROWSUM && SHARED_SUMS && q == NMF - 1) {
+                if (kk % WGN == wn)
+                    static_for<FM>([&](auto i_c) { rowsum[decltype(i_c)::value] = sum_bytes_signed(af[cur][decltype(i_c)::value], rowsum[decltype(i_c)::value]); });
             }
             if constexpr (q == NMF - 1) {
                 if constexpr (fetch) flip(nxt_c{}, c0{});
@@ -415,9 +431,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
     // ---- epilogue.  acc[i][j][r] belongs to pixel row i*32 + (lane & 31) and, with the row
     // permutation of the packed weights, channel j*32 + 16*(lane >> 5) + r of this wave's sub-tile.
     if constexpr (ROWSUM) {
-        if (wn == 0) {
+        if (SHARED_SUMS || wn == 0) {
 #pragma unroll
-            for (int i = 0; i < FM; ++i) rowsum_s[wk * 2 + fhalf][wm * WTM + i * 32 + frow] = rowsum[i];
+            for (int i = 0; i < FM; ++i) rowsum_s[(SHARED_SUMS ? wk * WGN + wn : wk) * 2 + fhalf][wm * WTM + i * 32 + frow] = rowsum[i];
         }
     }
     if (tid < BN) bias_s[tid] = bias_reg;
@@ -433,7 +449,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
             const int ml = wm * WTM + i * 32 + frow, m = m0 + ml;
             row_ok[i] = m < p.m;
             row_off[i] = row_ok[i] ? out_pixel_offset(p, m, plane) : 0;
-            ncorr[i] = ROWSUM ? -p.zw * (rowsum_s[0][ml] + rowsum_s[1][ml]) : 0;
+            ncorr[i] = 0;
+            if constexpr (ROWSUM) {
+#pragma unroll
+                for (int w = 0; w < SUM_PARTS; ++w) ncorr[i] += rowsum_s[w][ml];
+                ncorr[i] *= -p.zw;
+            }
         }
         // whole tiles with 16-byte aligned rows (the usual case) store without any per-store test
         const bool aligned16 = (p.ldc & 15) == 0 && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
@@ -496,10 +517,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
                         if (aligned16 && n + 16 <= p.n) {
                             *reinterpret_cast<uint4 *>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
                         } else {
-                            if constexpr (BM == 256 && BN == 256) {  // (no registers to spare for the dword form's copies)
-                                const int cnt = p.n - n < 16 ? p.n - n : 16;
-                                for (int t = 0; t < cnt; ++t) dst[t] = (uint8_t)(packed[t >> 2] >> (8 * (t & 3)));
-                            } else if (p.planar.out_plane) {
+                            if (p.planar.out_plane) {
                                 store_bytes_planar(p.out, p.planar, row_off[i], n, packed, p.n - n < 16 ? p.n - n : 16);
                             } else {
                                 store_bytes_any_alignment(dst, packed, p.n - n < 16 ? p.n - n : 16);
@@ -512,12 +530,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
         };
         // edge tiles and unusual requantization parameters take the general code
         if (rq.pc_multiplier) {
-            // (the 256 x 256 tile has no registers to spare for the per-channel terms: two-step order there)
-            constexpr bool pc_single_shift = !(BM == 256 && BN == 256);
-            if (pc_single_shift && rq.fast == 2)
-                emit(std::true_type{}, std::integral_constant<int, pc_single_shift ? 2 : 0>{}, std::true_type{});
-            else if (pc_single_shift && rq.fast == 1)
-                emit(std::true_type{}, std::integral_constant<int, pc_single_shift ? 1 : 0>{}, std::true_type{});
+            if (rq.fast == 2)
+                emit(std::true_type{}, std::integral_constant<int, 2>{}, std::true_type{});
+            else if (rq.fast == 1)
+                emit(std::true_type{}, std::integral_constant<int, 1>{}, std::true_type{});
             else
                 emit(std::true_type{}, std::integral_constant<int, 0>{}, std::true_type{});
         } else if (rq.fast && aligned16 && m0 + BM <= p.m && n0 + BN <= p.n) {
@@ -557,7 +573,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
         int corr = 0;
         if constexpr (ROWSUM) {
 #pragma unroll
-            for (int w = 0; w < WGK * 2; ++w) corr += rowsum_s[w][ml];
+            for (int w = 0; w < SUM_PARTS; ++w) corr += rowsum_s[w][ml];
             corr *= p.zw;
         }
         const int32_t *pr = reinterpret_cast<const int32_t *>(stages) + ml * PART_ROW + nl;
@@ -668,12 +684,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 128 &
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int WGK, int SLAB, int STAGES>
+// TABLE_ONLY: plain matrices too are gathered by table
+template <int BM, int BN, int WGM, int WGN, int WGK, int SLAB, int STAGES, bool TABLE_ONLY = false>
 int launch_cfg(const TapProblem *ps, int count, hipStream_t stream) {
     const GemmProblem &p = ps[0];
     GemmBatch batch;
     for (int i = 0; i < count; ++i) static_cast<GemmProblem &>(batch.p[i]) = ps[i];
-    static_assert(STAGES * (BM + BN) * SLAB + WGK * 2 * BM * 4 + BN * 4 <= 160 * 1024 - 12288, "LDS budget with the largest k-table");
+    static_assert(STAGES * (BM + BN) * SLAB + WGK * (WGM * WGN * WGK == 8 ? WGN : 1) * 2 * BM * 4 + BN * 4 <= 160 * 1024 - 12288, "LDS budget with the largest k-table");
     int m_max = p.m;  // (table-driven problems of one launch may differ in their row counts: every kernel tests rows against its own problem's)
     for (int i = 1; i < count; ++i) m_max = ps[i].m > m_max ? ps[i].m : m_max;
     const int tiles_m = (m_max + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
@@ -710,28 +727,30 @@ int launch_cfg(const TapProblem *ps, int count, hipStream_t stream) {
     // with the split reduction serves it (1x1 layers with 320 .. 960 input channels); elsewhere it is gathered by table
     constexpr bool ragged_variant = BM == 64 && BN == 64;
     const bool whole = p.k == p.k_pad;
-    if (p.dense && whole) {
-        if (p.zw != 0)
-            hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 1, true>), dim3(grid), dim3(256), 0,
-                               stream, batch, count, tiles_m, tiles_n, gm, gn);
-        else
-            hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 1, false>), dim3(grid), dim3(256), 0,
-                               stream, batch, count, tiles_m, tiles_n, gm, gn);
+    if (!TABLE_ONLY && p.dense && whole) {
+        if constexpr (!TABLE_ONLY) {
+            if (p.zw != 0)
+                hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 1, true>), dim3(grid), dim3(WGM * WGN * WGK * 64), 0,
+                                   stream, batch, count, tiles_m, tiles_n, gm, gn);
+            else
+                hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 1, false>), dim3(grid), dim3(WGM * WGN * WGK * 64), 0,
+                                   stream, batch, count, tiles_m, tiles_n, gm, gn);
+        }
     } else if (p.dense && ragged_variant) {
         if constexpr (ragged_variant) {
             if (p.zw != 0)
-                hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 2, true>), dim3(grid), dim3(256), 0,
+                hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 2, true>), dim3(grid), dim3(WGM * WGN * WGK * 64), 0,
                                    stream, batch, count, tiles_m, tiles_n, gm, gn);
             else
-                hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 2, false>), dim3(grid), dim3(256), 0,
+                hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 2, false>), dim3(grid), dim3(WGM * WGN * WGK * 64), 0,
                                    stream, batch, count, tiles_m, tiles_n, gm, gn);
         }
     } else {
         if (p.zw != 0)
-            hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 0, true>), dim3(grid), dim3(256),
+            hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 0, true>), dim3(grid), dim3(WGM * WGN * WGK * 64),
                                ktab_bytes, stream, batch, count, tiles_m, tiles_n, gm, gn);
         else
-            hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 0, false>), dim3(grid), dim3(256),
+            hipLaunchKernelGGL((igemm_dma_kernel<BM, BN, WGM, WGN, WGK, SLAB, STAGES, 0, false>), dim3(grid), dim3(WGM * WGN * WGK * 64),
                                ktab_bytes, stream, batch, count, tiles_m, tiles_n, gm, gn);
     }
     EH_HIP(hipGetLastError());
@@ -810,10 +829,19 @@ GemmConfig igemm_dma_select(int32_t m, int32_t n, int32_t k, int32_t siblings) {
     const long t128 = (long)((m + 127) / 128) * ((n + 127) / 128) * siblings;
     const long t128x64 = (long)((m + 127) / 128) * ((n + 63) / 64) * siblings;
     const long t256x256 = (long)((m + 255) / 256) * ((n + 255) / 256) * siblings;
-    if (n > 128 && t256x256 >= 240) {
+    const int cols128 = (n + 127) / 128 * 128, cols256 = (n + 255) / 256 * 256;
+    if (n > 128 && t256x256 >= 240 && cols128 * 6 >= cols256 * 5 && (k > 512 || cols128 == cols256)) {
+        // (the largest tile does the same products on fewer bytes, but pads the columns further: 8192 x 4096 x 4096 130 us against 156
+        // on 128 x 128, 256 -> 256 3x3 at 64 x 28x28 41.5 against 44; with a quarter of the columns padding 1x1 328 -> 340 at 18 x 71x62
+        // 62 against 51, 3x3 12 -> 283 at 28 x 52x52 43.8 against 33.3; on short reductions any padding counts, 7974 x 192 x 1552
+        // 13.7 against 12.9)
         c.id = GEMM_DMA_256x256;
         c.slab = 128;
-    } else if (n > 64 && t256 >= 240) {
+    } else if (n > 64 && n <= 128 && k <= 128 && t256 >= 240 && t256 <= 512) {
+        // one slab: nothing to pipeline, and one round or two.  2x2 16 -> 72 at 28 x 57x57 13.86 us against 14.07 on 128 x 128 tiles, planar at 20 images 11.92
+        // against 12.22.  More rounds or longer reductions want two workgroups on a CU, one's stores under the other's products:
+        // 2x2 16 -> 128 at 64 x 57x57 20.96 here, 18.7 there; 5x5 16 -> 76 at 10 x 109x109 22.3 and 20.2; 8x8 stride 4 40 -> 55
+        // transposed at 16 x 38x38 57.2 and 53.8; 3x3 256 -> 96 at 16 x 56x56 22.3 either way.
         c.id = GEMM_DMA_256x128;
         c.slab = 128;
     } else if (n > 64 && t128 > 128) {
@@ -829,8 +857,14 @@ GemmConfig igemm_dma_select(int32_t m, int32_t n, int32_t k, int32_t siblings) {
         c.id = GEMM_DMA_64x64_SPLITK;
         c.slab = 256;
     }
-    (void)k;
     return c;
+}
+
+// how many tiles of bm x bn a launch of equally shaped problems has
+static long tiles_of(const TapProblem *ps, int count, int bm, int bn) {
+    int m_max = 0;
+    for (int i = 0; i < count; ++i) m_max = ps[i].m > m_max ? ps[i].m : m_max;
+    return (long)((m_max + bm - 1) / bm) * ((ps[0].n + bn - 1) / bn) * count;
 }
 
 int launch_igemm_dma(const TapProblem *ps, int count, hipStream_t stream) {
@@ -843,18 +877,21 @@ int launch_igemm_dma(const TapProblem *ps, int count, hipStream_t stream) {
                    "igemm_dma: a batch must hold equally shaped problems");
     }
     switch (p.cfg.id) {
-        case GEMM_DMA_256x256: return launch_cfg<256, 256, 2, 2, 1, 128, 2>(ps, count, stream);
-        case GEMM_DMA_256x128: return launch_cfg<256, 128, 2, 2, 1, 128, 3>(ps, count, stream);
-        case GEMM_DMA_128x128: return launch_cfg<128, 128, 2, 2, 1, 128, 2>(ps, count, stream);
+        case GEMM_DMA_256x256: return launch_cfg<256, 256, 2, 4, 1, 128, 2>(ps, count, stream);
+        case GEMM_DMA_256x128: return launch_cfg<256, 128, 4, 2, 1, 128, 2, true>(ps, count, stream);
+        case GEMM_DMA_128x128:
+            // Up to one tile per CU a workgroup has the CU to itself, and eight waves use it better than four (transposed convolution
+            // 256 -> 128 at 8 x 32x32, 256 tiles, 10.4 -> 9.75 us; 3x3 dilation 2 128 -> 128 at 32 x 28x28, 196 tiles, 10.8 -> 9.9; plain
+            // matrices are equal, 4096 x 1024 x 1024 9.0 either way); from there on two workgroups of four waves share it (3x3 128 -> 128
+            // at 64 x 28x28, 392 tiles, 13.5 us, with eight 14.3).
+            if (!(p.dense && p.k == p.k_pad) && tiles_of(ps, count, 128, 128) <= 256) return launch_cfg<128, 128, 4, 2, 1, 128, 2, true>(ps, count, stream);
+            return launch_cfg<128, 128, 2, 2, 1, 128, 2>(ps, count, stream);
         case GEMM_DMA_128x64: return launch_cfg<128, 64, 4, 1, 1, 128, 2>(ps, count, stream);
         case GEMM_DMA_64x64_SPLITK: {
             // Two stages take half the LDS, so two workgroups share a CU: for reductions of one or two slabs (deeper
             // staging has nothing to prefetch) and for launches with more tiles than CUs (the second workgroup's
             // prologue and epilogue hide behind the first one's loop instead of forming a second round).
-            int m_max = p.m;
-            for (int i = 1; i < count; ++i) m_max = ps[i].m > m_max ? ps[i].m : m_max;
-            const long tiles = (long)((m_max + 63) / 64) * ((p.n + 63) / 64) * count;
-            if (p.k_pad / 256 <= 2 || tiles > 256) return launch_cfg<64, 64, 1, 1, 4, 256, 2>(ps, count, stream);
+            if (p.k_pad / 256 <= 2 || tiles_of(ps, count, 64, 64) > 256) return launch_cfg<64, 64, 1, 1, 4, 256, 2>(ps, count, stream);
             return launch_cfg<64, 64, 1, 1, 4, 256, 4>(ps, count, stream);
         }
         default: break;

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as O
-from harness import eden, gpu_fc, synth
+from harness import eden, gpu_conv, gpu_fc, synth, to_eh_requant
 
 pytestmark = pytest.mark.gpu
 SEED = 0xEDE2 + 16 * 23
@@ -56,3 +56,24 @@ def test_a_pair_per_channel(deconv, n, c, h, cout, k, stride):
     plan.destroy()
     assert np.array_equal(got, want)
     assert want.std() > 4
+
+
+# row sums (weights around a zero point of their own), shared by the waves of a row block where a SIMD runs two of them
+@pytest.mark.parametrize("n,c,h,cout,k,dil,kernel", [
+    (21, 128, 28, 121, 3, 2, "dma_128x128"),   # at most one tile per CU
+    (13, 16, 71, 250, 5, 1, "dma_256x256"),
+    (20, 16, 57, 72, 2, 1, "dma_256x128"),     # one slab
+    (30, 16, 57, 72, 3, 2, "dma_128x128"),     # more tiles than CUs
+])
+def test_row_sums(n, c, h, cout, k, dil, kernel):
+    print("row sums", n, c, h, cout, k, dil, kernel, flush=True)
+    pad = dil * (k - 1) // 2
+    s = O.conv_shape(n, c, h, h, cout, k, k, pad=(pad,) * 4, dil=(dil, dil))
+    desc = eden.conv_desc(n, c, h, h, cout, k, k, (1, 1), (pad,) * 4, (dil, dil), layout=eden.NHWC)
+    assert eden.conv_kernels(desc, launched=True) == [kernel]
+    x, w = synth.fill_u8((n, c, h, h), SEED + 8), synth.fill_u8((cout, c, k, k), SEED + 9)
+    b = synth.fill_i32((cout,), SEED + 10, -1000, 1000)
+    q = O.make_quant(0.02, 131, 0.005, 117, 0.02 * 0.005 * 74 * 74 * (c * k * k) ** 0.5 / 40, 120)
+    want, got = O.conv2d(x, w, b, s, q), gpu_conv(x, w, b, s, to_eh_requant(q), layout=eden.NHWC)
+    assert np.array_equal(got, want)
+    assert want.std() > 20
