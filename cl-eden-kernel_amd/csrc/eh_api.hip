@@ -143,6 +143,7 @@ struct GemmPart {
     int64_t so = 0, sc = 0;   // source weight strides (out channel, in channel)
     int64_t w_base = 0;       // element offset of this part in the source weights
     int32_t bias_base = 0;    // first output channel
+    int32_t c0 = 0, c_real = 0;  // first channel in the caller's tensor, and channels per tap there
     TapProblem proto{};      // geometry; pointers and quantization filled per run
 
     void release() {
@@ -572,11 +573,34 @@ struct GemmOp {
     }
     static constexpr int kInlineParts = 8;  // a run over at most this many parts allocates no host memory
 
+    // Which form of the caller's own tensor the launches of a run can read, where the kernels otherwise get a copy with padded
+    // channels or with the channels last (gemm_few_tiles_direct has the rule).
+    int32_t direct_form() const {
+        if (parts.empty() || (pad_cg_to == 0 && layout != EH_NCHW)) return INPUT_CHUNKS;
+        const int32_t form = layout == EH_NCHW ? INPUT_PLANAR : INPUT_RAGGED;
+        if ((int64_t)in_n * in_c * in_hw < 16 || (layout == EH_NCHW && !stores_planar())) return INPUT_CHUNKS;
+        for (auto &g : parts) {
+            const bool order = g.cfg.id == GEMM_FEW_TILES || g.cfg.id == GEMM_THIN || g.cfg.id == GEMM_CONV3X3 || g.cfg.id == GEMM_SKINNY;
+            if (!order || g.slices || g.n_period || g.block_cin || g.vec != 16 || g.k <= 0 || g.cin % 16 != 0 ||
+                !gemm_few_tiles_direct(g.proto.m, g.n, g.k, (int32_t)parts.size(), form))
+                return INPUT_CHUNKS;
+        }
+        return form;
+    }
+
     // One part's kernel argument for channels-last tensors `in` / `out`, with the quantization parameters refold() left in `q`
     // (planar_out: `out` is a planar tensor that the kernels write themselves)
-    TapProblem problem(const GemmPart &g, const uint8_t *in, uint8_t *out, const uint8_t *residual, const AddDev *radd, bool planar_out = false) const {
+    // (form: what `in` is)
+    TapProblem problem(const GemmPart &g, const uint8_t *in, uint8_t *out, const uint8_t *residual, const AddDev *radd, bool planar_out = false,
+                       int32_t form = INPUT_CHUNKS) const {
         TapProblem p = g.proto;
         p.a = in;
+        if (form != INPUT_CHUNKS) {
+            p.form = form;
+            p.cin = in_c;
+            p.tap.c0 = g.c0;
+            p.c_last = g.c_real - (p.tap.chunks - 1) * 16;
+        }
         p.b = g.b;
         p.bias = g.folded;
         p.fillbuf = fillbuf;
@@ -623,7 +647,10 @@ struct GemmOp {
         uint8_t *const st_pad = staging ? staging + (layout == EH_NCHW ? stage_in_bytes() + stage_out_bytes() : 0) : stage_pad;
         const bool planar_out = stores_planar();
         bool padded = false;
-        if (layout == EH_NCHW) {
+        const int32_t form = direct_form();
+        if (layout == EH_NCHW && form != INPUT_CHUNKS) {
+            // (planar_out: see direct_form)
+        } else if (layout == EH_NCHW) {
             // (the channel padding as part of the same pass)
             padded = pad_cg_to != 0 && pad_groups == 1;
             uint8_t *const to = padded ? st_pad : st_in;
@@ -633,7 +660,7 @@ struct GemmOp {
             in = to;
             if (!planar_out) out = st_out;
         }
-        if (pad_cg_to && !padded) {
+        if (pad_cg_to && !padded && form == INPUT_CHUNKS) {
             // (q holds the uint8-equivalent input zero point after refold(); int8 tensors store it minus 128)
             if ((rc = launch_pad_channels(in, st_pad, (int64_t)in_n * in_hw, pad_groups, pad_cg, pad_cg_to,
                                           (uint32_t)(q.zp_in & 0xFF) ^ (io_signed ? 0x80u : 0u), stream)))
@@ -648,9 +675,9 @@ struct GemmOp {
         TapProblem *const problems = many.empty() ? inline_problems : many.data();
         int filled = 0;
         for (auto &g : parts) {
-            EH_REQUIRE((reinterpret_cast<uintptr_t>(in) & (uintptr_t)(g.vec - 1)) == 0,
+            EH_REQUIRE(form != INPUT_CHUNKS || (reinterpret_cast<uintptr_t>(in) & (uintptr_t)(g.vec - 1)) == 0,
                        "input pointer is not aligned to %d bytes", g.vec);
-            const TapProblem whole = problem(g, in, out, fuse ? residual : nullptr, radd, planar_out);
+            const TapProblem whole = problem(g, in, out, fuse ? residual : nullptr, radd, planar_out, form);
             if (g.slices == 0) {
                 problems[filled++] = whole;
                 continue;
@@ -1180,6 +1207,8 @@ static int conv_plan_build(eh_conv_plan *pl, const eh_conv_desc *d, hipStream_t 
         part.k = taps * cig;
         part.vec = pick_vec(cig, pixel_c);
         part.bias_base = g * cog;
+        part.c_real = padded ? cig_real : cig;
+        part.c0 = g * part.c_real;
         if (d->weight_layout == EH_W_OIHW) {
             part.so = (int64_t)cig_real * taps;
             part.sc = taps;
@@ -1252,7 +1281,7 @@ static int report_kernels(const GemmOp &op, int32_t *kernel_ids, int32_t cap, bo
     for (size_t i = 0; launched && i < op.parts.size();) {
         std::vector<TapProblem> problems;  // (a sliced part is launched by itself, by the kernel it is planned for)
         while (i + problems.size() < op.parts.size() && op.parts[i + problems.size()].slices == 0)
-            problems.push_back(op.problem(op.parts[i + problems.size()], nullptr, nullptr, nullptr, nullptr));
+            problems.push_back(op.problem(op.parts[i + problems.size()], nullptr, nullptr, nullptr, nullptr, false, op.direct_form()));
         for (size_t j = 0; j < problems.size();) {
             int32_t id;
             const int run = igemm_next_launch(problems.data() + j, (int)(problems.size() - j), &id);
@@ -1434,6 +1463,7 @@ int eh_fc_q8_plan(eh_fc_plan **plan, int32_t m, int32_t k, int32_t n, int32_t fl
         part.n = n;
         part.cin = k;
         part.cin_real = pass == 1 ? k_real : 0;
+        part.c_real = k_real;
         part.taps = 1;
         part.k = k;
         part.vec = pick_vec(k, k);
@@ -1602,6 +1632,8 @@ static int deconv_plan_build(eh_deconv_plan *pl, const eh_conv_desc *d, hipStrea
                 part.k = part.taps * cig;
                 part.vec = pick_vec(cig, pixel_c);
                 part.bias_base = g * cog;
+                part.c_real = cig_real;
+                part.c0 = g * cig_real;
                 std::vector<int32_t> tap_off(part.taps > 0 ? part.taps : 0);
                 if (d->weight_layout == EH_W_IOHW) {
                     part.so = (int64_t)d->kh * d->kw;

@@ -314,6 +314,13 @@ int igemm_next_launch(const TapProblem *ps, int count, int32_t *kernel_id) {
     *kernel_id = p.cfg.id;
     int run = 1;
     if (p.m <= 0 || p.n <= 0) return run;
+    if (p.form != INPUT_CHUNKS) {  // the caller's tensor as it is: the kernel for few tiles, whatever the plan's own is
+        *kernel_id = GEMM_FEW_TILES;
+        while (run < count && run < GemmBatch::MAX && p.residual == nullptr && ps[run].residual == nullptr && ps[run].form == p.form && ps[run].n == p.n &&
+               ps[run].k_pad == p.k_pad && ps[run].zw == p.zw && ps[run].rq.fast == p.rq.fast && ps[run].c_last == p.c_last)
+            ++run;
+        return run;
+    }
     if (is_dma(p.cfg.id))
         // (row counts may differ where nothing depends on them: table-driven problems; the launch covers the largest)
         while (run < count && run < GemmBatch::MAX && ps[run].cfg.id == p.cfg.id && (ps[run].m == p.m || (!p.dense && !p.partial)) && ps[run].n == p.n &&

@@ -42,6 +42,7 @@ struct FewProblem {
         AddDev radd;
         PlanarOut planar;
     };
+    int32_t c_last;
     RequantDev rq;
 
     FewProblem() {}
@@ -49,8 +50,9 @@ struct FewProblem {
         : a(p.a), b(p.b), bias(p.bias), out(p.out), residual(p.residual), m(p.m), n(p.n), k(p.k), k_pad(p.k_pad), h(p.h), w(p.w), cin(p.cin), ho(p.ho), wo(p.wo),
           stride_h(p.stride_h), stride_w(p.stride_w), y_base(p.y_base), x_base(p.x_base), div_plane(p.div_plane), div_wo(p.div_wo), tap(p.tap), fill(p.fill),
           a_xor(p.a_xor), out_xor(p.out_xor), zw(p.zw), out_h(p.out_h), out_w(p.out_w), out_sy(p.out_sy), out_sx(p.out_sx), out_y0(p.out_y0), out_x0(p.out_x0),
-          ldc(p.ldc), radd(p.radd), rq(p.rq) {}  // (radd's bytes are `planar` where that is in use)
+          ldc(p.ldc), radd(p.radd), c_last(p.c_last), rq(p.rq) {}  // (radd's bytes are `planar` where that is in use)
 };
+static_assert(sizeof(FewProblem) == 328, "c_last lies in what alignment leaves free: 3x3 on 256 channels at 14 x 14, one image, 5.31 us; in front of the union 5.41");
 struct FewBatch {
     FewProblem p[GemmBatch::MAX];
 };
@@ -86,13 +88,38 @@ __device__ __forceinline__ void quad_transpose(int &c0, int &c1, int &c2, int &c
     swap2(c1, c3);
 }
 
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef v4i v4i_any_alignment __attribute__((aligned(1)));
+
+// sixteen bytes shifted down by `bytes` of them (0 .. 15)
+__device__ __forceinline__ v4i shift_bytes_down(v4i v, uint32_t bytes) {
+    const uint64_t lo = (uint64_t)(uint32_t)v.x | (uint64_t)(uint32_t)v.y << 32, hi = (uint64_t)(uint32_t)v.z | (uint64_t)(uint32_t)v.w << 32;
+    const uint32_t n = bytes * 8, part = n & 63u;
+    const uint64_t down = part ? lo >> part | hi << (64u - part) : lo, top = hi >> part;
+    const uint64_t a = n < 64u ? down : top, b = n < 64u ? top : 0u;
+    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)(uint32_t)b, (int)(uint32_t)(b >> 32)};
+}
+// the low `count` (0 or less .. 16 or more) of sixteen bytes' places, word d of the four
+__device__ __forceinline__ uint32_t byte_mask(int count, int d) {
+    const int left = count - 4 * d;
+    return left >= 4 ? ~0u : left <= 0 ? 0u : (1u << (8 * left)) - 1u;
+}
+
 // GROUPS: 128-byte groups of the reduction a wave has on their way together.  TAPS: the reduction runs over kernel taps that
 // may lie outside the image (else: one tap inside it).  ROWSUM: the weights' zero point is not 128.  FAST: every
-// requantization pair in use is inside the single-shift form's range.  BATCHED: equally shaped problems along grid z.
-template <int GROUPS, bool TAPS, bool ROWSUM, bool FAST, bool BATCHED>
+// requantization pair in use is inside the single-shift form's range (or is told at run time).  BATCHED: equally shaped
+// problems along grid z.  FORM: where the chunks are (InputForm).
+//
+// Ragged and planar tensors used to be brought into whole chunks by a launch of their own, which for a small layer costs as much as the
+// layer (figures at gemm_few_tiles_direct).
+// A ragged chunk is sixteen bytes at any address; what lies behind the tap's channels is replaced by the input zero point, the
+// byte that the padded copy held, and a chunk that would end behind the tensor is read from sixteen bytes before its end and
+// shifted down.  A planar chunk is sixteen single bytes a plane apart, which neighbouring lanes read from neighbouring pixels.
+template <int GROUPS, bool TAPS, bool ROWSUM, bool FAST, bool BATCHED, int FORM>
 __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::conditional_t<BATCHED, FewBatch, FewProblem> arg, const int m_blocks, const int n_blocks,
                                                                 const int tiles_per_xcd, const int m_fastest) {
     const FewProblem &p = problem_of(arg);
+    static_assert(FORM != INPUT_PLANAR || GROUPS <= 3, "a planar group is many loads on their way already");
     __shared__ __align__(16) int32_t part_s[kWaves][64 * kLanePitch];
     __shared__ int32_t sum_s[ROWSUM ? kWaves * 2 : 1][32];
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, half = lane >> 5;
@@ -103,7 +130,10 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
     const int slow = __builtin_amdgcn_readfirstlane(tile / (m_fastest ? m_blocks : n_blocks));
     const int fast_i = tile - slow * (m_fastest ? m_blocks : n_blocks);
     const int mb = m_fastest ? fast_i : slow, nb = m_fastest ? slow : fast_i;
-    const int groups = (p.k_pad + 127) >> 7, chunks = p.k_pad >> 4;
+    // products of 32 bytes to a group; PLANAR: one, for the registers that single bytes take and so that more waves have a share
+    // (3x3 21 -> 21 at 3 x 65x47 5.95 us with two, 5.06 with one)
+    constexpr int STEPS = FORM == INPUT_PLANAR ? 1 : 4;
+    const int groups = (p.k_pad + STEPS * 32 - 1) >> (STEPS == 1 ? 5 : 7), chunks = p.k_pad >> 4;
 
     // ---- where this lane's pixel reads
     const int m_in = mb * 32 + r;
@@ -114,7 +144,10 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
         const int oy = (int)fastdiv((uint32_t)rem, p.div_wo), ox = rem - oy * p.wo;
         iy0 = oy * p.stride_h + p.y_base;
         ix0 = ox * p.stride_w + p.x_base;
-        base = ((img * p.h + iy0) * p.w + ix0) * p.cin + p.tap.c0;
+        if constexpr (FORM == INPUT_PLANAR)
+            base = ((img * p.cin + p.tap.c0) * p.h + iy0) * p.w + ix0;
+        else
+            base = ((img * p.h + iy0) * p.w + ix0) * p.cin + p.tap.c0;
     }
     // Activation loads: four neighbouring lanes fetch 64 contiguous bytes of ONE pixel (the cache answers a 64-byte piece
     // per cycle; four pixels' pieces take four), pixel by pixel of the four, and exchange them afterwards.
@@ -152,41 +185,89 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
         }
     };
 
+    uint32_t last_start = 0;  // RAGGED: where the last sixteen bytes of the tensor start (the host leaves smaller tensors to the padded copy)
+    if constexpr (FORM == INPUT_RAGGED) last_start = fastdiv((uint32_t)p.m, p.div_plane) * (uint32_t)(p.h * p.w) * (uint32_t)p.cin - 16u;
     for (int g0 = wave; g0 < groups; g0 += kWaves * GROUPS) {
-        // Group g is the reduction's bytes 128 g .. 128 g + 127: chunks 8 g + 4 half + u meet in its u-th product.
-        v4i bf[GROUPS][4], af[GROUPS][4];
-        uint32_t inside[GROUPS];
+        // Group g is the reduction's bytes 128 g .. 128 g + 127: chunks 8 g + 4 half + u meet in its u-th product.  (PLANAR: a quarter of that.)
+        v4i bf[GROUPS][STEPS], af[GROUPS][STEPS];
+        uint32_t inside[GROUPS];   // bit px: pixel px's tap lies inside; RAGGED: bits 8 + 4 px on by how many bytes its chunk was read too early
+        int valid[GROUPS];         // RAGGED: bytes of the chunk that are the tap's own
         bool exists[GROUPS];
 #pragma unroll
         for (int u = 0; u < GROUPS; ++u) {
             const int g = g0 + u * kWaves;
             if (g >= groups) break;  // (uniform across the wave)
-            // the chunk this lane fetches for each of the four pixels
-            const int chunk = g * 8 + half * 4 + (lane & 3);
-            exists[u] = chunk * 16 < p.k;
-            int dy = 0, dx = 0, off = chunk * 16;
-            if constexpr (TAPS) {
-                const int tap = (int)fastdiv((uint32_t)chunk, p.tap.div_chunks), c = chunk - tap * p.tap.chunks;
-                const int ty = (int)fastdiv((uint32_t)tap, p.tap.div_nx), tx = tap - ty * p.tap.nx;
-                dy = p.tap.dy0 + ty * p.tap.dys;
-                dx = p.tap.dx0 + tx * p.tap.dxs;
-                off = (dy * p.w + dx) * p.cin + c * 16;
-            }
-            inside[u] = 0;
-            auto fetch = [&](auto px_c, int b, int iy, int ix) {
-                constexpr int px = decltype(px_c)::value;
-                bool ok = exists[u];
-                if constexpr (TAPS) ok = ok && (unsigned)(iy + dy) < (unsigned)p.h && (unsigned)(ix + dx) < (unsigned)p.w;
-                inside[u] |= (uint32_t)ok << px;
-                af[u][px] = *reinterpret_cast<const v4i *>(p.a + (size_t)(ok ? b + off : 0));
+            auto place = [&](int chunk, int &dy, int &dx, int &c) {
+                c = chunk;
+                dy = dx = 0;
+                if constexpr (TAPS) {
+                    const int tap = (int)fastdiv((uint32_t)chunk, p.tap.div_chunks);
+                    const int ty = (int)fastdiv((uint32_t)tap, p.tap.div_nx), tx = tap - ty * p.tap.nx;
+                    c = chunk - tap * p.tap.chunks;
+                    dy = p.tap.dy0 + ty * p.tap.dys;
+                    dx = p.tap.dx0 + tx * p.tap.dxs;
+                }
             };
-            fetch(std::integral_constant<int, 0>{}, q_base.x, q_iy.x, q_ix.x);
-            fetch(std::integral_constant<int, 1>{}, q_base.y, q_iy.y, q_ix.y);
-            fetch(std::integral_constant<int, 2>{}, q_base.z, q_iy.z, q_ix.z);
-            fetch(std::integral_constant<int, 3>{}, q_base.w, q_iy.w, q_ix.w);
+            inside[u] = 0;
+            valid[u] = 16;
+            if constexpr (FORM == INPUT_PLANAR) {
+                // product t's chunk of this lane's own pixel, byte by byte
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int wc = g * 8 + half * 4 + t;
+                for (int t = 0; t < STEPS; ++t) {
+                    const int chunk = (g * 2 + half) * STEPS + t;
+                    int dy, dx, c;
+                    place(chunk, dy, dx, c);
+                    exists[u] = chunk * 16 < p.k;
+                    bool ok = exists[u];
+                    if constexpr (TAPS) ok = ok && (unsigned)(iy0 + dy) < (unsigned)p.h && (unsigned)(ix0 + dx) < (unsigned)p.w;
+                    const int here = c == p.tap.chunks - 1 ? p.c_last : 16;
+                    const uint32_t plane = (uint32_t)(p.h * p.w);
+                    uint32_t at = ok ? (uint32_t)(base + dy * p.w + dx) + (uint32_t)(c * 16) * plane : 0u;
+                    u16x2 b[8];  // (two to a register)
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) {
+                        b[j >> 1][j & 1] = p.a[at];
+                        at += ok && j + 1 < here ? plane : 0u;
+                    }
+                    // (taps outside the image and bytes behind the tap's channels: the input zero point; past the reduction: zero after the flip)
+                    const uint32_t other = exists[u] ? p.fill : p.a_xor;
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const uint32_t mask = ok ? byte_mask(here, d) : 0u;
+                        const uint32_t w = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b[2 * d + 1]), __builtin_bit_cast(uint32_t, b[2 * d]), 0x06040200u);
+                        af[u][t][d] = (int)(((w & mask) | (other & ~mask)) ^ p.a_xor);
+                    }
+                }
+            } else {
+                // the chunk this lane fetches for each of the four pixels
+                const int chunk = g * 8 + half * 4 + (lane & 3);
+                exists[u] = chunk * 16 < p.k;
+                int dy, dx, c;
+                place(chunk, dy, dx, c);
+                int off = chunk * 16;
+                if constexpr (TAPS) off = (dy * p.w + dx) * p.cin + c * 16;
+                if constexpr (FORM == INPUT_RAGGED) valid[u] = c == p.tap.chunks - 1 ? p.c_last : 16;
+                auto fetch = [&](auto px_c, int b, int iy, int ix) {
+                    constexpr int px = decltype(px_c)::value;
+                    bool ok = exists[u];
+                    if constexpr (TAPS) ok = ok && (unsigned)(iy + dy) < (unsigned)p.h && (unsigned)(ix + dx) < (unsigned)p.w;
+                    inside[u] |= (uint32_t)ok << px;
+                    if constexpr (FORM == INPUT_RAGGED) {
+                        const uint32_t at = ok ? (uint32_t)(b + off) : 0u, from = at < last_start ? at : last_start;
+                        inside[u] |= (at - from) << (8 + 4 * px);
+                        af[u][px] = *reinterpret_cast<const v4i_any_alignment *>(p.a + from);
+                    } else {
+                        af[u][px] = *reinterpret_cast<const v4i *>(p.a + (size_t)(ok ? b + off : 0));
+                    }
+                };
+                fetch(std::integral_constant<int, 0>{}, q_base.x, q_iy.x, q_ix.x);
+                fetch(std::integral_constant<int, 1>{}, q_base.y, q_iy.y, q_ix.y);
+                fetch(std::integral_constant<int, 2>{}, q_base.z, q_iy.z, q_ix.z);
+                fetch(std::integral_constant<int, 3>{}, q_base.w, q_iy.w, q_ix.w);
+            }
+#pragma unroll
+            for (int t = 0; t < STEPS; ++t) {
+                const int wc = (g * 2 + half) * STEPS + t;
                 bf[u][t] = wsrc[(size_t)(wc < chunks ? wc : chunks - 1) * 32];  // (past the packed rows: multiplied by zeros)
             }
         }
@@ -194,34 +275,53 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
 #pragma unroll
         for (int u = 0; u < GROUPS; ++u) {
             if (g0 + u * kWaves >= groups) break;
-            // taps outside the image read the input zero point; bytes past the reduction the one the flip turns into 0
-            const int other = (int)(exists[u] ? p.fill ^ p.a_xor : 0u), flip = (int)p.a_xor;
+            if constexpr (FORM == INPUT_PLANAR) {
+                if constexpr (ROWSUM) {
 #pragma unroll
-            for (int px = 0; px < 4; ++px) {
-                const bool ok = (inside[u] >> px) & 1u;
-                af[u][px].x = ok ? af[u][px].x ^ flip : other;
-                af[u][px].y = ok ? af[u][px].y ^ flip : other;
-                af[u][px].z = ok ? af[u][px].z ^ flip : other;
-                af[u][px].w = ok ? af[u][px].w ^ flip : other;
-            }
-            if constexpr (ROWSUM) {
-                // (summed before the exchange: of pixel px by the lane that fetched it)
+                    for (int t = 0; t < STEPS; ++t)
+#pragma unroll
+                        for (int d = 0; d < 4; ++d) rowsum[0] = __builtin_amdgcn_sdot4(af[u][t][d], 0x01010101, rowsum[0], false);
+                }
+            } else {
+                // taps outside the image read the input zero point; bytes past the reduction the one the flip turns into 0
+                const int other = (int)(exists[u] ? p.fill ^ p.a_xor : 0u), flip = (int)p.a_xor;
+                if constexpr (FORM == INPUT_RAGGED) {
+                    if (__builtin_amdgcn_ballot_w64(inside[u] >> 8 != 0)) {  // (only where the wave reads the tensor's last bytes)
+#pragma unroll
+                        for (int px = 0; px < 4; ++px) af[u][px] = shift_bytes_down(af[u][px], (inside[u] >> (8 + 4 * px)) & 15u);
+                    }
+                }
+                uint32_t mask[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) mask[d] = FORM == INPUT_RAGGED ? byte_mask(valid[u], d) : ~0u;
 #pragma unroll
                 for (int px = 0; px < 4; ++px) {
-                    rowsum[px] = __builtin_amdgcn_sdot4(af[u][px].x, 0x01010101, rowsum[px], false);
-                    rowsum[px] = __builtin_amdgcn_sdot4(af[u][px].y, 0x01010101, rowsum[px], false);
-                    rowsum[px] = __builtin_amdgcn_sdot4(af[u][px].z, 0x01010101, rowsum[px], false);
-                    rowsum[px] = __builtin_amdgcn_sdot4(af[u][px].w, 0x01010101, rowsum[px], false);
+                    const bool ok = (inside[u] >> px) & 1u;
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const uint32_t v = (uint32_t)(af[u][px][d] ^ flip);
+                        af[u][px][d] = ok ? (int)(FORM == INPUT_RAGGED ? (v & mask[d]) | ((uint32_t)other & ~mask[d]) : v) : other;
+                    }
+                }
+                if constexpr (ROWSUM) {
+                    // (summed before the exchange: of pixel px by the lane that fetched it)
+#pragma unroll
+                    for (int px = 0; px < 4; ++px) {
+                        rowsum[px] = __builtin_amdgcn_sdot4(af[u][px].x, 0x01010101, rowsum[px], false);
+                        rowsum[px] = __builtin_amdgcn_sdot4(af[u][px].y, 0x01010101, rowsum[px], false);
+                        rowsum[px] = __builtin_amdgcn_sdot4(af[u][px].z, 0x01010101, rowsum[px], false);
+                        rowsum[px] = __builtin_amdgcn_sdot4(af[u][px].w, 0x01010101, rowsum[px], false);
+                    }
+                }
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    int c0 = af[u][0][d], c1 = af[u][1][d], c2 = af[u][2][d], c3 = af[u][3][d];
+                    quad_transpose(c0, c1, c2, c3, odd, high);
+                    af[u][0][d] = c0, af[u][1][d] = c1, af[u][2][d] = c2, af[u][3][d] = c3;
                 }
             }
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                int c0 = af[u][0][d], c1 = af[u][1][d], c2 = af[u][2][d], c3 = af[u][3][d];
-                quad_transpose(c0, c1, c2, c3, odd, high);
-                af[u][0][d] = c0, af[u][1][d] = c1, af[u][2][d] = c2, af[u][3][d] = c3;
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[u][t], af[u][t], acc, 0, 0, 0);
+            for (int t = 0; t < STEPS; ++t) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[u][t], af[u][t], acc, 0, 0, 0);
         }
     }
     request_finish();  // (a wave without a step of its own)
@@ -230,7 +330,7 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
 #pragma unroll
     for (int g = 0; g < 4; ++g) *reinterpret_cast<int4 *>(mine + g * 4) = make_int4(acc[g * 4], acc[g * 4 + 1], acc[g * 4 + 2], acc[g * 4 + 3]);
     if constexpr (ROWSUM) {
-        quad_transpose(rowsum[0], rowsum[1], rowsum[2], rowsum[3], odd, high);  // now four lanes' shares of this lane's own pixel
+        if constexpr (FORM != INPUT_PLANAR) quad_transpose(rowsum[0], rowsum[1], rowsum[2], rowsum[3], odd, high);  // now four lanes' shares of this lane's own pixel
         sum_s[wave * 2 + half][r] = rowsum[0] + rowsum[1] + rowsum[2] + rowsum[3];
     }
     __syncthreads();
@@ -266,7 +366,7 @@ __global__ __launch_bounds__(kWaves * 64) void few_tiles_kernel(const std::condi
             o1 = requant_u8_as<mode>(x1, rq);
         }
     };
-    if constexpr (!FAST)
+    if (!FAST || (FORM != INPUT_CHUNKS && rq.fast == 0))
         produce(std::integral_constant<int, 0>{});
     else if (rq.fast == 2)
         produce(std::integral_constant<int, 2>{});
@@ -323,15 +423,34 @@ bool gemm_few_tiles_instead(const GemmProblem &p) {
     return p.cfg.id == GEMM_THIN || p.cfg.id == GEMM_CONV3X3;
 }
 
+// Against the copy and the kernel that reads it, us (start of the line: tiles, bytes of a tap's reduction with its padding):
+//   ragged   7, 176 of 128 x 175 x 88 7.7 -> 3.8; 352, 288 of 3x3 24 -> 64 at 6 x 28x28 7.6 -> 4.5; 875, 96 of 4000 x 90 x 200 7.7 -> 6.8; 774, 288
+//            of 3x3 24 -> 168 at 11 x 17x22 7.8 -> 7.0; 752, 512 of 6000 x 500 x 128 9.3 either way; 1252, 288 7.9 -> 8.7; 1120, 1008 9.1 -> 9.9
+//   planar   287, 288 of 3x3 21 -> 21 at 3 x 65x47 7.8 -> 5.2; 150, 864 of 3x3 96 -> 96 at 4 x 20x20 7.7 -> 7.0; 100, 1152 7.5 -> 7.2; 784, 256 of 1x1
+//            256 -> 128 at 32 x 14x14 9.3 -> 6.7; 588, 288 7.1 -> 7.8; 294, 800 8.4 -> 9.1; 800, 160 7.8 -> 8.1
+// (planar 1x1 layers of one product keep to two rounds: 980 tiles 6.5 .. 7.6 either way)
+bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t problems, int32_t form) {
+    const long tiles = m > 0 ? few_tiles_count(m, n) * problems : 0;
+    if (tiles <= 0 || k > 8192) return false;
+    if (form == INPUT_RAGGED) return tiles <= 512 || (tiles <= 1024 && k <= 448);
+    const long rounds = (tiles + 255) / 256;
+    return rounds <= 2 ? k * rounds <= 1152 : tiles < 800 && k > 32 && k <= 256;
+}
+
 int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream) {
     const TapProblem &p = ps[0];
     EH_REQUIRE(count >= 1 && count <= GemmBatch::MAX, "few_tiles: batch of %d", count);
     int m_max = p.m;
     for (int i = 0; i < count; ++i) {
         EH_REQUIRE(ps[i].k_pad == p.k_pad && ps[i].n == p.n && ps[i].zw == p.zw && ps[i].rq.fast == p.rq.fast && ps[i].vec == 16 &&
-                       (ps[i].k & 15) == 0 && (ps[i].k_pad & 31) == 0 && ps[i].k_pad >= ps[i].k && ps[i].k > 0 && ps[i].k % (ps[i].tap.chunks * 16) == 0,
+                       (ps[i].k & 15) == 0 && (ps[i].k_pad & 31) == 0 && ps[i].k_pad >= ps[i].k && ps[i].k > 0 && ps[i].k % (ps[i].tap.chunks * 16) == 0 &&
+                       ps[i].form == p.form && ps[i].c_last == p.c_last && ps[i].c_last >= 1 && ps[i].c_last <= 16,
                    "few_tiles: unsupported problem");
-        EH_REQUIRE((reinterpret_cast<uintptr_t>(ps[i].a) & 15) == 0 && (ps[i].cin & 15) == 0 && (ps[i].tap.c0 & 15) == 0, "few_tiles: unaligned activations");
+        if (p.form != INPUT_CHUNKS)
+            EH_REQUIRE((int64_t)(ps[i].m / (ps[i].ho * ps[i].wo)) * ps[i].h * ps[i].w * ps[i].cin >= 16 && ps[i].tap.c0 + (ps[i].tap.chunks - 1) * 16 + ps[i].c_last <= ps[i].cin,
+                       "few_tiles: channels %d .. of %d", ps[i].tap.c0, ps[i].cin);
+        else
+            EH_REQUIRE((reinterpret_cast<uintptr_t>(ps[i].a) & 15) == 0 && (ps[i].cin & 15) == 0 && (ps[i].tap.c0 & 15) == 0, "few_tiles: unaligned activations");
         m_max = ps[i].m > m_max ? ps[i].m : m_max;
     }
     const int m_blocks = (m_max + 31) / 32, n_blocks = (p.n + 31) / 32;
@@ -340,7 +459,7 @@ int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream) {
     const int per_xcd = (int)((tiles + 7) / 8);
     const int m_fastest = (long)p.n * p.k >= (long)p.m * p.cin ? 1 : 0;  // the larger operand's blocks run slowest
     const dim3 grid((unsigned)(per_xcd * 8), 1, (unsigned)count), block(kWaves * 64);
-    const int groups = ((p.k_pad + 127) / 128 + kWaves - 1) / kWaves;  // of the longest-working wave
+    const int groups = ((p.k_pad + (p.form == INPUT_PLANAR ? 31 : 127)) / (p.form == INPUT_PLANAR ? 32 : 128) + kWaves - 1) / kWaves;  // of the longest-working wave
     // one tap at the pixel itself, on an image it cannot leave
     bool inside = true;
     for (int i = 0; i < count; ++i)
@@ -349,19 +468,23 @@ int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream) {
     FewBatch batch;
     if (count > 1)
         for (int i = 0; i < count; ++i) batch.p[i] = ps[i];
-    auto launch = [&](auto groups_c, auto taps_c, auto rowsum_c, auto fast_c) {
-        constexpr int S = decltype(groups_c)::value;
+    auto launch = [&](auto groups_c, auto taps_c, auto rowsum_c, auto fast_c, auto form_c) {
+        constexpr int S = decltype(groups_c)::value, I = decltype(form_c)::value;
         constexpr bool T = decltype(taps_c)::value, R = decltype(rowsum_c)::value, F = decltype(fast_c)::value;
         if (count > 1)
-            hipLaunchKernelGGL((few_tiles_kernel<S, T, R, F, true>), grid, block, 0, stream, batch, m_blocks, n_blocks, per_xcd, m_fastest);
+            hipLaunchKernelGGL((few_tiles_kernel<S, T, R, F, true, I>), grid, block, 0, stream, batch, m_blocks, n_blocks, per_xcd, m_fastest);
         else
-            hipLaunchKernelGGL((few_tiles_kernel<S, T, R, F, false>), grid, block, 0, stream, FewProblem(p), m_blocks, n_blocks, per_xcd, m_fastest);
+            hipLaunchKernelGGL((few_tiles_kernel<S, T, R, F, false, I>), grid, block, 0, stream, FewProblem(p), m_blocks, n_blocks, per_xcd, m_fastest);
     };
     auto with_fast = [&](auto groups_c, auto taps_c, auto rowsum_c) {
-        if (p.rq.fast != 0)
-            launch(groups_c, taps_c, rowsum_c, std::true_type{});
+        if (p.form == INPUT_RAGGED)
+            launch(groups_c, taps_c, rowsum_c, std::true_type{}, std::integral_constant<int, INPUT_RAGGED>{});
+        else if (p.form == INPUT_PLANAR)
+            launch(groups_c, taps_c, rowsum_c, std::true_type{}, std::integral_constant<int, INPUT_PLANAR>{});
+        else if (p.rq.fast != 0)
+            launch(groups_c, taps_c, rowsum_c, std::true_type{}, std::integral_constant<int, INPUT_CHUNKS>{});
         else
-            launch(groups_c, taps_c, rowsum_c, std::false_type{});
+            launch(groups_c, taps_c, rowsum_c, std::false_type{}, std::integral_constant<int, INPUT_CHUNKS>{});
     };
     auto with_rowsum = [&](auto groups_c, auto taps_c) {
         if (p.zw != 0)

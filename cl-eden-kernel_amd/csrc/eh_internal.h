@@ -544,9 +544,18 @@ __device__ __forceinline__ void store_bytes_planar(uint8_t *out, const PlanarOut
     }
 }
 
+// How the kernel for few tiles finds a tap's 16-channel chunks.
+enum InputForm {
+    INPUT_CHUNKS = 0,   // every tap is whole aligned chunks (the caller's tensor, or a padded copy of it)
+    INPUT_RAGGED = 1,   // channels-last rows of any length at any alignment: `cin` bytes per pixel, the last chunk of a tap holds c_last
+    INPUT_PLANAR = 2,   // one plane per channel, `cin` of them per image, the last chunk of a tap holds c_last
+};
+
 // A problem as the host hands it to the launchers.  Only the kernel for few tiles is given the taps' geometry.
 struct TapProblem : GemmProblem {
     TapGeom tap;
+    int32_t c_last = 16;
+    int32_t form = INPUT_CHUNKS;
 };
 
 // Equally shaped problems of one operator that go out as one launch (kernel argument).
@@ -576,6 +585,8 @@ int launch_gemm_skinny(const GemmProblem &p, hipStream_t stream);
 // few output tiles (eh_gemm_few.hip): whether a problem whose weights are packed in fragment order should run there, and the launch
 bool gemm_few_tiles_applies(int64_t m, int64_t n, int64_t k, int32_t siblings);
 bool gemm_few_tiles_instead(const GemmProblem &p);  // ... although it was planned for another kernel of the same weight order
+// ... reading the caller's own tensor in form `form` where the plan's kernels would read a padded or channels-last copy of it
+bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t problems, int32_t form);
 int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream);  // `count` equally shaped problems as one launch
 // few input channels, a kernel row per reduction step (eh_conv_rows.hip)
 bool conv_rows_applies(int32_t cin_group, int32_t pixel_stride, int32_t kh, int32_t kw);
