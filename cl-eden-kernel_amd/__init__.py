@@ -387,7 +387,7 @@ def conv_dw_block_preferred(pw, dw):
 
 
 def conv_dw_block_tile(pw, dw, rows_per_tile=0, cols_per_tile=0):
-    """(rows, columns, blocks of 32 channels, depthwise stage on the matrix cores) of the tile that a fused launch of the pair takes"""
+    """(rows, columns, blocks of 32 channels, depthwise stage in units of sixteen outputs) of the tile that a fused launch of the pair takes"""
     out = [C.c_int32() for _ in range(4)]
     check(load().eh_conv_dw_block_tile(pw.handle, dw.handle, rows_per_tile, cols_per_tile, *(C.byref(v) for v in out)))
     return tuple(v.value for v in out[:3]) + (bool(out[3].value),)

@@ -13,12 +13,16 @@
 //      (pixel block, channel block) pairs are dealt out evenly over the four waves), requantized exactly as the
 //      pointwise operator does it and written as uint8 into an LDS image [row][column][channel]; pixels outside the
 //      image are written as the depthwise operator's input zero point, which is what its padding reads;
-//   2. after one barrier the threads compute the depthwise outputs from that image, four horizontally adjacent output
-//      pixels of four channels per thread, with the arithmetic of the stand-alone depthwise kernel (8-bit dot products,
-//      signed or unsigned form), and store them.
-//      Small tiles (a network on few images) do this stage on the matrix cores: a thread's sixteen outputs are a chain of some 300
-//      vector instructions that a workgroup of few such threads waits for.  28x28 32 -> 192 at stride 2, two images, 5.4 -> 4.2 us
-//      (pwdw_block_geometry has the rule and both sides of it).
+//   2. after one barrier the waves compute the depthwise outputs from that image on the matrix cores and store them.  One 16x16x64
+//      product takes 16 pixels and, per pixel, 16 channels at up to four columns of a kernel row; its other operand is diagonal.
+//      A wave takes 16 channels and walks down 16 columns of the tile (or 8 in two strips of rows, or 4 in four): an input row is
+//      read once, multiplied by each kernel row that it meets, and the vector units are left with the requantization, some 20
+//      instructions for 256 outputs.  (As 8-bit dot products, which want every channel's three rows gathered into a word first, a
+//      thread's sixteen outputs were 300.)  Dot products -> walk, us: 24 -> 144 at 56x56, 23 images 16.1 -> 11.8; 64 -> 384 at
+//      58x58, 16 images 32.7 -> 23; 16 -> 96 at 83x83, 21 images 21.4 -> 13.6; 56 -> 336 at 31x31, 18 images 13.4 -> 9.3; 120 -> 720
+//      at 12x12, 18 images 9.2 -> 7.0; a pair per channel, 16 -> 96 at 104x97, 28 images 34.1 -> 26.6, 80 -> 480 at 36x36, 16 images
+//      20.4 -> 15.0; at stride 2, where the expansion is most of the work, 24 -> 144 at 56x56, 32 images 11.3 and 11.3.
+//      Tiles of few outputs are taken sixteen outputs at a time instead, wherever their rows end (pwdw_block_geometry has the rule).
 // The rows and columns two neighbouring workgroups both need (the halo) are computed twice; nothing else is.  Tiles are
 // cut in both directions because the halo of a stride-2 window costs (2 TH + 1)(2 TW + 1) / (4 TH TW): 1.53 for one full
 // row of 28 outputs, 1.21 for 4 x 7.
@@ -38,39 +42,27 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 namespace {
 
-__device__ __forceinline__ int udot4(uint32_t a, uint32_t b, int acc) { return (int)__builtin_amdgcn_udot4(a, b, (uint32_t)acc, false); }
-
-// the four channels of a column's three rows as four words of three bytes each (byte 3 zero)
-__device__ __forceinline__ void column_words(uint32_t r0, uint32_t r1, uint32_t r2, uint32_t (&out)[4]) {
-    const uint32_t t01 = __builtin_amdgcn_perm(r1, r0, 0x05010400u);
-    const uint32_t t23 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
-    out[0] = __builtin_amdgcn_perm(r2, t01, 0x0c040100u);
-    out[1] = __builtin_amdgcn_perm(r2, t01, 0x0c050302u);
-    out[2] = __builtin_amdgcn_perm(r2, t23, 0x0c060100u);
-    out[3] = __builtin_amdgcn_perm(r2, t23, 0x0c070302u);
-}
-
 // S: depthwise stride.  FORM: how the depthwise stage multiplies (DwForm).  ROWSUM: the pointwise weights' zero point is not 128, so a pixel's byte sum enters.
 // QM: pointwise requantization, 0 two-step order, 1 / 2 the single-shift forms.  KS: reduction steps of the pointwise
 // stage when they are 1, 2 or 3 (a lane then keeps its pixel's operand bytes in registers across the channel blocks),
 // 0 for any number (read from LDS for every product).
 enum class DwForm {
-    DOT,   // 8-bit dot products of a - 128 and w - zp_w
-    FOLD,  // ... of the raw bytes: the unsigned form, for weights of any range
-    MATRIX // on the matrix cores, weights of any range
+    UNITS,  // small tiles: sixteen outputs of the tile, wherever its rows end, by sixteen channels
+    WALK    // the others: sixteen columns, down the tile's rows
 };
-template <int S, DwForm FORM, bool ROWSUM, int QM, int KS, bool PC>
+// PC: one multiplier and shift per channel in both operators; the depthwise ones in the single-shift form, or in two steps.
+enum class Pairs { TENSOR, CHANNEL, CHANNEL_TWO_STEP };
+template <int S, DwForm FORM, bool ROWSUM, int QM, int KS, Pairs PAIRS>
 __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, const DwProblem dw, const BlockGeom g) {
-    constexpr bool FOLD = FORM == DwForm::FOLD, MATRIX = FORM == DwForm::MATRIX;
+    constexpr bool WALK = FORM == DwForm::WALK, PC = PAIRS != Pairs::TENSOR, DW_TWO_STEP = PAIRS == Pairs::CHANNEL_TWO_STEP;
     const int ksteps = KS ? KS : g.ks;
     extern __shared__ __align__(16) uint8_t lds_raw[];
     v4i *b_s = reinterpret_cast<v4i *>(lds_raw);                              // [nb][ks][64 lanes]: pointwise weights, fragment order
     int32_t *bias_s = reinterpret_cast<int32_t *>(lds_raw + (size_t)g.nb * ksteps * 1024);  // [nb * 32]
-    // PC (one multiplier and shift per channel in both operators): the pointwise stage's pairs beside the bias; the shifts as the
-    // bytes that requant4_channel wants or, two-step, as they are
+    // PC: the pointwise stage's pairs beside the bias; the shifts as the bytes that requant4_channel wants or, two-step, as they are
     int32_t *pcm_s = bias_s + g.nb * 32, *pcf_s = pcm_s + g.nb * 32;
     uint8_t *pce_s = reinterpret_cast<uint8_t *>(pcf_s);
-    uint8_t *img_s = lds_raw + g.image_off;                                   // [ih][iwp][cpitch] uint8 (xor 0x80 for the signed form)
+    uint8_t *img_s = lds_raw + g.image_off;                                   // [ih][iwp][cpitch] uint8 xor 0x80: operands
     const int nb_first = blockIdx.y * g.nb;                                   // this workgroup's channel range
     const int c_first = nb_first * 32;
     const int c_here = g.c - c_first < g.nb * 32 ? g.c - c_first : g.nb * 32;  // channels of the range that exist (a multiple of 16)
@@ -90,10 +82,11 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
     const int iy_first = oy0 * S - dw.pad_t, ix_first = ox_first * S - dw.pad_l;  // image coordinates of the LDS image's corner
     uint8_t *a_s = lds_raw + g.a_off;  // [pixels][a_pitch]: the input pixels' reduction bytes as signed operands (a ^ 0x80), 0 past the reduction length
 
-    // MATRIX: units of (chunk of 16 channels, 16 output pixels), a contiguous share per wave; lane (i, q) holds the weights of
-    // channel i of the chunk in kernel column q.  A wave's first chunk is requested ahead of everything else.
+    // The depthwise stage's units of (chunk of 16 channels, 16 output pixels or columns of output pixels), a contiguous share per
+    // wave; lane (i, q) holds the weights of channel i of the chunk in kernel column q.  A wave's first chunk is requested ahead
+    // of everything else.
     const int lane16 = lane & 15, quarter = lane >> 4, cpad = (g.c + 15) & ~15;
-    const int out_pixels = g.th * g.tw, groups = (out_pixels + 15) >> 4, w_uniform = __builtin_amdgcn_readfirstlane(wave);
+    const int out_pixels = g.th * g.tw, groups = WALK ? g.walk_groups : (out_pixels + 15) >> 4, w_uniform = __builtin_amdgcn_readfirstlane(wave);
     const int unit_first = ((c_here >> 4) * groups * w_uniform) >> 2, unit_last = ((c_here >> 4) * groups * (w_uniform + 1)) >> 2;
     struct DwPart {
         uint32_t w[3], neg;  // by kernel row; minus what the stored weights lack (dw_pack_mfma_kernel)
@@ -114,9 +107,7 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
     };
     int chunk = unit_first / groups, group = unit_first - chunk * groups;
     DwPart part{};
-    if constexpr (MATRIX) {
-        if (unit_first < unit_last) part = request_dw(chunk);
-    }
+    if (unit_first < unit_last) part = request_dw(chunk);
 
     // ---- stage 0: weights, bias and the tile's input pixels into LDS (8-byte pieces: pixels start on 8-byte boundaries)
     auto inside_image = [&](int q, int &iy, int &ix) {
@@ -161,7 +152,7 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
     }
 
     // ---- stage 1: the expanded pixels into the LDS image.  Units of (pixel block, channel block), a contiguous share per wave.
-    const uint32_t flip_store = FOLD ? 0u : 0x80808080u;  // the signed depthwise forms read a - 128
+    const uint32_t flip_store = 0x80808080u;  // the depthwise stage multiplies a - 128
     const uint32_t pad_word = ((uint32_t)dw.zp_in * 0x01010101u) ^ flip_store;
     const int blocks = (g.pixels + 31) >> 5;
     const RequantDev rq = pw.rq;
@@ -253,40 +244,113 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
     __syncthreads();
 
     // ---- stage 2: the depthwise outputs from the LDS image
-    // four channels' accumulators to four bytes
-    auto finish = [&](int a0, int a1, int a2, int a3, const int4 &m, const int4 &sh) {
-        const RequantDev &drq = dw.rq;
-        if constexpr (PC) {
-            // (the caller clears `fast` unless every pair fits the four-channel form)
-            if (drq.fast == 2) return requant4_channel<2>(a0, a1, a2, a3, m, channel_shift_bytes(sh), drq);
-            if (drq.fast) return requant4_channel<1>(a0, a1, a2, a3, m, channel_shift_bytes(sh), drq);
-            return pack_bytes(requant_u8_channel(a0, m.x, sh.x, drq), requant_u8_channel(a1, m.y, sh.y, drq), requant_u8_channel(a2, m.z, sh.z, drq),
-                              requant_u8_channel(a3, m.w, sh.w, drq));
-        }
-        if (drq.fast == 2) return requant4_fast<2>(a0, a1, a2, a3, 0, drq);
-        if (drq.fast) return requant4_fast<1>(a0, a1, a2, a3, 0, drq);
-        return pack_bytes(requant_u8(a0, drq), requant_u8(a1, drq), requant_u8(a2, drq), requant_u8(a3, drq));
+    // As in eh_dwconv_mfma.hip: lane (i, q) fetches the sixteen channels of output pixel i's window at kernel column q, one
+    // 16-byte piece per kernel row, and three products against diagonal weights leave every lane with four neighbouring
+    // channels of one pixel.
+    const int column = quarter < 3 ? quarter : 2;  // (the fourth column's weights are zero: any pixel will do)
+    auto diagonal = [&](uint32_t byte) {
+        const int v = (int)(byte << (8 * (lane16 & 3))), d = lane16 >> 2;
+        return v4i{d == 0 ? v : 0, d == 1 ? v : 0, d == 2 ? v : 0, d == 3 ? v : 0};
     };
-    if constexpr (MATRIX) {
-        // As in eh_dwconv_mfma.hip: lane (i, q) fetches the sixteen channels of output pixel i's window at kernel column q, one
-        // 16-byte piece per kernel row, and three products against diagonal weights leave every lane with four neighbouring
-        // channels of one pixel.
-        const int column = quarter < 3 ? quarter : 2;  // (the fourth column's weights are zero: any pixel will do)
-        auto diagonal = [&](uint32_t byte) {
-            const int v = (int)(byte << (8 * (lane16 & 3))), d = lane16 >> 2;
-            return v4i{d == 0 ? v : 0, d == 1 ? v : 0, d == 2 ? v : 0, d == 3 ? v : 0};
-        };
-        for (int left = unit_last - unit_first; left > 0; group = 0, ++chunk) {
-            v4i wf[3];
+    auto product = [](const v4i &w, const v4i &x, const v4i &acc) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(w, x, acc, 0, 0, 0); };
+    const auto out = __builtin_amdgcn_make_buffer_rsrc(dw.out, 0, (int)((uint32_t)dw.n * (uint32_t)dw.ho * (uint32_t)dw.wo * (uint32_t)dw.cout), 0x00020000);
+    const uint32_t out_pitch = (uint32_t)dw.wo * (uint32_t)dw.cout;
+    for (int left = unit_last - unit_first; left > 0; group = 0, ++chunk) {
+        v4i wf[3];
 #pragma unroll
-            for (int ky = 0; ky < 3; ++ky) wf[ky] = diagonal(part.w[ky]);
-            const v4i df = diagonal(quarter < 3 ? part.neg : 0u);
-            const bool lacks = __builtin_amdgcn_ballot_w64(part.neg != 0) != 0;
-            const DwPart now = part;
-            const int last_group = left < groups - group ? group + left : groups;
-            left -= last_group - group;
-            if (left > 0) part = request_dw(chunk + 1);  // (on its way under this chunk's products)
-            const int c0 = c_first + chunk * 16;
+        for (int ky = 0; ky < 3; ++ky) wf[ky] = diagonal(part.w[ky]);
+        const v4i df = diagonal(quarter < 3 ? part.neg : 0u);
+        const bool lacks = __builtin_amdgcn_ballot_w64(part.neg != 0) != 0;
+        const DwPart now = part;
+        const uint32_t shift_bytes = PC && !DW_TWO_STEP ? channel_shift_bytes(now.shift) : 0u;
+        // four channels' accumulators to four bytes
+        const RequantDev &drq = dw.rq;
+        auto finish = [&](auto mode_c, const v4i &a) {
+            constexpr int MODE = decltype(mode_c)::value;  // single-shift form 1 or 2, or the two steps
+            if constexpr (PC && MODE != 0)
+                return requant4_channel<MODE>(a.x, a.y, a.z, a.w, now.mult, shift_bytes, drq);
+            else if constexpr (PC)
+                return pack_bytes(requant_u8_channel(a.x, now.mult.x, now.shift.x, drq), requant_u8_channel(a.y, now.mult.y, now.shift.y, drq),
+                                  requant_u8_channel(a.z, now.mult.z, now.shift.z, drq), requant_u8_channel(a.w, now.mult.w, now.shift.w, drq));
+            else if constexpr (MODE != 0)
+                return requant4_fast<MODE>(a.x, a.y, a.z, a.w, 0, drq);
+            else
+                return pack_bytes(requant_u8(a.x, drq), requant_u8(a.y, drq), requant_u8(a.z, drq), requant_u8(a.w, drq));
+        };
+        auto with_mode = [&](auto body) {
+            if constexpr (DW_TWO_STEP)
+                body(std::integral_constant<int, 0>{});
+            else if (drq.fast == 2)
+                body(std::integral_constant<int, 2>{});
+            else if (PC || drq.fast != 0)  // (the caller clears `fast` unless every channel's pair fits the four-channel form)
+                body(std::integral_constant<int, 1>{});
+            else
+                body(std::integral_constant<int, 0>{});
+        };
+        const v4i bias = v4i{now.bias.x, now.bias.y, now.bias.z, now.bias.w}, none = v4i{0, 0, 0, 0};
+        const int last_group = left < groups - group ? group + left : groups;
+        left -= last_group - group;
+        if (left > 0) part = request_dw(chunk + 1);  // (on its way under this chunk's products)
+        const int c0 = c_first + chunk * 16;
+        if constexpr (WALK) {
+            // lanes 0-15 are 16 columns, or 8 in two strips of rows, or 4 in four
+            const int strip = lane16 >> g.walk_log, rows = g.th >> (4 - g.walk_log);
+            auto walk = [&](auto mode_c, auto lacks_c) {
+                constexpr bool LACKS = decltype(lacks_c)::value;
+                for (int grp = group; grp < last_group; ++grp) {
+                    const int px = (grp << g.walk_log) + lane16 - (strip << g.walk_log), oy = oy0 + strip * rows, ox = ox_first + px;
+                    const int at = px * S + column < g.iwp ? px * S + column : g.iwp - 1;  // (columns past the tile: not stored)
+                    const uint8_t *src = img_s + (strip * rows * S * g.iwp + at) * cpitch + chunk * 16;
+                    const int src_pitch = g.iwp * cpitch;
+                    const int rows_here = px < g.tw && ox < dw.wo ? dw.ho - oy : 0;
+                    uint32_t dst = ((img * (uint32_t)dw.ho + (uint32_t)oy) * (uint32_t)dw.wo + (uint32_t)ox) * (uint32_t)dw.cout + (uint32_t)(c0 + quarter * 4);
+                    auto next = [&] {
+                        const v4i x = *reinterpret_cast<const v4i *>(src);
+                        src += src_pitch;
+                        return x;
+                    };
+                    auto store = [&](const v4i &acc, int o) {
+                        const uint32_t v = finish(mode_c, acc);
+                        // (what is not the tile's is sent past the tensor's end, where the hardware drops it: no branch per row)
+                        __builtin_amdgcn_raw_buffer_store_b32(v, out, (int)(o < rows_here ? dst : 0xFFFFFFF0u), 0, 0);
+                        dst += out_pitch;
+                    };
+                    // an input row is multiplied by every kernel row it meets: two, or one, output rows are on their way beside the one it ends
+                    if constexpr (S == 1) {
+                        v4i x = next(), a0 = product(wf[0], x, bias), l0 = LACKS ? product(df, x, none) : none;
+                        x = next();
+                        v4i a1 = product(wf[1], x, a0), l1 = LACKS ? product(df, x, l0) : none;
+                        a0 = product(wf[0], x, bias);
+                        if constexpr (LACKS) l0 = product(df, x, none);
+                        for (int o = 0; o < rows; ++o) {
+                            x = next();
+                            v4i done = product(wf[2], x, a1);
+                            a1 = product(wf[1], x, a0);
+                            a0 = product(wf[0], x, bias);
+                            if constexpr (LACKS) {
+                                done -= product(df, x, l1);
+                                l1 = product(df, x, l0);
+                                l0 = product(df, x, none);
+                            }
+                            store(done, o);
+                        }
+                    } else {
+                        v4i x = next(), a = product(wf[0], x, bias), l = LACKS ? product(df, x, none) : none;
+                        for (int o = 0; o < rows; ++o) {
+                            const v4i x1 = next(), x2 = next();
+                            v4i done = product(wf[2], x2, product(wf[1], x1, a));
+                            a = product(wf[0], x2, bias);
+                            if constexpr (LACKS) {
+                                done -= product(df, x2, product(df, x1, l));
+                                l = product(df, x2, none);
+                            }
+                            store(done, o);
+                        }
+                    }
+                }
+            };
+            with_mode([&](auto mode_c) { lacks ? walk(mode_c, std::true_type{}) : walk(mode_c, std::false_type{}); });
+        } else {
             for (int grp = group; grp < last_group; ++grp) {
                 const int p = grp * 16 + lane16, pc = p < out_pixels ? p : out_pixels - 1;
                 const int row = (int)fastdiv((uint32_t)pc, g.div_tw), col = pc - row * g.tw, oy = oy0 + row, ox = ox_first + col;
@@ -294,89 +358,21 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
                 v4i x[3];
 #pragma unroll
                 for (int ky = 0; ky < 3; ++ky) x[ky] = *reinterpret_cast<const v4i *>(src + ky * g.iwp * cpitch);
-                v4i acc = v4i{now.bias.x, now.bias.y, now.bias.z, now.bias.w};
+                v4i acc = bias;
 #pragma unroll
-                for (int ky = 0; ky < 3; ++ky) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[ky], x[ky], acc, 0, 0, 0);
+                for (int ky = 0; ky < 3; ++ky) acc = product(wf[ky], x[ky], acc);
                 if (lacks) {
-                    v4i lack = v4i{0, 0, 0, 0};
+                    v4i lack = none;
 #pragma unroll
-                    for (int ky = 0; ky < 3; ++ky) lack = __builtin_amdgcn_mfma_i32_16x16x64_i8(df, x[ky], lack, 0, 0, 0);
+                    for (int ky = 0; ky < 3; ++ky) lack = product(df, x[ky], lack);
                     acc -= lack;
                 }
-                const uint32_t o = finish(acc.x, acc.y, acc.z, acc.w, now.mult, now.shift);
+                uint32_t o = 0;
+                with_mode([&](auto mode_c) { o = finish(mode_c, acc); });
                 if (p < out_pixels && oy < dw.ho && ox < dw.wo)
                     *reinterpret_cast<uint32_t *>(dw.out + (((img * (uint32_t)dw.ho + (uint32_t)oy) * (uint32_t)dw.wo + (uint32_t)ox) * (uint32_t)dw.cout +
                                                             (uint32_t)(c0 + quarter * 4))) = o;
             }
-        }
-        return;
-    }
-    constexpr int TW = 4, IW = (TW - 1) * S + 3;  // a thread's four adjacent output pixels
-    const uint32_t cq_count = (uint32_t)c_here >> 2;
-    const uint32_t units = (uint32_t)g.units_per_cq * cq_count;
-    const uint32_t cq_first = (uint32_t)c_first >> 2;
-    const FastDiv div_cq = blockIdx.y + 1 == gridDim.y ? g.div_cq_last : g.div_cq;
-    for (uint32_t u = (uint32_t)tid; u < units; u += 256u) {
-        const uint32_t t = fastdiv(u, div_cq);
-        const uint32_t cql = u - t * cq_count, cq = cq_first + cql;  // channel quad within the range, and in the layer
-        const uint32_t row = fastdiv(t, g.div_tx);
-        const int tx = (int)(t - row * (uint32_t)g.tiles_x);
-        const int oy = oy0 + (int)row, lx0 = tx * TW, ox0 = ox_first + lx0;  // lx0: first column within the workgroup's tile
-        if (oy >= dw.ho) continue;
-        uint32_t in[3][IW];
-#pragma unroll
-        for (int ky = 0; ky < 3; ++ky)
-#pragma unroll
-            for (int x = 0; x < IW; ++x) {
-                int col = lx0 * S + x;
-                col = col < g.iwp ? col : g.iwp - 1;  // columns past the last window belong to outputs that are not stored
-                in[ky][x] = *reinterpret_cast<const uint32_t *>(img_s + (((int)row * S + ky) * g.iwp + col) * cpitch + (int)cql * 4);
-            }
-        int4 wk[3];
-#pragma unroll
-        for (int kx = 0; kx < 3; ++kx) wk[kx] = *reinterpret_cast<const int4 *>((FOLD ? dw.w_fold : dw.w_trip) + ((uint32_t)kx * (uint32_t)dw.cout + cq * 4u));
-        const int4 b4 = *reinterpret_cast<const int4 *>((FOLD ? dw.bias_fold : dw.bias_trip) + cq * 4u);
-        int4 dm = make_int4(0, 0, 0, 0), ds = dm;  // PC: the depthwise stage's four pairs
-        if constexpr (PC) {
-            dm = *reinterpret_cast<const int4 *>(dw.rq.pc_multiplier + cq * 4u);
-            ds = *reinterpret_cast<const int4 *>(dw.rq.pc_shift + cq * 4u);
-        }
-        uint32_t colw[IW][4];
-        int cs[FOLD ? IW : 1][4];
-#pragma unroll
-        for (int x = 0; x < IW; ++x) {
-            column_words(in[0][x], in[1][x], in[2][x], colw[x]);
-            if constexpr (FOLD) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) cs[x][c] = udot4(colw[x][c], 0x00010101u, 0);
-            }
-        }
-        uint8_t *dst = dw.out + (((img * (uint32_t)dw.ho + (uint32_t)oy) * (uint32_t)dw.wo + (uint32_t)ox0) * (uint32_t)dw.cout + cq * 4u);
-#pragma unroll
-        for (int j = 0; j < TW; ++j) {
-            int acc0 = b4.x, acc1 = b4.y, acc2 = b4.z, acc3 = b4.w;
-#pragma unroll
-            for (int kx = 0; kx < 3; ++kx) {
-                if constexpr (FOLD) {
-                    acc0 = udot4(colw[j * S + kx][0], (uint32_t)wk[kx].x, acc0);
-                    acc1 = udot4(colw[j * S + kx][1], (uint32_t)wk[kx].y, acc1);
-                    acc2 = udot4(colw[j * S + kx][2], (uint32_t)wk[kx].z, acc2);
-                    acc3 = udot4(colw[j * S + kx][3], (uint32_t)wk[kx].w, acc3);
-                } else {
-                    acc0 = __builtin_amdgcn_sdot4((int)colw[j * S + kx][0], wk[kx].x, acc0, false);
-                    acc1 = __builtin_amdgcn_sdot4((int)colw[j * S + kx][1], wk[kx].y, acc1, false);
-                    acc2 = __builtin_amdgcn_sdot4((int)colw[j * S + kx][2], wk[kx].z, acc2, false);
-                    acc3 = __builtin_amdgcn_sdot4((int)colw[j * S + kx][3], wk[kx].w, acc3, false);
-                }
-            }
-            if constexpr (FOLD) {
-                acc0 += __mul24(-dw.zp_w, cs[j * S][0] + cs[j * S + 1][0] + cs[j * S + 2][0]);
-                acc1 += __mul24(-dw.zp_w, cs[j * S][1] + cs[j * S + 1][1] + cs[j * S + 2][1]);
-                acc2 += __mul24(-dw.zp_w, cs[j * S][2] + cs[j * S + 1][2] + cs[j * S + 2][2]);
-                acc3 += __mul24(-dw.zp_w, cs[j * S][3] + cs[j * S + 1][3] + cs[j * S + 2][3]);
-            }
-            const uint32_t o = finish(acc0, acc1, acc2, acc3, dm, ds);
-            if (lx0 + j < g.tw && ox0 + j < dw.wo) *reinterpret_cast<uint32_t *>(dst + (uint32_t)j * (uint32_t)dw.cout) = o;
         }
     }
 }
@@ -411,14 +407,14 @@ bool pwdw_block_takes(const DwProblem &dw) {
 
 // The pointwise problem is a one-tap problem of at most eight 32-byte reduction steps on whole dense images whose
 // weights are packed in fragment order, the depthwise one a 3x3 channels-last layer of stride 1 or 2 on the pointwise
-// output with the 8-bit dot product weights at hand; uint8 tensors; one requantization pair per operator, or one pair per
+// output with the matrix form of its weights at hand; uint8 tensors; one requantization pair per operator, or one pair per
 // channel in both.
 bool pwdw_block_applies(const GemmProblem &pw, const DwProblem &dw) {
     if (pw.cfg.id != GEMM_THIN || pw.k_pad > 256 || pw.k > pw.k_pad || (pw.k & 7) != 0 || (pw.cin & 7) != 0 || pw.k != pw.cin) return false;
     if (pw.stride_h != 1 || pw.stride_w != 1 || pw.y_base != 0 || pw.x_base != 0 || pw.ho != pw.h || pw.wo != pw.w) return false;
     if (pw.a_xor != 0x80808080u || pw.out_xor != 0u || pw.residual) return false;
     if ((pw.rq.pc_multiplier != nullptr) != (dw.rq.pc_multiplier != nullptr)) return false;
-    if (!pwdw_block_takes(dw) || dw.c != pw.n || dw.h != pw.h || dw.w_ != pw.w || (!dw.w_trip && !dw.w_fold)) return false;
+    if (!pwdw_block_takes(dw) || dw.c != pw.n || dw.h != pw.h || dw.w_ != pw.w || dw.w_mm == nullptr) return false;
     if ((size_t)dw.n * dw.h * dw.w_ * pw.cin >= (1ull << 31) || (size_t)dw.n * dw.ho * dw.wo * dw.cout >= (1ull << 31)) return false;
     return block_lds_bytes(1, pw.k_pad / 32, 3, 3 * dw.stride_w + 3, dw.c, nullptr, nullptr) <= kBlockLdsMax;  // one row of four outputs, one channel block
 }
@@ -456,6 +452,69 @@ bool pwdw_block_preferred(const GemmProblem &pw, const DwProblem &dw) {
     return pwdw_block_applies(pw, dw) && pwdw_block_listed(dw.n, dw.h, dw.w_, pw.k, dw.c, dw.stride_h);
 }
 
+namespace {
+
+// The tile of a launch whose depthwise stage walks: the one that takes the least time by a count of its waves' instructions, each of
+// which takes a SIMD some 2.3 + 1.1 w ns for the w waves it holds; a set of workgroups that a CU holds at a time (registers leave
+// room for five, with a pair per channel four) takes a microsecond beside that.  The coefficients are fitted to 3900 tiles of eighteen
+// layers; for those layers the tile chosen is 3 % slower than the fastest on average and 8 % at most.
+bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, int cols_per_tile, int *th, int *tw, int *nb, int *walk_log) {
+    const int S = dw.stride_h, ks = pw.k_pad / 32, nb_all = (dw.c + 31) / 32, chunks_all = dw.c / 16;
+    const double epilogue = pw.rq.pc_multiplier ? 1.42 : 1.0;
+    const int held = pw.rq.pc_multiplier ? 4 : 5;
+    auto shares = [](int a, int b) { return (a + b - 1) / b; };
+    double best = -1;
+    for (const size_t lds_max : {(size_t)64 * 1024, kBlockLdsMax}) {  // (above 64 KiB a launch sets an attribute of the kernel first)
+        for (int cn = 1; cn <= nb_all; ++cn) {
+            const int ranges = shares(nb_all, cn);
+            if ((ranges - 1) * cn >= nb_all) continue;  // the same ranges with fewer blocks each
+            const int chunks = cn * 2 < chunks_all ? cn * 2 : chunks_all;
+            for (int lg = 4; lg >= 2; --lg) {
+                const int strips = 16 >> lg;
+                if (rows_per_tile > 0 && rows_per_tile % strips != 0) continue;
+                // tiles down the image and across it, as equal as whole strips and columns allow
+                for (int down = 1, ch_before = 0; down <= dw.ho; ++down) {
+                    const int ch = rows_per_tile > 0 ? rows_per_tile : shares(dw.ho, down * strips) * strips;
+                    if (ch == ch_before) {
+                        if (rows_per_tile > 0 || ch == strips) break;
+                        continue;
+                    }
+                    ch_before = ch;
+                    for (int across = 1, cw_before = 0; across <= dw.wo; ++across) {
+                        const int cw = cols_per_tile > 0 ? cols_per_tile : shares(dw.wo, across);
+                        if (cw == cw_before) {
+                            if (cols_per_tile > 0 || cw == 1) break;
+                            continue;
+                        }
+                        cw_before = cw;
+                        const int pixels = ((ch - 1) * S + 3) * ((cw - 1) * S + 3);
+                        const size_t lds = block_lds_bytes(cn, ks, (ch - 1) * S + 3, (cw - 1) * S + 3, dw.c, nullptr, nullptr);
+                        if (lds > lds_max) continue;
+                        const double wave = 10 + 40.0 * cn + 40.0 * shares(pixels * ks * 4, 256) + shares(shares(pixels, 32) * cn, 4) * (67.0 * epilogue + 5.5 * ks) +
+                                            shares(chunks * shares(cw, 1 << lg), 4) * (52.0 + 26.0 * epilogue * (ch / strips));
+                        const double per_cu = (double)dw.n * shares(dw.ho, ch) * shares(dw.wo, cw) * ranges / 256.0;
+                        const int fit = (int)((160 * 1024) / lds), most = fit < held ? fit : held, full = (int)(per_cu / most);
+                        auto time = [&](int waves) { return wave * (2.3 + 1.07 * waves) + 800; };
+                        const int rest = (int)(per_cu - full * most + 0.999);
+                        const double cost = full * time(most) + (rest > 0 ? time(rest) : 0);
+                        if (best < 0 || cost < best) {
+                            best = cost;
+                            *th = ch;
+                            *tw = cw;
+                            *nb = cn;
+                            *walk_log = lg;
+                        }
+                    }
+                }
+            }
+        }
+        if (best >= 0) return true;
+    }
+    return false;
+}
+
+}  // namespace
+
 bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, int cols_per_tile, BlockGeom *geom) {
     const int S = dw.stride_h;
     BlockGeom g;
@@ -470,10 +529,10 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     // the one that computes the fewest pixel slots wins, counting the slots that pixel blocks of 32 and output tiles of
     // four leave empty and, at a lower weight, the input bytes staged again for every channel range.
     int th = rows_per_tile, tw = cols_per_tile, nb = nb_all;
-    // Form of the depthwise stage.  The matrix form works in units of sixteen output pixels by sixteen channels, spread over the four
-    // waves, the vector form in units of four by four, some 300 instructions each, one to a thread: with few of them a workgroup waits
-    // for that chain, however few threads walk it.  With more than a matrix unit to a wave it is a matter of their fill and of their
-    // epilogue, which a pair per channel doubles.  The same tiles, vector -> matrix form, us (with a pair per channel):
+    // Form of the depthwise stage.  Units of sixteen output pixels by sixteen channels, spread over the four waves, suit a tile of few of
+    // them, whose rows a walk would leave half of its lanes without; with more than one or two to a wave it is a matter of their fill
+    // and of their epilogue, which a pair per channel doubles.  The line was drawn against 8-bit dot products, sixteen outputs to a
+    // thread, whose place the walk has taken.  The same tiles, dot products -> units, us (with a pair per channel):
     //   up to 3 units  28x28 32 -> 192 stride 2, 2 images 5.4 -> 4.2 (6.1 -> 4.6), stride 1, 2 images 4.6 -> 4.3 (4.9 -> 4.6),
     //                  7x7 160 -> 960, 1 image 5.3 -> 4.55 (6.1 -> 5.05)
     //   4              56x56 24 -> 144 stride 2, 4 images 5.4 -> 4.75 (6.1 -> 5.5), 28x28 32 -> 192 stride 1, 4 images 4.7 -> 4.8
@@ -488,7 +547,7 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     auto quads_of = [&](int blocks) { return blocks * 8 < dw.c / 4 ? blocks * 8 : dw.c / 4; };
     auto matrix_form = [&](int rows, int cols, int blocks) {
         const int groups = (rows * cols + 15) / 16, units = groups * (quads_of(blocks) / 4);
-        return dw.w_mm != nullptr && units <= (!per_channel ? 8 : S == 2 ? 6 : 3) && (units <= 4 || rows * cols > groups * 8);
+        return units <= (!per_channel ? 8 : S == 2 ? 6 : 3) && (units <= 4 || rows * cols > groups * 8);
     };
     {
         double best = -1;
@@ -509,7 +568,7 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
                         const int px = ih * iw;
                         const double tiles = (double)dw.n * ((dw.ho + ch - 1) / ch) * ((dw.wo + cw - 1) / cw);
                         const double stage1 = (double)((px + 31) / 32 * 32) * tiles / ((double)dw.n * dw.h * dw.w_);   // pixel slots computed per real pixel
-                        // A tile of up to 128 vector units (half the threads) is priced by whole groups of sixteen outputs, a slot of them at
+                        // A tile of up to 128 groups of four outputs by four channels is priced by whole groups of sixteen outputs, a slot of them at
                         // three quarters, whichever form will run it: by the vector form's own slots the search prefers tiles of two outputs
                         // or four, whose chain is as long and whose halo is larger.  Tiles by groups and by slots, us (with a pair per
                         // channel): both matrix, 56x56 24 -> 144 stride 2, one image 4.15 and 4.5 (4.6 and 5.0); matrix and vector, 28x28
@@ -533,29 +592,25 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
         tw = best_tw;
         nb = best_nb;
     }
+    g.matrix = matrix_form(th, tw, nb) ? 1 : 0;
+    g.walk_log = g.walk_groups = 0;
+    if (!g.matrix && !walk_tile(pw, dw, rows_per_tile, cols_per_tile, &th, &tw, &nb, &g.walk_log)) return false;
     g.nb = nb;
-    if (!(th >= 1 && th <= dw.ho && tw >= 1 && tw <= dw.wo)) return false;
     g.th = th;
     g.tw = tw;
     g.ih = (th - 1) * S + 3;
     g.iwp = (tw - 1) * S + 3;
     g.pixels = g.ih * g.iwp;
-    g.tiles_x = (tw + 3) / 4;
     g.tiles_y = (dw.ho + th - 1) / th;
     g.tiles_w = (dw.wo + tw - 1) / tw;
     g.total_tiles = dw.n * g.tiles_y * g.tiles_w;
-    g.units_per_cq = th * g.tiles_x;
+    if (!g.matrix) g.walk_groups = (tw + (1 << g.walk_log) - 1) >> g.walk_log;
     g.div_iwp = make_fastdiv((uint32_t)g.iwp);
-    g.div_tx = make_fastdiv((uint32_t)g.tiles_x);
     g.div_tw = make_fastdiv((uint32_t)tw);
     g.div_tiles_y = make_fastdiv((uint32_t)g.tiles_y);
     g.div_tiles_w = make_fastdiv((uint32_t)g.tiles_w);
     g.div_ppp = make_fastdiv((uint32_t)(g.ks * 4));
-    const int ranges = (nb_all + g.nb - 1) / g.nb;
-    g.div_cq = make_fastdiv((uint32_t)(g.nb * 8 < g.c / 4 ? g.nb * 8 : g.c / 4));
-    g.div_cq_last = make_fastdiv((uint32_t)((g.c - (ranges - 1) * g.nb * 32) / 4));
     g.cpitch = block_image_pitch(g.nb, g.c);
-    g.matrix = matrix_form(th, tw, nb) ? 1 : 0;
     const size_t lds = block_lds_bytes(g.nb, g.ks, g.ih, g.iwp, g.c, &g.a_off, &g.image_off);
     if (lds > kBlockLdsMax) return false;
     *geom = g;
@@ -563,13 +618,10 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
 }
 
 // `g`: what pwdw_block_geometry gave for the pair (the search over tiles costs the host as much as the launch: callers keep it)
-int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, const BlockGeom &g, hipStream_t stream) {
-    EH_REQUIRE(pwdw_block_applies(pw, caller_dw), "block: the two operators do not fit the fused kernel");
-    EH_REQUIRE((reinterpret_cast<uintptr_t>(pw.a) & 7) == 0 && (reinterpret_cast<uintptr_t>(caller_dw.out) & 3) == 0, "block: unaligned tensors");
-    EH_REQUIRE(g.c == caller_dw.c && g.ks == pw.k_pad / 32, "block: geometry of another pair");
-    DwProblem dw = caller_dw;
-    if (dw.w_trip) dw.w_fold = nullptr;                 // the signed form where it applies, as the stand-alone launcher decides
-    if (dw.w_fold) dw.zp_w += dw.w_signed ? 128 : 0;    // zero point of the uint8 values the unsigned form multiplies
+int launch_pwdw_block(const GemmProblem &pw, const DwProblem &dw, const BlockGeom &g, hipStream_t stream) {
+    EH_REQUIRE(pwdw_block_applies(pw, dw), "block: the two operators do not fit the fused kernel");
+    EH_REQUIRE((reinterpret_cast<uintptr_t>(pw.a) & 7) == 0 && (reinterpret_cast<uintptr_t>(dw.out) & 3) == 0, "block: unaligned tensors");
+    EH_REQUIRE(g.c == dw.c && g.ks == pw.k_pad / 32, "block: geometry of another pair");
     const int S = dw.stride_h;
     const size_t lds = (size_t)g.image_off + (size_t)g.ih * g.iwp * g.cpitch;
     if (g.total_tiles <= 0) return EH_OK;
@@ -586,7 +638,10 @@ int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, const B
         return (int)EH_OK;
     };
     auto launch = [&](auto s_c, auto form_c, auto rowsum_c, auto qm_c, auto ks_c) {
-        return pw.rq.pc_multiplier ? launch_pc(s_c, form_c, rowsum_c, qm_c, ks_c, std::true_type{}) : launch_pc(s_c, form_c, rowsum_c, qm_c, ks_c, std::false_type{});
+        using std::integral_constant;
+        if (!pw.rq.pc_multiplier) return launch_pc(s_c, form_c, rowsum_c, qm_c, ks_c, integral_constant<Pairs, Pairs::TENSOR>{});
+        return dw.rq.fast ? launch_pc(s_c, form_c, rowsum_c, qm_c, ks_c, integral_constant<Pairs, Pairs::CHANNEL>{})
+                          : launch_pc(s_c, form_c, rowsum_c, qm_c, ks_c, integral_constant<Pairs, Pairs::CHANNEL_TWO_STEP>{});
     };
     auto with_ks = [&](auto s_c, auto form_c, auto rowsum_c, auto qm_c) {
         if (g.ks == 1) return launch(s_c, form_c, rowsum_c, qm_c, std::integral_constant<int, 1>{});
@@ -603,8 +658,7 @@ int launch_pwdw_block(const GemmProblem &pw, const DwProblem &caller_dw, const B
         return pw.zw != 0 ? with_qm(s_c, form_c, std::true_type{}) : with_qm(s_c, form_c, std::false_type{});
     };
     auto with_form = [&](auto s_c) {
-        if (g.matrix) return with_rowsum(s_c, std::integral_constant<DwForm, DwForm::MATRIX>{});
-        return dw.w_trip ? with_rowsum(s_c, std::integral_constant<DwForm, DwForm::DOT>{}) : with_rowsum(s_c, std::integral_constant<DwForm, DwForm::FOLD>{});
+        return g.matrix ? with_rowsum(s_c, std::integral_constant<DwForm, DwForm::UNITS>{}) : with_rowsum(s_c, std::integral_constant<DwForm, DwForm::WALK>{});
     };
     const int rc = S == 1 ? with_form(std::integral_constant<int, 1>{}) : with_form(std::integral_constant<int, 2>{});
     if (rc) return rc;

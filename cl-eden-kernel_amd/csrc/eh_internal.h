@@ -702,13 +702,11 @@ struct BlockGeom {
     int32_t nb;          // channel blocks of 32 per workgroup (grid y walks the ranges); bytes per pixel of the LDS image = 32 nb
     int32_t ks;          // reduction steps of 32 bytes of the pointwise stage
     int32_t cpitch;      // bytes per pixel of the LDS image
-    int32_t tiles_x;     // depthwise tiles of four output columns per row of the workgroup's tile
-    int32_t units_per_cq;  // th * tiles_x: depthwise thread-units per channel quad
-    int32_t matrix;      // the depthwise stage runs on the matrix cores (see pwdw_block_geometry)
+    int32_t matrix;      // the depthwise stage takes sixteen outputs at a time (small tiles; see pwdw_block_geometry)
+    int32_t walk_log, walk_groups;  // otherwise: log2 of the columns a wave walks down, and such groups per tile
     int32_t total_tiles; // n * tiles_y * tiles_w
     int32_t a_pitch;     // LDS bytes per input pixel: 32 ks + 16 (the slack spreads the fragment reads over the banks)
-    FastDiv div_iwp, div_tx, div_tw, div_tiles_y, div_tiles_w, div_ppp;
-    FastDiv div_cq, div_cq_last;  // by the channel quads of a full range, and of the last one
+    FastDiv div_iwp, div_tw, div_tiles_y, div_tiles_w, div_ppp;
     uint32_t a_off;      // byte offset of the staged input pixels
     uint32_t image_off;  // byte offset of the LDS image behind the staged weights, bias and input pixels
 };
