@@ -1,7 +1,7 @@
 // Depthwise uint8 convolution with 5x5 and 7x7 windows on the matrix cores (gfx950), channels-last tensors.
 //
 // On the vector units such a window is bound by instructions: 8-bit dot products need every channel's taps gathered into
-// words first, 30 instructions per output at 5x5 (64 images of 144 channels at 56x56: 39 us, 24 here; the bytes take 11).
+// words first, 30 instructions per output at 5x5 (64 images of 144 channels at 56x56: 39 us, 22.6 here; the bytes take 11).
 // The matrix form needs no gather.  One 16x16x64 product takes 16 pixels and, per pixel, 64 bytes: the 16 channels of a
 // 16-byte piece at four neighbouring taps of a kernel row, read as they lie in memory; the other operand is diagonal
 // (channel i of tap t only reaches output channel i), so 15 of 16 products multiply zeros, and 25 taps still cost seven
@@ -99,6 +99,7 @@ __global__ __launch_bounds__(256) void dw_mfma_kernel(const DwProblem p, const D
     const int fill = (int)(((uint32_t)p.zp_in * 0x01010101u) ^ 0x80808080u);
     const uint32_t base = (uint32_t)img * (uint32_t)(p.h * p.w_ * p.c) + (uint32_t)chunk0 * 16u;
     const int line = g.cols * g.ch_per;  // 16-byte pieces of a tile row
+    const auto in = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(p.in), 0, (int)g.in_bytes, 0x00020000);
     constexpr int BATCH = 4;             // rows a thread has on their way
     auto fetch = [&](auto inside_c, auto whole_c) {
         constexpr bool INSIDE = decltype(inside_c)::value, WHOLE = decltype(whole_c)::value;
@@ -107,35 +108,48 @@ __global__ __launch_bounds__(256) void dw_mfma_kernel(const DwProblem p, const D
         for (int e = tid - y_first * line; e < line; e += (int)blockDim.x) {  // (one turn where a step takes whole rows)
             const int x = (int)fastdiv((uint32_t)e, g.div_ch), c = e - x * g.ch_per, ix = ix0 + x;
             const bool exists = INSIDE || ((unsigned)ix < (unsigned)p.w_ && c < n_chunks);
-            // A piece that does not exist is read from the nearest one that does: with the loads in branches of their own the
-            // compiler waited for each before it made the next.  (144 channels at 56x56, 64 images: 5x5 25.6 -> 24.7 us, at stride 2
-            // 16.0 -> 14.7, 7x7 36.3 -> 32.8; 88 at 100x100, 7x7 stride 2, 44 images 26.5 -> 22.6.)
+            // A piece that does not exist is loaded without a branch of its own: with one the compiler waited for each load before it
+            // made the next.  (144 channels at 56x56, 64 images: 5x5 25.6 -> 24.7 us, at stride 2 16.0 -> 14.7, 7x7 36.3 -> 32.8; 88
+            // at 100x100, 7x7 stride 2, 44 images 26.5 -> 22.6.)  Of pixels of whole pieces it is sent past the tensor's end, where
+            // the bounds check gives zero, and the XOR that makes operands makes it the fill: one select in place of the clamps and
+            // four more.  (The first and third again: 23.8 -> 22.6, 32.6 -> 30.2.)
             const int ixc = ix < 0 ? 0 : (ix < p.w_ ? ix : p.w_ - 1), cc = c < n_chunks ? c : 0;
-            const uint32_t off0 = base + (uint32_t)((INSIDE ? ix : ixc) * p.c + (INSIDE ? c : cc) * 16), pitch = (uint32_t)(p.w_ * p.c);
+            const uint32_t off0 = base + (uint32_t)((WHOLE ? ix : ixc) * p.c + (WHOLE ? c : cc) * 16), pitch = (uint32_t)(p.w_ * p.c);
             uint8_t *to = lds + c * g.plane + x * 16;
             for (int y0 = y_first; y0 < g.rows; y0 += g.rows_per_step * BATCH) {
                 v4i v[BATCH];
+                int mask[BATCH];
 #pragma unroll
                 for (int b = 0; b < BATCH; ++b) {
-                    const int y = y0 + b * g.rows_per_step, yc = y < g.rows ? y : g.rows - 1;
-                    int iy = iy0 + yc;
-                    if constexpr (!INSIDE) iy = iy < 0 ? 0 : (iy < p.h ? iy : p.h - 1);
-                    const uint32_t off = off0 + (uint32_t)iy * pitch;
-                    if (WHOLE || off + 16u <= g.in_bytes) {
-                        v[b] = *reinterpret_cast<const v4i_a4 *>(p.in + off);
-                    } else {  // the tensor's last pixel, where it ends inside a piece
-                        v[b] = v4i{0, 0, 0, 0};
+                    const int y = y0 + b * g.rows_per_step;
+                    if constexpr (WHOLE) {
+                        const bool there = y < g.rows && (INSIDE || (exists && (unsigned)(iy0 + y) < (unsigned)p.h));
+                        mask[b] = there ? flip : fill;
+                        v[b] = __builtin_amdgcn_raw_buffer_load_b128(in, (int)(there ? off0 + (uint32_t)(iy0 + y) * pitch : 0xFFFFFFF0u), 0, 0);
+                    } else {
+                        int iy = iy0 + (y < g.rows ? y : g.rows - 1);
+                        iy = iy < 0 ? 0 : (iy < p.h ? iy : p.h - 1);
+                        const uint32_t off = off0 + (uint32_t)iy * pitch;
+                        if (off + 16u <= g.in_bytes) {
+                            v[b] = *reinterpret_cast<const v4i_a4 *>(p.in + off);
+                        } else {  // the tensor's last pixel, where it ends inside a piece
+                            v[b] = v4i{0, 0, 0, 0};
 #pragma unroll
-                        for (int d = 0; d < 3; ++d)
-                            if (off + 4u * d + 4u <= g.in_bytes) v[b][d] = *reinterpret_cast<const int *>(p.in + off + 4u * d);
+                            for (int d = 0; d < 3; ++d)
+                                if (off + 4u * d + 4u <= g.in_bytes) v[b][d] = *reinterpret_cast<const int *>(p.in + off + 4u * d);
+                        }
                     }
                 }
 #pragma unroll
                 for (int b = 0; b < BATCH; ++b) {
                     const int y = y0 + b * g.rows_per_step;
-                    const bool there = INSIDE || (exists && (unsigned)(iy0 + y) < (unsigned)p.h);
-                    if (y < g.rows)
-                        *reinterpret_cast<v4i *>(to + y * g.cols * 16) = v4i{there ? v[b].x ^ flip : fill, there ? v[b].y ^ flip : fill, there ? v[b].z ^ flip : fill, there ? v[b].w ^ flip : fill};
+                    if constexpr (WHOLE) {
+                        v[b] ^= v4i{mask[b], mask[b], mask[b], mask[b]};
+                    } else {
+                        const bool there = exists && (unsigned)(iy0 + y) < (unsigned)p.h;
+                        v[b] = v4i{there ? v[b].x ^ flip : fill, there ? v[b].y ^ flip : fill, there ? v[b].z ^ flip : fill, there ? v[b].w ^ flip : fill};
+                    }
+                    if (y < g.rows) *reinterpret_cast<v4i *>(to + y * g.cols * 16) = v[b];
                 }
             }
         }
