@@ -432,7 +432,9 @@ bool pwdw_block_applies(const GemmProblem &pw, const DwProblem &dw) {
 //    28     32 -> 192        2      -1.1
 // (changes within +-1.5 are noise.  With the listed pairs fused the pass takes 324.6; 14 x 14 64 -> 384 alone runs in 6.6 us against 8.0
 // for the two launches, 28 x 28 32 -> 192 in 9.2 against 9.2 and at stride 2 in 6.8 against 7.8, 56 x 56 24 -> 144 in 20.9 against 21.1.)
-// A shape that is not in the table runs as two launches.
+// A shape that is not in the table runs as two launches.  (The figures are from before the depthwise stage's walk; timed alone since, two
+// launches against one, us: 96 -> 576 at 14x14, 32 images 11.0 and 8.5, at stride 2 9.8 and 7.7, 160 -> 960 at 7x7, 32 images 10.0 and 8.4,
+// 24 -> 144 at 56x56, 32 images 18.0 and 16.9.  The answer is part of the interface and has been left as it was.)
 bool pwdw_block_listed(int32_t images, int32_t image_h, int32_t image_w, int32_t in_channels, int32_t expanded_channels, int32_t stride) {
     // Below 32 images a launch is mostly latency, and one launch instead of two wins for the whole network:
     // MobileNetV2 with all 16 fitting pairs fused against the listed ones, 144 against 162 us at batch 1, 168 against 176
@@ -463,44 +465,56 @@ bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, in
     const double epilogue = pw.rq.pc_multiplier ? 1.42 : 1.0;
     const int held = pw.rq.pc_multiplier ? 4 : 5;
     auto shares = [](int a, int b) { return (a + b - 1) / b; };
+    // tiles across the image and down it, as equal as columns and whole strips allow, the largest first.  (A launch finds its tile the
+    // first time it runs: what a candidate needs is worked out ahead of the loops, and shapes that cannot win are not looked at.)
+    constexpr int MOST = 24;
+    struct Cut {
+        int size, pieces;
+    } across[MOST], down[3][MOST];
+    int n_across = 0, n_down[3] = {0, 0, 0};
+    auto cut = [&](int extent, int fixed, int unit, Cut *to, int *count) {
+        if (fixed > 0) {
+            if (fixed % unit == 0) to[(*count)++] = Cut{fixed, shares(extent, fixed)};
+            return;
+        }
+        for (int pieces = 1; pieces <= extent && *count < MOST; ++pieces) {
+            const int size = shares(extent, pieces * unit) * unit;
+            if (size > 64 || (*count > 0 && to[*count - 1].size == size)) continue;
+            to[(*count)++] = Cut{size, shares(extent, size)};
+            if (size == unit) break;
+        }
+    };
+    cut(dw.wo, cols_per_tile, 1, across, &n_across);
+    for (int lg = 4; lg >= 2; --lg) cut(dw.ho, rows_per_tile, 16 >> lg, down[4 - lg], &n_down[4 - lg]);
     double best = -1;
     for (const size_t lds_max : {(size_t)64 * 1024, kBlockLdsMax}) {  // (above 64 KiB a launch sets an attribute of the kernel first)
         for (int cn = 1; cn <= nb_all; ++cn) {
             const int ranges = shares(nb_all, cn);
             if ((ranges - 1) * cn >= nb_all) continue;  // the same ranges with fewer blocks each
             const int chunks = cn * 2 < chunks_all ? cn * 2 : chunks_all;
+            const size_t lds_fixed = block_lds_bytes(cn, ks, 0, 0, dw.c, nullptr, nullptr), lds_pixel = (size_t)(ks * 32 + 16 + block_image_pitch(cn, dw.c));
             for (int lg = 4; lg >= 2; --lg) {
-                const int strips = 16 >> lg;
-                if (rows_per_tile > 0 && rows_per_tile % strips != 0) continue;
-                // tiles down the image and across it, as equal as whole strips and columns allow
-                for (int down = 1, ch_before = 0; down <= dw.ho; ++down) {
-                    const int ch = rows_per_tile > 0 ? rows_per_tile : shares(dw.ho, down * strips) * strips;
-                    if (ch == ch_before) {
-                        if (rows_per_tile > 0 || ch == strips) break;
-                        continue;
-                    }
-                    ch_before = ch;
-                    for (int across = 1, cw_before = 0; across <= dw.wo; ++across) {
-                        const int cw = cols_per_tile > 0 ? cols_per_tile : shares(dw.wo, across);
-                        if (cw == cw_before) {
-                            if (cols_per_tile > 0 || cw == 1) break;
-                            continue;
-                        }
-                        cw_before = cw;
-                        const int pixels = ((ch - 1) * S + 3) * ((cw - 1) * S + 3);
-                        const size_t lds = block_lds_bytes(cn, ks, (ch - 1) * S + 3, (cw - 1) * S + 3, dw.c, nullptr, nullptr);
+                for (int i = 0; i < n_down[4 - lg]; ++i) {
+                    const Cut d = down[4 - lg][i];
+                    const int ih = (d.size - 1) * S + 3;
+                    const double walk = 52.0 + 26.0 * epilogue * (d.size >> (4 - lg)), groups_of_tiles = (double)dw.n * d.pieces * ranges / 256.0;
+                    for (int j = 0; j < n_across; ++j) {
+                        const Cut a = across[j];
+                        const int pixels = ih * ((a.size - 1) * S + 3);
+                        const size_t lds = lds_fixed + (size_t)pixels * lds_pixel + 15;
                         if (lds > lds_max) continue;
-                        const double wave = 10 + 40.0 * cn + 40.0 * shares(pixels * ks * 4, 256) + shares(shares(pixels, 32) * cn, 4) * (67.0 * epilogue + 5.5 * ks) +
-                                            shares(chunks * shares(cw, 1 << lg), 4) * (52.0 + 26.0 * epilogue * (ch / strips));
-                        const double per_cu = (double)dw.n * shares(dw.ho, ch) * shares(dw.wo, cw) * ranges / 256.0;
+                        const double per_cu = groups_of_tiles * a.pieces;
+                        if (best >= 0 && pixels < 64 && per_cu > held) break;  // (small tiles only where larger ones would leave CUs idle)
+                        const double wave = 10 + 40.0 * cn + 40.0 * ((pixels * ks * 4 + 255) >> 8) + ((((pixels + 31) >> 5) * cn + 3) >> 2) * (67.0 * epilogue + 5.5 * ks) +
+                                            ((chunks * ((a.size + (1 << lg) - 1) >> lg) + 3) >> 2) * walk;
                         const int fit = (int)((160 * 1024) / lds), most = fit < held ? fit : held, full = (int)(per_cu / most);
                         auto time = [&](int waves) { return wave * (2.3 + 1.07 * waves) + 800; };
                         const int rest = (int)(per_cu - full * most + 0.999);
                         const double cost = full * time(most) + (rest > 0 ? time(rest) : 0);
                         if (best < 0 || cost < best) {
                             best = cost;
-                            *th = ch;
-                            *tw = cw;
+                            *th = d.size;
+                            *tw = a.size;
                             *nb = cn;
                             *walk_log = lg;
                         }
@@ -549,24 +563,30 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
         const int groups = (rows * cols + 15) / 16, units = groups * (quads_of(blocks) / 4);
         return units <= (!per_channel ? 8 : S == 2 ? 6 : 3) && (units <= 4 || rows * cols > groups * 8);
     };
-    {
+    // (A layer of so many units leaves more of them to each workgroup that the chip holds.)
+    const bool large = rows_per_tile == 0 && cols_per_tile == 0 && (double)dw.n * dw.ho * dw.wo * dw.c > 768.0 * 12 * 256;
+    if (!large) {
+        int across[65];
+        for (int cw = 1; cw <= dw.wo && cw <= 64; ++cw) across[cw] = (dw.wo + cw - 1) / cw;
         double best = -1;
         int best_th = 1, best_tw = dw.wo < 4 ? dw.wo : 4, best_nb = 1;
         for (int pass = 0; pass < 3 && best < 0; ++pass)  // later passes: fewer workgroups, then anything that fits at all
             for (int cn = 1; cn <= nb_all; ++cn) {
                 const int ranges = (nb_all + cn - 1) / cn;
                 if ((ranges - 1) * cn >= nb_all) continue;  // the same ranges with fewer blocks each
-                for (int ch = 1; ch <= dw.ho && ch <= 16; ++ch)
+                const size_t lds_fixed = block_lds_bytes(cn, g.ks, 0, 0, dw.c, nullptr, nullptr), lds_pixel = (size_t)block_image_pitch(cn, dw.c);
+                for (int ch = 1; ch <= dw.ho && ch <= 16; ++ch) {
+                    const int down = (dw.ho + ch - 1) / ch;
                     for (int cw = 1; cw <= dw.wo && cw <= 64; ++cw) {
                         if (rows_per_tile > 0 && ch != rows_per_tile) continue;
                         if (cols_per_tile > 0 && cw != cols_per_tile) continue;
                         const int ih = (ch - 1) * S + 3, iw = (cw - 1) * S + 3;
-                        const size_t lds = block_lds_bytes(cn, g.ks, ih, iw, dw.c, nullptr, nullptr);
+                        const size_t lds = lds_fixed + (((size_t)ih * iw * (g.ks * 32 + 16) + 15) & ~(size_t)15) + (size_t)ih * iw * lds_pixel;
                         if (pass < 2 ? lds * 4 > 144 * 1024 : lds > kBlockLdsMax) continue;
-                        const long wgs = (long)dw.n * ((dw.ho + ch - 1) / ch) * ((dw.wo + cw - 1) / cw) * ranges;
+                        const long wgs = (long)dw.n * down * across[cw] * ranges;
                         if (pass == 0 && wgs < 768) continue;
                         const int px = ih * iw;
-                        const double tiles = (double)dw.n * ((dw.ho + ch - 1) / ch) * ((dw.wo + cw - 1) / cw);
+                        const double tiles = (double)dw.n * down * across[cw];
                         const double stage1 = (double)((px + 31) / 32 * 32) * tiles / ((double)dw.n * dw.h * dw.w_);   // pixel slots computed per real pixel
                         // A tile of up to 128 groups of four outputs by four channels is priced by whole groups of sixteen outputs, a slot of them at
                         // three quarters, whichever form will run it: by the vector form's own slots the search prefers tiles of two outputs
@@ -586,13 +606,14 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
                             best_nb = cn;
                         }
                     }
+                }
             }
         if (best < 0) return false;
         th = best_th;
         tw = best_tw;
         nb = best_nb;
     }
-    g.matrix = matrix_form(th, tw, nb) ? 1 : 0;
+    g.matrix = !large && matrix_form(th, tw, nb) ? 1 : 0;
     g.walk_log = g.walk_groups = 0;
     if (!g.matrix && !walk_tile(pw, dw, rows_per_tile, cols_per_tile, &th, &tw, &nb, &g.walk_log)) return false;
     g.nb = nb;
