@@ -769,7 +769,7 @@ struct eh_dwconv_plan {
     // every pixel with repeats of its last channel, the weights of the extra channels are zero, and the result is
     // computed into an image of the padded width, from which the caller's channels are copied out.
     int32_t cout_caller = 0;        // `cout` counts the padded channels; this is what the caller's tensors hold
-    bool planar = false;            // the caller's tensors are NCHW
+    bool planar = false;            // the caller's tensors are NCHW, and the kernels' are not
     uint8_t *stage_in = nullptr, *stage_out = nullptr;
     // geometry of the latest fused launch behind a pointwise layer, and what it was chosen for
     BlockGeom block{};
@@ -1908,7 +1908,11 @@ int eh_dwconv2d_u8_plan(eh_dwconv_plan **plan, const eh_conv_desc *desc, const v
         return EH_INVALID_PARAMS;
     }
     hipStream_t s = as_stream(stream);
-    rc = dev_alloc(&pl->w_copy, (size_t)pl->cout * pl->taps);
+    if (pl->planar && dw_planar_applies(dw_problem(pl, nullptr, nullptr))) {
+        pl->planar = false;
+        pl->d.layout = EH_NCHW;
+    }
+    rc = dev_alloc(&pl->w_copy, (size_t)pl->cout * pl->taps + 4);
     if (!rc && (pl->rep_dm || pl->planar)) rc = dev_alloc(&pl->stage_in, (size_t)desc->n * desc->h * desc->w * pl->cout + 256);
     if (!rc && (pl->planar || pl->cout != pl->cout_caller)) rc = dev_alloc(&pl->stage_out, (size_t)desc->n * pl->ho * pl->wo * pl->cout + 256);
     if (!rc) rc = dev_alloc(&pl->bias_copy, (size_t)pl->cout);

@@ -376,6 +376,136 @@ __global__ __launch_bounds__(256) void dw3x3_nhwc_tile4_dot4_kernel(const DwProb
     }
 }
 
+// Planar tensors, K x K windows, stride S, no dilation: a thread owns four horizontally adjacent outputs of R rows of one plane.
+//
+// A row of a plane is what 8-bit dot products want: an output's taps of a kernel row are neighbouring bytes, with no gather.  The thread
+// loads the aligned words of each input row under its windows, shifts them to its first column by one byte alignment each, and replaces
+// what lies outside the image by masks that are the same for all its rows.  Weights are the caller's bytes as uint8; their zero point
+// enters through the windows' sums.  Bound by those instructions on large tensors, some 25 per output at 5x5.
+// Before -> here, us.  Through channels-last and back, three launches: 3x3 29 images of 232 channels at 8x7 9.7 -> 4.0, 32 of 144 at 56x56
+// 27.3 -> 13.0; 5x5 64 of 144 at 56x56 53.0 -> 37.5; 7x7 2 of 520 at 13x7 11.5 -> 3.6.  One output to a thread, where the channels were no
+// multiple of four or had a multiplier: 5x5 3 of 171 at 103x103 76 -> 11.2, 7x7 8 of 64 x 2 at 40x40 35.8 -> 6.2.
+template <int K, int S, int R, bool PC>
+__global__ __launch_bounds__(256) void dw_planar_kernel(const DwProblem p, const uint32_t total, const int quads, const int bands, const FastDiv div_quads,
+                                                        const FastDiv div_bands, const FastDiv div_cout, const FastDiv div_dm) {
+    constexpr int F = (K + 3) / 4, ND = (3 * S + 4 * F - 1) / 4 + 1, ROWS = (R - 1) * S + K;  // words per kernel row, per input row; input rows
+    const uint32_t idx = xcd_contiguous_block() * 256u + threadIdx.x;
+    if (idx >= total) return;
+    const uint32_t r = fastdiv(idx, div_quads), plane = fastdiv(r, div_bands);
+    const int ox0 = (int)(idx - r * (uint32_t)quads) * 4, oy0 = (int)(r - plane * (uint32_t)bands) * R;
+    const uint32_t img = fastdiv(plane, div_cout), oc = plane - img * (uint32_t)p.cout;
+    const uint32_t in_plane = img * (uint32_t)p.c + fastdiv(oc, div_dm);
+    const int ix0 = ox0 * S - p.pad_l, iy0 = oy0 * S - p.pad_t;
+    // the tensor from the word that it starts in to the one that it ends in: an aligned word with a byte of the tensor may be read whole
+    const uint32_t lead = (uint32_t)reinterpret_cast<uintptr_t>(p.in) & 3u;
+    const auto in = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(p.in) - lead, 0,
+                                                      (int)((lead + (uint32_t)p.n * (uint32_t)p.c * (uint32_t)p.h * (uint32_t)p.w_ + 3u) & ~3u), 0x00020000);
+    const uint32_t fill = (uint32_t)p.zp_in * 0x01010101u;
+    uint32_t keep[ND], pad[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {  // bytes of word i left of the image, and those up to its right edge
+        const int lo = -ix0 - 4 * i, hi = p.w_ - ix0 - 4 * i;
+        const uint32_t below = lo <= 0 ? 0u : lo >= 4 ? ~0u : (1u << (8 * lo)) - 1u, upto = hi <= 0 ? 0u : hi >= 4 ? ~0u : (1u << (8 * hi)) - 1u;
+        keep[i] = upto & ~below;
+        pad[i] = fill & ~keep[i];
+    }
+    // kernel rows as words of uint8 taps, zero past the last one
+    const uint32_t w_flip = p.w_signed ? 0x80808080u : 0u;
+    const uint8_t *w = p.w + (size_t)oc * (K * K);
+    uint32_t wk[K][F];
+#pragma unroll
+    for (int ky = 0; ky < K; ++ky)
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            const int taps = K - 4 * f < 4 ? K - 4 * f : 4;
+            const uint32_t v = *reinterpret_cast<const u32_any_alignment *>(w + ky * K + f * 4);  // (the plan's copy ends in four bytes of slack)
+            wk[ky][f] = (v ^ w_flip) & (taps == 4 ? ~0u : (1u << (8 * taps)) - 1u);
+        }
+    const int bias = p.bias_folded[oc];
+    ChannelQuad quad{};
+    if constexpr (PC) {
+        const int m = p.rq.pc_multiplier[oc], sh = p.rq.pc_shift[oc];
+        quad.m = make_int4(m, m, m, m);
+        quad.s = make_int4(sh, sh, sh, sh);
+    }
+    int acc[R][4], sum[R][4];
+#pragma unroll
+    for (int o = 0; o < R; ++o)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            acc[o][j] = bias;
+            sum[o][j] = 0;
+        }
+    const int row0 = (int)(lead + in_plane * (uint32_t)(p.h * p.w_)) + ix0;
+#pragma unroll
+    for (int row = 0; row < ROWS; ++row) {
+        const int iy = iy0 + row;
+        const bool exists = (unsigned)iy < (unsigned)p.h;
+        const int off = exists ? row0 + iy * p.w_ : 0, at = off < 0 ? 0 : off;  // (below zero: the tensor's first row, left of it)
+        uint32_t d[ND + 1], x[ND];
+        const int from = at & ~3;
+        if constexpr (ND == 2) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b96(in, from, 0, 0);
+            d[0] = v[0], d[1] = v[1], d[2] = v[2];
+        } else {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(in, from, 0, 0);
+            d[0] = v[0], d[1] = v[1], d[2] = v[2], d[3] = v[3];
+            if constexpr (ND == 4) d[4] = __builtin_amdgcn_raw_buffer_load_b32(in, from + 16, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i) x[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], (uint32_t)at);
+        if (off < 0) {
+#pragma unroll
+            for (int i = ND - 1; i >= 0; --i) x[i] = __builtin_amdgcn_alignbyte(x[i], i ? x[i - 1] : 0u, (uint32_t)(4 + off));
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i) x[i] = exists ? ((x[i] ^ p.io_flip) & keep[i]) | pad[i] : fill;
+        uint32_t win[4][F];
+        int row_sum[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            row_sum[j] = 0;
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                const int b = j * S + f * 4;
+                win[j][f] = (b & 3) == 0 ? x[b >> 2] : __builtin_amdgcn_alignbyte((b >> 2) + 1 < ND ? x[(b >> 2) + 1 < ND ? (b >> 2) + 1 : 0] : 0u, x[b >> 2], b & 3);
+                const int taps = K - 4 * f < 4 ? K - 4 * f : 4;
+                row_sum[j] = udot4(win[j][f], 0x01010101u >> (8 * (4 - taps)), row_sum[j]);
+            }
+        }
+#pragma unroll
+        for (int ky = 0; ky < K; ++ky) {
+            if (row < ky || (row - ky) % S != 0 || (row - ky) / S >= R) continue;
+            const int o = (row - ky) / S;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                for (int f = 0; f < F; ++f) acc[o][j] = udot4(win[j][f], wk[ky][f], acc[o][j]);
+                sum[o][j] += row_sum[j];
+            }
+        }
+    }
+    const int zw = p.zp_w + (p.w_signed ? 128 : 0);
+    const RequantDev rq = p.rq;
+    const uint32_t out_plane = plane * (uint32_t)(p.ho * p.wo);
+#pragma unroll
+    for (int o = 0; o < R; ++o) {
+        if (oy0 + o >= p.ho) break;
+        int a[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = acc[o][j] - __mul24(zw, sum[o][j]);  // (49 bytes times a zero point of at most 383)
+        const uint32_t v = (PC && rq.fast ? requant4_channel_fast(a[0], a[1], a[2], a[3], rq, quad) : requant4<PC>(a[0], a[1], a[2], a[3], rq, quad)) ^ p.io_flip;
+        uint8_t *dst = p.out + (out_plane + (uint32_t)(oy0 + o) * (uint32_t)p.wo + (uint32_t)ox0);
+        if (ox0 + 4 <= p.wo) {
+            *reinterpret_cast<u32_any_alignment *>(dst) = v;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (ox0 + j < p.wo) dst[j] = (uint8_t)(v >> (8 * j));
+        }
+    }
+}
+
 // One output element per thread; any depth multiplier, dilation, channel count.
 // NHWC = true: channel fastest.  NHWC = false: planar NCHW, x fastest.
 template <bool NHWC>
@@ -609,9 +739,43 @@ int launch_dwconv_nhwc(const DwProblem &caller_p, hipStream_t stream) {
     return EH_OK;
 }
 
+// (what a plan that keeps a caller's planar tensors planar has to be)
+bool dw_planar_applies(const DwProblem &p) {
+    return p.kh == p.kw && (p.kh == 3 || p.kh == 5 || p.kh == 7) && p.dil_h == 1 && p.dil_w == 1 && p.stride_h == p.stride_w &&
+           (p.stride_h == 1 || p.stride_h == 2) && p.pad_l >= 0 && p.pad_l <= 3 && p.pad_t >= 0 && (size_t)p.n * p.c * p.h * p.w_ < (1ull << 31) - 64 &&
+           (size_t)p.n * p.cout * p.ho * p.wo < (1ull << 31) - 64;
+}
+
+static int launch_dw_planar(const DwProblem &p, hipStream_t stream) {
+    const int quads = (p.wo + 3) / 4;
+    const long threads = (long)p.n * p.cout * quads;
+    // Four rows to a thread share their input rows' loads and shifts; a launch that they would not fill has one.  One row and four, us, by
+    // the threads of four: 6272 5x5 stride 2 4.3 and 5.6; 8320 7x7 3.6 and 4.9; 26912 3x3 4.0 and 4.0; 61440 7x7 stride 2 7.4 and 6.6;
+    // 122880 5x5 6.9 and 6.1; 225792 3x3 6.8 and 5.6.
+    const bool four = threads * ((p.ho + 3) / 4) >= 32768;
+    auto launch = [&](auto k_c, auto s_c, auto r_c, auto pc_c) {
+        constexpr int R = decltype(r_c)::value;
+        const int bands = (p.ho + R - 1) / R;
+        const uint32_t total = (uint32_t)(threads * bands);
+        hipLaunchKernelGGL((dw_planar_kernel<decltype(k_c)::value, decltype(s_c)::value, R, decltype(pc_c)::value>), dim3(((total + 255) / 256 + 7) / 8 * 8), dim3(256), 0,
+                           stream, p, total, quads, bands, make_fastdiv((uint32_t)quads), make_fastdiv((uint32_t)bands), make_fastdiv((uint32_t)p.cout),
+                           make_fastdiv((uint32_t)p.dm));
+    };
+    using std::integral_constant;
+    auto with_rows = [&](auto k_c, auto s_c) {
+        auto with_pairs = [&](auto r_c) { p.rq.pc_multiplier ? launch(k_c, s_c, r_c, std::true_type{}) : launch(k_c, s_c, r_c, std::false_type{}); };
+        four ? with_pairs(integral_constant<int, 4>{}) : with_pairs(integral_constant<int, 1>{});
+    };
+    auto with_stride = [&](auto k_c) { p.stride_h == 1 ? with_rows(k_c, integral_constant<int, 1>{}) : with_rows(k_c, integral_constant<int, 2>{}); };
+    p.kh == 3 ? with_stride(integral_constant<int, 3>{}) : p.kh == 5 ? with_stride(integral_constant<int, 5>{}) : with_stride(integral_constant<int, 7>{});
+    EH_HIP(hipGetLastError());
+    return EH_OK;
+}
+
 int launch_dwconv_nchw(const DwProblem &p, hipStream_t stream) {
     const long outs = (long)p.n * p.ho * p.wo * p.cout;
     if (outs <= 0) return EH_OK;
+    if (dw_planar_applies(p)) return launch_dw_planar(p, stream);
     const long blocks = (outs + 255) / 256;
     EH_REQUIRE(blocks < (1l << 31), "depthwise: grid too large");
     hipLaunchKernelGGL((dw_scalar_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, stream, p, outs);

@@ -679,6 +679,7 @@ int launch_dw_pack_trip(const uint8_t *w, const int32_t *bias, int32_t *w_trip, 
 int launch_dw_pack_fold(const uint8_t *w, const int32_t *bias, int32_t *w_fold, int32_t *bias_fold, int32_t cout, int32_t zp_in,
                         int32_t zp_w_u8, int32_t w_signed, hipStream_t stream);
 int launch_dwconv_nhwc(const DwProblem &p, hipStream_t stream);
+bool dw_planar_applies(const DwProblem &p);  // by its geometry: launch_dwconv_nchw has a kernel for it that is worth no transposition
 int launch_dwconv_nchw(const DwProblem &p, hipStream_t stream);
 // 5x5 and 7x7 windows on the matrix cores (eh_dwconv_mfma.hip)
 size_t dw_mfma_weight_bytes(int32_t cout, int32_t k);
