@@ -262,9 +262,15 @@ __device__ __forceinline__ void column_words(uint32_t r0, uint32_t r1, uint32_t 
 // TW + 2 D columns.  0: any dilation, read from the problem; no column is shared then and the tile reads three groups of
 // TW adjacent columns, one per kernel column (what remains shared is the index arithmetic, the weights and the
 // border tests).
+// GATHER: a pixel of the input holds p.gather_c channels, any number from four on, each read by as many output channels as the
+// multiplier says, and one of the output p.out_c; p.c and p.cout count those of the padded weights.  A thread loads the word of a pixel that holds its quad's
+// input channels from where it lies and brings the channels to their places with one permute.  (Before, by a copy of the input with
+// each channel as often as it is read and whole quads, and a copy of the result without the padding, us: 103
+// channels at 22x22, 3 images 10.2 -> 3.9; 143 at 56x56, 32 images 31.6 -> 15.7; 119 at 40x40 stride 2, int8 with a pair per channel, 58
+// images 19.1 -> 7.1; 112 x 2 at 86x86 stride 2, 60 images 96 -> 27; 50 x 2 at 28x28, 4 images 7.7 -> 4.0.)
 __device__ __forceinline__ int udot4(uint32_t a, uint32_t b, int acc) { return (int)__builtin_amdgcn_udot4(a, b, (uint32_t)acc, false); }
 
-template <int S, bool FLIP, int TW = 4, bool PC = false, bool FOLD = false, int D = 1>
+template <int S, bool FLIP, int TW = 4, bool PC = false, bool FOLD = false, int D = 1, bool GATHER = false>
 __global__ __launch_bounds__(256) void dw3x3_nhwc_tile4_dot4_kernel(const DwProblem p, const uint32_t total, const int tiles_x,
                                                                     const FastDiv div_cq, const FastDiv div_tiles, const FastDiv div_ho) {
     static_assert(D == 1 || S == 1, "dilated tiles are stride 1");
@@ -288,22 +294,40 @@ __global__ __launch_bounds__(256) void dw3x3_nhwc_tile4_dot4_kernel(const DwProb
     const uint32_t fill = ((uint32_t)p.zp_in * 0x01010101u) ^ (FOLD ? 0u : 0x80808080u);
     // uint8 tensors hold a, int8 tensors a - 128: the signed form wants a - 128, the unsigned one a
     constexpr bool flip_loaded = FOLD ? FLIP : !FLIP;
-    const uint32_t base = img * (uint32_t)(p.h * p.w_ * p.c) + cq * 4u;
+    const int in_c = GATHER ? p.gather_c : p.c, out_c = GATHER ? p.out_c : p.cout;
+    uint32_t first = cq * 4u, select = 0;
+    if constexpr (GATHER) {
+        // the word of a pixel that holds the quad's input channels, the last one that lies in the pixel whole, and their places in it
+        const uint32_t channel = fastdiv(first, p.gather_div);
+        const uint32_t start = channel < (uint32_t)in_c - 4u ? channel : (uint32_t)in_c - 4u;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t oc = first + j < (uint32_t)out_c ? first + j : (uint32_t)out_c - 1u;
+            select |= (fastdiv(oc, p.gather_div) - start) << (8 * j);
+        }
+        first = start;
+    }
+    const uint32_t base = img * (uint32_t)(p.h * p.w_ * in_c) + first;
+    using Word = std::conditional_t<GATHER, const u32_any_alignment, const uint32_t>;
+    auto load = [&](const uint8_t *from) {
+        const uint32_t v = *reinterpret_cast<Word *>(from);
+        return GATHER ? __builtin_amdgcn_perm(0u, v, select) : v;
+    };
 
     // (row pitch and pixel offsets stay below 2^24, which the launcher checks: 24-bit multiplies run at full rate,
     // 32-bit ones at a quarter of it)
-    const int row_pitch = p.w_ * p.c;
+    const int row_pitch = p.w_ * in_c;
     uint32_t in[3][IW];
     const bool inside = iy0 >= 0 && iy0 + 2 * dil < p.h && ix0 >= 0 && ix0 + x_offset(IW - 1) < p.w_;
     if (__builtin_amdgcn_ballot_w64(!inside) == 0) {
         // every window of the wave lies inside the image (most waves): no clamps, no selects, offsets that differ
         // between the loads by wave-uniform amounts; a wave with one window on the border takes the general path whole
-        const uint8_t *src = p.in + (base + (uint32_t)__mul24(iy0, row_pitch) + (uint32_t)__mul24(ix0, p.c));
+        const uint8_t *src = p.in + (base + (uint32_t)__mul24(iy0, row_pitch) + (uint32_t)__mul24(ix0, in_c));
 #pragma unroll
         for (int ky = 0; ky < 3; ++ky)
 #pragma unroll
             for (int x = 0; x < IW; ++x) {
-                const uint32_t v = *reinterpret_cast<const uint32_t *>(src + (uint32_t)(ky * dil * row_pitch + x_offset(x) * p.c));
+                const uint32_t v = load(src + (uint32_t)(ky * dil * row_pitch + x_offset(x) * in_c));
                 in[ky][x] = flip_loaded ? v ^ 0x80808080u : v;
             }
     } else {
@@ -314,7 +338,7 @@ __global__ __launch_bounds__(256) void dw3x3_nhwc_tile4_dot4_kernel(const DwProb
             const int ix = ix0 + x_offset(x);
             col_ok[x] = (unsigned)ix < (unsigned)p.w_;
             const int ixc = ix < 0 ? 0 : (ix >= p.w_ ? p.w_ - 1 : ix);
-            col_off[x] = base + (uint32_t)__mul24(ixc, p.c);
+            col_off[x] = base + (uint32_t)__mul24(ixc, in_c);
         }
 #pragma unroll
         for (int ky = 0; ky < 3; ++ky) {
@@ -324,7 +348,7 @@ __global__ __launch_bounds__(256) void dw3x3_nhwc_tile4_dot4_kernel(const DwProb
             const uint32_t row_off = (uint32_t)__mul24(iyc, row_pitch);
 #pragma unroll
             for (int x = 0; x < IW; ++x) {
-                const uint32_t v = *reinterpret_cast<const uint32_t *>(p.in + (row_off + col_off[x]));
+                const uint32_t v = load(p.in + (row_off + col_off[x]));
                 in[ky][x] = row_ok && col_ok[x] ? (flip_loaded ? v ^ 0x80808080u : v) : fill;
             }
         }
@@ -343,7 +367,7 @@ __global__ __launch_bounds__(256) void dw3x3_nhwc_tile4_dot4_kernel(const DwProb
             for (int c = 0; c < 4; ++c) cs[x][c] = udot4(col[x][c], 0x00010101u, 0);
         }
     }
-    uint8_t *dst = p.out + (((img * (uint32_t)p.ho + (uint32_t)oy) * (uint32_t)p.wo + (uint32_t)ox0) * (uint32_t)p.cout + cq * 4u);
+    uint8_t *dst = p.out + (((img * (uint32_t)p.ho + (uint32_t)oy) * (uint32_t)p.wo + (uint32_t)ox0) * (uint32_t)out_c + cq * 4u);
     const RequantDev rq = p.rq;
     const ChannelQuad quad = load_channel_quad<PC>(rq, cq * 4u);
 #pragma unroll
@@ -372,7 +396,21 @@ __global__ __launch_bounds__(256) void dw3x3_nhwc_tile4_dot4_kernel(const DwProb
         }
         uint32_t o = PC ? requant4_channel_fast(acc0, acc1, acc2, acc3, rq, quad) : requant4<false>(acc0, acc1, acc2, acc3, rq, quad);
         if (FLIP) o ^= 0x80808080u;
-        if (ox0 + j < p.wo) *reinterpret_cast<uint32_t *>(dst + (uint32_t)j * (uint32_t)p.cout) = o;
+        if (ox0 + j < p.wo) {
+            uint8_t *const to = dst + (uint32_t)j * (uint32_t)out_c;
+            if constexpr (GATHER) {
+                const int left = out_c - (int)cq * 4;
+                if (left >= 4) {
+                    *reinterpret_cast<u32_any_alignment *>(to) = o;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        if (i < left) to[i] = (uint8_t)(o >> (8 * i));
+                }
+            } else {
+                *reinterpret_cast<uint32_t *>(to) = o;
+            }
+        }
     }
 }
 
@@ -735,6 +773,35 @@ int launch_dwconv_nhwc(const DwProblem &caller_p, hipStream_t stream) {
         EH_REQUIRE(blocks < (1l << 31), "depthwise: grid too large");
         hipLaunchKernelGGL((dw_scalar_kernel<true>), dim3((unsigned)blocks), dim3(256), 0, stream, p, outs);
     }
+    EH_HIP(hipGetLastError());
+    return EH_OK;
+}
+
+// The problem of a plan whose kernels' channels are not its tensors': the dot product form of 3x3 layers without dilation.
+bool dw_gather_applies(const DwProblem &p) {
+    return p.kh == 3 && p.kw == 3 && p.dil_h == 1 && p.dil_w == 1 && p.stride_h == p.stride_w && (p.stride_h == 1 || p.stride_h == 2) && (p.w_trip || p.w_fold) &&
+           (p.rq.pc_multiplier == nullptr || p.rq.fast) && (long)p.w_ * p.c < (1l << 23) && p.h < (1 << 23) && p.gather_c >= 4 &&
+           (size_t)p.n * p.h * p.w_ * p.c < (1ull << 31) && (size_t)p.n * p.ho * p.wo * p.cout < (1ull << 31);
+}
+
+int launch_dw_gather(const DwProblem &caller_p, hipStream_t stream) {
+    DwProblem p = caller_p;
+    const bool fold = p.w_trip == nullptr, pc = p.rq.pc_multiplier != nullptr, flip = p.io_flip != 0;
+    if (fold) p.zp_w += p.w_signed ? 128 : 0;
+    const int tiles_x = (p.wo + 3) / 4;
+    const long total = (long)p.n * p.ho * tiles_x * (p.c >> 2);
+    if (total <= 0) return EH_OK;
+    auto pick = [&](auto stride_c) {
+        constexpr int S = decltype(stride_c)::value;
+        if (fold)
+            return pc ? (flip ? dw3x3_nhwc_tile4_dot4_kernel<S, true, 4, true, true, 1, true> : dw3x3_nhwc_tile4_dot4_kernel<S, false, 4, true, true, 1, true>)
+                      : (flip ? dw3x3_nhwc_tile4_dot4_kernel<S, true, 4, false, true, 1, true> : dw3x3_nhwc_tile4_dot4_kernel<S, false, 4, false, true, 1, true>);
+        return pc ? (flip ? dw3x3_nhwc_tile4_dot4_kernel<S, true, 4, true, false, 1, true> : dw3x3_nhwc_tile4_dot4_kernel<S, false, 4, true, false, 1, true>)
+                  : (flip ? dw3x3_nhwc_tile4_dot4_kernel<S, true, 4, false, false, 1, true> : dw3x3_nhwc_tile4_dot4_kernel<S, false, 4, false, false, 1, true>);
+    };
+    auto kernel = p.stride_h == 1 ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, 2>{});
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(((total + 255) / 256 + 7) / 8 * 8)), dim3(256), 0, stream, p, (uint32_t)total, tiles_x,
+                       make_fastdiv((uint32_t)(p.c >> 2)), make_fastdiv((uint32_t)tiles_x), make_fastdiv((uint32_t)p.ho));
     EH_HIP(hipGetLastError());
     return EH_OK;
 }

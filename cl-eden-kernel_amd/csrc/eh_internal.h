@@ -671,6 +671,10 @@ struct DwProblem {
     int32_t w_signed;            // weight bytes are int8
     uint32_t io_flip;            // 0x80808080 when input and output hold int8 values (computed as value + 128), else 0
     RequantDev rq;               // rq.pc_multiplier / rq.pc_shift: [cout + 4] when set
+    // launch_dw_gather: channels per pixel of the tensors, where c and cout are those of padded weights with multiplier 1, and
+    // division by the depth multiplier
+    int32_t gather_c, out_c;
+    FastDiv gather_div;
 };
 int launch_dw_pack(const uint8_t *w, const int32_t *bias, int32_t *w_pair, int32_t *bias_folded, int32_t cout,
                    int32_t taps, int32_t zp_in, int32_t zp_w, int32_t w_signed, hipStream_t stream);
@@ -679,6 +683,8 @@ int launch_dw_pack_trip(const uint8_t *w, const int32_t *bias, int32_t *w_trip, 
 int launch_dw_pack_fold(const uint8_t *w, const int32_t *bias, int32_t *w_fold, int32_t *bias_fold, int32_t cout, int32_t zp_in,
                         int32_t zp_w_u8, int32_t w_signed, hipStream_t stream);
 int launch_dwconv_nhwc(const DwProblem &p, hipStream_t stream);
+bool dw_gather_applies(const DwProblem &p);
+int launch_dw_gather(const DwProblem &p, hipStream_t stream);
 bool dw_planar_applies(const DwProblem &p);  // by its geometry: launch_dwconv_nchw has a kernel for it that is worth no transposition
 int launch_dwconv_nchw(const DwProblem &p, hipStream_t stream);
 // 5x5 and 7x7 windows on the matrix cores (eh_dwconv_mfma.hip)
