@@ -472,7 +472,7 @@ bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, in
         int size, pieces;
     } across[MOST], down[3][MOST];
     int n_across = 0, n_down[3] = {0, 0, 0};
-    auto cut = [&](int extent, int fixed, int unit, Cut *to, int *count) {
+    auto cut = [&](int extent, int fixed, int unit, int narrowest, Cut *to, int *count) {
         if (fixed > 0) {
             if (fixed % unit == 0) to[(*count)++] = Cut{fixed, shares(extent, fixed)};
             return;
@@ -480,12 +480,13 @@ bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, in
         for (int pieces = 1; pieces <= extent && *count < MOST; ++pieces) {
             const int size = shares(extent, pieces * unit) * unit;
             if (size > 64 || (*count > 0 && to[*count - 1].size == size)) continue;
+            if (size < narrowest && *count > 0) break;
             to[(*count)++] = Cut{size, shares(extent, size)};
             if (size == unit) break;
         }
     };
-    cut(dw.wo, cols_per_tile, 1, across, &n_across);
-    for (int lg = 4; lg >= 2; --lg) cut(dw.ho, rows_per_tile, 16 >> lg, down[4 - lg], &n_down[4 - lg]);
+    cut(dw.wo, cols_per_tile, 1, 4, across, &n_across);  // (of four columns or more: a walk takes no fewer at a time)
+    for (int lg = 4; lg >= 2; --lg) cut(dw.ho, rows_per_tile, 16 >> lg, 1, down[4 - lg], &n_down[4 - lg]);
     double best = -1;
     for (const size_t lds_max : {(size_t)64 * 1024, kBlockLdsMax}) {  // (above 64 KiB a launch sets an attribute of the kernel first)
         for (int cn = 1; cn <= nb_all; ++cn) {
@@ -504,7 +505,7 @@ bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, in
                         const size_t lds = lds_fixed + (size_t)pixels * lds_pixel + 15;
                         if (lds > lds_max) continue;
                         const double per_cu = groups_of_tiles * a.pieces;
-                        if (best >= 0 && pixels < 64 && per_cu > held) break;  // (small tiles only where larger ones would leave CUs idle)
+                        if (best >= 0 && pixels < 80 && per_cu > held) break;  // (small tiles only where larger ones would leave CUs idle)
                         const double wave = 10 + 40.0 * cn + 40.0 * ((pixels * ks * 4 + 255) >> 8) + ((((pixels + 31) >> 5) * cn + 3) >> 2) * (67.0 * epilogue + 5.5 * ks) +
                                             ((chunks * ((a.size + (1 << lg) - 1) >> lg) + 3) >> 2) * walk;
                         const int fit = (int)((160 * 1024) / lds), most = fit < held ? fit : held, full = (int)(per_cu / most);
