@@ -424,15 +424,16 @@ bool gemm_few_tiles_instead(const GemmProblem &p) {
 }
 
 // Against the copy and the kernel that reads it, us (start of the line: tiles, bytes of a tap's reduction with its padding):
-//   ragged   7, 176 of 128 x 175 x 88 7.7 -> 3.8; 352, 288 of 3x3 24 -> 64 at 6 x 28x28 7.6 -> 4.5; 875, 96 of 4000 x 90 x 200 7.7 -> 6.8; 774, 288
-//            of 3x3 24 -> 168 at 11 x 17x22 7.8 -> 7.0; 752, 512 of 6000 x 500 x 128 9.3 either way; 1252, 288 7.9 -> 8.7; 1120, 1008 9.1 -> 9.9
+//   ragged   7, 176 of 128 x 175 x 88 7.7 -> 3.8; 352, 288 of 3x3 24 -> 64 at 6 x 28x28 7.6 -> 4.5; in a replayed graph, where a second launch is
+//            cheaper, 512, 288 of 3x3 21 -> 21 at 4 x 64x64 6.6 -> 4.9; 640 of it 6.6 -> 6.7; 1024 6.7 -> 7.5; 1024, 144 of 3x3 15 -> 21 6.3 -> 7.3;
+//            1024, 64 of 1x1 45 -> 21 6.0 -> 6.6, 160 9.5 -> 6.8, 256 14.1 -> 6.8; 768, 400 5.8 either way
 //   planar   287, 288 of 3x3 21 -> 21 at 3 x 65x47 7.8 -> 5.2; 150, 864 of 3x3 96 -> 96 at 4 x 20x20 7.7 -> 7.0; 100, 1152 7.5 -> 7.2; 784, 256 of 1x1
 //            256 -> 128 at 32 x 14x14 9.3 -> 6.7; 588, 288 7.1 -> 7.8; 294, 800 8.4 -> 9.1; 800, 160 7.8 -> 8.1
 // (planar 1x1 layers of one product keep to two rounds: 980 tiles 6.5 .. 7.6 either way)
 bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t problems, int32_t form) {
     const long tiles = m > 0 ? few_tiles_count(m, n) * problems : 0;
     if (tiles <= 0 || k > 8192) return false;
-    if (form == INPUT_RAGGED) return tiles <= 512 || (tiles <= 1024 && k <= 448);
+    if (form == INPUT_RAGGED) return tiles <= 512 || (tiles <= 1024 && k > 144 && k <= 256);
     const long rounds = (tiles + 255) / 256;
     return rounds <= 2 ? k * rounds <= 1152 : tiles < 800 && k > 32 && k <= 256;
 }
