@@ -117,23 +117,33 @@ __global__ __launch_bounds__(256) void pwdw_block_kernel(const GemmProblem pw, c
         return (unsigned)iy < (unsigned)pw.h && (unsigned)ix < (unsigned)pw.w;
     };
     {
-        // The input pixels first, then the weights as direct-to-LDS copies, all on their way at once beside the bias.  (The pieces four
-        // at a time behind the weights' copies, from clamped addresses without a branch, cost a small launch more instructions than they
-        // save trips: 40 -> 240 at 20x20 stride 2, six images, 5.13 us as here, 5.44 like that; 48 -> 288 at 33x33, four images 5.57
-        // and 5.81; 64 -> 384 at 14x14, eight images 5.46 and 5.69.)
+        // The input pixels first, then the weights as direct-to-LDS copies, all on their way at once beside the bias.  A thread of a tile
+        // that walks has two pieces on their way at a time, from clamped addresses without a branch: 24 -> 144 at 56x56 stride 2, 32
+        // images, four pieces to a thread, 10.95 us one at a time and 10.8 so, on cold tensors 13.6 and 12.8.  (Four at a time cost a small
+        // tile more instructions than they save trips: 40 -> 240 at 20x20 stride 2, six images, 5.13 us one at a time, 5.44 like that; 48
+        // -> 288 at 33x33, four images 5.57 and 5.81; 64 -> 384 at 14x14, eight images 5.46 and 5.69.)
         const int ppp = ksteps * 4;  // 8-byte pieces per pixel
         const int pieces = g.pixels * ppp;
-        for (int i = tid; i < pieces; i += 256) {
-            const int q = KS ? i / (KS * 4) : (int)fastdiv((uint32_t)i, g.div_ppp), piece = i - q * ppp;
-            int iy, ix;
-            uint2 v = make_uint2(0u, 0u);  // bytes past the reduction length, and whole pixels outside the image: operand 0
-            if (inside_image(q, iy, ix) && piece * 8 < pw.k) {
-                v = *reinterpret_cast<const uint2 *>(pw.a + (((img * (uint32_t)pw.h + (uint32_t)iy) * (uint32_t)pw.w + (uint32_t)ix) * (uint32_t)pw.cin +
-                                                               (uint32_t)pw.a_offset + (uint32_t)piece * 8u));
-                v.x ^= pw.a_xor;
-                v.y ^= pw.a_xor;
+        constexpr int BATCH = WALK ? 2 : 1;
+        for (int i0 = tid; i0 < pieces; i0 += 256 * BATCH) {
+            uint2 v[BATCH];
+            uint32_t to[BATCH];
+            bool exists[BATCH];
+#pragma unroll
+            for (int b = 0; b < BATCH; ++b) {
+                const int i = i0 + b * 256, q = KS ? i / (KS * 4) : (int)fastdiv((uint32_t)i, g.div_ppp), piece = i - q * ppp;
+                int iy, ix;
+                exists[b] = inside_image(q, iy, ix) && piece * 8 < pw.k;
+                to[b] = (uint32_t)(q * g.a_pitch + piece * 8);
+                v[b] = make_uint2(0u, 0u);
+                const uint32_t from = ((img * (uint32_t)pw.h + (uint32_t)iy) * (uint32_t)pw.w + (uint32_t)ix) * (uint32_t)pw.cin + (uint32_t)pw.a_offset + (uint32_t)piece * 8u;
+                if (WALK || exists[b]) v[b] = *reinterpret_cast<const uint2 *>(pw.a + (exists[b] ? from : 0u));
             }
-            *reinterpret_cast<uint2 *>(a_s + q * g.a_pitch + piece * 8) = v;
+#pragma unroll
+            for (int b = 0; b < BATCH; ++b) {  // bytes past the reduction length, and whole pixels outside the image: operand 0
+                const uint2 w = exists[b] ? make_uint2(v[b].x ^ pw.a_xor, v[b].y ^ pw.a_xor) : make_uint2(0u, 0u);
+                if (b == 0 || i0 + b * 256 < pieces) *reinterpret_cast<uint2 *>(a_s + to[b]) = w;
+            }
         }
         dma_linear<4>(pw.b + (size_t)nb_first * ksteps * 1024, lds_offset(lds_raw), nb_here * ksteps, w_uniform, lane);
         for (int i = tid; i < nb_here * 32; i += 256) bias_s[i] = pw.bias[c_first + i];
