@@ -477,7 +477,7 @@ bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, in
     auto shares = [](int a, int b) { return (a + b - 1) / b; };
     // tiles across the image and down it, as equal as columns and whole strips allow, the largest first.  (A launch finds its tile the
     // first time it runs: what a candidate needs is worked out ahead of the loops, and shapes that cannot win are not looked at.)
-    constexpr int MOST = 24;
+    constexpr int MOST = 32;  // rows and columns
     struct Cut {
         int size, pieces;
     } across[MOST], down[3][MOST];
@@ -487,12 +487,11 @@ bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, in
             if (fixed % unit == 0) to[(*count)++] = Cut{fixed, shares(extent, fixed)};
             return;
         }
-        for (int pieces = 1; pieces <= extent && *count < MOST; ++pieces) {
-            const int size = shares(extent, pieces * unit) * unit;
-            if (size > 64 || (*count > 0 && to[*count - 1].size == size)) continue;
-            if (size < narrowest && *count > 0) break;
-            to[(*count)++] = Cut{size, shares(extent, size)};
-            if (size == unit) break;
+        const int whole = shares(extent, unit) * unit;
+        for (int size = whole < MOST ? whole : MOST; size >= unit; size -= unit) {
+            const int even = shares(extent, shares(extent, size) * unit) * unit;
+            if (*count > 0 && (even == to[*count - 1].size || even < narrowest)) continue;
+            to[(*count)++] = Cut{even, shares(extent, even)};
         }
     };
     cut(dw.wo, cols_per_tile, 1, 4, across, &n_across);  // (of four columns or more: a walk takes no fewer at a time)

@@ -15,6 +15,8 @@ SEED = 0x3A1C
 CASES = [
     # n, h, w, cin, c, stride, rows, cols, depthwise zp_w, depthwise output scale
     (24, 28, 28, 24, 144, 1, 0, 0, 128, 0.4),    # the tile chosen here; differences fit int8
+    (1, 230, 205, 8, 64, 1, 0, 0, 100, 0.4),     # ... of an image of many tiles either way
+    (1, 300, 290, 8, 128, 2, 0, 0, 100, 0.4),
     (2, 23, 37, 24, 144, 1, 8, 16, 0, 0.4),      # whole column groups; differences up to 255
     (1, 23, 37, 40, 240, 2, 5, 13, 255, 0.4),    # an odd number of rows: 16 columns only; differences down to -255
     (2, 17, 19, 16, 96, 1, 6, 9, 100, 0.4),      # nine columns
