@@ -21,19 +21,19 @@ CALL_LIB = os.path.join(HERE, "_call" + sysconfig.get_config_var("EXT_SUFFIX")) 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+             # Every joining block of a conditional restores the execution mask itself.  Left to itself the compiler drops the restore
+             # where an enclosing conditional ends right behind it, and then, short of registers, puts a spilled value's reload or a
+             # register copy between the two, where the lanes that need it are off: the per-channel epilogue of a 256 x 256 tile wrote to
+             # addresses made of stale registers.  tests/test_exec_restore.py reads the built code for such instructions, but sees
+             # a joining block only where a branch leads to it, so no file goes without the restores.
+             "-mllvm", "-amdgpu-remove-redundant-endcf=0",
              "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
 
 
 # MFMA results straight into ordinary registers for the kernels whose epilogue is the bottleneck (no AGPR -> VGPR
 # copy per output); the big-tile GEMM keeps its accumulators in the AGPR half of the register file
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-# Every joining block of a conditional restores the execution mask itself.  Left to itself the compiler drops the restore where
-# an enclosing conditional ends right behind it, and then, out of registers, puts a spilled value's reload between the two,
-# where the lanes that need it are off: the per-channel epilogue of a 256 x 256 tile wrote to addresses made of stale registers.
-# tests/test_exec_restore.py reads all built code for such reloads; the other files have none and keep the shorter code (3x3
-# patch kernel 9.48 us without the restores, 9.54 with them).
-MASK_RESTORES = ["-mllvm", "-amdgpu-remove-redundant-endcf=0"]
-PER_FILE_FLAGS = {"eh_gemm_dma.hip": MASK_RESTORES, "eh_gemm_thin.hip": VGPR_FORM, "eh_block.hip": VGPR_FORM, "eh_conv_c3.hip": VGPR_FORM, "eh_conv_rows.hip": VGPR_FORM, "eh_dwconv_mfma.hip": VGPR_FORM}
+PER_FILE_FLAGS = {"eh_gemm_thin.hip": VGPR_FORM, "eh_block.hip": VGPR_FORM, "eh_conv_c3.hip": VGPR_FORM, "eh_conv_rows.hip": VGPR_FORM, "eh_dwconv_mfma.hip": VGPR_FORM}
 
 RESOURCES = os.path.join(OBJ, "kernel_resources.txt")
 
