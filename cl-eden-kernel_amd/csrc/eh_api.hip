@@ -395,6 +395,12 @@ static int upload_padded_pairs(int32_t *d_mult, int32_t *d_shift, const int32_t 
     return EH_OK;
 }
 
+// whether two pieces of memory share no byte
+static bool lie_apart(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+    const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+    return a0 + a_bytes <= b0 || b0 + b_bytes <= a0;
+}
+
 struct GemmOp {
     std::vector<GemmPart> parts;
     int32_t *bias_copy = nullptr;  // the operator's own copy of the int32 bias
@@ -574,7 +580,8 @@ struct GemmOp {
     static constexpr int kInlineParts = 8;  // a run over at most this many parts allocates no host memory
 
     // Which form of the caller's own tensor the launches of a run can read, where the kernels otherwise get a copy with padded
-    // channels or with the channels last (gemm_few_tiles_direct has the rule).
+    // channels or with the channels last (gemm_few_tiles_direct has the rule).  A run whose output lies on its input reads the copy,
+    // which the plan's staging is kept for: workgroups store while others still read.
     int32_t direct_form() const {
         if (parts.empty() || (pad_cg_to == 0 && layout != EH_NCHW)) return INPUT_CHUNKS;
         const int32_t form = layout == EH_NCHW ? INPUT_PLANAR : INPUT_RAGGED;
@@ -647,7 +654,8 @@ struct GemmOp {
         uint8_t *const st_pad = staging ? staging + (layout == EH_NCHW ? stage_in_bytes() + stage_out_bytes() : 0) : stage_pad;
         const bool planar_out = stores_planar();
         bool padded = false;
-        const int32_t form = direct_form();
+        const bool apart = lie_apart(input, (size_t)in_n * in_c * in_hw, output, (size_t)in_n * cout * out_hw);
+        const int32_t form = apart ? direct_form() : (int32_t)INPUT_CHUNKS;
         if (layout == EH_NCHW && form != INPUT_CHUNKS) {
             // (planar_out: see direct_form)
         } else if (layout == EH_NCHW) {
