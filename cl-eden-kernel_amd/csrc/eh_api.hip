@@ -2064,7 +2064,10 @@ int eh_dwconv2d_u8_run(eh_dwconv_plan *plan, const void *input, void *output, co
         direct.gather_c = plan->rep_c;
         direct.out_c = plan->cout_caller;
         direct.gather_div = make_fastdiv((uint32_t)plan->rep_dm);
-        if (dw_gather_applies(direct)) return launch_dw_gather(direct, s);
+        // (an output on its input: the copy is read, as workgroups store while others still read)
+        if (dw_gather_applies(direct) &&
+            lie_apart(input, (size_t)d.n * d.h * d.w * plan->rep_c, output, (size_t)d.n * plan->ho * plan->wo * plan->cout_caller))
+            return launch_dw_gather(direct, s);
         // (multiplier 1: only the rows' tails are new, and the copy reads whole dwords)
         rc = plan->rep_dm == 1 ? launch_pad_channels(static_cast<const uint8_t *>(input), plan->stage_in, (int64_t)d.n * d.h * d.w, 1, plan->rep_c, plan->cout, 0, s)
                                : launch_replicate_channels(static_cast<const uint8_t *>(input), plan->stage_in, (int64_t)d.n * d.h * d.w, plan->rep_c,

@@ -27,16 +27,24 @@ def in_place(plan, x, out_bytes, q, shift):
     ("deconv", 2, 23, 15, 17, 3, eden.NHWC, 0),
     ("deconv", 2, 23, 15, 17, 3, eden.NCHW, 0),
     ("fc", 1, 113, 97, 113, 1, eden.NHWC, 0),      # 97 rows
+    ("dw", 2, 33, 41, 33, 3, eden.NHWC, 0),
+    ("dw", 2, 33, 41, 33, 3, eden.NHWC, 33 * 41),
+    ("dw", 2, 22, 41, 44, 3, eden.NHWC, 0),        # a multiplier
 ])
 def test_in_place(kind, n, c, h, cout, k, layout, shift):
     print("in place", kind, n, c, h, cout, k, layout, shift, flush=True)
-    q = O.make_quant(0.02, 131, 0.005, 117, float(0.02 * 0.005 * 74 * 74 * np.sqrt(c * k * k) / 40), 120)
+    q = O.make_quant(0.02, 131, 0.005, 117, float(0.02 * 0.005 * 74 * 74 * np.sqrt((1 if kind == "dw" else c) * k * k) / 40), 120)
     b, pad = synth.fill_i32((cout,), SEED + 1, -1000, 1000), (k // 2,) * 4
     d_b = eden.DeviceBuffer(host=b)
     if kind == "fc":
         x, w = synth.fill_u8((h, c), SEED), synth.fill_u8((cout, c), SEED + 2)
         want, d_w = O.fc(x, w, b, q), eden.DeviceBuffer(host=w)
         plan = eden.FcPlan(h, c, cout, d_w, d_b, to_eh_requant(q))
+    elif kind == "dw":
+        x, w = synth.fill_u8((n, c, h, h), SEED), synth.fill_u8((cout, 1, k, k), SEED + 2)
+        want = O.dwconv2d(x, w, b, O.conv_shape(n, c, h, h, cout, k, k, pad=pad, groups=c, dm=cout // c), q)
+        d_w = eden.DeviceBuffer(host=w)
+        plan = eden.DwConvPlan(eden.conv_desc(n, c, h, h, cout, k, k, (1, 1), pad, dm=cout // c, layout=layout), d_w, d_b, to_eh_requant(q))
     else:
         deconv = kind == "deconv"
         x, w = synth.fill_u8((n, c, h, h), SEED), synth.fill_u8((c, cout, k, k) if deconv else (cout, c, k, k), SEED + 2)
@@ -44,7 +52,7 @@ def test_in_place(kind, n, c, h, cout, k, layout, shift):
         desc = eden.conv_desc(n, c, h, h, cout, k, k, (1, 1), pad, layout=layout, weight_layout=eden.W_IOHW if deconv else eden.W_OIHW)
         d_w = eden.DeviceBuffer(host=w)
         plan = (eden.DeconvPlan if deconv else eden.ConvPlan)(desc, d_w, d_b, to_eh_requant(q))
-        if layout == eden.NHWC:
-            x, want = x.transpose(0, 2, 3, 1), want.transpose(0, 2, 3, 1)
+    if kind != "fc" and layout == eden.NHWC:
+        x, want = x.transpose(0, 2, 3, 1), want.transpose(0, 2, 3, 1)
     got = in_place(plan, x, want.size, to_eh_requant(q), shift).reshape(want.shape)
     assert np.array_equal(got, want), diff_report(got, want)

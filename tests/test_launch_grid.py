@@ -115,7 +115,7 @@ IN_PLACE = """
 import os
 def in_place(plan, in_bytes, out_bytes):
     d = eden.DeviceBuffer(nbytes=in_bytes + out_bytes)
-    for shift in (in_bytes, 0, in_bytes - 1):   # behind the input, on it, on its last byte
+    for shift in (in_bytes, 0, in_bytes - 4):   # behind the input, on it, on its last word
         print("run", file=open(os.environ["HIP_STUB_LOG"], "a"))
         plan.run(d, eden.BufferView(d, shift), q)
 """
@@ -127,10 +127,12 @@ def in_place(plan, in_bytes, out_bytes):
     ("eden.ConvPlan(eden.conv_desc(1, 64, 20, 20, 30, 1, 1, layout=eden.NCHW), buf(30, 64, 1, 1), bias(30), q)", 64 * 400, 30 * 400),
     ("eden.DeconvPlan(eden.conv_desc(2, 23, 15, 15, 17, 3, 3, (1, 1), (1,) * 4, layout=eden.NHWC, weight_layout=eden.W_IOHW), buf(23, 17, 3, 3), bias(17), q)", 2 * 23 * 225, 2 * 17 * 225),
     ("eden.FcPlan(97, 113, 113, buf(113, 113), bias(113), q)", 97 * 113, 97 * 113),
-], ids=["ragged", "planar", "planar_whole_channels", "transposed", "fc"])
+    ("eden.DwConvPlan(eden.conv_desc(2, 33, 21, 21, 33, 3, 3, (1, 1), (1,) * 4, dm=1, layout=eden.NHWC), buf(33, 1, 3, 3), bias(33), q)", 2 * 33 * 441, 2 * 33 * 441),
+    ("eden.DwConvPlan(eden.conv_desc(2, 22, 21, 21, 44, 3, 3, (1, 1), (1,) * 4, dm=2, layout=eden.NHWC), buf(44, 1, 3, 3), bias(44), q)", 2 * 22 * 441, 2 * 44 * 441),
+], ids=["ragged", "planar", "planar_whole_channels", "transposed", "fc", "depthwise_ragged", "depthwise_multiplier"])
 def test_an_output_on_its_input_reads_a_copy(stub, tmp_path, plan, in_bytes, out_bytes):
     program = "bias = lambda n: buf(n, dtype=np.int32)\n" + IN_PLACE + "in_place(%s, %d, %d)\n" % (plan, in_bytes, out_bytes)
     names = [r[0] for r in launches(stub, tmp_path, program)]
     at = [i for i, v in enumerate(names) if v == "run"] + [len(names)]
-    apart, on, last_byte = [names[at[i] + 1:at[i + 1]] for i in range(3)]
-    assert len(apart) == 1 and len(on) > 1 and "few_tiles" not in on[0] and on == last_byte, (apart, on, last_byte)
+    apart, on, last_word = [names[at[i] + 1:at[i + 1]] for i in range(3)]
+    assert len(apart) == 1 and len(on) > 1 and on[0].split("kernel")[0] not in apart[0] and on == last_word, (apart, on, last_word)
