@@ -770,14 +770,15 @@ struct eh_dwconv_plan {
     bool trip_valid = false;    // w_trip / bias_trip match the current zero points
     // Staging.  `d` describes what the kernels run: channels-last tensors with depth multiplier 1.  A caller's depth
     // multiplier m > 1 (channels-last) is met by a copy of the input with every channel m times in a row, so that
-    // output channel j reads channel j of the copy; a caller's planar tensors (multiplier 1) by the two transpositions
-    // the convolution plans use.  Both only where the output channels are a multiple of 4 (the four-channel kernels).
+    // output channel j reads channel j of the copy; a caller's planar tensors (multiplier 1) that no kernel reads as they are by the two
+    // transpositions the convolution plans use.  Both only where the output channels are a multiple of 4 (the four-channel kernels).
     int32_t rep_c = 0, rep_dm = 0;  // the caller's channel count and depth multiplier when the input is replicated
     // ... and output channels that are no multiple of 4 (channels-last) by rounding them up: the copy of the input ends
     // every pixel with repeats of its last channel, the weights of the extra channels are zero, and the result is
     // computed into an image of the padded width, from which the caller's channels are copied out.
     int32_t cout_caller = 0;        // `cout` counts the padded channels; this is what the caller's tensors hold
     bool planar = false;            // the caller's tensors are NCHW, and the kernels' are not
+    bool planar_direct = false;     // ... and so are the kernels', which read a copy (stage_in) where the output lies on the input
     uint8_t *stage_in = nullptr, *stage_out = nullptr;
     // geometry of the latest fused launch behind a pointwise layer, and what it was chosen for
     BlockGeom block{};
@@ -1918,10 +1919,11 @@ int eh_dwconv2d_u8_plan(eh_dwconv_plan **plan, const eh_conv_desc *desc, const v
     hipStream_t s = as_stream(stream);
     if (pl->planar && dw_planar_applies(dw_problem(pl, nullptr, nullptr))) {
         pl->planar = false;
+        pl->planar_direct = true;
         pl->d.layout = EH_NCHW;
     }
     rc = dev_alloc(&pl->w_copy, (size_t)pl->cout * pl->taps + 4);
-    if (!rc && (pl->rep_dm || pl->planar)) rc = dev_alloc(&pl->stage_in, (size_t)desc->n * desc->h * desc->w * pl->cout + 256);
+    if (!rc && (pl->rep_dm || pl->planar || pl->planar_direct)) rc = dev_alloc(&pl->stage_in, (size_t)desc->n * desc->h * desc->w * pl->cout + 256);
     if (!rc && (pl->planar || pl->cout != pl->cout_caller)) rc = dev_alloc(&pl->stage_out, (size_t)desc->n * pl->ho * pl->wo * pl->cout + 256);
     if (!rc) rc = dev_alloc(&pl->bias_copy, (size_t)pl->cout);
     if (!rc && pl->cout != pl->cout_caller && !g_dry_run) {  // the extra channels: zero weights, zero bias
@@ -2083,6 +2085,12 @@ int eh_dwconv2d_u8_run(eh_dwconv_plan *plan, const void *input, void *output, co
         if ((rc = launch_nchw2nhwc(static_cast<const uint8_t *>(input), plan->stage_in, d.n, d.c, d.h * d.w, s))) return rc;
         if ((rc = launch_dwconv_nhwc(dw_problem(plan, plan->stage_in, plan->stage_out), s))) return rc;
         return launch_nhwc2nchw(plan->stage_out, static_cast<uint8_t *>(output), d.n, plan->cout, plan->ho * plan->wo, s);
+    } else if (plan->planar_direct) {
+        const size_t in_bytes = (size_t)d.n * d.c * d.h * d.w;
+        if (!lie_apart(input, in_bytes, output, (size_t)d.n * plan->cout * plan->ho * plan->wo)) {
+            EH_HIP(hipMemcpyAsync(plan->stage_in, input, in_bytes, hipMemcpyDeviceToDevice, s));
+            input = plan->stage_in;
+        }
     }
     const DwProblem p = dw_problem(plan, input, output);
     return d.layout == EH_NHWC ? launch_dwconv_nhwc(p, s) : launch_dwconv_nchw(p, s);

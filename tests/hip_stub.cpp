@@ -1,6 +1,8 @@
 // A stand-in for the HIP runtime, for programs without a GPU (LD_PRELOAD): "device" memory is host memory, copies happen at
 // once, kernels do not run.  Each launch adds a line to the file that HIP_STUB_LOG names:
 //     <kernel> <grid x> <grid y> <grid z> <dynamic LDS bytes>
+// and with HIP_STUB_COPIES set each copy on a stream
+//     copy <bytes> 1 1 0
 // A kernel whose name holds HIP_STUB_FULL is said to fit 8 workgroups to a CU, any other one 4.
 #include <cstdio>
 #include <cstdlib>
@@ -56,7 +58,14 @@ int hipFree(void *p) { return free(p), 0; }
 int hipHostMalloc(void **p, size_t bytes, unsigned) { return allocate(p, bytes); }
 int hipHostFree(void *p) { return free(p), 0; }
 int hipMemcpy(void *dst, const void *src, size_t bytes, int) { return memmove(dst, src, bytes), 0; }
-int hipMemcpyAsync(void *dst, const void *src, size_t bytes, int, void *) { return memmove(dst, src, bytes), 0; }
+int hipMemcpyAsync(void *dst, const void *src, size_t bytes, int, void *) {
+    if (getenv("HIP_STUB_COPIES"))
+        if (FILE *f = getenv("HIP_STUB_LOG") ? fopen(getenv("HIP_STUB_LOG"), "a") : nullptr) {
+            fprintf(f, "copy %zu 1 1 0\n", bytes);
+            fclose(f);
+        }
+    return memmove(dst, src, bytes), 0;
+}
 int hipMemset(void *p, int value, size_t bytes) { return memset(p, value, bytes), 0; }
 int hipMemsetAsync(void *p, int value, size_t bytes, void *) { return memset(p, value, bytes), 0; }
 int hipFuncSetAttribute(const void *, int, int) { return 0; }

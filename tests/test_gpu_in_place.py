@@ -30,6 +30,9 @@ def in_place(plan, x, out_bytes, q, shift):
     ("dw", 2, 33, 41, 33, 3, eden.NHWC, 0),
     ("dw", 2, 33, 41, 33, 3, eden.NHWC, 33 * 41),
     ("dw", 2, 22, 41, 44, 3, eden.NHWC, 0),        # a multiplier
+    ("dw", 2, 24, 41, 24, 3, eden.NCHW, 0),
+    ("dw", 2, 24, 41, 24, 5, eden.NCHW, 41 * 41),
+    ("dw", 1, 64, 56, 64, 7, eden.NCHW, 0),        # four rows to a thread
 ])
 def test_in_place(kind, n, c, h, cout, k, layout, shift):
     print("in place", kind, n, c, h, cout, k, layout, shift, flush=True)

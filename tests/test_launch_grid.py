@@ -113,6 +113,7 @@ assert forms == [%d, %d, %d], forms
 
 IN_PLACE = """
 import os
+os.environ["HIP_STUB_COPIES"] = "1"
 def in_place(plan, in_bytes, out_bytes):
     d = eden.DeviceBuffer(nbytes=in_bytes + out_bytes)
     for shift in (in_bytes, 0, in_bytes - 4):   # behind the input, on it, on its last word
@@ -129,7 +130,10 @@ def in_place(plan, in_bytes, out_bytes):
     ("eden.FcPlan(97, 113, 113, buf(113, 113), bias(113), q)", 97 * 113, 97 * 113),
     ("eden.DwConvPlan(eden.conv_desc(2, 33, 21, 21, 33, 3, 3, (1, 1), (1,) * 4, dm=1, layout=eden.NHWC), buf(33, 1, 3, 3), bias(33), q)", 2 * 33 * 441, 2 * 33 * 441),
     ("eden.DwConvPlan(eden.conv_desc(2, 22, 21, 21, 44, 3, 3, (1, 1), (1,) * 4, dm=2, layout=eden.NHWC), buf(44, 1, 3, 3), bias(44), q)", 2 * 22 * 441, 2 * 44 * 441),
-], ids=["ragged", "planar", "planar_whole_channels", "transposed", "fc", "depthwise_ragged", "depthwise_multiplier"])
+    ("eden.DwConvPlan(eden.conv_desc(2, 24, 21, 21, 24, 3, 3, (1, 1), (1,) * 4, dm=1, layout=eden.NCHW), buf(24, 1, 3, 3), bias(24), q)", 2 * 24 * 441, 2 * 24 * 441),
+    ("eden.DwConvPlan(eden.conv_desc(2, 24, 21, 21, 24, 7, 7, (2, 2), (3,) * 4, dm=1, layout=eden.NCHW), buf(24, 1, 7, 7), bias(24), q)", 2 * 24 * 441, 2 * 24 * 121),
+], ids=["ragged", "planar", "planar_whole_channels", "transposed", "fc", "depthwise_ragged", "depthwise_multiplier",
+        "depthwise_planar", "depthwise_planar_7x7_stride_2"])
 def test_an_output_on_its_input_reads_a_copy(stub, tmp_path, plan, in_bytes, out_bytes):
     program = "bias = lambda n: buf(n, dtype=np.int32)\n" + IN_PLACE + "in_place(%s, %d, %d)\n" % (plan, in_bytes, out_bytes)
     names = [r[0] for r in launches(stub, tmp_path, program)]
