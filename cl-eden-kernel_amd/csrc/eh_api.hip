@@ -541,7 +541,8 @@ struct GemmOp {
 
     // Whether the plan's kernels write a planar output themselves, instead of a channels-last image that a transposition
     // then reads (a launch and two trips of the output).  Every epilogue that holds sixteen channels of a pixel per lane has
-    // the form, but for the largest tiles (no registers to spare) and the second launches of sliced reductions.  Transposed ->
+    // the form, but for the largest tiles (240 of them, the fewest of a launch, are beyond the line for tiled kernels below; the form would
+    // make them spill) and the second launches of sliced reductions.  Transposed ->
     // written, us, whole runs, over 16 .. 512 output channels, planes of 7x7 .. 224x224 and 1 .. 64 images:
     //   kernels that finish wave by wave gain at every size, some 3 us on small outputs, and at worst break even:
     //     one tap      64 -> 256 at 56x56, 4 / 64 images (3.2 / 51 MB) 11.8 -> 9.5 / 47.3 -> 40.7; 64 -> 256 at 112x112, 64 images (206 MB) 185 -> 115

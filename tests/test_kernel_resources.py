@@ -53,3 +53,9 @@ def test_other_hot_kernels_keep_their_occupancy(needle, max_scratch, min_occupan
     assert hits
     for f, name, vgprs, agprs, scratch, occ in hits:
         assert scratch <= max_scratch and occ >= min_occupancy, (name, scratch, occ)
+
+
+def test_no_kernel_uses_scratch_memory():
+    """What spills is reloaded where the allocator finds room, also between a conditional's end and the restore of the execution
+    mask (see test_exec_restore.py): no kernel does."""
+    assert not [(name, scratch) for f, name, vgprs, agprs, scratch, occ in rows() if scratch]
