@@ -469,7 +469,10 @@ namespace {
 // The tile of a launch whose depthwise stage walks: the one that takes the least time by a count of its waves' instructions, each of
 // which takes a SIMD some 2.3 + 1.1 w ns for the w waves it holds; a set of workgroups that a CU holds at a time (registers leave
 // room for five, with a pair per channel four) takes a microsecond beside that.  The coefficients are fitted to 3900 tiles of eighteen
-// layers; for those layers the tile chosen is 3 % slower than the fastest on average and 8 % at most.
+// layers; for those layers the tile chosen is 3 % slower than the fastest on average and 8 % at most.  How many workgroups a CU gets is
+// counted as the hardware deals them out: an eighth of the tiles, rounded up, to an XCD of 32 CUs, and LDS in pieces of 1280 bytes.  Without
+// the one, 152 -> 912 at 17x17, 11 images, a pair per channel, had 65 workgroups to an XCD where 64 fit, 15.3 us (9.55 now); without the other 24 ->
+// 144 at 77x77 stride 2, 22 images, had two of 54336 bytes to a CU where three were counted on, 17.8 us (13.8).  364 drawn pairs: 1.8 % faster.
 bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, int cols_per_tile, int *th, int *tw, int *nb, int *walk_log) {
     const int S = dw.stride_h, ks = pw.k_pad / 32, nb_all = (dw.c + 31) / 32, chunks_all = dw.c / 16;
     const double epilogue = pw.rq.pc_multiplier ? 1.42 : 1.0;
@@ -507,17 +510,17 @@ bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, in
                 for (int i = 0; i < n_down[4 - lg]; ++i) {
                     const Cut d = down[4 - lg][i];
                     const int ih = (d.size - 1) * S + 3;
-                    const double walk = 52.0 + 26.0 * epilogue * (d.size >> (4 - lg)), groups_of_tiles = (double)dw.n * d.pieces * ranges / 256.0;
+                    const double walk = 52.0 + 26.0 * epilogue * (d.size >> (4 - lg));
                     for (int j = 0; j < n_across; ++j) {
                         const Cut a = across[j];
                         const int pixels = ih * ((a.size - 1) * S + 3);
                         const size_t lds = lds_fixed + (size_t)pixels * lds_pixel + 15;
                         if (lds > lds_max) continue;
-                        const double per_cu = groups_of_tiles * a.pieces;
+                        const double per_cu = (double)(((long)dw.n * d.pieces * a.pieces + 7) / 8 * ranges) / 32.0;  // (of an XCD with all its tiles)
                         if (best >= 0 && pixels < 80 && per_cu > held) break;  // (small tiles only where larger ones would leave CUs idle)
                         const double wave = 10 + 40.0 * cn + 40.0 * ((pixels * ks * 4 + 255) >> 8) + ((((pixels + 31) >> 5) * cn + 3) >> 2) * (67.0 * epilogue + 5.5 * ks) +
                                             ((chunks * ((a.size + (1 << lg) - 1) >> lg) + 3) >> 2) * walk;
-                        const int fit = (int)((160 * 1024) / lds), most = fit < held ? fit : held, full = (int)(per_cu / most);
+                        const int fit = (int)((160 * 1024) / ((lds + 1279) / 1280 * 1280)), most = fit < held ? fit : held, full = (int)(per_cu / most);
                         auto time = [&](int waves) { return wave * (2.3 + 1.07 * waves) + 800; };
                         const int rest = (int)(per_cu - full * most + 0.999);
                         const double cost = full * time(most) + (rest > 0 ? time(rest) : 0);

@@ -111,6 +111,38 @@ assert forms == [%d, %d, %d], forms
     launches(stub, tmp_path, program)
 
 
+@pytest.mark.parametrize("shape", [
+    # n, cin, expanded, height, width, stride, a pair per channel
+    (11, 152, 912, 17, 17, 1, True),     # 65 workgroups to an XCD that holds 64
+    (7, 96, 576, 37, 37, 1, True),       # 99, 96
+    (22, 24, 144, 77, 77, 2, False),     # three workgroups of 54336 bytes fill 160 KB, and two of the 55040 that are given out
+    (37, 40, 240, 75, 79, 1, False),     # 54080
+    (4, 72, 432, 106, 106, 2, False),    # 54592
+])
+def test_rounds_of_a_fused_launch_are_counted_as_the_hardware_deals_them_out(stub, tmp_path, shape):
+    """The tile of a fused launch is chosen by its rounds of workgroups: those that the launch has on XCDs of 32 CUs with whole tiles and LDS in
+    pieces of 1280 bytes are no more than an even split of everything would have."""
+    program = """
+import os
+n, cin, c, h, w, stride, pairs = %r
+pw = eden.ConvPlan(eden.conv_desc(n, cin, h, w, c, 1, 1, layout=eden.NHWC), buf(c, cin, 1, 1), buf(c, dtype=np.int32), q)
+dw = eden.DwConvPlan(eden.conv_desc(n, c, h, w, c, 3, 3, (stride,) * 2, (1,) * 4, dm=1, layout=eden.NHWC), buf(c, 1, 3, 3), buf(c, dtype=np.int32), q)
+for plan in (pw, dw):
+    plan.set_perchannel(*((np.full(c, q.multiplier), np.full(c, q.shift)) if pairs else (None, None)))
+ho, wo = (h - 1) // stride + 1, (w - 1) // stride + 1
+eden.conv_dw_block_run(pw, dw, buf(n, h, w, cin), eden.DeviceBuffer(nbytes=n * ho * wo * c), q, eden.make_requant(0.02, 5, 0.004, 121, 0.03, 5))
+rows, cols = eden.conv_dw_block_tile(pw, dw)[:2]
+print("tiles", n * -(-ho // rows) * -(-wo // cols), file=open(os.environ["HIP_STUB_LOG"], "a"))
+""" % (shape,)
+    log = launches(stub, tmp_path, program)
+    (_, x, y, _, lds), = [l for l in log if "pwdw_block_kernel" in l[0]]
+    tiles, held = log[-1][1], 4 if shape[-1] else 5   # by their registers
+    ceil = lambda a, b: -(-a // b)
+    even = ceil(tiles * y, 256 * min(held, 163840 // lds))
+    dealt = ceil(ceil(tiles, 8) * y, 32 * min(held, 163840 // (ceil(lds, 1280) * 1280)))
+    assert x == ceil(tiles, 8) * 8 and dealt <= even, (tiles, y, lds, dealt, even)
+
+
 IN_PLACE = """
 import os
 os.environ["HIP_STUB_COPIES"] = "1"
