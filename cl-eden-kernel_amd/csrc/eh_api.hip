@@ -590,7 +590,7 @@ struct GemmOp {
         for (auto &g : parts) {
             const bool order = g.cfg.id == GEMM_FEW_TILES || g.cfg.id == GEMM_THIN || g.cfg.id == GEMM_CONV3X3 || g.cfg.id == GEMM_SKINNY;
             if (!order || g.slices || g.n_period || g.block_cin || g.vec != 16 || g.k <= 0 || g.cin % 16 != 0 ||
-                !gemm_few_tiles_direct(g.proto.m, g.n, g.k, (int32_t)parts.size(), form))
+                !gemm_few_tiles_direct(g.proto.m, g.n, g.k, g.taps, (int32_t)parts.size(), form))
                 return INPUT_CHUNKS;
         }
         return form;

@@ -423,19 +423,29 @@ bool gemm_few_tiles_instead(const GemmProblem &p) {
     return p.cfg.id == GEMM_THIN || p.cfg.id == GEMM_CONV3X3;
 }
 
-// Against the copy and the kernel that reads it, us (start of the line: tiles, bytes of a tap's reduction with its padding):
-//   ragged   7, 176 of 128 x 175 x 88 7.7 -> 3.8; 352, 288 of 3x3 24 -> 64 at 6 x 28x28 7.6 -> 4.5; in a replayed graph, where a second launch is
-//            cheaper, 512, 288 of 3x3 21 -> 21 at 4 x 64x64 6.6 -> 4.9; 640 of it 6.6 -> 6.7; 1024 6.7 -> 7.5; 1024, 144 of 3x3 15 -> 21 6.3 -> 7.3;
-//            1024, 64 of 1x1 45 -> 21 6.0 -> 6.6, 160 9.5 -> 6.8, 256 14.1 -> 6.8; 768, 400 5.8 either way
-//   planar   287, 288 of 3x3 21 -> 21 at 3 x 65x47 7.8 -> 5.2; 150, 864 of 3x3 96 -> 96 at 4 x 20x20 7.7 -> 7.0; 100, 1152 7.5 -> 7.2; 784, 256 of 1x1
-//            256 -> 128 at 32 x 14x14 9.3 -> 6.7; 588, 288 7.1 -> 7.8; 294, 800 8.4 -> 9.1; 800, 160 7.8 -> 8.1
-// (planar 1x1 layers of one product keep to two rounds: 980 tiles 6.5 .. 7.6 either way)
-bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t problems, int32_t form) {
+// Against the copy and the kernel that reads it.  Drawn layers (some 1500, on both sides of every line; a replayed graph, where a second
+// launch is cheapest), the time of reading directly over that of the copy; k: a tap's reduction with its padding, times the taps:
+//   ragged  up to one round of tiles  k to 2500 0.60 .. 1.03; 2700 .. 3500 0.79 .. 1.06; beyond 0.86 .. 1.13, as four lanes' pieces of a pixel
+//                                     meet more cache lines than whole chunks do.  Rows few enough for the few-row kernel: k 2000 .. 2560 0.73 .. 1.07,
+//                                     2600 .. 3000 0.82 .. 1.14, 3500 .. 3650 1.05 .. 1.23
+//           up to two                 k 400 .. 1024 0.66 .. 0.84; 1150 .. 1570 0.88 .. 1.33; one tap 600 .. 2208 0.39 .. 0.91
+//           up to four                one tap, k 190 .. 240 0.69 .. 0.79; 144 1.08; 3x3 288 1.06, 864 1.12
+//   planar  up to one                 k to 576 0.50 .. 0.97; 720 .. 1000 0.80 .. 1.28 (most of 7x7 on 16 channels 1.01 .. 1.18); 1100 .. 1600 1.04 .. 1.70,
+//                                     4000 2.0 .. 2.8: sixteen loads to a chunk.  One tap 0.51 .. 1.01 to 1072
+//           up to two                 k to 576 0.39 .. 1.16, of 40 three above 1.03; 640 .. 860 0.90 .. 1.35
+//           800 tiles                 k 48 .. 160 0.57 .. 0.84; 288 .. 1150 1.10 .. 1.31; 800 tiles, 160 7.8 -> 8.1 us
+// (planar 1x1 layers of one product keep to two rounds: 980 tiles 6.5 .. 7.6 us either way)
+bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t taps, int32_t problems, int32_t form) {
     const long tiles = m > 0 ? few_tiles_count(m, n) * problems : 0;
-    if (tiles <= 0 || k > 8192) return false;
-    if (form == INPUT_RAGGED) return tiles <= 512 || (tiles <= 1024 && k > 144 && k <= 256);
-    const long rounds = (tiles + 255) / 256;
-    return rounds <= 2 ? k * rounds <= 1152 : tiles < 800 && k > 32 && k <= 256;
+    if (tiles <= 0) return false;
+    const bool one_tap = taps == 1;
+    if (form == INPUT_RAGGED) {
+        if (tiles <= 256) return k <= (one_tap && m <= 16 ? 2560 : 3500);
+        if (tiles <= 512) return k <= (one_tap ? 2208 : 1024);
+        return tiles <= 1024 && one_tap && k > 144 && k <= 256;
+    }
+    if (tiles <= 256) return k <= (one_tap ? 1152 : 576);
+    return tiles <= 512 ? k <= 576 : tiles < 800 && k > 32 && k <= 256;
 }
 
 int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream) {

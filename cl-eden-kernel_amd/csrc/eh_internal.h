@@ -586,7 +586,7 @@ int launch_gemm_skinny(const GemmProblem &p, hipStream_t stream);
 bool gemm_few_tiles_applies(int64_t m, int64_t n, int64_t k, int32_t siblings);
 bool gemm_few_tiles_instead(const GemmProblem &p);  // ... although it was planned for another kernel of the same weight order
 // ... reading the caller's own tensor in form `form` where the plan's kernels would read a padded or channels-last copy of it
-bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t problems, int32_t form);
+bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t taps, int32_t problems, int32_t form);
 int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream);  // `count` equally shaped problems as one launch
 // few input channels, a kernel row per reduction step (eh_conv_rows.hip)
 bool conv_rows_applies(int32_t cin_group, int32_t pixel_stride, int32_t kh, int32_t kw);

@@ -143,6 +143,44 @@ print("tiles", n * -(-ho // rows) * -(-wo // cols), file=open(os.environ["HIP_ST
     assert x == ceil(tiles, 8) * 8 and dealt <= even, (tiles, y, lds, dealt, even)
 
 
+@pytest.mark.parametrize("plan,in_bytes,out_bytes,direct", [
+    # rows few enough for the few-row kernel: k to 2560
+    ("fc(3, 2555, 798)", 3 * 2555, 3 * 798, True),
+    ("fc(3, 3609, 798)", 3 * 3609, 3 * 798, False),
+    ("fc(21, 3480, 294)", 21 * 3480, 21 * 294, True),
+    # one round of tiles: k to 3500
+    ("conv(1, 378, 9, 40, 3)", 378 * 81, 40 * 81, True),
+    ("conv(1, 426, 13, 11, 3)", 426 * 169, 11 * 169, False),
+    # two: k to 1024, one tap to 2208
+    ("conv(4, 97, 42, 45, 3)", 4 * 97 * 1764, 4 * 45 * 1764, True),
+    ("conv(4, 21, 42, 45, 7)", 4 * 21 * 1764, 4 * 45 * 1764, False),
+    ("fc(637, 2204, 477)", 637 * 2204, 637 * 477, True),
+    # four: one tap only
+    ("conv(2, 238, 66, 42, 1)", 2 * 238 * 4356, 2 * 42 * 4356, True),
+    ("conv(2, 50, 66, 42, 2)", 2 * 50 * 4356, 2 * 42 * 65 * 65, False),
+    # planar: k to 576, one tap to 1152
+    ("conv(1, 60, 20, 40, 3, eden.NCHW)", 60 * 400, 40 * 400, True),
+    ("conv(1, 80, 20, 40, 3, eden.NCHW)", 80 * 400, 40 * 400, False),
+    ("conv(1, 880, 20, 40, 1, eden.NCHW)", 880 * 400, 40 * 400, True),
+    ("conv(1, 1168, 20, 40, 1, eden.NCHW)", 1168 * 400, 40 * 400, False),
+])
+def test_ragged_and_planar_tensors_are_read_as_they_are_where_that_is_faster(stub, tmp_path, plan, in_bytes, out_bytes, direct):
+    program = """
+bias = lambda n: buf(n, dtype=np.int32)
+def fc(m, k, n):
+    return eden.FcPlan(m, k, n, buf(n, k), bias(n), q)
+def conv(n, c, h, cout, k, layout=eden.NHWC):
+    return eden.ConvPlan(eden.conv_desc(n, c, h, h, cout, k, k, (1, 1), ((k - 1) // 2,) * 4, layout=layout), buf(cout, c, k, k), bias(cout), q)
+plan = %s
+import os
+print("run", file=open(os.environ["HIP_STUB_LOG"], "a"))
+plan.run(eden.DeviceBuffer(nbytes=%d), eden.DeviceBuffer(nbytes=%d), q)
+""" % (plan, in_bytes, out_bytes)
+    names = [r[0] for r in launches(stub, tmp_path, program)]
+    names = names[names.index("run") + 1:]
+    assert (len(names) == 1 and "few_tiles" in names[0]) if direct else len(names) > 1, names
+
+
 IN_PLACE = """
 import os
 os.environ["HIP_STUB_COPIES"] = "1"
