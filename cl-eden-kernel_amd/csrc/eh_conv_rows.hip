@@ -231,7 +231,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KH <= 7 ? 4
                             if constexpr (mode == 0)
                                 return requant_u8_channel(x, mult, shift, rq);
                             else
-                                return requant_u8_channel_fast<mode>(x, mult, shift, rq);
+                                return requant_u8_channel_words<mode>(x, mult, shift, rq);
                         };
                         packed[g] = pack_bytes(one(acc[g * 4 + 0], cm.x, cs.x), one(acc[g * 4 + 1], cm.y, cs.y), one(acc[g * 4 + 2], cm.z, cs.z),
                                                one(acc[g * 4 + 3], cm.w, cs.w)) ^

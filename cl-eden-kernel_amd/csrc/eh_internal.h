@@ -215,6 +215,21 @@ __host__ __device__ __forceinline__ uint32_t requant_u8_channel_fast(int32_t x, 
     return (uint32_t)v;
 }
 
+// The same for shifts of two and more (what a plan with `fast` set and pairs of channel_pair_is_fast(.., -2) has), with the channel's term
+// by a 32-bit shift.  A 64-bit shift whose amount lies in the last of a wave's registers gives wrong results now and then: the 7x7
+// first-layer kernel's did, for the sixteenth channel of every block (the compiler knows of it on gfx90a, not here).
+// tests/test_wide_shifts.py reads all built code for such shifts.
+template <int MODE>
+__host__ __device__ __forceinline__ uint32_t requant_u8_channel_words(int32_t x, int32_t multiplier, int32_t shift, const RequantDev &r) {
+    const int32_t rs = -shift;
+    const int64_t nudge = (MODE != 2 && x < 0) ? (1ll << 30) - (1ll << 31) : 1ll << 30;
+    const int32_t h = (int32_t)(((int64_t)x * (int64_t)multiplier + nudge) >> 32);
+    int32_t v = (h + (int32_t)((uint32_t)(1 + 2 * r.zp_out) << (rs - 2))) >> (rs - 1);
+    v = v < r.act_min ? r.act_min : v;
+    v = v > r.act_max ? r.act_max : v;
+    return (uint32_t)v;
+}
+
 // Four channels at a time, for shifts of two and more.  With z = 1 + 2 zp the numerator's channel term is z 2^(rs - 2) in the high
 // word, so with h the high word of x M + 2^30 (2^31 less where x < 0)
 //     result + zp = (h + z 2^(rs - 2)) >> (rs - 1) = ((h >> (rs - 2)) + z) >> 1,
