@@ -53,9 +53,10 @@ __device__ __forceinline__ v4i one_byte(uint32_t byte, int at) {
 constexpr int kernel_columns(int k) { return (k + 3) / 4 * 4; }
 
 // K: window.  S: stride.  TH: output rows per strip.  PC: one multiplier and shift per channel.  MODE: single-shift form of
-// the requantization (1, 2) or the two-step form (0).
+// the requantization (1, 2) or the two-step form (0).  (One form has a register more than four waves per SIMD leave it: 224 channels at 32x64, 7x7, 35 images
+// 22.4 us, held to four waves 19.8.)
 template <int K, int S, int TH, bool PC, int MODE>
-__global__ __launch_bounds__(256) void dw_mfma_kernel(const DwProblem p, const DwTile g) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 7 && S == 1 && TH == 4 && !PC && MODE == 2 ? 4 : 1))) void dw_mfma_kernel(const DwProblem p, const DwTile g) {
     constexpr int KF = kernel_columns(K), ROWS = (TH - 1) * S + K;
     constexpr bool COLUMN = K == 5;             // the fifth kernel column by itself
     constexpr int FX = KF / 4, FR = COLUMN ? 1 : FX;  // operands per input row; those that run along the row
