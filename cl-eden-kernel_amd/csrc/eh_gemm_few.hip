@@ -423,7 +423,7 @@ bool gemm_few_tiles_instead(const GemmProblem &p) {
     return p.cfg.id == GEMM_THIN || p.cfg.id == GEMM_CONV3X3;
 }
 
-// Against the copy and the kernel that reads it.  Drawn layers (some 1500, on both sides of every line; a replayed graph, where a second
+// Against the copy and the kernel that reads it.  Drawn layers (some 1700, on both sides of every line; a replayed graph, where a second
 // launch is cheapest), the time of reading directly over that of the copy; k: a tap's reduction with its padding, times the taps:
 //   ragged  up to one round of tiles  k to 2500 0.60 .. 1.03; 2700 .. 3500 0.79 .. 1.06; beyond 0.86 .. 1.13, as four lanes' pieces of a pixel
 //                                     meet more cache lines than whole chunks do.  Rows few enough for the few-row kernel: k 2000 .. 2560 0.73 .. 1.07,
@@ -432,7 +432,8 @@ bool gemm_few_tiles_instead(const GemmProblem &p) {
 //           up to four                one tap, k 190 .. 240 0.69 .. 0.79; 144 1.08; 3x3 288 1.06, 864 1.12
 //   planar  up to one                 k to 576 0.50 .. 0.97; 720 .. 1000 0.80 .. 1.28 (most of 7x7 on 16 channels 1.01 .. 1.18); 1100 .. 1600 1.04 .. 1.70,
 //                                     4000 2.0 .. 2.8: sixteen loads to a chunk.  One tap 0.51 .. 1.01 to 1072
-//           up to two                 k to 576 0.39 .. 1.16, of 40 three above 1.03; 640 .. 860 0.90 .. 1.35
+//           up to two                 k 288 0.70 .. 0.94; 400 0.84 .. 1.19, 0.97 on average; 432 0.76 .. 1.07; 576 0.82 .. 1.20; 640 .. 860 0.90 .. 1.35.  One tap
+//                                     0.33 .. 0.96 to 576
 //           800 tiles                 k 48 .. 160 0.57 .. 0.84; 288 .. 1150 1.10 .. 1.31; 800 tiles, 160 7.8 -> 8.1 us
 // (planar 1x1 layers of one product keep to two rounds: 980 tiles 6.5 .. 7.6 us either way)
 bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t taps, int32_t problems, int32_t form) {
@@ -445,7 +446,7 @@ bool gemm_few_tiles_direct(int64_t m, int64_t n, int64_t k, int32_t taps, int32_
         return tiles <= 1024 && one_tap && k > 144 && k <= 256;
     }
     if (tiles <= 256) return k <= (one_tap ? 1152 : 576);
-    return tiles <= 512 ? k <= 576 : tiles < 800 && k > 32 && k <= 256;
+    return tiles <= 512 ? k <= (one_tap ? 576 : 432) : tiles < 800 && k > 32 && k <= 256;
 }
 
 int launch_gemm_few_tiles(const TapProblem *ps, int count, hipStream_t stream) {

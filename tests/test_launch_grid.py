@@ -161,6 +161,8 @@ print("tiles", n * -(-ho // rows) * -(-wo // cols), file=open(os.environ["HIP_ST
     # planar: k to 576, one tap to 1152
     ("conv(1, 60, 20, 40, 3, eden.NCHW)", 60 * 400, 40 * 400, True),
     ("conv(1, 80, 20, 40, 3, eden.NCHW)", 80 * 400, 40 * 400, False),
+    ("conv(4, 48, 48, 20, 3, eden.NCHW)", 4 * 48 * 2304, 4 * 20 * 2304, True),    # 288 tiles: to 432
+    ("conv(4, 64, 48, 20, 3, eden.NCHW)", 4 * 64 * 2304, 4 * 20 * 2304, False),
     ("conv(1, 880, 20, 40, 1, eden.NCHW)", 880 * 400, 40 * 400, True),
     ("conv(1, 1168, 20, 40, 1, eden.NCHW)", 1168 * 400, 40 * 400, False),
 ])
