@@ -22,7 +22,7 @@
 //      58x58, 16 images 32.7 -> 23; 16 -> 96 at 83x83, 21 images 21.4 -> 13.6; 56 -> 336 at 31x31, 18 images 13.4 -> 9.3; 120 -> 720
 //      at 12x12, 18 images 9.2 -> 7.0; a pair per channel, 16 -> 96 at 104x97, 28 images 34.1 -> 26.6, 80 -> 480 at 36x36, 16 images
 //      20.4 -> 15.0; at stride 2, where the expansion is most of the work, 24 -> 144 at 56x56, 32 images 11.3 and 11.3.
-//      Tiles of few outputs are taken sixteen outputs at a time instead, wherever their rows end (pwdw_block_geometry has the rule).
+//      Small tiles that a caller asks for are taken sixteen outputs at a time instead, wherever their rows end (pwdw_block_geometry has the rule).
 // The rows and columns two neighbouring workgroups both need (the halo) are computed twice; nothing else is.  Tiles are
 // cut in both directions because the halo of a stride-2 window costs (2 TH + 1)(2 TW + 1) / (4 TH TW): 1.53 for one full
 // row of 28 outputs, 1.21 for 4 x 7.
@@ -47,7 +47,7 @@ namespace {
 // stage when they are 1, 2 or 3 (a lane then keeps its pixel's operand bytes in registers across the channel blocks),
 // 0 for any number (read from LDS for every product).
 enum class DwForm {
-    UNITS,  // small tiles: sixteen outputs of the tile, wherever its rows end, by sixteen channels
+    UNITS,  // small tiles on request: sixteen outputs of the tile, wherever its rows end, by sixteen channels
     WALK    // the others: sixteen columns, down the tile's rows
 };
 // PC: one multiplier and shift per channel in both operators; the depthwise ones in the single-shift form, or in two steps.
@@ -549,85 +549,23 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
     g.ks = pw.k_pad / 32;
     g.a_pitch = g.ks * 32 + 16;
     const int nb_all = (dw.c + 31) / 32;
-    // Tile shape and channel blocks per workgroup.  A workgroup's three stages run one after the other, so the stages
-    // of different workgroups have to overlap on a CU: the shapes considered leave room for four or more workgroups in
-    // a CU's LDS (measured: tiles of twice that size take twice as long at a batch of 256, however little halo they
-    // recompute) and, where the problem is large enough, give the launch at least three workgroups per CU.  Among those
-    // the one that computes the fewest pixel slots wins, counting the slots that pixel blocks of 32 and output tiles of
-    // four leave empty and, at a lower weight, the input bytes staged again for every channel range.
-    int th = rows_per_tile, tw = cols_per_tile, nb = nb_all;
-    // Form of the depthwise stage.  Units of sixteen output pixels by sixteen channels, spread over the four waves, suit a tile of few of
-    // them, whose rows a walk would leave half of its lanes without; with more than one or two to a wave it is a matter of their fill
-    // and of their epilogue, which a pair per channel doubles.  The line was drawn against 8-bit dot products, sixteen outputs to a
-    // thread, whose place the walk has taken.  The same tiles, dot products -> units, us (with a pair per channel):
-    //   up to 3 units  28x28 32 -> 192 stride 2, 2 images 5.4 -> 4.2 (6.1 -> 4.6), stride 1, 2 images 4.6 -> 4.3 (4.9 -> 4.6),
-    //                  7x7 160 -> 960, 1 image 5.3 -> 4.55 (6.1 -> 5.05)
-    //   4              56x56 24 -> 144 stride 2, 4 images 5.4 -> 4.75 (6.1 -> 5.5), 28x28 32 -> 192 stride 1, 4 images 4.7 -> 4.8
-    //                  (5.25 -> 5.4), 14x14 64 -> 384, 4 images 4.9 -> 4.8 (5.35 -> 5.5), 7x7 160 -> 960, 4 images 5.4 -> 5.2 (5.85 -> 5.8)
-    //   6, full        56x56 24 -> 144 stride 2, 6 images 5.8 -> 5.1 (6.6 -> 6.0), 28x28 32 -> 192, 8 images 6.2 -> 6.0 (6.8 -> 7.1), at
-    //                  stride 2, 24 images 6.5 -> 6.0 (7.4 -> 7.15)
-    //   6, half full   28x28 32 -> 192 stride 2, 8 images 5.2 -> 5.35 (5.6 -> 6.4), 14x14 96 -> 576, 4 images 5.2 -> 5.7 (5.9 -> 6.7)
-    //   8, full        14x14 96 -> 576, 8 images 5.9 -> 5.6 (6.6 -> 6.7), 64 -> 384, 16 images 6.0 -> 6.05 (6.85 -> 7.3)
-    //   9 and 10, full 56x56 24 -> 144 stride 2, 12 images 7.1 -> 7.5 (8.4 -> 9.2), 14x14 96 -> 576, 12 images 6.5 -> 6.6 (7.3 -> 8.0),
-    //                  33x33 48 -> 288, 4 images 5.8 -> 6.2 (6.5 -> 7.6)
-    const bool per_channel = pw.rq.pc_multiplier != nullptr;
-    auto quads_of = [&](int blocks) { return blocks * 8 < dw.c / 4 ? blocks * 8 : dw.c / 4; };
-    auto matrix_form = [&](int rows, int cols, int blocks) {
-        const int groups = (rows * cols + 15) / 16, units = groups * (quads_of(blocks) / 4);
-        return units <= (!per_channel ? 8 : S == 2 ? 6 : 3) && (units <= 4 || rows * cols > groups * 8);
-    };
-    // (A layer of so many units leaves more of them to each workgroup that the chip holds.)
-    const bool large = rows_per_tile == 0 && cols_per_tile == 0 && (double)dw.n * dw.ho * dw.wo * dw.c > 768.0 * 12 * 256;
-    if (!large) {
-        int across[65];
-        for (int cw = 1; cw <= dw.wo && cw <= 64; ++cw) across[cw] = (dw.wo + cw - 1) / cw;
-        double best = -1;
-        int best_th = 1, best_tw = dw.wo < 4 ? dw.wo : 4, best_nb = 1;
-        for (int pass = 0; pass < 3 && best < 0; ++pass)  // later passes: fewer workgroups, then anything that fits at all
-            for (int cn = 1; cn <= nb_all; ++cn) {
-                const int ranges = (nb_all + cn - 1) / cn;
-                if ((ranges - 1) * cn >= nb_all) continue;  // the same ranges with fewer blocks each
-                const size_t lds_fixed = block_lds_bytes(cn, g.ks, 0, 0, dw.c, nullptr, nullptr), lds_pixel = (size_t)block_image_pitch(cn, dw.c);
-                for (int ch = 1; ch <= dw.ho && ch <= 16; ++ch) {
-                    const int down = (dw.ho + ch - 1) / ch;
-                    for (int cw = 1; cw <= dw.wo && cw <= 64; ++cw) {
-                        if (rows_per_tile > 0 && ch != rows_per_tile) continue;
-                        if (cols_per_tile > 0 && cw != cols_per_tile) continue;
-                        const int ih = (ch - 1) * S + 3, iw = (cw - 1) * S + 3;
-                        const size_t lds = lds_fixed + (((size_t)ih * iw * (g.ks * 32 + 16) + 15) & ~(size_t)15) + (size_t)ih * iw * lds_pixel;
-                        if (pass < 2 ? lds * 4 > 144 * 1024 : lds > kBlockLdsMax) continue;
-                        const long wgs = (long)dw.n * down * across[cw] * ranges;
-                        if (pass == 0 && wgs < 768) continue;
-                        const int px = ih * iw;
-                        const double tiles = (double)dw.n * down * across[cw];
-                        const double stage1 = (double)((px + 31) / 32 * 32) * tiles / ((double)dw.n * dw.h * dw.w_);   // pixel slots computed per real pixel
-                        // A tile of up to 128 groups of four outputs by four channels is priced by whole groups of sixteen outputs, a slot of them at
-                        // three quarters, whichever form will run it: by the vector form's own slots the search prefers tiles of two outputs
-                        // or four, whose chain is as long and whose halo is larger.  Tiles by groups and by slots, us (with a pair per
-                        // channel): both matrix, 56x56 24 -> 144 stride 2, one image 4.15 and 4.5 (4.6 and 5.0); matrix and vector, 28x28
-                        // 32 -> 192 stride 2, 16 images 5.0 and 5.8 (5.8 and 6.6); both vector, 56x56 24 -> 144 stride 2, two images 5.0 and
-                        // 5.15 (5.3 and 5.35), 14x14 96 -> 576 stride 2, 24 images 6.2 and 6.3 (7.15 and 7.1).
-                        const bool small = ch * ((cw + 3) / 4) * quads_of(cn) <= 128;
-                        const double slots = small ? 0.75 * ((ch * cw + 15) / 16 * 16) : (double)(ch * ((cw + 3) / 4 * 4));
-                        const double stage2 = slots * tiles / ((double)dw.n * dw.ho * dw.wo);  // output slots per real output
-                        const double restage = (double)px * tiles * ranges * (g.ks * 32) / ((double)dw.n * dw.h * dw.w_ * dw.c);  // staged input bytes per expanded byte
-                        const double cost = stage1 + 0.5 * stage2 + 2.0 * restage;
-                        if (best < 0 || cost < best) {
-                            best = cost;
-                            best_th = ch;
-                            best_tw = cw;
-                            best_nb = cn;
-                        }
-                    }
-                }
-            }
-        if (best < 0) return false;
-        th = best_th;
-        tw = best_tw;
-        nb = best_nb;
+    if (rows_per_tile > (dw.ho < 16 ? dw.ho : 16) || cols_per_tile > (dw.wo < 64 ? dw.wo : 64)) return false;
+    int th = rows_per_tile, tw = cols_per_tile, nb = 0;
+    g.matrix = g.walk_log = g.walk_groups = 0;
+    if (rows_per_tile > 0 && cols_per_tile > 0) {
+        // A tile of the caller's may suit the units of sixteen outputs: a walk takes 16 columns at a time, or 8, or 4, and leaves the lanes of the
+        // others idle.  Channel blocks of a unit's workgroup: as many as leave room for four workgroups in a CU's LDS, or as fit.
+        for (const size_t lds_max : {(size_t)36 * 1024, kBlockLdsMax})
+            for (int cn = nb_all; cn >= 1 && nb == 0; --cn)
+                if (((nb_all + cn - 1) / cn - 1) * cn < nb_all && block_lds_bytes(cn, g.ks, (th - 1) * S + 3, (tw - 1) * S + 3, dw.c, nullptr, nullptr) <= lds_max) nb = cn;
+        if (nb == 0) return false;
+        // The line, on 900 requested tiles of drawn layers of up to 1.5 GFLOP, walk over units by the units of a workgroup (with a pair per channel): 2
+        // 0.98 (1.02), 4 1.03 (1.03), 6 1.17 and half full ones 1.21 (0.97 and 1.07), 8 full 0.96 (0.96), 12 full 0.92 (0.99), beyond 0.77 (0.73).
+        // Tiles of this library's own choice walk: 144 drawn layers whose tiles had been of few units took 0.73 .. 1.06 of the time, 0.91 on
+        // average and 0.95 with a pair per channel, with the tile of walk_tile.
+        const int groups = (th * tw + 15) / 16, chunks = nb * 2 < dw.c / 16 ? nb * 2 : dw.c / 16, units = groups * chunks;
+        g.matrix = units <= (pw.rq.pc_multiplier == nullptr ? 8 : S == 2 ? 6 : 3) && (units <= 4 || th * tw > groups * 8) ? 1 : 0;
     }
-    g.matrix = !large && matrix_form(th, tw, nb) ? 1 : 0;
-    g.walk_log = g.walk_groups = 0;
     if (!g.matrix && !walk_tile(pw, dw, rows_per_tile, cols_per_tile, &th, &tw, &nb, &g.walk_log)) return false;
     g.nb = nb;
     g.th = th;
