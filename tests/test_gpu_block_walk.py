@@ -24,8 +24,8 @@ CASES = [
     (1, 9, 40, 8, 112, 1, 9, 20, 90, 0.4),       # the whole height; a last block of sixteen channels
     (3, 14, 14, 96, 576, 1, 7, 14, 120, 0.4),    # three reduction steps
     (2, 15, 15, 160, 192, 1, 8, 15, 0, 0.4),     # five
-    (1, 31, 33, 24, 80, 1, 16, 33, 60, 0.00002), # scales above one half: the two-step form
-    (1, 31, 33, 24, 80, 2, 16, 17, 200, 0.00002),
+    (1, 31, 33, 24, 80, 1, 16, 33, 60, 0.0003),  # 0.6, above one half: the two-step form
+    (1, 31, 33, 24, 80, 2, 16, 17, 200, 0.00025),
 ]
 
 
@@ -39,6 +39,10 @@ def test_walking_depthwise_stage_matches_oracle(case, per_channel, act_min_at_ze
     b1, b2 = synth.fill_i32((c,), SEED + 2, -1000, 1000), synth.fill_i32((c,), SEED + 4, -1000, 1000)
     w2 = synth.fill_u8((c, 1, 3, 3), SEED + 3)
     q1 = O.make_quant(0.02, 117, 0.004, 121, 0.03, 5, O.ACT_RELU6, True)
+    two_step = scale < 0.001
+    if two_step:   # small operands, so that results at such a scale are bytes of their own and not the clamp's
+        w2, b2 = (zp_w + w2.astype(np.int16) % 3 - 1).astype(np.uint8), b2 // 20
+        q1 = O.make_quant(0.02, 117, 0.004, 121, 0.5, 5, O.ACT_RELU6, True)
     q2 = O.make_quant(0.03, 5, 0.006, zp_w, scale, 128, O.ACT_RELU, act_min_at_zero_point)
     ho, wo = (h + 2 - 3) // stride + 1, (w + 2 - 3) // stride + 1
     d1 = eden.conv_desc(n, cin, h, w, c, 1, 1, layout=eden.NHWC)
@@ -55,4 +59,5 @@ def test_walking_depthwise_stage_matches_oracle(case, per_channel, act_min_at_ze
     eden.conv_dw_block_run(pw, dw, d_x, d_o, e1, e2, rows, cols)
     got = d_o.download((n, ho, wo, c))
     assert np.array_equal(got, want), diff_report(got, want)
+    assert not two_step or ((want > 0) & (want < 255)).mean() > 0.9
     assert act_min_at_zero_point or want.std() > 1   # (differences down to -255 leave nothing above the zero point)

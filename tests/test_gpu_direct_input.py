@@ -1,5 +1,5 @@
 """The kernel for few tiles on tensors that it reads as they are: channel counts off 16 (chunks at any address, the last ones ending behind
-the tensor) and planar tensors, against the oracle.  The tensors lie at the end of their allocation's own bytes, one byte in, so that
+the tensor) and planar tensors, uint8 and int8, of convolutions, transposed ones and with a fused residual add, against the oracle.  The tensors lie at the end of their allocation's own bytes, one byte in, so that
 no alignment is there by chance."""
 import numpy as np
 import pytest
@@ -65,3 +65,50 @@ def test_conv(n, c, h, w, cout, k, stride, dil, groups, layout, pc):
     got = d_o.download((n, cout, ho, wo)) if layout == eden.NCHW else d_o.download((n, ho, wo, cout)).transpose(0, 3, 1, 2)
     plan.destroy()
     assert np.array_equal(got, want), diff_report(got, want)
+
+
+@pytest.mark.parametrize("layout", [eden.NHWC, eden.NCHW])
+@pytest.mark.parametrize("deconv,n,c,h,w,cout,k,stride", [(False, 2, 21, 9, 7, 13, 3, 1), (False, 1, 37, 12, 11, 40, 1, 1), (False, 3, 10, 8, 13, 9, 5, 2),
+                                                        (True, 2, 23, 7, 9, 17, 3, 1), (True, 1, 40, 6, 5, 24, 3, 2), (True, 2, 20, 5, 6, 33, 4, 2)])
+def test_int8_and_transposed(deconv, n, c, h, w, cout, k, stride, layout):
+    print("int8", deconv, n, c, h, w, cout, k, stride, layout, flush=True)
+    pad = ((k - stride) // 2 if deconv else k // 2,) * 4
+    s = O.conv_shape(n, c, h, w, cout, k, k, stride=(stride, stride), pad=pad)
+    x, b = synth.fill_u8((n, c, h, w), SEED + 8), synth.fill_i32((cout,), SEED + 10, -1000, 1000)
+    wt = synth.fill_u8((c, cout, k, k) if deconv else (cout, c, k, k), SEED + 9)
+    x, wt = (x.astype(np.int16) - 128).astype(np.int8), (wt.astype(np.int16) - 128).astype(np.int8)
+    s_out = float(0.02 * 0.005 * 74.0 * 74.0 * np.sqrt(c * max(1, k // stride if deconv else k) ** 2) / 40.0)
+    want = (O.deconv2d_s8 if deconv else O.conv2d_s8)(x, wt, b, s, O.make_quant_s8(0.02, -11, 0.005, 3, s_out, -3))
+    q = eden.make_requant_s8(0.02, -11, 0.005, 3, s_out, -3)
+    desc = eden.conv_desc(n, c, h, w, cout, k, k, (stride, stride), pad, layout=layout | eden.IO_SIGNED, weight_layout=(eden.W_IOHW if deconv else eden.W_OIHW) | eden.W_SIGNED)
+    assert set(eden.conv_kernels(desc, deconv, launched=True)) == {"few_tiles"}
+    nhwc = layout == eden.NHWC
+    flat = np.ascontiguousarray(x.transpose(0, 2, 3, 1) if nhwc else x).view(np.uint8).reshape(-1)
+    d_x = eden.BufferView(eden.DeviceBuffer(host=np.concatenate([[7], flat]).astype(np.uint8)), 1)
+    d_w, d_b, d_o = eden.DeviceBuffer(host=wt), eden.DeviceBuffer(host=b), eden.DeviceBuffer(nbytes=want.size)
+    (eden.DeconvPlan if deconv else eden.ConvPlan)(desc, d_w, d_b, q).run(d_x, d_o, q)
+    ho, wo = want.shape[2:]
+    got = (d_o.download((n, ho, wo, cout)).transpose(0, 3, 1, 2) if nhwc else d_o.download((n, cout, ho, wo))).view(np.int8)
+    assert np.array_equal(got, want), diff_report(got, want)
+    assert want.std() > 4
+
+
+@pytest.mark.parametrize("n,c,h,w,cout,k", [(2, 21, 9, 7, 13, 1), (1, 37, 12, 11, 48, 1), (2, 26, 9, 9, 32, 3)])
+def test_residual_add(n, c, h, w, cout, k):
+    print("residual", n, c, h, w, cout, k, flush=True)
+    pad = (k // 2,) * 4
+    s = O.conv_shape(n, c, h, w, cout, k, k, pad=pad)
+    x, b = synth.fill_u8((n, c, h, w), SEED + 11), synth.fill_i32((cout,), SEED + 12, -1000, 1000)
+    wt, res = synth.fill_u8((cout, c, k, k), SEED + 13), synth.fill_u8((n, cout, h, w), SEED + 14)
+    s_out = float(0.02 * 0.005 * 74.0 * 74.0 * np.sqrt(c * k * k) / 40.0)
+    q = O.make_quant(0.02, 131, 0.005, 117, s_out, 120)
+    want = O.add(res, O.conv2d(x, wt, b, s, q), O.make_add_quant(0.05, 120, s_out, 120, 0.07, 128))
+    aq, e = eden.make_add_requant(0.05, 120, s_out, 120, 0.07, 128), to_eh_requant(q)
+    d_x = eden.BufferView(eden.DeviceBuffer(host=np.concatenate([[7], x.transpose(0, 2, 3, 1).ravel()]).astype(np.uint8)), 1)
+    d_w, d_b, d_r = eden.DeviceBuffer(host=wt), eden.DeviceBuffer(host=b), eden.DeviceBuffer(host=res.transpose(0, 2, 3, 1))
+    d_o = eden.DeviceBuffer(nbytes=want.size)
+    plan = eden.ConvPlan(eden.conv_desc(n, c, h, w, cout, k, k, (1, 1), pad, layout=eden.NHWC), d_w, d_b, e)
+    plan.run_add(d_x, d_r, d_o, e, aq)
+    got = d_o.download((n, h, w, cout)).transpose(0, 3, 1, 2)
+    assert np.array_equal(got, want), diff_report(got, want)
+    assert want.std() > 4

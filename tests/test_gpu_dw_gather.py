@@ -1,11 +1,13 @@
 """Channels-last 3x3 depthwise layers whose channels are no multiple of four or have a multiplier, straight from the caller's
 tensors: bit for bit the oracle, at a last quad of one, two and three channels, pixels of four channels and just beyond, quads whose
-input channels are one, two or four, multipliers that leave a quad's edges inside a channel's repeats, tensors at any byte."""
+input channels are one, two or four, multipliers that leave a quad's edges inside a channel's repeats, tensors at any byte; pairs that differ
+from channel to channel; and not a byte beside the result.  (test_launch_grid.py holds that these cases take the gathering kernel.)"""
 import numpy as np
 import pytest
 
 import oracle_lib as O
-from harness import diff_report, eden, synth, to_eh_requant
+from harness import diff_report, eden, synth
+from test_gpu_dw_planar import problem
 
 pytestmark = pytest.mark.gpu
 SEED = 0xD6A7
@@ -25,36 +27,27 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("form", ["u8", "u8pc", "s8"])
+@pytest.mark.parametrize("form", ["u8", "u8pc", "s8", "s8pc"])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(str(v) for v in c))
 def test_unpadded_depthwise_matches_oracle(case, form):
     n, c, dm, h, w, stride, lead = case
-    k = 3
     print("dw gather", case, form, flush=True)
-    cout, pad = c * dm, (k // 2,) * 4
-    s = O.conv_shape(n, c, h, w, cout, k, k, stride=(stride, stride), pad=pad, groups=c, dm=dm)
-    x, wt = synth.fill_u8((n, c, h, w), SEED + h), synth.fill_u8((cout, 1, k, k), SEED + c)
-    bias = synth.fill_i32((cout,), SEED + 1, -2000, 2000)
-    ho, wo = (h + 2 * pad[0] - k) // stride + 1, (w + 2 * pad[0] - k) // stride + 1
-    signed, layout = form == "s8", eden.NHWC
-    if signed:
-        q = O.make_quant_s8(0.02, 9, 0.004, 0, 0.05 * k, -4)
-        x, wt = x.view(np.int8), wt.view(np.int8)
-        want = O.dwconv2d_s8(x, wt, bias, s, q)
-        layout |= eden.IO_SIGNED
-    else:
-        q = O.make_quant(0.02, 117, 0.004, 121, 0.05 * k, 128)
-        want = O.dwconv2d(x, wt, bias, s, q)
-    e = to_eh_requant(q)
-    weight_layout = eden.W_OIHW | (eden.W_SIGNED if signed else 0)
-    desc = eden.conv_desc(n, c, h, w, cout, k, k, stride=(stride, stride), pad=pad, dm=dm, layout=layout, weight_layout=weight_layout)
-    d_w, d_b = eden.DeviceBuffer(host=wt), eden.DeviceBuffer(host=bias)
+    cout, pad = c * dm, (1, 1, 1, 1)
+    s = O.conv_shape(n, c, h, w, cout, 3, 3, stride=(stride, stride), pad=pad, groups=c, dm=dm)
+    ho, wo = O.conv_out_hw(s)
+    x, wt, e, pairs, want = problem(s, form, SEED + h, SEED + c, 0.15)
+    desc = eden.conv_desc(n, c, h, w, cout, 3, 3, stride=(stride, stride), pad=pad, dm=dm, layout=eden.NHWC | (eden.IO_SIGNED if x.dtype == np.int8 else 0),
+                          weight_layout=eden.W_OIHW | (eden.W_SIGNED if wt.dtype == np.int8 else 0))
+    d_w, d_b = eden.DeviceBuffer(host=wt), eden.DeviceBuffer(host=synth.fill_i32((cout,), 0xD3A1 + 1, -2000, 2000))
     plan = eden.DwConvPlan(desc, d_w, d_b, e)
-    if form == "u8pc":   # the tensors' own pair for every channel: the same results through the per-channel code
-        plan.set_perchannel(np.full(cout, e.multiplier), np.full(cout, e.shift))
-    padded = np.concatenate([np.full(lead, 7, np.uint8), x.view(np.uint8).transpose(0, 2, 3, 1).ravel()])
-    d_x, d_o = eden.DeviceBuffer(host=padded), eden.DeviceBuffer(nbytes=n * cout * ho * wo + 8)
+    if pairs:
+        plan.set_perchannel(*pairs)
+    count = n * cout * ho * wo
+    padded = np.concatenate([np.full(lead, 7, np.uint8), np.ascontiguousarray(x.transpose(0, 2, 3, 1)).view(np.uint8).ravel()])
+    d_x, d_o = eden.DeviceBuffer(host=padded), eden.DeviceBuffer(host=np.full(count + 8, 0xA5, np.uint8))
     plan.run(eden.BufferView(d_x, lead), eden.BufferView(d_o, lead), e)
-    got = d_o.download((n * cout * ho * wo + 8,))[lead:lead + n * cout * ho * wo].reshape(n, ho, wo, cout).transpose(0, 3, 1, 2).view(want.dtype)
+    whole = d_o.download((count + 8,))
+    got = whole[lead:lead + count].reshape(n, ho, wo, cout).transpose(0, 3, 1, 2).view(want.dtype)
     assert np.array_equal(got, want), diff_report(got, want)
-    assert n * cout * ho * wo < 64 or want.std() > 1
+    assert (whole[:lead] == 0xA5).all() and (whole[lead + count:] == 0xA5).all()
+    assert count < 64 or want.std() > 1

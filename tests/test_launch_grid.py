@@ -1,6 +1,7 @@
 """What is launched, without a GPU: the library runs on a stand-in for the HIP runtime (tests/hip_stub.cpp) that notes each
 launch's kernel and grid."""
 import os
+import re
 import subprocess
 import sys
 
@@ -139,6 +140,40 @@ print("tiles", n * -(-ho // rows) * -(-wo // cols), file=open(os.environ["HIP_ST
     even = ceil(tiles * y, 256 * min(held, 163840 // lds))
     dealt = ceil(ceil(tiles, 8) * y, 32 * min(held, 163840 // (ceil(lds, 1280) * 1280)))
     assert x == ceil(tiles, 8) * 8 and dealt <= even, (tiles, y, lds, dealt, even)
+
+
+@pytest.mark.parametrize("module,kernel", [("test_gpu_dw_planar", r"dw_planar_kernelI"), ("test_gpu_dw_gather", r"dw3x3_nhwc_tile4_dot4_kernelI.*ELb1EEEv")])
+def test_depthwise_tensors_are_read_as_they_are(stub, tmp_path, module, kernel):
+    """The cases of the two tests against the oracle take the kernels that those tests are for, in every form."""
+    program = """
+import os
+sys.path.insert(0, %r)
+import %s as m
+for case in m.CASES:
+    n, c, dm, h, w = case[:5]
+    planar = m.__name__.endswith("planar")
+    k, stride = (case[5], case[6]) if planar else (3, case[5])
+    pad = case[8] if len(case) > 8 else (k // 2,) * 4
+    for signed in (False, True):
+        e = eden.make_requant_s8(0.02, 9, 0.004, 0, 0.1, -4) if signed else q
+        desc = eden.conv_desc(n, c, h, w, c * dm, k, k, stride=(stride, stride), pad=pad, dm=dm, layout=(eden.NCHW if planar else eden.NHWC) | (eden.IO_SIGNED if signed else 0),
+                              weight_layout=eden.W_OIHW | (eden.W_SIGNED if signed else 0))
+        plan = eden.DwConvPlan(desc, buf(c * dm, 1, k, k), buf(c * dm, dtype=np.int32), e)
+        ho, wo = (h + pad[0] + pad[1] - k) // stride + 1, (w + pad[2] + pad[3] - k) // stride + 1
+        x, o = eden.DeviceBuffer(nbytes=n * c * h * w), eden.DeviceBuffer(nbytes=n * c * dm * ho * wo)
+        for pairs in (False, True):
+            if pairs:
+                plan.set_perchannel(np.full(c * dm, 1 << 30), np.full(c * dm, -6))
+            print("run", file=open(os.environ["HIP_STUB_LOG"], "a"))
+            plan.run(x, o, e)
+            print("end", file=open(os.environ["HIP_STUB_LOG"], "a"))
+""" % (HERE, module)
+    names, runs = [r[0] for r in launches(stub, tmp_path, program)], []
+    while "run" in names:
+        start, end = names.index("run"), names.index("end")
+        runs.append(names[start + 1:end])
+        names = names[end + 1:]
+    assert len(runs) >= 40 and all(len(r) == 1 and re.search(kernel, r[0]) for r in runs), [r for r in runs if len(r) != 1 or not re.search(kernel, r[0])][:3]
 
 
 @pytest.mark.parametrize("plan,in_bytes,out_bytes,direct", [
