@@ -2116,7 +2116,7 @@ int eh_conv_dw_block_applies(const eh_conv_plan *pointwise, const eh_dwconv_plan
     if (op.pad_cg_to != 0 || op.parts[0].slices != 0) return 0;
     if (depthwise->d.layout != EH_NHWC || depthwise->io_signed || depthwise->rep_dm || depthwise->planar) return 0;
     if ((op.pc_multiplier != nullptr) != (depthwise->pc_multiplier != nullptr)) return 0;  // one pair per operator, or one per channel in both
-    if (depthwise->d.n != pointwise->d.n || !(depthwise->w_trip || depthwise->w_fold)) return 0;
+    if (depthwise->d.n != pointwise->d.n) return 0;
     // geometry and kernel family are checked on the problems themselves; the pointers and parameters of a run do not enter
     const GemmProblem pw = op.problem(op.parts[0], nullptr, nullptr, nullptr, nullptr);
     const DwProblem dw = dw_problem(depthwise, nullptr, nullptr);

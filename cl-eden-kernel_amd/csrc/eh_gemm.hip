@@ -306,7 +306,7 @@ static int launch_staged(const GemmProblem &p, hipStream_t stream) {
 }
 
 static bool is_dma(int32_t id) {
-    return id == GEMM_DMA_256x256 || id == GEMM_DMA_256x128 || id == GEMM_DMA_128x128 || id == GEMM_DMA_128x64 || id == GEMM_DMA_64x64_SPLITK;
+    return id == GEMM_DMA_256x256 || id == GEMM_DMA_128x128 || id == GEMM_DMA_128x64 || id == GEMM_DMA_64x64_SPLITK;
 }
 
 int igemm_next_launch(const TapProblem *ps, int count, int32_t *kernel_id) {

@@ -826,7 +826,6 @@ int launch_splitk_finish(const GemmProblem &p, const int32_t *partial, int32_t p
 // `siblings` equally shaped problems share one launch (convolution groups, deconvolution phases).
 GemmConfig igemm_dma_select(int32_t m, int32_t n, int32_t k, int32_t siblings) {
     GemmConfig c;
-    const long t256 = (long)((m + 255) / 256) * ((n + 127) / 128) * siblings;
     const long t128 = (long)((m + 127) / 128) * ((n + 127) / 128) * siblings;
     const long t128x64 = (long)((m + 127) / 128) * ((n + 63) / 64) * siblings;
     const long t256x256 = (long)((m + 255) / 256) * ((n + 255) / 256) * siblings;
@@ -838,15 +837,9 @@ GemmConfig igemm_dma_select(int32_t m, int32_t n, int32_t k, int32_t siblings) {
         // 13.7 against 12.9)
         c.id = GEMM_DMA_256x256;
         c.slab = 128;
-    } else if (n > 64 && n <= 128 && k <= 128 && t256 >= 240 && t256 <= 512) {
-        // one slab: nothing to pipeline, and one round or two.  2x2 16 -> 72 at 28 x 57x57 13.86 us against 14.07 on 128 x 128 tiles, planar at 20 images 11.92
-        // against 12.22.  More rounds or longer reductions want two workgroups on a CU, one's stores under the other's products:
-        // 2x2 16 -> 128 at 64 x 57x57 20.96 here, 18.7 there; 5x5 16 -> 76 at 10 x 109x109 22.3 and 20.2; 8x8 stride 4 40 -> 55
-        // transposed at 16 x 38x38 57.2 and 53.8; 3x3 256 -> 96 at 16 x 56x56 22.3 either way.
-        c.id = GEMM_DMA_256x128;
-        c.slab = 128;
     } else if (n > 64 && t128 > 128) {
-        // (more than 128 of these are more than 512 split-reduction tiles, i.e. three of those per CU on some CUs: from there
+        // (256 x 128 tiles lost to these at every size measured: the last ones that were chosen, one slab and one or two rounds of them, took 1.04 of
+        // the time over 60 drawn layers, 1.16 at most, 2x2 32 -> 104 at 14 x 77x77 16.5 us and 14.2 here.  More than 128 of these are more than 512 split-reduction tiles, i.e. three of those per CU on some CUs: from there
         // on one round of 128 x 128 tiles is as fast or faster at every reduction length measured, 1.5x at 18 KiB; up to
         // 128 the split-reduction tiles win, 17.9 against 26.0 us at 100 tiles and a 4.5 KiB reduction)
         c.id = GEMM_DMA_128x128;
@@ -879,7 +872,6 @@ int launch_igemm_dma(const TapProblem *ps, int count, hipStream_t stream) {
     }
     switch (p.cfg.id) {
         case GEMM_DMA_256x256: return launch_cfg<256, 256, 2, 4, 1, 128, 2>(ps, count, stream);
-        case GEMM_DMA_256x128: return launch_cfg<256, 128, 4, 2, 1, 128, 2, true>(ps, count, stream);
         case GEMM_DMA_128x128:
             // Up to one tile per CU a workgroup has the CU to itself, and eight waves use it better than four (transposed convolution
             // 256 -> 128 at 8 x 32x32, 256 tiles, 10.4 -> 9.75 us; 3x3 dilation 2 128 -> 128 at 32 x 28x28, 196 tiles, 10.8 -> 9.9; plain

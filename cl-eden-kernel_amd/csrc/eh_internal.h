@@ -455,8 +455,7 @@ struct KUnit {
 // Kernel shape chosen for a problem when its weights are packed.
 enum GemmConfigId {
     GEMM_STAGED = 0,            // register-staged kernel, any channel count; weights row-major [n_pad][k_pad]
-    GEMM_DMA_256x128 = 1,       // direct-to-LDS kernels; weights in swizzled 1 KiB blocks (see packed_b_offset)
-    GEMM_DMA_128x128 = 2,
+    GEMM_DMA_128x128 = 2,       // direct-to-LDS kernels; weights in swizzled 1 KiB blocks (see packed_b_offset)
     GEMM_DMA_128x64 = 3,
     GEMM_DMA_64x64_SPLITK = 4,
     GEMM_DMA_256x256 = 5,

@@ -310,8 +310,8 @@ int eh_conv2d_u8_plan(eh_conv_plan **plan, const eh_conv_desc *desc, const void 
  * same weight order as the one-tap, the 3x3 patch and the few-row kernel, where that is the faster one. */
 typedef enum eh_kernel_id {
     EH_KERNEL_STAGED = 0,         /* register-staged implicit GEMM, any channel count               */
-    EH_KERNEL_DMA_256x128 = 1,    /* direct-to-LDS implicit GEMM tiles                              */
-    EH_KERNEL_DMA_128x128 = 2,
+    EH_KERNEL_DMA_256x128 = 1,    /* (no part is planned for it any more)                           */
+    EH_KERNEL_DMA_128x128 = 2,    /* direct-to-LDS implicit GEMM tiles                              */
     EH_KERNEL_DMA_128x64 = 3,
     EH_KERNEL_DMA_64x64_SPLITK = 4,
     EH_KERNEL_DMA_256x256 = 5,

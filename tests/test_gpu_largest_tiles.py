@@ -62,7 +62,7 @@ def test_a_pair_per_channel(deconv, n, c, h, cout, k, stride):
 @pytest.mark.parametrize("n,c,h,cout,k,dil,kernel", [
     (21, 128, 28, 121, 3, 2, "dma_128x128"),   # at most one tile per CU
     (13, 16, 71, 250, 5, 1, "dma_256x256"),
-    (20, 16, 57, 72, 2, 1, "dma_256x128"),     # one slab
+    (20, 16, 57, 72, 2, 1, "dma_128x128"),     # one slab
     (30, 16, 57, 72, 3, 2, "dma_128x128"),     # more tiles than CUs
 ])
 def test_row_sums(n, c, h, cout, k, dil, kernel):
