@@ -541,8 +541,7 @@ struct GemmOp {
 
     // Whether the plan's kernels write a planar output themselves, instead of a channels-last image that a transposition
     // then reads (a launch and two trips of the output).  Every epilogue that holds sixteen channels of a pixel per lane has
-    // the form, but for the largest tiles (240 of them, the fewest of a launch, are beyond the line for tiled kernels below; the form would
-    // make them spill) and the second launches of sliced reductions.  Transposed ->
+    // the form, but for the largest tiles, which it would make spill, and the second launches of sliced reductions.  Transposed ->
     // written, us, whole runs, over 16 .. 512 output channels, planes of 7x7 .. 224x224 and 1 .. 64 images:
     //   kernels that finish wave by wave gain at every size, some 3 us on small outputs, and at worst break even:
     //     one tap      64 -> 256 at 56x56, 4 / 64 images (3.2 / 51 MB) 11.8 -> 9.5 / 47.3 -> 40.7; 64 -> 256 at 112x112, 64 images (206 MB) 185 -> 115
@@ -550,16 +549,16 @@ struct GemmOp {
     //                  80.4 -> 80.8, 64 images (206 MB) 324 -> 284
     //     first layers 3 -> 64 at 224x224 stride 2, 64 images (51 MB) 3x3 45.9 -> 38.4, 7x7 59.3 -> 54.4
     //     few tiles    5x5, 64 -> 256 at 28x28, 1 image 10.4 -> 7.7
-    //   the tiled kernels, whose workgroups finish together, gain while the output is small (128x128 tiles: 5x5, 64 -> 256 at 14x14, 64 images,
-    //   3.2 MB 21.0 -> 19.1; 256 -> 512 at 56x56, 4 images, 6.4 MB 17.5 -> 14.2) and lose on 256x128 tiles beyond (256 -> 256 at 56x56, 16 images,
-    //   12.8 MB 30.3 -> 37.6; 5x5, 64 -> 96 at 112x112, 16 images, 19 MB 94 -> 110); at the line those tiles go both ways
-    //   (20 images at 56x56, 6.0 MB: 5x5, 64 -> 96 33.2 -> 31.6, 256 -> 96 23.6 -> 26.0)
+    //   the tiled kernels too: 150 drawn layers of 0.5 .. 24 MiB took 0.56 .. 0.98 of the time, 0.80 on average and as much above 6 MiB as below
+    //   (128 x 128 tiles 0.79, 7.4 MiB 68.0 -> 65.6, 12.5 MiB 44.0 -> 37.0; 128 x 64 tiles 0.87)
+    //   the register-staged kernel is held to the 6 MiB that it was measured up to
     bool stores_planar() const {
         bool all = layout == EH_NCHW && (int64_t)in_n * out_hw < (1ll << 31);
         const bool small = (int64_t)in_n * out_hw * cout <= (6ll << 20);
         for (auto &g : parts) {
             const bool per_wave = g.cfg.id == GEMM_THIN || g.cfg.id == GEMM_FEW_TILES || g.cfg.id == GEMM_CONV3X3 || g.cfg.id == GEMM_C3K3 || g.cfg.id == GEMM_ROWS;
-            all = all && g.slices == 0 && g.n_period == 0 && (per_wave || (small && g.cfg.id != GEMM_SKINNY && g.cfg.id != GEMM_DMA_256x256));
+            const bool tiled = g.cfg.id == GEMM_DMA_128x128 || g.cfg.id == GEMM_DMA_128x64 || g.cfg.id == GEMM_DMA_64x64_SPLITK;
+            all = all && g.slices == 0 && g.n_period == 0 && (per_wave || tiled || (small && g.cfg.id == GEMM_STAGED));
         }
         return all;
     }

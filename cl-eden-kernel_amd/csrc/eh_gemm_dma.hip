@@ -517,7 +517,7 @@ __global__ __launch_bounds__(WGM * WGN * WGK * 64) __attribute__((amdgpu_waves_p
                         if (aligned16 && n + 16 <= p.n) {
                             *reinterpret_cast<uint4 *>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
                         } else {
-                            constexpr bool planar_form = !(BM == 256 && BN == 256);  // (planar outputs of this tile are too large to gain: see stores_planar)
+                            constexpr bool planar_form = !(BM == 256 && BN == 256);  // (it would make this tile spill: see stores_planar)
                             if (planar_form && p.planar.out_plane) {
                                 if constexpr (planar_form) store_bytes_planar(p.out, p.planar, row_off[i], n, packed, p.n - n < 16 ? p.n - n : 16);
                             } else {
