@@ -442,13 +442,16 @@ bool pwdw_block_applies(const GemmProblem &pw, const DwProblem &dw) {
 //    28     32 -> 192        2      -1.1
 // (changes within +-1.5 are noise.  With the listed pairs fused the pass takes 324.6; 14 x 14 64 -> 384 alone runs in 6.6 us against 8.0
 // for the two launches, 28 x 28 32 -> 192 in 9.2 against 9.2 and at stride 2 in 6.8 against 7.8, 56 x 56 24 -> 144 in 20.9 against 21.1.)
-// A shape that is not in the table runs as two launches.  (The figures are from before the depthwise stage's walk; timed alone since, two
-// launches against one, us: 96 -> 576 at 14x14, 32 images 11.0 and 8.5, at stride 2 9.8 and 7.7, 160 -> 960 at 7x7, 32 images 10.0 and 8.4,
-// 24 -> 144 at 56x56, 32 images 18.0 and 16.9.  The answer is part of the interface and has been left as it was.)
+// A shape that is not in the table runs as two launches.  (The figures are from before the depthwise stage's walk.  Since then, alone in a
+// replayed graph, two launches against one, us: 32 images, 96 -> 576 at 14x14 8.5 and 8.4, at stride 2 7.0 and 7.3, 160 -> 960 at 7x7 7.1 and 6.8,
+// 24 -> 144 at 56x56 18.6 and 17.0, 16 -> 96 at 112x112 35.8 and 33.6, at stride 2 23.7 and 23.0; 64 images, 24 -> 144 at 56x56 29.9 and 27.1, 96 -> 576 12.4
+// and 11.6, 160 -> 960 8.7 and 8.9; 44 images, 16 -> 96 at 88x88 32.2 and 33.4.  Inside the network these pairs have not been timed again.)
 bool pwdw_block_listed(int32_t images, int32_t image_h, int32_t image_w, int32_t in_channels, int32_t expanded_channels, int32_t stride) {
     // Below 32 images a launch is mostly latency, and one launch instead of two wins for the whole network:
     // MobileNetV2 with all 16 fitting pairs fused against the listed ones, 144 against 162 us at batch 1, 168 against 176
     // at 4, 206 against 222 at 8, 246 against 260 at 16, 288 against 294 at 24; at 32 it is a draw, 324.2 against 324.6.
+    // (With the walk also alone and on large tensors: 31 images, 16 -> 96 at 112x112 34.8 and 34.3, 32 -> 192 at 56x56 21.5 and 19.8; 16 images, 24 -> 144
+    // at 112x112 29.9 and 27.0, 16 -> 96 at 112x112 22.4 and 21.3; one image, 24 -> 144 at 224x224 11.3 and 9.7.)
     if (images < 32) return true;
     if (image_h != image_w) return false;
     struct Shape {

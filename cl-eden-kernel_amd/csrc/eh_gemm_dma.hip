@@ -18,7 +18,7 @@
 // every 8 clocks, two waves together one every 2 to 5 (measured, ns per vector instruction and SIMD: one wave 3.35, two 1.1 for
 // additions and logic, 2.4 for three-operand forms, four 1.1 and 2.1).  The 256 x 256 tile therefore has eight waves of 128 x 64
 // instead of four of 128 x 128: its registers then hold the per-channel forms and the dword stores of output rows off 16-byte
-// boundaries, whose absence (a byte at a time) cost 1x1 96 -> 168 behind its expansion at 44 x 88x88 251 -> 105 us in all and the
+// boundaries, whose absence (a byte at a time) cost 1x1 96 -> 168 behind its expansion at 44 x 88x88 247 -> 99 us in all and the
 // transposed convolution 16x16 stride 8, 48 -> 40 at 4 x 45x45, 81 -> 30 us.  On whole rows the two are equal: 8192 x 4096 x 4096
 // is held by power (random bytes 121.5 us, all zero 88).  WGK > 1 splits the
 // slab along the reduction axis between waves (each wave still owns the whole

@@ -332,16 +332,20 @@ int eh_deconv2d_u8_launch_kernels(const eh_conv_desc *desc, int32_t *kernel_ids,
 int eh_conv2d_u8_set_perchannel(eh_conv_plan *plan, const int32_t *multipliers, const int32_t *shifts, int32_t count,
                                 void *stream);
 int eh_conv2d_u8_repack(eh_conv_plan *plan, const void *weight, const void *bias, const eh_requant *q, void *stream);
+/* Input and output must not share memory: workgroups store while others still read.  (A plan that holds a staging image of its
+ * input, because its tensors are planar or its channels are no multiple of its kernel's, works from that image where they
+ * do; so do the depthwise and fully connected plans of such tensors.  No other plan does.) */
 int eh_conv2d_u8_run(eh_conv_plan *plan, const void *input, void *output, const eh_requant *q, void *stream);
 /* eh_conv2d_u8_run for callers that must not allocate (code under graph capture, tight serving loops, harnesses
  * that forbid it): no counterpart in the reference.  Calls no hipMalloc / hipFree and allocates no host memory.  A
- * planar (EH_NCHW) plan computes channels-last between two layout conversions; here the two channels-last staging
- * images live in a static device array of EH_STATIC_SCRATCH_BYTES that each GPU holds from the moment the library
+ * planar (EH_NCHW) plan may have to compute channels-last, between one or two layout conversions; here the two channels-last
+ * staging images live in a static device array of EH_STATIC_SCRATCH_BYTES that each GPU holds from the moment the library
  * is loaded on it, instead of in the plan's own buffers; so does the channel-padded copy of the input that a plan
  * with a channel count off the multiples of 16 reads (see EH_EXACT_CHANNELS).  Any other EH_NHWC plan needs no staging
  * and runs as eh_conv2d_u8_run does.  Fails with EH_INVALID_PARAMS, launching nothing, when the staging
  * (planar: n*c*h*w + n*cout*ho*wo bytes; padded: n*h*w*groups*ceil16(c/groups); each rounded up to 256 plus 256)
- * exceeds the array or the plan runs as more than 8 problems (groups, slices of a long reduction).  What a plan
+ * exceeds the array, also where the plan's kernels read and write the caller's tensors as they are and touch none of it, or the
+ * plan runs as more than 8 problems (groups, slices of a long reduction).  What a plan
  * allocated when it was made (packed weights, the int32 image of a sliced reduction) stays the plan's.  Every call on a GPU shares that GPU's array: calls that overlap in time on one GPU (two streams, two
  * threads) race; calls ordered on one stream do not.  Results are bit for bit those of eh_conv2d_u8_run.  The first
  * launch of a persistent-grid kernel variant (the one-tap and the few-channel first-layer kernels) at a given LDS size
@@ -388,8 +392,7 @@ int eh_dwconv2d_u8_destroy(eh_dwconv_plan *plan);
  * `_preferred` says whether the one launch is also the faster choice for the pair's shape (1) or the two launches
  * are (0): below 32 images per launch every fitting pair (a launch is mostly latency there, and a whole network
  * measured faster with all of them fused at every batch from 1 to 24); from 32 images on a table of shapes timed
- * inside a network, kept beside the kernel: a caller that fuses wherever `_preferred` says so never loses to the
- * two launches on a measured shape, and unmeasured shapes stay unfused.
+ * inside a network, kept beside the kernel, and unmeasured shapes stay unfused (there are faster ones in one launch among them).
  * rows_per_tile, cols_per_tile: the tile of output pixels a workgroup owns, 0 lets the library choose.
  * q_pointwise->zp_out must equal q_depthwise->zp_in (they describe the same tensor). */
 int eh_conv_dw_block_applies(const eh_conv_plan *pointwise, const eh_dwconv_plan *depthwise);
