@@ -22,7 +22,8 @@
 //      58x58, 16 images 32.7 -> 23; 16 -> 96 at 83x83, 21 images 21.4 -> 13.6; 56 -> 336 at 31x31, 18 images 13.4 -> 9.3; 120 -> 720
 //      at 12x12, 18 images 9.2 -> 7.0; a pair per channel, 16 -> 96 at 104x97, 28 images 34.1 -> 26.6, 80 -> 480 at 36x36, 16 images
 //      20.4 -> 15.0; at stride 2, where the expansion is most of the work, 24 -> 144 at 56x56, 32 images 11.3 and 11.3.
-//      Small tiles that a caller asks for are taken sixteen outputs at a time instead, wherever their rows end (pwdw_block_geometry has the rule).
+//      Small tiles at stride 2, and those that a caller asks for, are taken sixteen outputs at a time instead, wherever their rows end
+//      (units_tile and pwdw_block_geometry have the rules).
 // The rows and columns two neighbouring workgroups both need (the halo) are computed twice; nothing else is.  Tiles are
 // cut in both directions because the halo of a stride-2 window costs (2 TH + 1)(2 TW + 1) / (4 TH TW): 1.53 for one full
 // row of 28 outputs, 1.21 for 4 x 7.
@@ -47,7 +48,7 @@ namespace {
 // stage when they are 1, 2 or 3 (a lane then keeps its pixel's operand bytes in registers across the channel blocks),
 // 0 for any number (read from LDS for every product).
 enum class DwForm {
-    UNITS,  // small tiles on request: sixteen outputs of the tile, wherever its rows end, by sixteen channels
+    UNITS,  // small tiles at stride 2 or on request: sixteen outputs of the tile, wherever its rows end, by sixteen channels
     WALK    // the others: sixteen columns, down the tile's rows
 };
 // PC: one multiplier and shift per channel in both operators; the depthwise ones in the single-shift form, or in two steps.
@@ -476,7 +477,7 @@ namespace {
 // counted as the hardware deals them out: an eighth of the tiles, rounded up, to an XCD of 32 CUs, and LDS in pieces of 1280 bytes.  Without
 // the one, 152 -> 912 at 17x17, 11 images, a pair per channel, had 65 workgroups to an XCD where 64 fit, 15.3 us (9.55 now); without the other 24 ->
 // 144 at 77x77 stride 2, 22 images, had two of 54336 bytes to a CU where three were counted on, 17.8 us (13.8).  364 drawn pairs: 1.8 % faster.
-bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, int cols_per_tile, int *th, int *tw, int *nb, int *walk_log) {
+bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, int cols_per_tile, int *th, int *tw, int *nb, int *walk_log, double *time_taken) {
     const int S = dw.stride_h, ks = pw.k_pad / 32, nb_all = (dw.c + 31) / 32, chunks_all = dw.c / 16;
     const double epilogue = pw.rq.pc_multiplier ? 1.42 : 1.0;
     const int held = pw.rq.pc_multiplier ? 4 : 5;
@@ -538,9 +539,58 @@ bool walk_tile(const GemmProblem &pw, const DwProblem &dw, int rows_per_tile, in
                 }
             }
         }
+        *time_taken = best;
         if (best >= 0) return true;
     }
     return false;
+}
+
+// The tile of a stride-2 launch whose depthwise stage takes sixteen outputs at a time, where that is the faster one than the tile that walks, of
+// which `walk` is the time: at stride 2 a walk meets a wave's columns in rows twice as long and keeps few of its lanes busy on a small tile.  One
+// group of outputs to a tile, up to eight chunks of sixteen channels, a workgroup or more to every CU and no second round of them (smaller launches
+// are latency either way).  Priced as walk_tile prices, but by the mean of the channel ranges, of which the last may be short; the coefficients
+// are fitted to 700 drawn stride-2 layers with every such tile timed, and so are the prices up to which units are taken: with one reduction step 1.06
+// of the walk's, with more 0.94, where units' time is 0.98 of the walk's from there to 1.00 and 1.07 at most; launches of more than 1.28 million outputs
+// took 1.02 .. 1.11.  836 other drawn stride-2 layers: 308 take units, 0.96 of the walk's time on average, 0.87 .. 1.07, four of them above 1.04.
+// us, walk and units:
+// 24 -> 144 at 56x56, seven images 5.47 and 4.89, a pair per channel at 48x48, nine images 6.08 and 5.37; 16 -> 96 at 64x64, six images
+// 5.07 and 4.53.  At stride 1 the walk takes 0.88 of the units' time, 0.95 with a pair per channel.
+bool units_tile(const GemmProblem &pw, const DwProblem &dw, double walk, int *th, int *tw, int *nb) {
+    const int ks = pw.k_pad / 32, nb_all = (dw.c + 31) / 32, chunks_all = dw.c / 16;
+    const double epilogue = pw.rq.pc_multiplier ? 1.42 : 1.0;
+    if ((int64_t)dw.n * dw.ho * dw.wo * dw.c > 5000 * 256) return false;
+    bool found = false;
+    walk *= ks == 1 ? 1.06 : 0.94;  // (the prices of the two forms meet there: timed, see above)
+    for (int cn = 1; cn <= 4 && cn <= nb_all; ++cn) {
+        const int ranges = (nb_all + cn - 1) / cn;
+        if ((ranges - 1) * cn >= nb_all) continue;  // the same ranges with fewer blocks each
+        const int last_blocks = nb_all - (ranges - 1) * cn, last_chunks = chunks_all - (ranges - 1) * cn * 2;
+        for (int rows = 1; rows <= 8 && rows <= dw.ho; ++rows)
+            for (int cols = (8 + rows - 1) / rows < 3 ? 3 : (8 + rows - 1) / rows; cols * rows <= 16 && cols <= dw.wo; ++cols) {
+                const int ih = (rows - 1) * 2 + 3, iw = (cols - 1) * 2 + 3, pixels = ih * iw;
+                const size_t lds = block_lds_bytes(cn, ks, ih, iw, dw.c, nullptr, nullptr);
+                if (lds > (size_t)64 * 1024) continue;
+                const long tiles = (long)dw.n * ((dw.ho + rows - 1) / rows) * ((dw.wo + cols - 1) / cols);
+                const double per_cu = (double)((tiles + 7) / 8 * ranges) / 32.0;
+                const int fit = (int)((160 * 1024) / ((lds + 1279) / 1280 * 1280)), most = fit < 5 ? fit : 5;
+                if (per_cu < 1 || per_cu > 5) continue;
+                auto range = [&](int blocks, int chunks) {
+                    return 10 + 40.0 * blocks + 40.0 * ((pixels * ks * 4 + 255) >> 8) + ((((pixels + 31) >> 5) * blocks + 3) >> 2) * (67.0 * epilogue + 5.5 * ks) +
+                           ((chunks + 3) >> 2) * (40.0 + 12.0 * epilogue);
+                };
+                const double wave = ((ranges - 1) * range(cn, cn * 2) + range(last_blocks, last_chunks)) / ranges;
+                auto time = [&](int waves) { return wave * (2.3 + 1.07 * waves) + 800; };
+                const int full = (int)(per_cu / most), rest = (int)(per_cu - full * most + 0.999);
+                const double cost = full * time(most) + (rest > 0 ? time(rest) : 0);
+                if (cost >= walk) continue;
+                walk = cost;
+                *th = rows;
+                *tw = cols;
+                *nb = cn;
+                found = true;
+            }
+    }
+    return found;
 }
 
 }  // namespace
@@ -564,12 +614,12 @@ bool pwdw_block_geometry(const GemmProblem &pw, const DwProblem &dw, int rows_pe
         if (nb == 0) return false;
         // The line, on 900 requested tiles of drawn layers of up to 1.5 GFLOP, walk over units by the units of a workgroup (with a pair per channel): 2
         // 0.98 (1.02), 4 1.03 (1.03), 6 1.17 and half full ones 1.21 (0.97 and 1.07), 8 full 0.96 (0.96), 12 full 0.92 (0.99), beyond 0.77 (0.73).
-        // Tiles of this library's own choice walk: 144 drawn layers whose tiles had been of few units took 0.73 .. 1.06 of the time, 0.91 on
-        // average and 0.95 with a pair per channel, with the tile of walk_tile.
         const int groups = (th * tw + 15) / 16, chunks = nb * 2 < dw.c / 16 ? nb * 2 : dw.c / 16, units = groups * chunks;
         g.matrix = units <= (pw.rq.pc_multiplier == nullptr ? 8 : S == 2 ? 6 : 3) && (units <= 4 || th * tw > groups * 8) ? 1 : 0;
     }
-    if (!g.matrix && !walk_tile(pw, dw, rows_per_tile, cols_per_tile, &th, &tw, &nb, &g.walk_log)) return false;
+    double time_taken = 0;
+    if (!g.matrix && !walk_tile(pw, dw, rows_per_tile, cols_per_tile, &th, &tw, &nb, &g.walk_log, &time_taken)) return false;
+    if (rows_per_tile <= 0 && cols_per_tile <= 0 && S == 2 && units_tile(pw, dw, time_taken, &th, &tw, &nb)) g.matrix = 1, g.walk_log = 0;
     g.nb = nb;
     g.th = th;
     g.tw = tw;

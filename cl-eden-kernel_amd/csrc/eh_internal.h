@@ -723,7 +723,7 @@ struct BlockGeom {
     int32_t nb;          // channel blocks of 32 per workgroup (grid y walks the ranges); bytes per pixel of the LDS image = 32 nb
     int32_t ks;          // reduction steps of 32 bytes of the pointwise stage
     int32_t cpitch;      // bytes per pixel of the LDS image
-    int32_t matrix;      // the depthwise stage takes sixteen outputs at a time (small tiles on request; see pwdw_block_geometry)
+    int32_t matrix;      // the depthwise stage takes sixteen outputs at a time (small tiles; see units_tile and pwdw_block_geometry)
     int32_t walk_log, walk_groups;  // otherwise: log2 of the columns a wave walks down, and such groups per tile
     int32_t total_tiles; // n * tiles_y * tiles_w
     int32_t a_pitch;     // LDS bytes per input pixel: 32 ks + 16 (the slack spreads the fragment reads over the banks)

@@ -403,8 +403,8 @@ int eh_conv_dw_block_preferred(const eh_conv_plan *pointwise, const eh_dwconv_pl
  * shape: whether the pair fits is `_applies`' business). */
 int eh_conv_dw_block_listed(int32_t images, int32_t image_h, int32_t image_w, int32_t in_channels, int32_t expanded_channels, int32_t stride);
 /* The tile that a fused launch of the two plans takes: output rows and columns and blocks of 32 channels per workgroup,
- * and whether its depthwise stage takes the tile's outputs sixteen at a time, as small tiles that are asked for do
- * (1), or walks down its columns (0). */
+ * and whether its depthwise stage takes the tile's outputs sixteen at a time, as small tiles at stride 2 or that are
+ * asked for do (1), or walks down its columns (0). */
 int eh_conv_dw_block_tile(eh_conv_plan *pointwise, eh_dwconv_plan *depthwise, int32_t rows_per_tile, int32_t cols_per_tile, int32_t *rows, int32_t *cols,
                           int32_t *channel_blocks, int32_t *matrix);
 int eh_conv_dw_block_run(eh_conv_plan *pointwise, eh_dwconv_plan *depthwise, const void *input, void *output,

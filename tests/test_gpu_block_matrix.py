@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 SEED = 0xB10D
 
 CASES = [
-    # n, h, w, cin, c, stride, rows, cols, depthwise zp_w, on the matrix cores with one pair per tensor / per channel
+    # n, h, w, cin, c, stride, rows, cols (0: the library's), depthwise zp_w, on the matrix cores with one pair per tensor / per channel
     (1, 3, 3, 8, 16, 1, 1, 1, 128, True, True),       # one output per workgroup, one chunk: three waves without work
     (2, 9, 7, 16, 48, 1, 3, 5, 0, True, True),        # fifteen pixels; differences up to 255
     (1, 9, 7, 24, 48, 2, 4, 4, 255, True, True),      # sixteen pixels; differences down to -255
@@ -29,6 +29,10 @@ CASES = [
     (2, 8, 8, 24, 64, 2, 2, 4, 127, True, True),      # ... at stride 2
     (2, 8, 8, 24, 64, 1, 3, 3, 127, True, False),     # of nine
     (1, 5, 6, 16, 16, 1, 5, 6, 90, True, True),       # the whole image in one workgroup
+    (4, 28, 28, 32, 128, 2, 0, 0, 100, True, True),   # the library's own tile at stride 2: fifteen pixels, one channel block
+    (6, 31, 29, 24, 144, 2, 0, 0, 0, True, True),     # ... ten, ranges of four chunks and one of one
+    (3, 39, 41, 40, 240, 2, 0, 0, 255, True, True),   # ... twelve, two reduction steps, ranges of four chunks and one of three
+    (2, 21, 23, 160, 960, 2, 0, 0, 127, True, True),  # ... nine, five steps
 ]
 
 

@@ -82,20 +82,20 @@ plan = eden.DwConvPlan(d, buf(d.cout, 1, d.kh, d.kw), buf(d.cout, dtype=np.int32
     assert sum("dw_pack_mfma_kernel" in l[0] for l in launches(stub, tmp_path, program)) == packs
 
 
-@pytest.mark.parametrize("shape,tile,tensor,channel", [
-    # n, cin, expanded, extent, stride; rows and columns asked for
-    ((1, 32, 64, 28, 2), (2, 4), 1, 1),      # four units of sixteen outputs by sixteen channels, half full
-    ((1, 32, 96, 28, 2), (2, 4), 0, 0),      # six, half full
-    ((4, 24, 144, 56, 2), (2, 8), 0, 0),     # nine at stride 2
-    ((4, 16, 96, 14, 1), (4, 4), 1, 0),      # six, full
-    ((4, 32, 128, 28, 2), (4, 4), 1, 0),     # eight, full
-    ((4, 16, 64, 28, 1), (3, 5), 1, 0),      # four
-    ((4, 16, 48, 28, 1), (3, 5), 1, 1),      # three
-    ((4, 96, 576, 14, 1), (7, 14), 0, 0),    # many
+@pytest.mark.parametrize("shape,tile,tensor,channel,own", [
+    # n, cin, expanded, extent, stride; rows and columns asked for; whether the library's own tile takes units
+    ((1, 32, 64, 28, 2), (2, 4), 1, 1, 0),      # four units of sixteen outputs by sixteen channels, half full
+    ((1, 32, 96, 28, 2), (2, 4), 0, 0, 0),      # six, half full
+    ((4, 24, 144, 56, 2), (2, 8), 0, 0, 1),     # nine at stride 2
+    ((4, 16, 96, 14, 1), (4, 4), 1, 0, 0),      # six, full
+    ((4, 32, 128, 28, 2), (4, 4), 1, 0, 1),     # eight, full
+    ((4, 16, 64, 28, 1), (3, 5), 1, 0, 0),      # four
+    ((4, 16, 48, 28, 1), (3, 5), 1, 1, 0),      # three
+    ((4, 96, 576, 14, 1), (7, 14), 0, 0, 0),    # many
 ])
-def test_form_of_the_fused_launchs_depthwise_stage(stub, tmp_path, shape, tile, tensor, channel):
+def test_form_of_the_fused_launchs_depthwise_stage(stub, tmp_path, shape, tile, tensor, channel, own):
     """Units of sixteen outputs for small tiles that are asked for, with one pair per tensor and with one per channel, where they are the faster
-    form; tiles of the library's own choice walk; the plan notices that its pairs and the requested tile have changed."""
+    form; tiles of the library's own choice walk, but for some at stride 2; the plan notices that its pairs and the requested tile have changed."""
     program = """
 n, cin, c, h, stride = %r
 pw = eden.ConvPlan(eden.conv_desc(n, cin, h, h, c, 1, 1, layout=eden.NHWC), buf(c, cin, 1, 1), buf(c, dtype=np.int32), q)
@@ -105,8 +105,8 @@ for pairs in (False, True, False):
     for plan in (pw, dw):
         plan.set_perchannel(*((np.full(c, q.multiplier), np.full(c, q.shift)) if pairs else (None, None)))
     forms += [eden.conv_dw_block_tile(pw, dw, *%r)[3], eden.conv_dw_block_tile(pw, dw)[3]]
-assert forms == [%d, 0, %d, 0, %d, 0], forms
-""" % (shape, tile, tensor, channel, tensor)
+assert forms == [%d, %d, %d, %d, %d, %d], forms
+""" % (shape, tile, tensor, own, channel, own, tensor, own)
     launches(stub, tmp_path, program)
 
 
